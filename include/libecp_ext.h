@@ -167,9 +167,8 @@ int libecp_batch_quadrature_ms(libecp_batch *b, double *ms, int *samples);
    "t2_head" (PS93 levels of the type-2 small-grid kernel before the entries
    still open are rerun compacted; 15, the default: no split; 0: 6 with
    fused launches, no split otherwise), "t2_tail_grid",
-   "fb2_split" (waves sharing one (triplet, primitive pair) of the type-2
-   large-grid fallback; 0, the default: 3 for jobs of up to a million
-   (triplet, pair) items, 1 for larger ones).  "t1_spec" (fused launches: 1, the default, starts
+   "fb2_split" (shares a triplet's type-2 fallback entries are split into,
+   each with its own waves; 0, the default: by the job's size).  "t1_spec" (fused launches: 1, the default, starts
    the type-1 large-grid fallback beside the small-grid tail on every entry
    the head left open; 0 after the tail on the failed entries).  "t2_spec"
    (fused launches with a type-2 head: 1 starts the type-2 large-grid

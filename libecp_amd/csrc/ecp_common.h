@@ -90,7 +90,8 @@ typedef struct {
 typedef struct {
   int atom;      /* global atom index of the ECP centre */
   int L;         /* local channel label; semi-local channels 0..L-1 */
-  int g0, ng;    /* Gaussians [g0, g0+ng) */
+  int g0, ng;    /* Gaussians [g0, g0+ng), ordered by channel l (input order inside a channel) */
+  int gl[ECP_MAX_L + 2];   /* channel l's Gaussians: [g0 + gl[l], g0 + gl[l + 1]) */
   int mol;
   int end[ECP_MAX_L + 1];  /* progressive potential cut-off per semi-local channel */
   int UL_off;    /* offset (doubles) of the U_L table in ULtab */

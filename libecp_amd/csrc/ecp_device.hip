@@ -143,24 +143,55 @@ __device__ __forceinline__ double ecp_pow(double r, double n) {
   return ecp_pow_general(r, n);
 }
 
-__device__ double eval_ecp(const ecp_gauss *__restrict__ g, int ng, int l, double r) {
+// U_l(r): the channel's own Gaussians only (C.gl; the host orders a centre's
+// Gaussians by channel), where a scan over all of them would read and test
+// every one for each channel
+__device__ __forceinline__ double eval_ecp(const DevJob &J, int centre, int l, double r) {
   double pot = 0.0;
   const double r2 = r * r;
-  for (int i = 0; i < ng; i++) {
-    if (g[i].l == l) pot += ecp_pow(r, g[i].n) * g[i].d * exp(-g[i].a * r2);
-  }
+  const ecp_centre *__restrict__ C = J.cent + centre;
+  const ecp_gauss *__restrict__ g = J.gauss + C->g0;
+  const int end = C->gl[l + 1];
+  for (int i = C->gl[l]; i < end; i++) pot += ecp_pow(r, g[i].n) * g[i].d * exp(-g[i].a * r2);
   return pot;
 }
 
-template <int J>
-struct RecC {
-  static constexpr double v = double(J) / (2.0 * J + 1.0);
-};
+// x / D, correctly rounded, in three operations: q = RN(x RN(1 / D)) is
+// within one unit in the last place of the quotient, its remainder x - q D
+// is exact in a fused multiply-add, and RN(q + r RN(1 / D)) is then the
+// rounded quotient (Markstein, IBM J. Res. Dev. 34 (1990) 111).  The
+// compiler's general FP64 division takes about a dozen instructions, one of
+// them at a quarter of the rate.  Finite x away from the underflow range.
+template <int D>
+__device__ __forceinline__ double div_const(double x) {
+  if constexpr ((D & (D - 1)) == 0) {
+    return x * (1.0 / D);  // exact
+  } else {
+    constexpr double y = 1.0 / D;
+    const double q = x * y;
+    return __builtin_fma(__builtin_fma(-double(D), q, x), y, q);
+  }
+}
 
 // K_0..K_LM at z (bessel.c:102-199): leading term below 1e-7, 5-term Taylor
 // series about the nearest table abscissa below 16 (derivatives by the
 // recurrence K_j' = j/(2j+1)(K_{j-1} - K_{j+1}) - K_j + K_{j+1}), asymptotic
 // series above.
+template <int LM, int L>
+__device__ __forceinline__ void bessel_asymptotic(double (&A)[LM + 1], double (&K)[LM + 1]) {
+  if constexpr (L <= LM) {
+    double f = L * (L + 1);
+#pragma unroll
+    for (int i = 1; i < L; i++) {
+      K[L] += f * A[i];
+      f *= (L + i + 1) * (L - i);
+    }
+    A[L] = div_const<L>(-A[0] * A[L - 1]);
+    K[L] += f * A[L];
+    bessel_asymptotic<LM, L + 1>(A, K);
+  }
+}
+
 template <int LM>
 __device__ __forceinline__ void bessel_k(const double *__restrict__ tab, double z, double (&K)[LM + 1]) {
   if (z < 1.0E-7) {
@@ -176,7 +207,7 @@ __device__ __forceinline__ void bessel_k(const double *__restrict__ tab, double 
   } else if (z < 16.0) {
     constexpr int ML = LM + 5;
     const int index = (int)floor(z * 100.0 + 0.5);
-    const double dz = z - index / 100.0;
+    const double dz = z - div_const<100>((double)index);
     const double *row = tab + (size_t)index * ECP_BESSEL_STRIDE;
     double d[ML + 2];
 #pragma unroll
@@ -184,10 +215,13 @@ __device__ __forceinline__ void bessel_k(const double *__restrict__ tab, double 
     d[ML + 1] = 0.0;
 #pragma unroll
     for (int l = 0; l <= LM; l++) K[l] = d[l];
-    double scale = 1.0;
+    // dz^i / i!, each factor divided in turn
+    const double sc1 = dz, sc2 = div_const<2>(sc1 * dz), sc3 = div_const<3>(sc2 * dz), sc4 = div_const<4>(sc3 * dz),
+                 sc5 = div_const<5>(sc4 * dz);
 #pragma unroll
     for (int i = 1; i <= 5; i++) {
       const int top = ML - i;
+      const double scale = i == 1 ? sc1 : i == 2 ? sc2 : i == 3 ? sc3 : i == 4 ? sc4 : sc5;
       double prev = d[0];
       d[0] = d[1] - d[0];
 #pragma unroll
@@ -197,7 +231,6 @@ __device__ __forceinline__ void bessel_k(const double *__restrict__ tab, double 
         d[j] = cj * (prev - d[j + 1]) - cur + d[j + 1];
         prev = cur;
       }
-      scale = scale * dz / i;
 #pragma unroll
       for (int j = 0; j <= LM; j++) K[j] += scale * d[j];
     }
@@ -206,17 +239,7 @@ __device__ __forceinline__ void bessel_k(const double *__restrict__ tab, double 
     A[0] = 0.5 / z;
 #pragma unroll
     for (int l = 0; l <= LM; l++) K[l] = A[0];
-#pragma unroll
-    for (int l = 1; l <= LM; l++) {
-      double f = l * (l + 1);
-#pragma unroll
-      for (int i = 1; i < l; i++) {
-        K[l] += f * A[i];
-        f *= (l + i + 1) * (l - i);
-      }
-      A[l] = -A[0] * A[l - 1] / l;
-      K[l] += f * A[l];
-    }
+    bessel_asymptotic<LM, 1>(A, K);
   }
 }
 
@@ -374,14 +397,13 @@ __device__ void utab_rows(const DevTables &T, const DevJob &J, int c, int row, i
   if (row > C.L) return;
   const int n = chunk * 128 + (int)threadIdx.x;
   if (n >= SO) return;
-  const ecp_gauss *g = J.gauss + C.g0;
   const double r = T.xs[n];
   if (row == C.L) {
-    J.UL[C.UL_off + n] = eval_ecp(g, C.ng, C.L, r);
+    J.UL[C.UL_off + n] = eval_ecp(J, c, C.L, r);
     return;
   }
   const int l = row;
-  double P = (n <= C.end[l]) ? eval_ecp(g, C.ng, l, r) : 0.0;
+  double P = (n <= C.end[l]) ? eval_ecp(J, c, l, r) : 0.0;
   const size_t rs = J.ptmajor ? 1 : SO;  // stride between the powers k
   double *dst = J.Ut + C.Ut_off + (size_t)l * J.UK * SO + (J.ptmajor ? (size_t)n * J.UK : (size_t)n);
   dst[0] = P;
@@ -886,92 +908,96 @@ __device__ __forceinline__ Fm06 fm06(double zeta_p, double P) {
   return m;
 }
 
-// First large-grid index n with r_n > max(dAC, dBC) and the exponent below
-// the numerical zero: the screening break of type1.c:222-225 /
-// type2.c:479-481; `order` if there is none.  expo(r) is evaluated by the
-// caller's functor with the same arithmetic as the integrand.
-// The predicate "r_n > max(dAC, dBC) and expo(r_n) < minExp" is monotone in
-// n (r_n increases with n, and beyond both centres the exponent decreases;
-// every rounding step is monotone), so its first true index is found with
-// two wave-wide probes instead of a scan: 64 samples at stride
-// ceil(order / 64) bracket it, then the 64 points ending at the first true
-// sample locate it.
+// Point of slot `lane` in a round of PSM92 point pairs [c0, c1): pair c0 +
+// lane / 2, left in even lanes, right in odd ones; in the first round (the
+// pairs of levels 1 to 5, 31 of them) the centre is in lane 62.  -1: none.
+__device__ __forceinline__ int psm92_point(const DevTables &T, int c0, int c1, int lane, bool first) {
+  const int k = c0 + (lane >> 1);
+  if (first && lane == 62) return T.s92.centre;
+  if (k >= c1) return -1;
+  return (lane & 1) ? T.p92r[k] : T.p92l[k];
+}
+
+// PSM92 levels [0, psm92_first) in the first round: centre and 31 pairs
+__device__ __forceinline__ int psm92_first(const DevTables &T) { return min(6, T.s92.nlevels); }
+
+// v(left) + v(right) of the wave's point pairs, in both lanes of each pair
+__device__ __forceinline__ double pair_sum(double v) {
+  // quad_perm [1, 0, 3, 2]: the neighbour's value
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0xB1, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0xB1, 0xF, 0xF, true);
+  return v + __hiloint2double(hi, lo);
+}
+
+// The exponents of the three points of PSM92 levels 0 and 1 are all below
+// the numerical zero: every integral of the pair is then 0 at level 0 and
+// converges with the result 0 at level 1 (0 <= 0 in its test).
 template <typename Expo>
-__device__ int fm06_break(const DevTables &T, const Fm06 &M, double dAC, double dBC, double minExp, Expo expo) {
-  const int order = T.lorder;
-  auto pred = [&](int n) {
-    const double r = M.i1 * T.xl[n] + M.i2;
-    return r > dAC && r > dBC && expo(r) < minExp;
-  };
-  const int stride = (order + 63) / 64;
-  const int ns = min(order - 1, ((int)threadIdx.x + 1) * stride - 1);
-  const unsigned long long b1 = __ballot(pred(ns));
-  if (!b1) return order;
-  const int k0 = __ffsll((long long)b1) - 1;
-  const int hi = min(order - 1, (k0 + 1) * stride - 1);
-  const int n = hi - 63 + (int)threadIdx.x;
-  const unsigned long long b2 = __ballot(n >= 0 && pred(n));
-  return hi - 63 + (__ffsll((long long)b2) - 1);
+__device__ __forceinline__ bool psm92_dead(const DevTables &T, const Fm06 &M, double minExp, Expo expo) {
+  if (T.s92.nlevels < 2) return false;
+  const double e0 = expo(M.i1 * T.xl[T.s92.centre] + M.i2), e1 = expo(M.i1 * T.xl[T.p92l[0]] + M.i2),
+               e2 = expo(M.i1 * T.xl[T.p92r[0]] + M.i2);
+  return !(e0 >= minExp) && !(e1 >= minExp) && !(e2 >= minExp);
 }
 
-// PSM92 evaluation rounds: the points of consecutive levels are evaluated by
-// the wave together when they fit (levels 0-1: 3 points, 2-5: 60, 6: 64);
-// larger levels go in chunks of 32 point pairs.  Within a round the centre
-// (level 0) takes slot 0 and pair k of level lv the slots roff + 2k (left)
-// and roff + 2k + 1 (right), roff being the points of the round's earlier
-// levels.  Summation order inside each level is unchanged.
-__device__ __forceinline__ int psm92_points(int lv) { return lv == 0 ? 1 : (1 << lv); }
-
-// hw: the slots of a round (lanes per integration, 16, 32 or 64); levels
-// 2 .. l2 - 1 take 2^l2 - 4 <= hw of them
-__device__ __forceinline__ int psm92_round_end(int lv, int nlev, int hw = 64) {
-  const int l2 = hw >= 64 ? 6 : hw >= 32 ? 5 : 4;
-  return min(nlev, lv == 0 ? 2 : (lv == 2 ? l2 : lv + 1));
-}
-
-// grid index evaluated by `slot` in the round [l0, l1); -1 for none (a slot
-// past the round, or a right point past the screening end)
-__device__ __forceinline__ int psm92_round_point(const DevTables &T, int l0, int l1, int slot, int end) {
-  int o = 0;
-  for (int lv = l0; lv < l1; lv++) {
-    const int np = psm92_points(lv);
-    if (slot < o + np) {
-      if (lv == 0) return T.s92.centre;
-      const int pair = T.s92.lvl_begin[lv] + ((slot - o) >> 1);
-      if (((slot - o) & 1) == 0) return T.p92l[pair];
-      const int ri = T.p92r[pair];
-      return ri <= end ? ri : -1;
-    }
-    o += np;
+// An integral's PSM92 state (gc_integrators.c:38-86)
+struct Psm92 {
+  double I, p, q;
+  __device__ __forceinline__ void step() {
+    q = 2 * p;
+    p = 2 * I;
   }
-  return -1;
-}
+  // after a level: converged? (*res: the integral)
+  __device__ __forceinline__ bool test(const DevTables &T, int l, double *res) const {
+    const double N = T.s92.lvl_n[l];
+    const double ee = I - p;
+    if (!(16 * ee * ee <= 3 * N * fabs(I - q) * T.tol)) return false;
+    *res = 16 * I / (3 * N);
+    return true;
+  }
+  // the first round: pair sums v[0 .. 30] of levels 1 to 5, the centre v[31]
+  __device__ __forceinline__ bool first_round(const DevTables &T, const double *v, double *res) {
+    I = p = v[31];
+    q = 0.0;
+    const int l1 = psm92_first(T);
+    for (int l = 1; l < l1; l++) {
+      step();
+      I = sum_in_order(I, v + T.s92.lvl_begin[l], T.s92.lvl_begin[l + 1] - T.s92.lvl_begin[l]);
+      if (test(T, l, res)) return true;
+    }
+    return false;
+  }
+};
 
 // type-1 fallback (type1.c:205-252): one wave per primitive pair with failed
-// Q entries.  Per level the wave evaluates the level's points of the
-// FM06-mapped PSM92 grid (Bessel functions, U_L, exponential) into LDS, then
-// each lane owning a failed entry sums them in the integrator's pair order
-// (gc_integrators.c:55-84) and applies the PSM92 test; the wave stops when
-// every entry has converged.  Points past the screening break contribute 0.
-constexpr int kKS = 65;     // LDS stride of per-point Bessel rows (bank spread)
-constexpr int kFb1TS = 33;  // LDS stride of a failed entry's pair sums (at most 32 pairs per call)
+// Q entries.  The wave's lanes evaluate the points of a round -- 31 point
+// pairs and the centre (levels 0 to 5) together, then 32 pairs at a time --
+// and form each open entry's pair sums (0 + f(left)) + f(right), a pair per
+// two lanes, into LDS; lane e adds those of entry e in the integrator's
+// order and applies the PSM92 test after each level.  Pairs whose points
+// of levels 0 and 1 are all numerically zero end there.
+// The reference's screening break (type1.c:222-225: no points from the first
+// one beyond both centres whose exponent is below the cut-off) needs no
+// search: beyond both centres the exponent only decreases, so every point it
+// drops is below the cut-off and contributes 0 here by its own test.
+constexpr int kFbTS = 33;  // LDS stride of an entry's pair sums (at most 32 per round)
 
 template <int LAB, bool SPEC = false>
 __device__ __forceinline__ void fb1_body(int bid, int nb, const DevTables &T, const DevJob &J,
                                          const T1Unit *__restrict__ units, double *__restrict__ qout,
                                          const unsigned long long *__restrict__ qfail, const int *__restrict__ fbq,
                                          const int *__restrict__ fbcount, unsigned char *__restrict__ status,
-                                         double *s_r, double *s_w, double *s_u, double *s_g, double *s_k,
-                                         double *s_t, int *s_e, const int *__restrict__ tq = nullptr,
+                                         double *s_t, const int *__restrict__ tq = nullptr,
                                          const int *__restrict__ tcount = nullptr,
                                          const unsigned long long *__restrict__ qopen = nullptr,
                                          double *__restrict__ qfb = nullptr,
                                          unsigned long long *__restrict__ qfbf = nullptr) {
-  // qfb != nullptr (speculative): besides the units whose small-grid
+  // SPEC (speculative): besides the units whose small-grid
   // integrals failed (fbq), every unit the tail takes (tq), for the entries
   // open after the head (qopen), started before the tail has decided them;
   // results to qfb, large-grid failures as an entry mask to qfbf, and the
   // assembly uses a result where the small grid failed
+  constexpr int NQ = nq_of(LAB);
   const int n1 = *fbcount;
   int count = n1;
   if constexpr (SPEC) count += *tcount;
@@ -996,145 +1022,78 @@ __device__ __forceinline__ void fb1_body(int bid, int nb, const DevTables &T, co
     const Fm06 M = fm06(zeta_p, (G.za * G.dAC + G.zb * G.dBC) / zeta_p);
     const double minExp = T.lnAcc1;
     auto expo_of = [&](double r) { return (G.z * r + G.s) * r + G.zd2; };
-    const int brk = fm06_break(T, M, G.dAC, G.dBC, minExp, expo_of);
-    const int end = brk - 1;
-    // this lane's failed entry (the lane-th set bit of mask)
-    int my_e = -1, my_l1 = 0, my_l2 = 0;
-    const int nfail = __popcll(mask);
-    {
-      int e = 0, seen = 0;
-      for (int l1 = 0; l1 <= LAB; l1++)
-        for (int l2 = l1; l2 >= 0; l2 -= 2, e++)
-          if ((mask >> e) & 1ull) {
-            if (seen == lane) {
-              my_e = e;
-              my_l1 = l1;
-              my_l2 = l2;
-            }
-            seen++;
-          }
+    double *out = (SPEC ? qfb : qout) + U.qoff;
+    bool open = lane < NQ && ((mask >> lane) & 1ull);
+    if (psm92_dead(T, M, minExp, expo_of)) {
+      if (open) out[lane] = 0.0;
+      if (SPEC && lane == 0) qfbf[u] = 0ull;
+      continue;
     }
-    const ecp_gauss *gs = J.gauss + Cn.g0;
-    auto eval = [&](int slot, int n) {
-      double r = 0.0, w = 0.0, uu = 0.0, g = 0.0;
+    Psm92 S{0.0, 0.0, 0.0};
+    double res = 0.0;
+    // rounds of point pairs [c0, c1): levels 0 to 5 first, then 32 pairs of
+    // level lv at a time
+    int lv = psm92_first(T), c0 = 0, c1 = T.s92.lvl_begin[lv];
+    for (;;) {
+      const bool first = c0 == 0;
+      const unsigned long long om = __ballot(open);
+      const int n = psm92_point(T, c0, c1, lane, first);
+      double w = 0.0, uu = 0.0, g = 0.0, r = 0.0;
       double K[LAB + 1];
 #pragma unroll
       for (int l = 0; l <= LAB; l++) K[l] = 0.0;
-      if (n >= 0 && n < brk) {
+      if (n >= 0) {
         r = M.i1 * T.xl[n] + M.i2;
         const double expo = expo_of(r);
         if (expo >= minExp) {
           g = exp(expo);
           bessel_k<LAB>(T.bessel, G.s * r, K);
-          uu = eval_ecp(gs, Cn.ng, Cn.L, r);
+          uu = eval_ecp(J, tr.centre, Cn.L, r);
           w = T.wl[n] * M.i1;
         }
       }
-      s_r[slot] = r;
-      s_w[slot] = w;
-      s_u[slot] = uu;
-      s_g[slot] = g;
-#pragma unroll
-      for (int l = 0; l <= LAB; l++) s_k[l * kKS + slot] = K[l];
-    };
-    auto fj = [&](int l1, int l2, int slot) {
+      // the open entries' pair sums
       double rn = 1.0;
-      for (int k = 0; k < l1; k++) rn = s_r[slot] * rn;
-      return s_w[slot] * ((((Cc * rn) * s_u[slot]) * s_k[l2 * kKS + slot]) * s_g[slot]);
-    };
-    auto f = [&](int slot) { return fj(my_l1, my_l2, slot); };
-    const bool mine = my_e >= 0;
-    if (mine) s_e[lane] = my_l1 | (my_l2 << 8);
-    double I = 0.0, p = 0.0, res = 0.0;
-    bool done = !mine;
-    auto test = [&](int l, double q) {
-      const double N = T.s92.lvl_n[l];
-      const double ee = I - p;
-      if (16 * ee * ee <= 3 * N * fabs(I - q) * T.tol) {
-        done = true;
-        res = 16 * I / (3 * N);
-      }
-    };
-    // pairs [kb, ke) of level l, pair k at slot0 + 2 (k - kb): the pair sums
-    // (0 + f(left)) + f(right) of every open entry by all lanes into s_t,
-    // then each entry's lane adds its own in pair order.  Called by the
-    // whole wave.
-    auto sum = [&](int l, int slot0, int kb, int ke) {
-      const int b0 = T.s92.lvl_begin[l], np = ke - kb;
-      const unsigned long long open = __ballot(mine && !done);
-      for (int i = lane; i < nfail * np; i += 64) {
-        const int j = i / np, k = i - j * np;
-        if (!((open >> j) & 1ull)) continue;
-        const int code = s_e[j];
-        double t = fj(code & 0xff, code >> 8, slot0 + 2 * k);
-        if (T.p92r[b0 + kb + k] <= end) t += fj(code & 0xff, code >> 8, slot0 + 2 * k + 1);
-        s_t[j * kFb1TS + k] = t;
+      int e = 0;
+#pragma unroll
+      for (int l1 = 0; l1 <= LAB; l1++) {
+        const double a = (Cc * rn) * uu;
+#pragma unroll
+        for (int l2 = l1; l2 >= 0; l2 -= 2, e++)
+          if ((om >> e) & 1ull) {
+            const double t = pair_sum(w * ((a * K[l2]) * g));
+            if (!(lane & 1)) s_t[e * kFbTS + (lane >> 1)] = t;
+          }
+        rn = r * rn;
       }
       __syncthreads();
-      if (mine && !done) I = sum_in_order(I, s_t + lane * kFb1TS, np);
-      __syncthreads();
-    };
-    int lv = 0;
-    while (lv < T.s92.nlevels && wave_any(!done)) {
-      const int l1 = psm92_round_end(lv, T.s92.nlevels);
-      if (l1 > lv + 1 || psm92_points(lv) <= 64) {
-        eval(lane, psm92_round_point(T, lv, l1, lane, end));
-        __syncthreads();
-        int roff = 0;
-        for (int l = lv; l < l1; l++) {
-          if (l == 0) {
-            if (mine) I = p = f(0);
-          } else {
-            double q = 0.0;
-            if (!done) {
-              q = 2 * p;
-              p = 2 * I;
-            }
-            sum(l, roff, 0, T.s92.lvl_begin[l + 1] - T.s92.lvl_begin[l]);
-            if (!done) test(l, q);
-          }
-          roff += psm92_points(l);
+      const bool level_end = !first && c1 == T.s92.lvl_begin[lv + 1];
+      if (open) {
+        bool done;
+        if (first) {
+          done = S.first_round(T, s_t + lane * kFbTS, &res);
+        } else {
+          S.I = sum_in_order(S.I, s_t + lane * kFbTS, c1 - c0);
+          done = level_end && S.test(T, lv, &res);
         }
-        __syncthreads();
-        lv = l1;
-      } else {
-        double q = 0.0;
-        if (!done) {
-          q = 2 * p;
-          p = 2 * I;
+        if (done) {
+          out[lane] = res;
+          open = false;
         }
-        const int b0 = T.s92.lvl_begin[lv], b1 = T.s92.lvl_begin[lv + 1];
-        for (int c0 = b0; c0 < b1; c0 += 32) {
-          const int nc = min(32, b1 - c0);
-          const int k = lane >> 1;
-          int n = -1;
-          if (k < nc) {
-            if ((lane & 1) == 0) n = T.p92l[c0 + k];
-            else if (T.p92r[c0 + k] <= end) n = T.p92r[c0 + k];
-          }
-          eval(lane, n);
-          __syncthreads();
-          sum(lv, 0, c0 - b0, c0 - b0 + nc);
-        }
-        if (!done) test(lv, q);
-        lv++;
       }
+      __syncthreads();
+      lv += level_end;
+      if (lv >= T.s92.nlevels || !wave_any(open)) break;
+      if (first || level_end) S.step();
+      c0 = c1;
+      c1 = min(c0 + 32, T.s92.lvl_begin[lv + 1]);
     }
     if constexpr (SPEC) {
-      if (mine && done) qfb[U.qoff + my_e] = res;
-      // the failed entries as a mask: one bit per lane that owns one
-      unsigned int lo = (mine && !done && my_e < 32) ? (1u << my_e) : 0u;
-      unsigned int hi = (mine && !done && my_e >= 32) ? (1u << (my_e - 32)) : 0u;
-      for (int o = 32; o > 0; o >>= 1) {
-        lo |= (unsigned int)__shfl_xor((int)lo, o, 64);
-        hi |= (unsigned int)__shfl_xor((int)hi, o, 64);
-      }
-      if (lane == 0) qfbf[u] = ((unsigned long long)hi << 32) | lo;
-    } else if (mine) {
-      if (done) qout[U.qoff + my_e] = res;
-      else status[2 * U.trip] = 1;
+      const unsigned long long failed = __ballot(open);
+      if (lane == 0) qfbf[u] = failed;
+    } else if (open) {
+      status[2 * U.trip] = 1;
     }
-    __syncthreads();
   }
 }
 
@@ -1143,10 +1102,8 @@ __global__ __launch_bounds__(64) void k_fb1(DevTables T, DevJob J, const T1Unit 
                                             double *__restrict__ qout, const unsigned long long *__restrict__ qfail,
                                             const int *__restrict__ fbq, const int *__restrict__ fbcount,
                                             unsigned char *__restrict__ status) {
-  __shared__ double s_r[64], s_w[64], s_u[64], s_g[64], s_k[(LAB + 1) * kKS], s_t[nq_of(LAB) * kFb1TS];
-  __shared__ int s_e[64];
-  fb1_body<LAB>(blockIdx.x, gridDim.x, T, J, units, qout, qfail, fbq, fbcount, status, s_r, s_w, s_u, s_g, s_k,
-                s_t, s_e);
+  __shared__ double s_t[nq_of(LAB) * kFbTS];
+  fb1_body<LAB>(blockIdx.x, gridDim.x, T, J, units, qout, qfail, fbq, fbcount, status, s_t);
 }
 
 // ---------------------------------------------------------------------------
@@ -1370,286 +1327,251 @@ __global__ __launch_bounds__(64) void k_type2_tail(DevTables T, DevJob J, T2Args
 }
 
 // type-2 fallback (calcT_FM06, type2.c:417-528): one wave per (triplet with
-// failed T entries, primitive pair).  The FM06-mapped points depend on the
-// pair only, so the wave evaluates each level's points once (K_a, K_b, the
-// exponential, and U_l for every channel l with failed entries) into LDS
-// for all failed entries of all the triplet's channels; lanes own the failed
-// entries (64 per pass) and sum the points in the integrator's pair order.
+// failed T entries, slot).  The FM06-mapped points depend on the primitive
+// pair only, so for each of its pairs the wave evaluates a round's points
+// once (31 point pairs and the centre, levels 0 to 5, then 32 pairs at a
+// time; a point per lane: exponential, weight and power of r in registers,
+// K_a, K_b and U_l of the channels with failed entries in the lane's own LDS
+// column) for all failed entries of all the triplet's channels.  The wave
+// takes the entries one after another: every lane forms the entry's
+// integrand at its point, two neighbouring lanes the pair sum, kFb2Chunk
+// entries at a time into LDS; then each entry's owner lane adds its own in
+// the integrator's order and tests after each level.
+// The lanes own points, not entries, so a triplet with few failed entries
+// keeps the wave as busy as one with many.  The primitive pairs whose points
+// of levels 0 and 1 are all numerically zero (half of them) are found first,
+// a pair per lane, and get their zeros without a wave's work; slot s of
+// `nslot` takes every nslot-th of the others.
 // Results per (entry, pair) go to fbT and are summed over pairs, in pair
-// order, by the assembly.// type-2 fallback (calcT_FM06, type2.c:417-528): one wave per (triplet with
-// failed T entries, primitive pair).  The FM06-mapped points depend on the
-// pair only, so the wave evaluates each level's points once (K_a, K_b, the
-// exponential, and U_l for every channel l with failed entries) into LDS
-// for all failed entries of all the triplet's channels; lanes own the
-// failed entries (64 per pass) and sum the points in the integrator's pair
-// With PACK, a triplet with at most 16 (32) failed entries runs four (two)
-// of its pairs per wave instead, one per lane group of HW = 16 (32) lanes,
-// so that the lanes summing are not a few of 64: the item of every fourth
-// (second) pair takes them, the others none; the groups share the wave's
-// rounds, each over its own pair's points.
-constexpr int kFb2PerLane = 1;
+// order, by the assembly.  No search for the screening break
+// (type2.c:479-481), as in the type-1 fallback.
+constexpr int kFb2Chunk = 16;  // entries whose pair sums are in LDS together
 constexpr int kFb2Cnt = 52;  // fbc[kFb2Cnt + c]: triplets queued for the type-2 fallback, class c
 constexpr int kFbcSlots = 80;  // queue counters per job
 static_assert(ECP_MAX_LAB < 16 && kFb2Cnt + kMaxLMB < kFbcSlots, "queue counter slots");
 
-template <int LMB, bool PACK>
+// OWN: entries owned per lane and pass
+template <int LMB, int OWN>
 __device__ __forceinline__ void fb2_body(int bid, int nb, const DevTables &T, const DevJob &J,
                                          const T2Group *__restrict__ groups, const int *__restrict__ tmpl,
-                                         const unsigned char *__restrict__ tfail, const int *__restrict__ fbq,
-                                         const int *__restrict__ fbcount, double *__restrict__ fbT,
-                                         unsigned char *__restrict__ status, const int *__restrict__ gcount,
-                                         const int *__restrict__ flist, const int *__restrict__ tgfirst,
-                                         int nsplit, double *s_r, double *s_w, double *s_cu, double *s_ex,
-                                         double *s_ka, double *s_kb, unsigned char *__restrict__ fbf2) {
+                                         const int *__restrict__ fbq, const int *__restrict__ fbcount,
+                                         double *__restrict__ fbT, unsigned char *__restrict__ status,
+                                         const int *__restrict__ gcount, const int *__restrict__ flist,
+                                         const int *__restrict__ tgfirst, int nslot, int nsplit, int share, double *s_cu,
+                                         double *s_rn, double *s_ka, double *s_kb, double *s_t,
+                                         unsigned char *__restrict__ fbf2) {
   const int lane = threadIdx.x;
-  // items (split, triplet, pair), split-major so that the grid-stride loop
-  // spreads every split over all workgroups; split k takes the passes k,
-  // k + nsplit, ...
-  const long per_split = (long)(*fbcount) * J.maxPairs;
+  const int count = *fbcount;
+  // items (split, slot, triplet): split k takes the k-th share of the entries
+  const long per_split = (long)count * nslot;
   const long total = per_split * nsplit;
   for (long it = bid; it < total; it += nb) {
     const int split = (int)(it / per_split);
-    const long r = it - split * per_split;
-    const int t = fbq[r / J.maxPairs];
-    const int pair = (int)(r % J.maxPairs);
+    const int rest = (int)(it - split * per_split);
+    const int slot = rest / count;
+    const int t = fbq[rest - slot * count];
     const ecp_triplet tr = J.trip[t];
     const ecp_shell Sa = J.shells[tr.sa], Sb = J.shells[tr.sb];
     const int npairs = Sa.K * Sb.K;
-    if (pair >= npairs) continue;
     const ecp_centre Cn = J.cent[tr.centre];
-    // the triplet's groups (one per semi-local channel l) and their failed
-    // entries; the points are shared by all of them
+    // the triplet's groups (one per semi-local channel l): their failed
+    // entries, listed one group after another
     const int g0 = tgfirst[t], L = Cn.L;
-    int gc[ECP_MAX_L], nfail = 0, lmax = 0;
+    int nfail = 0, lmax = 0;
+    unsigned int chan = 0;
     for (int l = 0; l < L; l++) {
-      gc[l] = gcount[g0 + l];
-      nfail += gc[l];
-      if (gc[l]) lmax = l;
+      const int c = gcount[g0 + l];
+      nfail += c;
+      if (c) {
+        lmax = l;
+        chan |= 1u << l;
+      }
     }
-    // this wave's passes: split, split + nsplit, ... (none: nothing to do)
-    if (split * 64 * kFb2PerLane >= nfail) continue;
-    // lane groups of HW = 1 << hwl lanes, group g on pair + g (a group past
-    // the triplet's pairs idles on pair's points)
-    const int hwl = !PACK ? 6 : nfail <= 16 ? 4 : nfail <= 32 ? 5 : 6;
-    if (PACK && (pair & ((64 >> hwl) - 1))) continue;
-    const int HW = PACK ? 1 << hwl : 64, NG = PACK ? 64 >> hwl : 1;
-    const int grp = PACK ? lane >> hwl : 0, sl = PACK ? lane & (HW - 1) : lane, base = PACK ? grp << hwl : 0;
-    const int mypair = pair + grp;
-    const bool gvalid = !PACK || mypair < npairs;
-    const int pq = gvalid ? mypair : pair;
-    const int pa = pq / Sb.K, pb = pq % Sb.K;
+    // shares of at least `share` entries, in whole chunks
+    const int ns = max(1, min(nsplit, (nfail + share - 1) / share));
+    const int per = ((nfail + ns - 1) / ns + kFb2Chunk - 1) / kFb2Chunk * kFb2Chunk;
+    const int e0 = split * per, e1 = min(nfail, e0 + per);
+    if (e0 >= e1) continue;
     const ecp_xyz rc = J.atoms[Cn.atom];
     const double dAC = dist(rc, J.atoms[Sa.atom]), dBC = dist(rc, J.atoms[Sb.atom]);
-    const double za = J.pa[Sa.prim + pa], zb = J.pa[Sb.prim + pb];
-    const double s1 = 2.0 * za * dAC, s2 = 2.0 * zb * dBC;
-    double Cc = J.pd[Sa.prim + pa] * J.pd[Sb.prim + pb];
-    // derivatives: times zeta^shift (type2.c:457-462)
-    for (int k = 0; k < tr.powa; k++) Cc *= za;
-    for (int k = 0; k < tr.powb; k++) Cc *= zb;
-    const double zeta_p = za + zb;
-    const Fm06 M = fm06(zeta_p, (za * dAC + zb * dBC) / zeta_p);
     const double minExp = T.lnAcc2;
-    auto expo_of = [&](double r) {
-      const double d1 = dAC - r, d2 = dBC - r;
-      return -za * d1 * d1 - zb * d2 * d2;
-    };
-    // the search is wave-wide: with lane groups on different pairs, the
-    // whole wave finds each group's break in turn
-    int brk = 0;
-    if (NG == 1) {
-      brk = fm06_break(T, M, dAC, dBC, minExp, expo_of);
-    } else {
-      for (int q = 0; q < NG; q++) {
-        const int pq2 = pair + q < npairs ? pair + q : pair;
-        const double za2 = J.pa[Sa.prim + pq2 / Sb.K], zb2 = J.pa[Sb.prim + pq2 % Sb.K];
-        const double zp2 = za2 + zb2;
-        const Fm06 M2 = fm06(zp2, (za2 * dAC + zb2 * dBC) / zp2);
-        const int b2 = fm06_break(T, M2, dAC, dBC, minExp, [&](double r) {
-          const double d1 = dAC - r, d2 = dBC - r;
-          return -za2 * d1 * d1 - zb2 * d2 * d2;
-        });
-        if (q == grp) brk = b2;
-      }
-    }
-    const int end = brk - 1;
-    const int laC = tr.la + lmax, lbC = tr.lb + lmax;
-    const ecp_gauss *gg = J.gauss + Cn.g0;
-    auto eval = [&](int slot, int n) {
-      double r = 0.0, w = 0.0, cu = 0.0, ex = 0.0;
-      bool live = false;
-      if (n >= 0 && n < brk) {
-        r = M.i1 * T.xl[n] + M.i2;
-        const double expo = expo_of(r);
-        if (expo >= minExp) {
-          live = true;
-          ex = exp(expo);
-          w = T.wl[n] * M.i1;
+    const int laC = tr.la + lmax, lbC = tr.lb + lmax, lab = tr.la + tr.lb;
+    for (int w0 = e0; w0 < e1; w0 += 64 * OWN) {
+      const int nhere = min(64 * OWN, e1 - w0);
+      // this lane's entries: packed (lambda1, lambda2, lambda3, l) and index
+      // in the job's T arrays
+      int code[OWN], eo[OWN];
+#pragma unroll
+      for (int i = 0; i < OWN; i++) {
+        code[i] = 0;
+        eo[i] = -1;
+        int kk = w0 + i * 64 + lane;
+        if (i * 64 + lane >= nhere) continue;
+        int l = 0, c = gcount[g0];
+        while (kk >= c) {
+          kk -= c;
+          c = gcount[g0 + ++l];
         }
+        const T2Group G = groups[g0 + l];
+        const int e = flist[G.eoff + kk];
+        code[i] = tmpl[G.tmpl + e] | (l << 24);
+        eo[i] = G.eoff + e;
       }
-      for (int l = 0; l < L; l++) {
-        if (!gc[l]) continue;
-        cu = live ? Cc * eval_ecp(gg, Cn.ng, l, r) : 0.0;
-        s_cu[l * 64 + slot] = cu;
-      }
-      s_r[slot] = r;
-      s_w[slot] = w;
-      s_ex[slot] = ex;
-      // one Bessel vector live at a time (register pressure)
-      {
-        double K[LMB + 1];
-#pragma unroll
-        for (int l = 0; l <= LMB; l++) K[l] = 0.0;
-        if (live) bessel_k<LMB>(T.bessel, s1 * r, K);
-#pragma unroll
-        for (int l = 0; l <= LMB; l++)
-          if (l <= laC) s_ka[l * kKS + slot] = K[l];
-      }
-      {
-        double K[LMB + 1];
-#pragma unroll
-        for (int l = 0; l <= LMB; l++) K[l] = 0.0;
-        if (live) bessel_k<LMB>(T.bessel, s2 * r, K);
-#pragma unroll
-        for (int l = 0; l <= LMB; l++)
-          if (l <= lbC) s_kb[l * kKS + slot] = K[l];
-      }
-    };
-    // the failed entries of all groups (listed by k_type2), group after
-    // group, HW per pass
-    for (int pass0 = split * HW * kFb2PerLane; pass0 < nfail; pass0 += HW * kFb2PerLane * nsplit) {
-      const int nhere = min(HW * kFb2PerLane, nfail - pass0);
-      int ent[kFb2PerLane], c1[kFb2PerLane], c2[kFb2PerLane], c3[kFb2PerLane], el[kFb2PerLane];
-      int eo[kFb2PerLane];  // the entry's index in the job's T arrays
-      double I[kFb2PerLane], p[kFb2PerLane], res[kFb2PerLane];
-      unsigned int done = 0;
-#pragma unroll
-      for (int j = 0; j < kFb2PerLane; j++) {
-        const int k = sl + HW * j;
-        ent[j] = -1;
-        el[j] = 0;
-        eo[j] = 0;
-        int code = 0;
-        if (gvalid && k < nhere) {
-          int kk = pass0 + k, l = 0;
-          while (kk >= gc[l]) kk -= gc[l++];
-          const T2Group G = groups[g0 + l];
-          ent[j] = flist[G.eoff + kk];
-          code = tmpl[G.tmpl + ent[j]];
-          el[j] = l;
-          eo[j] = G.eoff + ent[j];
+      for (int pb0 = 0; pb0 < npairs; pb0 += 64) {
+        bool mine_live = false;
+        if (pb0 + lane < npairs) {
+          const int pa = (pb0 + lane) / Sb.K, pb = (pb0 + lane) - pa * Sb.K;
+          const double za = J.pa[Sa.prim + pa], zb = J.pa[Sb.prim + pb];
+          const double zeta_p = za + zb;
+          const Fm06 M = fm06(zeta_p, (za * dAC + zb * dBC) / zeta_p);
+          mine_live = !psm92_dead(T, M, minExp, [&](double r) {
+            const double d1 = dAC - r, d2 = dBC - r;
+            return -za * d1 * d1 - zb * d2 * d2;
+          });
         }
-        c1[j] = code & 0xff;
-        c2[j] = (code >> 8) & 0xff;
-        c3[j] = (code >> 16) & 0xff;
-        if (ent[j] < 0) done |= 1u << j;
-        I[j] = p[j] = res[j] = 0.0;
-      }
-      const unsigned int all = (1u << kFb2PerLane) - 1u;
-      auto f = [&](int j, int slot) {
-        double rn = 1.0;
-        for (int k = 0; k < c3[j]; k++) rn = s_r[slot] * rn;
-        return s_w[slot] *
-               ((((s_cu[el[j] * 64 + slot] * rn) * s_ka[c1[j] * kKS + slot]) * s_kb[c2[j] * kKS + slot]) * s_ex[slot]);
-      };
-      __syncthreads();
-      auto test = [&](int l, const double (&q)[kFb2PerLane]) {
-        const double N = T.s92.lvl_n[l];
+        const int nc64 = min(64, npairs - pb0);
+        unsigned long long live = __ballot(mine_live);
+        unsigned long long dead = ~live & (nc64 == 64 ? ~0ull : (1ull << nc64) - 1ull);
+        // the zeros of the dead pairs: shared among the slots
+        for (int k = 0; dead; dead &= dead - 1ull, k++) {
+          if (k % nslot != slot) continue;
+          const int pair = pb0 + __ffsll((long long)dead) - 1;
 #pragma unroll
-        for (int j = 0; j < kFb2PerLane; j++) {
-          if (done & (1u << j)) continue;
-          const double ee = I[j] - p[j];
-          if (16 * ee * ee <= 3 * N * fabs(I[j] - q[j]) * T.tol) {
-            done |= 1u << j;
-            res[j] = 16 * I[j] / (3 * N);
+          for (int i = 0; i < OWN; i++)
+            if (eo[i] >= 0) fbT[(size_t)eo[i] * J.maxPairs + pair] = 0.0;
+        }
+        for (int k = 0; live; live &= live - 1ull, k++) {
+          if (k % nslot != slot) continue;
+          const int pair = pb0 + __ffsll((long long)live) - 1;
+          const int pa = pair / Sb.K, pb = pair - pa * Sb.K;
+          const double za = J.pa[Sa.prim + pa], zb = J.pa[Sb.prim + pb];
+          const double s1 = 2.0 * za * dAC, s2 = 2.0 * zb * dBC;
+          double Cc = J.pd[Sa.prim + pa] * J.pd[Sb.prim + pb];
+          // derivatives: times zeta^shift (type2.c:457-462)
+          for (int x = 0; x < tr.powa; x++) Cc *= za;
+          for (int x = 0; x < tr.powb; x++) Cc *= zb;
+          const double zeta_p = za + zb;
+          const Fm06 M = fm06(zeta_p, (za * dAC + zb * dBC) / zeta_p);
+          Psm92 S[OWN];
+          bool open[OWN];
+#pragma unroll
+          for (int i = 0; i < OWN; i++) {
+            S[i] = Psm92{0.0, 0.0, 0.0};
+            open[i] = eo[i] >= 0;
           }
-        }
-      };
-      // pair sums (0 + f(left)) + f(right) added to I in pair order; four
-      // pairs' sums are formed before they are added, so that their LDS
-      // reads overlap
-      auto sum = [&](int l, int slot0, int kb, int ke) {
-        const int b0 = T.s92.lvl_begin[l];
-#pragma unroll
-        for (int j = 0; j < kFb2PerLane; j++) {
-          if (done & (1u << j)) continue;
-          int k = kb;
-          for (; k + 4 <= ke; k += 4) {
-            double t[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-              t[i] = f(j, slot0 + 2 * (k + i - kb));
-              if (T.p92r[b0 + k + i] <= end) t[i] += f(j, slot0 + 2 * (k + i - kb) + 1);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; i++) I[j] += t[i];
-          }
-          for (; k < ke; k++) {
-            double t = f(j, slot0 + 2 * (k - kb));
-            if (T.p92r[b0 + k] <= end) t += f(j, slot0 + 2 * (k - kb) + 1);
-            I[j] += t;
-          }
-        }
-      };
-      int lv = 0;
-      while (lv < T.s92.nlevels && wave_any(done != all)) {
-        const int l1 = psm92_round_end(lv, T.s92.nlevels, HW);
-        if (l1 > lv + 1 || psm92_points(lv) <= HW) {
-          eval(base + sl, psm92_round_point(T, lv, l1, sl, end));
-          __syncthreads();
-          int roff = 0;
-          for (int l = lv; l < l1; l++) {
-            if (l == 0) {
-#pragma unroll
-              for (int j = 0; j < kFb2PerLane; j++)
-                if (!(done & (1u << j))) I[j] = p[j] = f(j, base);
-            } else {
-              double q[kFb2PerLane];
-#pragma unroll
-              for (int j = 0; j < kFb2PerLane; j++) {
-                q[j] = 2 * p[j];
-                p[j] = 2 * I[j];
+          // rounds of point pairs [c0, c1): levels 0 to 5 first, then 32
+          // pairs of level lv at a time
+          int lv = psm92_first(T), c0 = 0, c1 = T.s92.lvl_begin[lv];
+          for (;;) {
+            const bool first = c0 == 0;
+            const int n = psm92_point(T, c0, c1, lane, first);
+            double r = 0.0, w = 0.0, ex = 0.0;
+            bool on = false;
+            if (n >= 0) {
+              r = M.i1 * T.xl[n] + M.i2;
+              const double d1 = dAC - r, d2 = dBC - r;
+              const double expo = -za * d1 * d1 - zb * d2 * d2;
+              if (expo >= minExp) {
+                on = true;
+                ex = exp(expo);
+                w = T.wl[n] * M.i1;
               }
-              sum(l, base + roff, 0, T.s92.lvl_begin[l + 1] - T.s92.lvl_begin[l]);
-              test(l, q);
             }
-            roff += psm92_points(l);
-          }
-          __syncthreads();
-          lv = l1;
-        } else {
-          double q[kFb2PerLane];
+            for (int l = 0; l < L; l++)
+              if ((chan >> l) & 1u) s_cu[l * 64 + lane] = on ? Cc * eval_ecp(J, tr.centre, l, r) : 0.0;
+            {
+              double rn = 1.0;
+              for (int x = 0; x <= lab; x++) {
+                s_rn[x * 64 + lane] = rn;
+                rn = r * rn;
+              }
+            }
+            // one Bessel vector live at a time (register pressure)
+            {
+              double K[LMB + 1];
 #pragma unroll
-          for (int j = 0; j < kFb2PerLane; j++) {
-            q[j] = 2 * p[j];
-            p[j] = 2 * I[j];
-          }
-          const int b0 = T.s92.lvl_begin[lv], b1 = T.s92.lvl_begin[lv + 1];
-          for (int cb = b0; cb < b1; cb += HW / 2) {
-            const int nc = min(HW / 2, b1 - cb);
-            const int k = sl >> 1;
-            int n = -1;
-            if (k < nc) {
-              if ((sl & 1) == 0) n = T.p92l[cb + k];
-              else if (T.p92r[cb + k] <= end) n = T.p92r[cb + k];
+              for (int l = 0; l <= LMB; l++) K[l] = 0.0;
+              if (on) bessel_k<LMB>(T.bessel, s1 * r, K);
+#pragma unroll
+              for (int l = 0; l <= LMB; l++)
+                if (l <= laC) s_ka[l * 64 + lane] = K[l];
             }
-            eval(base + sl, n);
-            __syncthreads();
-            sum(lv, base, cb - b0, cb - b0 + nc);
-            __syncthreads();
+            {
+              double K[LMB + 1];
+#pragma unroll
+              for (int l = 0; l <= LMB; l++) K[l] = 0.0;
+              if (on) bessel_k<LMB>(T.bessel, s2 * r, K);
+#pragma unroll
+              for (int l = 0; l <= LMB; l++)
+                if (l <= lbC) s_kb[l * 64 + lane] = K[l];
+            }
+            const bool level_end = !first && c1 == T.s92.lvl_begin[lv + 1];
+            bool any = false;
+#pragma unroll
+            for (int i = 0; i < OWN; i++) {
+              const unsigned long long om = __ballot(open[i]);
+              for (int o = 0; o < 64; o += kFb2Chunk) {
+                unsigned int m = (unsigned int)(om >> o) & ((1u << kFb2Chunk) - 1u);
+                if (!m) continue;
+                // four entries at a time, so that their LDS reads overlap
+                // (fewer left: the last one again)
+                while (m) {
+                  int j[4];
+                  double cu[4], ka[4], kb[4], rn[4];
+#pragma unroll
+                  for (int x = 0; x < 4; x++) {
+                    j[x] = __ffs((int)m) - 1;
+                    if (m & (m - 1u)) m &= m - 1u;
+                    else if (x == 3) m = 0;
+                    const int cd = __builtin_amdgcn_readlane(code[i], o + j[x]);
+                    cu[x] = s_cu[(cd >> 24) * 64 + lane];
+                    rn[x] = s_rn[((cd >> 16) & 0xff) * 64 + lane];
+                    ka[x] = s_ka[(cd & 0xff) * 64 + lane];
+                    kb[x] = s_kb[((cd >> 8) & 0xff) * 64 + lane];
+                  }
+#pragma unroll
+                  for (int x = 0; x < 4; x++) {
+                    const double v = pair_sum(w * ((((cu[x] * rn[x]) * ka[x]) * kb[x]) * ex));
+                    if (!(lane & 1)) s_t[j[x] * kFbTS + (lane >> 1)] = v;
+                  }
+                }
+                __syncthreads();
+                if (open[i] && (unsigned)(lane - o) < (unsigned)kFb2Chunk) {
+                  const double *row = s_t + (lane - o) * kFbTS;
+                  double res = 0.0;
+                  bool done;
+                  if (first) {
+                    done = S[i].first_round(T, row, &res);
+                  } else {
+                    S[i].I = sum_in_order(S[i].I, row, c1 - c0);
+                    done = level_end && S[i].test(T, lv, &res);
+                  }
+                  if (done) {
+                    open[i] = false;
+                    fbT[(size_t)eo[i] * J.maxPairs + pair] = res;
+                  }
+                }
+                __syncthreads();
+              }
+              any = any || open[i];
+            }
+            lv += level_end;
+            if (lv >= T.s92.nlevels || !wave_any(any)) break;
+            if (first || level_end)
+#pragma unroll
+              for (int i = 0; i < OWN; i++) S[i].step();
+            c0 = c1;
+            c1 = min(c0 + 32, T.s92.lvl_begin[lv + 1]);
           }
-          test(lv, q);
-          lv++;
+#pragma unroll
+          for (int i = 0; i < OWN; i++) {
+            if (!open[i]) continue;
+            if (fbf2) fbf2[eo[i]] = 1;
+            else status[2 * t + 1] = 1;
+          }
         }
       }
-#pragma unroll
-      for (int j = 0; j < kFb2PerLane; j++) {
-        if (ent[j] < 0) continue;
-        if (done & (1u << j)) fbT[(size_t)eo[j] * J.maxPairs + mypair] = res[j];
-        else if (fbf2) fbf2[eo[j]] = 1;
-        else status[2 * t + 1] = 1;
-      }
     }
-    __syncthreads();
   }
 }
 
@@ -1729,18 +1651,16 @@ __global__ __launch_bounds__(64) void k_t1tail_fused(DevTables T, DevJob J, T1Se
 
 template <int MAXLAB, bool SPEC>
 __global__ __launch_bounds__(64) void k_fb1_fused(DevTables T, DevJob J, T1Set S, ClassMap cm) {
-  __shared__ double s_r[64], s_w[64], s_u[64], s_g[64], s_k[(MAXLAB + 1) * kKS], s_t[nq_of(MAXLAB) * kFb1TS];
-  __shared__ int s_e[64];
+  __shared__ double s_t[nq_of(MAXLAB) * kFbTS];
   const int i = class_entry(cm, blockIdx.x);
   const int c = cm.cls[i], bid = blockIdx.x - cm.bbeg[i], nb = cm.bbeg[i + 1] - cm.bbeg[i];
   const int ub = S.ubeg[c];
   switch (c) {
-#define X(L)                                                                                                   \
-  case L:                                                                                                      \
-    if constexpr (L <= MAXLAB)                                                                                 \
-      fb1_body<L, SPEC>(bid, nb, T, J, S.units + ub, S.q, S.qf + ub, S.fbq + ub, S.fbc + c, S.stat, s_r, s_w, s_u, \
-                        s_g, s_k, s_t, s_e, S.tq + ub, S.fbc + 32 + c, SPEC ? S.qopen + ub : nullptr, S.qfb,      \
-                        SPEC ? S.qfbf + ub : nullptr);                                                          \
+#define X(L)                                                                                                     \
+  case L:                                                                                                        \
+    if constexpr (L <= MAXLAB)                                                                                   \
+      fb1_body<L, SPEC>(bid, nb, T, J, S.units + ub, S.q, S.qf + ub, S.fbq + ub, S.fbc + c, S.stat, s_t, S.tq + ub, \
+                        S.fbc + 32 + c, SPEC ? S.qopen + ub : nullptr, S.qfb, SPEC ? S.qfbf + ub : nullptr);     \
     break;
     ECP_CASES_LAB(X)
 #undef X
@@ -1750,31 +1670,34 @@ __global__ __launch_bounds__(64) void k_fb1_fused(DevTables T, DevJob J, T1Set S
 struct T2Set {
   const T2Group *groups;
   const int *tmpl;
-  const unsigned char *tf;
   const int *fbq2;  // per class, the triplets with failed entries (nt apart)
   const int *fbc;
   double *fbT;
   unsigned char *stat;
   int nt;
   const int *gcount, *flist, *tgfirst;
-  int nsplit;
+  int nslot, nsplit, share;
+  int cu_rows, rn_rows, k_rows;  // LDS rows: U_l of the job's channels, powers of r, K of its largest class
   unsigned char *fbf2;  // speculative fallback: per entry, the large grid failed (nullptr: off)
 };
 
-// PACK: triplets with few failed entries run several pairs per wave (three
-// waves per SIMD kept: at two the uneven batch loses the gain)
-template <int MAXLMB, bool PACK>
-__global__ __launch_bounds__(64, PACK ? 3 : 1) void k_fb2_fused(DevTables T, DevJob J, T2Set S, ClassMap cm) {
-  __shared__ double s_r[64], s_w[64], s_cu[ECP_MAX_L * 64], s_ex[64];
-  __shared__ double s_ka[(MAXLMB + 1) * kKS], s_kb[(MAXLMB + 1) * kKS];
+// two entries per lane where registers set the waves per SIMD (three), four
+// in the larger classes, where the LDS rows do (two)
+template <int MAXLMB, int OWN = MAXLMB <= 7 ? 2 : 4>
+__global__ __launch_bounds__(64, MAXLMB <= 7 ? 3 : 2) void k_fb2_fused(DevTables T, DevJob J, T2Set S, ClassMap cm) {
+  // pair sums, then the points' columns: U rows for the job's channels, K
+  // rows for its largest class (fb2_lds)
+  extern __shared__ double lds[];
+  double *s_t = lds, *s_cu = lds + kFb2Chunk * kFbTS, *s_rn = s_cu + S.cu_rows * 64, *s_ka = s_rn + S.rn_rows * 64,
+         *s_kb = s_ka + S.k_rows * 64;
   const int i = class_entry(cm, blockIdx.x);
   const int c = cm.cls[i], bid = blockIdx.x - cm.bbeg[i], nb = cm.bbeg[i + 1] - cm.bbeg[i];
   switch (c) {
-#define X(L)                                                                                                   \
-  case L:                                                                                                      \
-    if constexpr (L <= MAXLMB)                                                                                 \
-      fb2_body<L, PACK>(bid, nb, T, J, S.groups, S.tmpl, S.tf, S.fbq2 + (size_t)L * S.nt, S.fbc + kFb2Cnt + L, S.fbT, \
-                  S.stat, S.gcount, S.flist, S.tgfirst, S.nsplit, s_r, s_w, s_cu, s_ex, s_ka, s_kb, S.fbf2);    \
+#define X(L)                                                                                                     \
+  case L:                                                                                                        \
+    if constexpr (L <= MAXLMB)                                                                                   \
+      fb2_body<L, OWN>(bid, nb, T, J, S.groups, S.tmpl, S.fbq2 + (size_t)L * S.nt, S.fbc + kFb2Cnt + L, S.fbT, S.stat, \
+                  S.gcount, S.flist, S.tgfirst, S.nslot, S.nsplit, S.share, s_cu, s_rn, s_ka, s_kb, s_t, S.fbf2); \
     break;
     ECP_CASES_LMB(X)
 #undef X
@@ -2500,6 +2423,7 @@ struct Prepared {
   int max_lab = 0, max_lmb = 0;
   int tcount2[kMaxLMB + 1] = {0};  // triplets per type-2 fallback class
   int max_cls2 = 0;
+  int max_ent2 = 0;  // T entries of a triplet, at most
   int *tclaim = nullptr;
   unsigned char *fbf2 = nullptr;  // per T entry: the speculative fallback failed on the large grid
   const unsigned char *tcls2 = nullptr;
@@ -3006,34 +2930,64 @@ void launch_fb1(ecp_dev *d, hipStream_t s, const DevTables &T, const DevJob &J, 
   }
 }
 
-// the type-2 fallback classes of cm in one grid; like the type-1 kernels,
-// three tiers bound the Bessel orders the grid holds: up to 7, 11 and 12
-// pack: several pairs per wave for triplets with few failed entries
-// (classes up to 7).  Less work in all, but each wave longer: it pays in
-// the throughput-bound per-class sequence of large jobs (the uneven batch
-// 1.4 % faster) and not on the fused sequence's critical chain (the medium
-// cluster 1.5 % slower).
-void launch_fb2_fused(ecp_dev *d, hipStream_t s, const T2Set &S2, const ClassMap &cm, bool pack) {
-  const Prepared &P = d->P;
-  const int nb = cm.bbeg[cm.n];
-  if (P.max_cls2 > 11) k_fb2_fused<12, false><<<nb, 64, 0, s>>>(d->T, P.J, S2, cm);
-  else if (P.max_cls2 > 7) k_fb2_fused<11, false><<<nb, 64, 0, s>>>(d->T, P.J, S2, cm);
-  else if (pack) k_fb2_fused<7, true><<<nb, 64, 0, s>>>(d->T, P.J, S2, cm);
-  else k_fb2_fused<7, false><<<nb, 64, 0, s>>>(d->T, P.J, S2, cm);
+// workgroup ranges of the classes with work; blocks(c) = workgroups of class c
+template <typename F>
+ClassMap class_map(int ncls, const int *count, F blocks) {
+  ClassMap cm{};
+  int b = 0;
+  for (int c = 0; c < ncls; c++) {
+    if (count[c] <= 0) continue;
+    const int nb = blocks(c);
+    if (nb <= 0) continue;
+    cm.cls[cm.n] = c;
+    cm.bbeg[cm.n] = b;
+    b += nb;
+    cm.n++;
+  }
+  cm.bbeg[cm.n] = b;
+  return cm;
 }
 
-// waves per (triplet, pair) of the type-2 fallback (fb2_split; 0: automatic,
-// 3 for jobs of up to kFb2SplitMaxItems (triplet, pair) items, where the
-// fallback's latency counts, 1 for larger, throughput-bound ones)
-constexpr long kFb2SplitMaxItems = 1000000;
+// the type-2 fallback classes of cm in one grid; like the type-1 kernels,
+// three tiers bound the Bessel orders the grid holds: up to 7, 11 and 12
+void launch_fb2_fused(ecp_dev *d, hipStream_t s, const T2Set &S2, const ClassMap &cm) {
+  const Prepared &P = d->P;
+  const int nb = cm.bbeg[cm.n];
+  // 13.1 KB for projectors up to f and class 6: twelve waves per CU, what
+  // the registers (168) allow
+  const size_t lds = sizeof(double) * (kFb2Chunk * kFbTS + (S2.cu_rows + S2.rn_rows + 2 * S2.k_rows) * 64);
+  if (P.max_cls2 > 11) k_fb2_fused<12><<<nb, 64, lds, s>>>(d->T, P.J, S2, cm);
+  else if (P.max_cls2 > 7) k_fb2_fused<11><<<nb, 64, lds, s>>>(d->T, P.J, S2, cm);
+  else k_fb2_fused<7><<<nb, 64, lds, s>>>(d->T, P.J, S2, cm);
+}
 
-int fb2_split(const ecp_dev *d, bool fused) {
-  (void)fused;
-  const int v = d->tune.fb2_split;
-  if (v > 0) return std::min(v, 8);
+// Waves per triplet of the type-2 fallback (nslot: its primitive pairs are
+// dealt to them) and the entries per wave (share), by the job's (triplet,
+// pair) items.  Many short waves where the fallback's latency counts, few
+// long ones where the wave's set-up (triplet, shells, entry list: a chain of
+// dependent reads) and the points evaluated once per share are what the chip
+// spends its time on.  Fallback alone, one wave per pair / three / one per
+// triplet at the shares given: the 50-atom cluster (72 k items) 120 / 150 /
+// 432 us, its gradient (222 k) 260 / 319 / 576, 20 atoms with g shells
+// (445 k) 1910 / 1557 / 2176, 256 uneven molecules (6.2 M) 5916 / 4208 /
+// 3917.  fb2_split > 0 sets the number of shares instead.
+void fb2_slots(const ecp_dev *d, T2Set &S) {
+  const int maxPairs = d->P.maxPairs;
   long items = 0;
-  for (int c = 0; c <= kMaxLMB; c++) items += (long)d->P.tcount2[c] * d->P.maxPairs;
-  return items <= kFb2SplitMaxItems ? 3 : 1;
+  for (int c = 0; c <= kMaxLMB; c++) items += (long)d->P.tcount2[c] * maxPairs;
+  S.nslot = items <= 300000 ? maxPairs : items <= 2000000 ? std::min(maxPairs, 3) : 1;
+  S.share = items <= 100000 ? 64 : items <= 300000 || d->P.max_cls2 <= 7 ? 128 : 256;
+  const int v = d->tune.fb2_split;
+  S.nsplit = v > 0 ? std::min(v, 8) : (d->P.max_ent2 + S.share - 1) / S.share;
+  S.cu_rows = d->P.max_L;
+  S.rn_rows = d->P.max_lab + 1;
+  S.k_rows = d->P.max_cls2 + 1;
+}
+
+ClassMap fb2_classes(const ecp_dev *d, const T2Set &S) {
+  return class_map(kMaxLMB + 1, d->P.tcount2, [&](int c) {
+    return (int)std::min<long>((long)d->P.tcount2[c] * S.nslot * S.nsplit, 8192);
+  });
 }
 
 // The kernel sequence of one evaluation, on resident inputs, one launch per
@@ -3071,24 +3025,6 @@ void launch_ang(ecp_dev *d, hipStream_t s) {
 // fuse = 2 (automatic): fused launches for jobs of up to this many type-1
 // primitive pairs (latency-bound: per-class launches hold few waves each)
 constexpr int kFuseAutoMaxUnits = 150000;
-
-// workgroup ranges of the classes with work; blocks(c) = workgroups of class c
-template <typename F>
-ClassMap class_map(int ncls, const int *count, F blocks) {
-  ClassMap cm{};
-  int b = 0;
-  for (int c = 0; c < ncls; c++) {
-    if (count[c] <= 0) continue;
-    const int nb = blocks(c);
-    if (nb <= 0) continue;
-    cm.cls[cm.n] = c;
-    cm.bbeg[cm.n] = b;
-    b += nb;
-    cm.n++;
-  }
-  cm.bbeg[cm.n] = b;
-  return cm;
-}
 
 // one type-1 class of the per-class sequence: small grid, fallback, assembly
 template <int c>
@@ -3170,14 +3106,12 @@ void enqueue(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
     // every fallback class in one persistent grid: the classes' items run
     // side by side instead of one class after another on this stream
     {
-      const int nsplit = fb2_split(d, false);
-      T2Set S2{P.grp, d->tmpl_dev, P.tf, P.fbq2, P.fbc, P.fbT, P.stat, P.nt, P.gflag, P.flist, P.tgf, nsplit};
-      const ClassMap cm2 = class_map(kMaxLMB + 1, P.tcount2, [&](int c) {
-        return (int)std::min<long>((long)P.tcount2[c] * P.maxPairs * nsplit, 8192);
-      });
+      T2Set S2{P.grp, d->tmpl_dev, P.fbq2, P.fbc, P.fbT, P.stat, P.nt, P.gflag, P.flist, P.tgf, 1, 1, 1, 0, 0, 0, nullptr};
+      fb2_slots(d, S2);
+      const ClassMap cm2 = fb2_classes(d, S2);
       if (cm2.n > 0) {
         Span sp(d, s, FAM_FB2);
-        launch_fb2_fused(d, s, S2, cm2, true);
+        launch_fb2_fused(d, s, S2, cm2);
       }
     }
     {
@@ -3332,15 +3266,13 @@ void enqueue_fused(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
     launch_type2(d, w[2], true, spec2, spec2 ? d->h2done : nullptr);
     (void)hipEventRecord(d->t2done, w[2]);
     (void)hipStreamWaitEvent(w[3], spec2 ? d->h2done : d->t2done, 0);
-    const int nsplit = fb2_split(d, true);
-    T2Set S2{P.grp, d->tmpl_dev, P.tf, P.fbq2, P.fbc, P.fbT, P.stat, P.nt, P.gflag, P.flist, P.tgf, nsplit};
-    S2.fbf2 = spec2 ? P.fbf2 : nullptr;
-    const ClassMap cm2 = class_map(kMaxLMB + 1, P.tcount2, [&](int c) {
-      return (int)std::min<long>((long)P.tcount2[c] * P.maxPairs * nsplit, 8192);
-    });
+    T2Set S2{P.grp, d->tmpl_dev, P.fbq2, P.fbc, P.fbT, P.stat, P.nt, P.gflag, P.flist, P.tgf, 1, 1, 1, 0, 0, 0,
+             spec2 ? P.fbf2 : nullptr};
+    fb2_slots(d, S2);
+    const ClassMap cm2 = fb2_classes(d, S2);
     if (cm2.n > 0) {
       Span sp(d, w[3], FAM_FB2);
-      launch_fb2_fused(d, w[3], S2, cm2, false);
+      launch_fb2_fused(d, w[3], S2, cm2);
     }
     (void)hipStreamWaitEvent(w[2], d->angdone, 0);
     {
@@ -3436,6 +3368,7 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
       P.tcount2[c2]++;
       P.max_cls2 = std::max(P.max_cls2, c2);
     }
+    const int ent0 = ntot2;
     for (int l = 0; l < job->cent[tr.centre].L; l++) {
       const int key = tmpl_key(la, lb, l);
       T2Group g{t, l, ntot2, d->tmpl_cnt[key], d->tmpl_off[key], std::max(la, lb) + l};
@@ -3446,6 +3379,7 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
       ntot2 += g.ne;
       P.lmb_count[g.lmb]++;
     }
+    P.max_ent2 = std::max(P.max_ent2, ntot2 - ent0);
   }
   P.ngroups = (int)groups.size();
   P.ntot2 = ntot2;

@@ -85,8 +85,8 @@ typedef struct {
                          (>= the level count, the default: no tail; 0: 6 with fused
                          launches, else none) */
   int t2_tail_grid;   /* most workgroups of the type-2 tail launch */
-  int fb2_split;      /* waves per (triplet, primitive pair) of the type-2 fallback, its 64-entry
-                         passes dealt round robin; 0: 3 for small jobs, 1 for large ones */
+  int fb2_split;      /* shares a triplet's type-2 fallback entries are split into, each with its
+                         own waves; 0: by the job's size */
   int t1_spec;        /* fused launches: the type-1 large-grid fallback starts after the head,
                          beside the tail, on every entry the head left open (1), or after the
                          tail on the failed ones only (0) */

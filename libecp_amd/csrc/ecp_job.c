@@ -243,6 +243,25 @@ static int trip_push(trip_vec *tv, const ecp_triplet *t) {
   return 0;
 }
 
+/* Orders a centre's Gaussians by channel, keeping the input order inside a
+   channel (the order its potential is summed in), and records where each
+   channel starts, so that a channel's potential visits its own Gaussians
+   only. */
+static void ecp_sort_channels(ecp_gauss *gauss, ecp_centre *Cn) {
+  ecp_gauss *g = gauss + Cn->g0;
+  for (int i = 1; i < Cn->ng; i++) {
+    const ecp_gauss x = g[i];
+    int j = i;
+    for (; j > 0 && g[j - 1].l > x.l; j--) g[j] = g[j - 1];
+    g[j] = x;
+  }
+  int i = 0;
+  for (int l = 0; l <= ECP_MAX_L + 1; l++) {
+    while (i < Cn->ng && g[i].l < l) i++;
+    Cn->gl[l] = i;
+  }
+}
+
 /* Derivative shifts of the basis angular momenta, in the reference's order
    (libecp.c:243-250): first derivatives (+1,0) (-1,0) (0,+1) (0,-1); second
    derivatives the ten pairs below. */
@@ -380,6 +399,7 @@ int ecp_job_build(const ecp_mol *mols, int nmol, int deriv, const ecp_static *st
         }
       }
       Cn->ng = gg - Cn->g0;
+      ecp_sort_channels(job->gauss, Cn);
       cc++;
     }
     job->trip_mol_begin[m] = tv.n;
