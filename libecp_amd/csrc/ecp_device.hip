@@ -35,6 +35,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -538,46 +539,93 @@ __device__ __forceinline__ void t1_geom(const DevJob &J, const ecp_triplet &tr, 
   G.z = -G.za - G.zb;
 }
 
+// FM06 linear map of the large grid for zeta_p, P (gc_integrators.c:316-331)
+struct Fm06 {
+  double i1, i2;
+};
+__device__ __forceinline__ Fm06 fm06(double zeta_p, double P) {
+  const double sigma = 1.0 / sqrt(zeta_p);
+  const double t = P - 7.0 * sigma;
+  const double rmin = (t > 0.0) ? t : 0.0;
+  const double rmax = P + 9.0 * sigma;
+  Fm06 m;
+  m.i1 = 0.5 * (rmax - rmin);
+  m.i2 = 0.5 * (rmax + rmin);
+  return m;
+}
+
+// The exponents of the three points of PSM92 levels 0 and 1 are all below
+// the numerical zero: every integral of the pair is then 0 at level 0 and
+// converges with the result 0 at level 1 (0 <= 0 in its test).
+template <typename Expo>
+__device__ __forceinline__ bool psm92_dead(const DevTables &T, const Fm06 &M, double minExp, Expo expo) {
+  if (T.s92.nlevels < 2) return false;
+  const double e0 = expo(M.i1 * T.xl[T.s92.centre] + M.i2), e1 = expo(M.i1 * T.xl[T.p92l[0]] + M.i2),
+               e2 = expo(M.i1 * T.xl[T.p92r[0]] + M.i2);
+  return !(e0 >= minExp) && !(e1 >= minExp) && !(e2 >= minExp);
+}
+
+// psm92_dead of a type-1 unit (the large grid of fb1_body)
+__device__ __forceinline__ bool t1_fb_dead(const DevTables &T, const T1Geom &G) {
+  const double zeta_p = G.za + G.zb;
+  const Fm06 M = fm06(zeta_p, (G.za * G.dAC + G.zb * G.dBC) / zeta_p);
+  return psm92_dead(T, M, T.lnAcc1, [&](double r) { return (G.z * r + G.s) * r + G.zd2; });
+}
+
+// Beyond this exponent exp overflows (from 709.78 on), whatever its last
+// bits: the point's integrand, exp(zd2) ... exp(expo) with exp(zd2) = 0 or
+// not, is infinite or not a number, and so is every level sum that holds it.
+constexpr double kOverflowExpo = 710.0;
+
+// A level sum that is infinite or not a number stays so, and no later level
+// passes the PS93 test: the entry has failed on the small grid.
+__device__ __forceinline__ bool t1_lost(double I) { return !(fabs(I) < INFINITY); }
+
+// A slot in a queue for every active lane: one atomic per wave
+__device__ __forceinline__ int queue_slot(int *count) {
+  const unsigned long long m = __ballot(true);
+  const int lane = threadIdx.x & 63;
+  int base = 0;
+  if (lane == __ffsll((long long)m) - 1) base = atomicAdd(count, __popcll(m));
+  return __builtin_amdgcn_readfirstlane(base) + __popcll(m & ((1ull << lane) - 1ull));
+}
+
 // Results of a finished primitive pair: converged entries, zeros for the
-// others, which go to the large-grid fallback queue.
+// others, which go to the large-grid fallback queue, unless the fallback
+// would end with zeros at once (t1_fb_dead: nine tenths of the failed pairs,
+// whose small-grid integrand overflows while the integral vanishes).
 template <int NQ>
-__device__ __forceinline__ void t1_finish(int u, const T1Unit &U, const double (&p)[NQ], unsigned long long done,
-                                          double *__restrict__ qout, unsigned long long *__restrict__ qfail,
-                                          int *__restrict__ fbq, int *__restrict__ fbcount,
-                                          unsigned char *__restrict__ fbflag) {
+__device__ __forceinline__ void t1_finish(const DevTables &T, const T1Geom &G, int u, const T1Unit &U,
+                                          const double (&p)[NQ], unsigned long long done, double *__restrict__ qout,
+                                          unsigned long long *__restrict__ qfail, int *__restrict__ fbq,
+                                          int *__restrict__ fbcount) {
   const unsigned long long all = (NQ >= 64) ? ~0ull : ((1ull << NQ) - 1ull);
   double *out = qout + U.qoff;
 #pragma unroll
   for (int e = 0; e < NQ; e++) out[e] = (done & (1ull << e)) ? p[e] : 0.0;
   const unsigned long long failed = all & ~done;
   qfail[u] = failed;
-  if (failed) {
-    fbq[atomicAdd(fbcount, 1)] = u;
-    fbflag[U.trip] = 1;
-  }
+  if (failed && !t1_fb_dead(T, G)) fbq[queue_slot(fbcount)] = u;
 }
 
-// Type-1 small grid, one lane per primitive pair (MODE 0: the whole PS93
-// sequence; MODE 1, head: levels [0, head), then a pair still open saves its
-// integrator state -- p, q, I per entry in planes of `plane` doubles at
-// state -- and its converged-entry mask and is queued for a tail kernel;
-// MODE 2, lane-serial tail: the queued pairs, compacted one per lane, resume
-// at level `head`).  Within a level each point pair's sum
-// T = (0 + f(left)) + f(right) is added to I in pair order, and the PS93
-// recurrences and test (gc_integrators.c:156-217) follow.
-template <int LAB, int MODE>
-__device__ __forceinline__ void type1_body(int bid, int nb, const DevTables &T, const DevJob &J,
+// Type-1 small grid, one lane per primitive pair: levels [0, head); a pair
+// still open then saves its integrator state -- p, q, I per entry in planes
+// of `plane` doubles at state -- and its converged-entry mask and is queued
+// for the tail (head >= the level count: the whole sequence, no tail).
+// Within a level each point pair's sum T = (0 + f(left)) + f(right) is added
+// to I in pair order, and the PS93 recurrences and test
+// (gc_integrators.c:156-217) follow.  Four fifths of the integrals converge
+// (nearly all to 0) by level 4, after 11 points, and hardly any at levels 5
+// to 7: the head ends there.
+template <int LAB>
+__device__ __forceinline__ void type1_body(int bid, const DevTables &T, const DevJob &J,
                                            const T1Unit *__restrict__ units, int nunits, double *__restrict__ qout,
                                            unsigned long long *__restrict__ qfail, int *__restrict__ fbq,
                                            int *__restrict__ fbcount, int head, double *__restrict__ state,
-                                           size_t plane, int *__restrict__ tq, int *__restrict__ tcount,
-                                           unsigned char *__restrict__ fbflag,
-                                           unsigned long long *__restrict__ qopen = nullptr) {
+                                           size_t plane, int *__restrict__ tq, int *__restrict__ tcount) {
   constexpr int NQ = nq_of(LAB);
-  const int count = MODE == 2 ? *tcount : nunits;
-  const int stride = MODE == 2 ? nb * 64 : count;
-  for (int it = bid * 64 + (int)threadIdx.x; it < count; it += stride) {
-    const int u = MODE == 2 ? tq[it] : it;
+  const int u = bid * 64 + (int)threadIdx.x;
+  if (u < nunits) {
     const T1Unit U = units[u];
     const ecp_triplet tr = J.trip[U.trip];
     const ecp_centre Cn = J.cent[tr.centre];
@@ -587,78 +635,59 @@ __device__ __forceinline__ void type1_body(int bid, int nb, const DevTables &T, 
     const double *__restrict__ UL = J.UL + Cn.UL_off;
     const int gs = tr.gs, ge = tr.ge;
     const double minExp = T.lnAcc1;
-    // w_n f(n) of one point for every entry, added into acc[] (type1.c:78-88
-    // integrand, tabulated only on [gs, ge) as type1.c:121-130)
-    auto f = [&](int n, double (&acc)[NQ]) {
-      if (n < gs || n >= ge) return;
+    // a point's factors (type1.c:78-88 integrand, tabulated only on [gs, ge)
+    // as type1.c:121-130): entry (l1, l2) is w ((C0 r^l1 U) K[l2]) g, all
+    // zero where the point contributes nothing
+    struct Point {
+      double r, w, U, g, K[LAB + 1];
+    };
+    auto point = [&](int n, bool use) {
+      Point Q;
+      Q.r = Q.w = Q.U = Q.g = 0.0;
+#pragma unroll
+      for (int l = 0; l <= LAB; l++) Q.K[l] = 0.0;
+      if (!use || n < gs || n >= ge) return Q;
       const double r = T.xs[n];
       const double expo = (G.z * r + G.s) * r;
-      if (!(expo >= minExp)) return;
-      const double g = exp(expo);
-      double K[LAB + 1];
-      bessel_k<LAB>(T.bessel, G.s * r, K);
-      const double Un = UL[n], wn = T.ws[n];
-      double rn = 1.0;
+      if (!(expo >= minExp)) return Q;
+      Q.r = r;
+      Q.g = exp(expo);
+      bessel_k<LAB>(T.bessel, G.s * r, Q.K);
+      Q.U = UL[n];
+      Q.w = T.ws[n];
+      return Q;
+    };
+    // each(e, (0 + f(left)) + f(right)) for every entry
+    auto pair = [&](const Point &a, const Point &b, auto each) {
+      double ra = 1.0, rb = 1.0;
       int e = 0;
 #pragma unroll
       for (int l1 = 0; l1 <= LAB; l1++) {
-        const double a = (C0 * rn) * Un;
+        const double ca = (C0 * ra) * a.U, cb = (C0 * rb) * b.U;
 #pragma unroll
-        for (int l2 = l1; l2 >= 0; l2 -= 2, e++) acc[e] += wn * ((a * K[l2]) * g);
-        rn *= r;
+        for (int l2 = l1; l2 >= 0; l2 -= 2, e++)
+          each(e, (0.0 + a.w * ((ca * a.K[l2]) * a.g)) + b.w * ((cb * b.K[l2]) * b.g));
+        ra *= a.r;
+        rb *= b.r;
       }
     };
-    double p[NQ], q[NQ], I[NQ], Tt[NQ];
-    unsigned long long done = 0ull;
+    double p[NQ], q[NQ], I[NQ];
+    unsigned long long done = 0ull, lost = 0ull;
     const unsigned long long all = (NQ >= 64) ? ~0ull : ((1ull << NQ) - 1ull);
-    int lv0 = 2, lv1 = T.s93.nlevels;
-    if (MODE == 2) {
-#pragma unroll
-      for (int e = 0; e < NQ; e++) {
-        p[e] = state[U.qoff + e];
-        q[e] = state[plane + U.qoff + e];
-        I[e] = state[2 * plane + U.qoff + e];
-      }
-      done = qfail[u];
-      lv0 = head;
-    } else {
-#pragma unroll
-      for (int e = 0; e < NQ; e++) Tt[e] = 0.0;
-      f(T.s93.centre, Tt);
-#pragma unroll
-      for (int e = 0; e < NQ; e++) {
-        p[e] = Tt[e];
-        Tt[e] = 0.0;
-      }
-      f(T.s93.first_l, Tt);
-      double t2[NQ];
-#pragma unroll
-      for (int e = 0; e < NQ; e++) t2[e] = 0.0;
-      f(T.s93.first_r, t2);
-#pragma unroll
-      for (int e = 0; e < NQ; e++) {
-        q[e] = Tt[e] + t2[e];
-        I[e] = p[e] + q[e];
-      }
-      if (MODE == 1) lv1 = min(head, T.s93.nlevels);
-    }
-    for (int lv = lv0; lv < lv1; lv++) {
+    const int lv1 = min(head, T.s93.nlevels);
+    pair(point(T.s93.centre, true), point(0, false), [&](int e, double t) { p[e] = t; });
+    pair(point(T.s93.first_l, true), point(T.s93.first_r, true), [&](int e, double t) {
+      q[e] = t;
+      I[e] = p[e] + t;
+    });
+    for (int lv = 2; lv < lv1; lv++) {
       const int j = T.s93.lvl_j[lv], nn = T.s93.lvl_n[lv];
       int cnt = 0;
       for (int k = T.s93.lvl_begin[lv]; k < T.s93.lvl_begin[lv + 1]; k++) {
         const int li = T.p93l[k], ri = T.p93r[k];
-#pragma unroll
-        for (int e = 0; e < NQ; e++) Tt[e] = 0.0;
-        if (li >= gs) {
-          cnt++;
-          f(li, Tt);
-        }
-        if (ri <= ge) {
-          cnt++;
-          f(ri, Tt);
-        }
-#pragma unroll
-        for (int e = 0; e < NQ; e++) I[e] += Tt[e];
+        const bool useL = li >= gs, useR = ri <= ge;
+        cnt += useL + useR;
+        pair(point(li, useL), point(ri, useR), [&](int e, double t) { I[e] += t; });
       }
 #pragma unroll
       for (int e = 0; e < NQ; e++) {
@@ -674,11 +703,24 @@ __device__ __forceinline__ void type1_body(int bid, int nb, const DevTables &T, 
         if (cnt > 0 && err < T.tol) {
           done |= (1ull << e);
           p[e] = 16 * q[e] / (3 * nn);
+        } else if (t1_lost(I[e])) {
+          lost |= (1ull << e);
         }
       }
-      if (done == all) break;
+      if ((done | lost) == all) break;
     }
-    if (MODE == 1 && done != all && lv1 < T.s93.nlevels) {
+    if ((done | lost) != all && lv1 < T.s93.nlevels) {
+      // an exponent that overflows in the tail's first level: nothing still
+      // open can converge, so there is no tail to run
+      for (int k = T.s93.lvl_begin[lv1]; k < T.s93.lvl_begin[lv1 + 1]; k++) {
+        const int li = T.p93l[k], ri = T.p93r[k];
+        const double rl = T.xs[li], rr = T.xs[ri];
+        if ((li >= gs && li < ge && (G.z * rl + G.s) * rl > kOverflowExpo) ||
+            (ri >= gs && ri < ge && (G.z * rr + G.s) * rr > kOverflowExpo))
+          lost = all;
+      }
+    }
+    if ((done | lost) != all && lv1 < T.s93.nlevels) {
 #pragma unroll
       for (int e = 0; e < NQ; e++) {
         state[U.qoff + e] = p[e];
@@ -686,23 +728,23 @@ __device__ __forceinline__ void type1_body(int bid, int nb, const DevTables &T, 
         state[2 * plane + U.qoff + e] = I[e];
       }
       qfail[u] = done;
-      // the entries still open, for a fallback that starts beside the tail
-      if (qopen) qopen[u] = all & ~done;
-      tq[atomicAdd(tcount, 1)] = u;
-      continue;
+      tq[queue_slot(tcount)] = u;
+      return;
     }
-    t1_finish<NQ>(u, U, p, done, qout, qfail, fbq, fbcount, fbflag);
+    t1_finish<NQ>(T, G, u, U, p, done, qout, qfail, fbq, fbcount);
   }
 }
 
-template <int LAB, int MODE>
-__global__ __launch_bounds__(64) void k_type1(DevTables T, DevJob J, const T1Unit *__restrict__ units, int nunits,
-                                              double *__restrict__ qout, unsigned long long *__restrict__ qfail,
-                                              int *__restrict__ fbq, int *__restrict__ fbcount, int head,
-                                              double *__restrict__ state, size_t plane, int *__restrict__ tq,
-                                              int *__restrict__ tcount, unsigned char *__restrict__ fbflag) {
-  type1_body<LAB, MODE>(blockIdx.x, gridDim.x, T, J, units, nunits, qout, qfail, fbq, fbcount, head, state, plane,
-                        tq, tcount, fbflag);
+// two waves per SIMD up to class 6 (256 registers), one above
+template <int LAB>
+__global__ __launch_bounds__(64, LAB <= 6 ? 2 : 1) void k_type1(DevTables T, DevJob J,
+                                                              const T1Unit *__restrict__ units, int nunits,
+                                                              double *__restrict__ qout,
+                                                              unsigned long long *__restrict__ qfail,
+                                                              int *__restrict__ fbq, int *__restrict__ fbcount,
+                                                              int head, double *__restrict__ state, size_t plane,
+                                                              int *__restrict__ tq, int *__restrict__ tcount) {
+  type1_body<LAB>(blockIdx.x, T, J, units, nunits, qout, qfail, fbq, fbcount, head, state, plane, tq, tcount);
 }
 
 // f + a[0] b[0] + a[sa] b[sb] + ... (n terms), accumulated in order; the
@@ -751,163 +793,6 @@ __device__ __forceinline__ double sum_in_order(double I, const double *v, int n)
   return I;
 }
 
-// Tail: one wave per primitive pair left open by the head, levels [head,
-// nlevels).  Lane k evaluates the k-th point pair of a round of levels (at
-// most 64 pairs per round; a level of the 383-point grid has at most 64) for
-// every Q entry and stores the pair sum T_k = (0 + f(left)) + f(right) in
-// LDS; lane e then adds each level's T_k
-// to its entry's I in pair order and applies the PS93 test, so the
-// arithmetic is that of the lane-serial integrator.
-constexpr int kTS = 65;  // LDS stride of the per-entry pair sums (bank spread)
-
-template <int LAB>
-__device__ __forceinline__ void t1tail_body(int bid, int nb, const DevTables &T, const DevJob &J,
-                                            const T1Unit *__restrict__ units, double *__restrict__ qout,
-                                            unsigned long long *__restrict__ qfail, int *__restrict__ fbq,
-                                            int *__restrict__ fbcount, int head, const double *__restrict__ state,
-                                            size_t plane, const int *__restrict__ tq, const int *__restrict__ tcount,
-                                            unsigned char *__restrict__ fbflag, double *s_T, bool spec = false) {
-  constexpr int NQ = nq_of(LAB);
-  static_assert(NQ <= 64, "one lane per Q entry");
-  const int count = *tcount;
-  const int lane = threadIdx.x;
-  for (int it = bid; it < count; it += nb) {
-    const int u = tq[it];
-    const T1Unit U = units[u];
-    const ecp_triplet tr = J.trip[U.trip];
-    const ecp_centre Cn = J.cent[tr.centre];
-    T1Geom G;
-    t1_geom(J, tr, U.pa, U.pb, G);
-    const double C0 = G.ca * G.cb * exp(G.zd2);
-    const double *__restrict__ UL = J.UL + Cn.UL_off;
-    const int gs = tr.gs, ge = tr.ge;
-    const double minExp = T.lnAcc1;
-    auto f = [&](int n, double (&acc)[NQ]) {
-      if (n < gs || n >= ge) return;
-      const double r = T.xs[n];
-      const double expo = (G.z * r + G.s) * r;
-      if (!(expo >= minExp)) return;
-      const double g = exp(expo);
-      double K[LAB + 1];
-      bessel_k<LAB>(T.bessel, G.s * r, K);
-      const double Un = UL[n], wn = T.ws[n];
-      double rn = 1.0;
-      int e = 0;
-#pragma unroll
-      for (int l1 = 0; l1 <= LAB; l1++) {
-        const double a = (C0 * rn) * Un;
-#pragma unroll
-        for (int l2 = l1; l2 >= 0; l2 -= 2, e++) acc[e] += wn * ((a * K[l2]) * g);
-        rn *= r;
-      }
-    };
-    const unsigned long long done0 = qfail[u];
-    double p = 0.0, q = 0.0, I = 0.0;
-    bool mydone = true;
-    if (lane < NQ) {
-      p = state[U.qoff + lane];
-      q = state[plane + U.qoff + lane];
-      I = state[2 * plane + U.qoff + lane];
-      mydone = (done0 >> lane) & 1ull;
-    }
-    // rounds of consecutive levels whose point pairs fit the wave together
-    // (levels 8-11: 48 pairs, 12-13: 64, 14: 64); the sums and tests then
-    // follow level by level, so only the evaluation is speculative
-    int lv = head;
-    while (lv < T.s93.nlevels) {
-      const int b0 = T.s93.lvl_begin[lv];
-      int l1 = lv + 1;
-      while (l1 < T.s93.nlevels && T.s93.lvl_begin[l1 + 1] - b0 <= 64) l1++;
-      const int tot = T.s93.lvl_begin[l1] - b0;
-      int cnt = 0;
-      if (lane < tot) {
-        const int li = T.p93l[b0 + lane], ri = T.p93r[b0 + lane];
-        double t[NQ];
-#pragma unroll
-        for (int e = 0; e < NQ; e++) t[e] = 0.0;
-        if (li >= gs) {
-          cnt++;
-          f(li, t);
-        }
-        if (ri <= ge) {
-          cnt++;
-          f(ri, t);
-        }
-#pragma unroll
-        for (int e = 0; e < NQ; e++) s_T[e * kTS + lane] = t[e];
-      }
-      const unsigned long long cmask = __ballot(cnt > 0);
-      __syncthreads();
-      bool stop = false;
-      for (int l = lv; l < l1; l++) {
-        const int o = T.s93.lvl_begin[l] - b0, np = T.s93.lvl_begin[l + 1] - T.s93.lvl_begin[l];
-        const unsigned long long lm = (np >= 64) ? ~0ull : (((1ull << np) - 1ull) << o);
-        const bool any = (cmask & lm) != 0ull;
-        if (lane < NQ) I = sum_in_order(I, s_T + lane * kTS + o, np);
-        if (!mydone) {
-          const int j = T.s93.lvl_j[l], nn = T.s93.lvl_n[l];
-          double err;
-          if (j == 0) {
-            p += (I - q);
-            err = 16 * fabs(q - 3 * p / 2) / (3 * nn);
-          } else {
-            err = 16 * fabs(I - 2 * q) / (3 * nn);
-            q = I;
-          }
-          if (any && err < T.tol) {
-            mydone = true;
-            p = 16 * q / (3 * nn);
-          }
-        }
-        if (!wave_any(!mydone)) {
-          stop = true;
-          break;
-        }
-      }
-      __syncthreads();
-      if (stop) break;
-      lv = l1;
-    }
-    if (lane < NQ) qout[U.qoff + lane] = mydone ? p : 0.0;
-    const unsigned long long failed = __ballot(lane < NQ && !mydone);
-    if (lane == 0) {
-      qfail[u] = failed;
-      if (failed) {
-        // spec: the fallback already runs over every unit of the tail
-        if (!spec) fbq[atomicAdd(fbcount, 1)] = u;
-        fbflag[U.trip] = 1;
-      }
-    }
-  }
-}
-
-template <int LAB>
-__global__ __launch_bounds__(64) void k_t1tail(DevTables T, DevJob J, const T1Unit *__restrict__ units,
-                                               double *__restrict__ qout, unsigned long long *__restrict__ qfail,
-                                               int *__restrict__ fbq, int *__restrict__ fbcount, int head,
-                                               const double *__restrict__ state, size_t plane,
-                                               const int *__restrict__ tq, const int *__restrict__ tcount,
-                                               unsigned char *__restrict__ fbflag) {
-  __shared__ double s_T[nq_of(LAB) * kTS];
-  t1tail_body<LAB>(blockIdx.x, gridDim.x, T, J, units, qout, qfail, fbq, fbcount, head, state, plane, tq, tcount,
-                   fbflag, s_T);
-}
-
-// FM06 linear map of the large grid for zeta_p, P (gc_integrators.c:316-331)
-struct Fm06 {
-  double i1, i2;
-};
-__device__ __forceinline__ Fm06 fm06(double zeta_p, double P) {
-  const double sigma = 1.0 / sqrt(zeta_p);
-  const double t = P - 7.0 * sigma;
-  const double rmin = (t > 0.0) ? t : 0.0;
-  const double rmax = P + 9.0 * sigma;
-  Fm06 m;
-  m.i1 = 0.5 * (rmax - rmin);
-  m.i2 = 0.5 * (rmax + rmin);
-  return m;
-}
-
 // Point of slot `lane` in a round of PSM92 point pairs [c0, c1): pair c0 +
 // lane / 2, left in even lanes, right in odd ones; in the first round (the
 // pairs of levels 1 to 5, 31 of them) the centre is in lane 62.  -1: none.
@@ -927,17 +812,6 @@ __device__ __forceinline__ double pair_sum(double v) {
   const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0xB1, 0xF, 0xF, true);
   const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0xB1, 0xF, 0xF, true);
   return v + __hiloint2double(hi, lo);
-}
-
-// The exponents of the three points of PSM92 levels 0 and 1 are all below
-// the numerical zero: every integral of the pair is then 0 at level 0 and
-// converges with the result 0 at level 1 (0 <= 0 in its test).
-template <typename Expo>
-__device__ __forceinline__ bool psm92_dead(const DevTables &T, const Fm06 &M, double minExp, Expo expo) {
-  if (T.s92.nlevels < 2) return false;
-  const double e0 = expo(M.i1 * T.xl[T.s92.centre] + M.i2), e1 = expo(M.i1 * T.xl[T.p92l[0]] + M.i2),
-               e2 = expo(M.i1 * T.xl[T.p92r[0]] + M.i2);
-  return !(e0 >= minExp) && !(e1 >= minExp) && !(e2 >= minExp);
 }
 
 // An integral's PSM92 state (gc_integrators.c:38-86)
@@ -969,141 +843,271 @@ struct Psm92 {
   }
 };
 
-// type-1 fallback (type1.c:205-252): one wave per primitive pair with failed
-// Q entries.  The wave's lanes evaluate the points of a round -- 31 point
+// type-1 fallback (type1.c:205-252) of one primitive pair with failed Q
+// entries (mask), by one wave: results to out.  The wave's lanes evaluate the points of a round -- 31 point
 // pairs and the centre (levels 0 to 5) together, then 32 pairs at a time --
 // and form each open entry's pair sums (0 + f(left)) + f(right), a pair per
 // two lanes, into LDS; lane e adds those of entry e in the integrator's
-// order and applies the PSM92 test after each level.  Pairs whose points
-// of levels 0 and 1 are all numerically zero end there.
+// order and applies the PSM92 test after each level.  (Pairs whose points
+// of levels 0 and 1 are all numerically zero do not come here: t1_fb_dead.)
 // The reference's screening break (type1.c:222-225: no points from the first
 // one beyond both centres whose exponent is below the cut-off) needs no
 // search: beyond both centres the exponent only decreases, so every point it
 // drops is below the cut-off and contributes 0 here by its own test.
 constexpr int kFbTS = 33;  // LDS stride of an entry's pair sums (at most 32 per round)
 
-template <int LAB, bool SPEC = false>
-__device__ __forceinline__ void fb1_body(int bid, int nb, const DevTables &T, const DevJob &J,
-                                         const T1Unit *__restrict__ units, double *__restrict__ qout,
-                                         const unsigned long long *__restrict__ qfail, const int *__restrict__ fbq,
-                                         const int *__restrict__ fbcount, unsigned char *__restrict__ status,
-                                         double *s_t, const int *__restrict__ tq = nullptr,
-                                         const int *__restrict__ tcount = nullptr,
-                                         const unsigned long long *__restrict__ qopen = nullptr,
-                                         double *__restrict__ qfb = nullptr,
-                                         unsigned long long *__restrict__ qfbf = nullptr) {
-  // SPEC (speculative): besides the units whose small-grid
-  // integrals failed (fbq), every unit the tail takes (tq), for the entries
-  // open after the head (qopen), started before the tail has decided them;
-  // results to qfb, large-grid failures as an entry mask to qfbf, and the
-  // assembly uses a result where the small grid failed
+template <int LAB>
+__device__ __forceinline__ void fb1_unit(const DevTables &T, const DevJob &J, const T1Unit &U, const ecp_triplet &tr,
+                                         int L, const T1Geom &G, unsigned long long mask, double *__restrict__ out,
+                                         unsigned char *__restrict__ status, double *s_t) {
   constexpr int NQ = nq_of(LAB);
-  const int n1 = *fbcount;
-  int count = n1;
-  if constexpr (SPEC) count += *tcount;
+  const int lane = threadIdx.x;
+  const double Cc = G.ca * G.cb;
+  const double zeta_p = G.za + G.zb;
+  const Fm06 M = fm06(zeta_p, (G.za * G.dAC + G.zb * G.dBC) / zeta_p);
+  const double minExp = T.lnAcc1;
+  auto expo_of = [&](double r) { return (G.z * r + G.s) * r + G.zd2; };
+  bool open = lane < NQ && ((mask >> lane) & 1ull);
+  Psm92 S{0.0, 0.0, 0.0};
+  double res = 0.0;
+      // rounds of point pairs [c0, c1): levels 0 to 5 first, then 32 pairs of
+      // level lv at a time
+      int lv = psm92_first(T), c0 = 0, c1 = T.s92.lvl_begin[lv];
+      for (;;) {
+        const bool first = c0 == 0;
+        const unsigned long long om = __ballot(open);
+        const int n = psm92_point(T, c0, c1, lane, first);
+        double w = 0.0, uu = 0.0, g = 0.0, r = 0.0;
+        double K[LAB + 1];
+  #pragma unroll
+        for (int l = 0; l <= LAB; l++) K[l] = 0.0;
+        if (n >= 0) {
+          r = M.i1 * T.xl[n] + M.i2;
+          const double expo = expo_of(r);
+          if (expo >= minExp) {
+            g = exp(expo);
+            bessel_k<LAB>(T.bessel, G.s * r, K);
+            uu = eval_ecp(J, tr.centre, L, r);
+            w = T.wl[n] * M.i1;
+          }
+        }
+        // the open entries' pair sums
+        double rn = 1.0;
+        int e = 0;
+  #pragma unroll
+        for (int l1 = 0; l1 <= LAB; l1++) {
+          const double a = (Cc * rn) * uu;
+  #pragma unroll
+          for (int l2 = l1; l2 >= 0; l2 -= 2, e++)
+            if ((om >> e) & 1ull) {
+              const double t = pair_sum(w * ((a * K[l2]) * g));
+              if (!(lane & 1)) s_t[e * kFbTS + (lane >> 1)] = t;
+            }
+          rn = r * rn;
+        }
+        __syncthreads();
+        const bool level_end = !first && c1 == T.s92.lvl_begin[lv + 1];
+        if (open) {
+          bool done;
+          if (first) {
+            done = S.first_round(T, s_t + lane * kFbTS, &res);
+          } else {
+            S.I = sum_in_order(S.I, s_t + lane * kFbTS, c1 - c0);
+            done = level_end && S.test(T, lv, &res);
+          }
+          if (done) {
+            out[lane] = res;
+            open = false;
+          }
+        }
+        __syncthreads();
+        lv += level_end;
+        if (lv >= T.s92.nlevels || !wave_any(open)) break;
+        if (first || level_end) S.step();
+        c0 = c1;
+        c1 = min(c0 + 32, T.s92.lvl_begin[lv + 1]);
+      }
+  if (open) status[2 * U.trip] = 1;
+}
+
+// Tail: one wave per primitive pair left open by the head, levels [head,
+// nlevels), in rounds of levels (at most 64 point pairs each; levels 5 to 11
+// have 58, 12 and 13, and 14, 64).  Lane k looks at the k-th pair's two
+// points; those inside the window whose exponent is above the cut-off -- a
+// third of them, a contiguous range of r -- are dealt to the lanes densely,
+// which evaluate them for every Q entry; the pair sums
+// T_k = (0 + f(left)) + f(right) form in LDS, and lane e then adds each
+// level's T_k to its entry's I in pair order and applies the PS93 test, so
+// the arithmetic is that of the lane-serial integrator.  Where a point's
+// exponent overflows, no entry can converge from its level on: nothing past
+// it is evaluated.  The wave then runs the large-grid fallback of the
+// entries that failed; the pairs that failed in the head (fbq) follow.
+constexpr int kTS = 65;  // LDS stride of the per-entry pair sums (bank spread)
+
+template <int LAB>
+__device__ __forceinline__ void t1tail_body(int bid, int nb, const DevTables &T, const DevJob &J,
+                                            const T1Unit *__restrict__ units, double *__restrict__ qout,
+                                            unsigned long long *__restrict__ qfail, const int *__restrict__ fbq,
+                                            const int *__restrict__ fbcount, int head,
+                                            const double *__restrict__ state, size_t plane,
+                                            const int *__restrict__ tq, const int *__restrict__ tcount,
+                                            unsigned char *__restrict__ status, double *s_T, int *s_pt) {
+  constexpr int NQ = nq_of(LAB);
+  static_assert(NQ <= 64, "one lane per Q entry");
+  const int ntail = *tcount, count = ntail + *fbcount;
   const int lane = threadIdx.x;
   for (int it = bid; it < count; it += nb) {
-    int u;
-    unsigned long long mask;
-    if (!SPEC || it < n1) {
-      u = fbq[it];
-      mask = qfail[u];
-    } else {
-      u = tq[it - n1];
-      mask = qopen[u];
-    }
+    const bool tail = it < ntail;
+    const int u = tail ? tq[it] : fbq[it - ntail];
     const T1Unit U = units[u];
     const ecp_triplet tr = J.trip[U.trip];
     const ecp_centre Cn = J.cent[tr.centre];
     T1Geom G;
     t1_geom(J, tr, U.pa, U.pb, G);
-    const double Cc = G.ca * G.cb;
-    const double zeta_p = G.za + G.zb;
-    const Fm06 M = fm06(zeta_p, (G.za * G.dAC + G.zb * G.dBC) / zeta_p);
+    const double C0 = G.ca * G.cb * exp(G.zd2);
+    const double *__restrict__ UL = J.UL + Cn.UL_off;
+    const int gs = tr.gs, ge = tr.ge;
     const double minExp = T.lnAcc1;
-    auto expo_of = [&](double r) { return (G.z * r + G.s) * r + G.zd2; };
-    double *out = (SPEC ? qfb : qout) + U.qoff;
-    bool open = lane < NQ && ((mask >> lane) & 1ull);
-    if (psm92_dead(T, M, minExp, expo_of)) {
-      if (open) out[lane] = 0.0;
-      if (SPEC && lane == 0) qfbf[u] = 0ull;
-      continue;
+    const unsigned long long done0 = qfail[u];
+    double p = 0.0, q = 0.0, I = 0.0;
+    bool mydone = true, lost = false;
+    if (tail && lane < NQ) {
+      p = state[U.qoff + lane];
+      q = state[plane + U.qoff + lane];
+      I = state[2 * plane + U.qoff + lane];
+      mydone = (done0 >> lane) & 1ull;
     }
-    Psm92 S{0.0, 0.0, 0.0};
-    double res = 0.0;
-    // rounds of point pairs [c0, c1): levels 0 to 5 first, then 32 pairs of
-    // level lv at a time
-    int lv = psm92_first(T), c0 = 0, c1 = T.s92.lvl_begin[lv];
-    for (;;) {
-      const bool first = c0 == 0;
-      const unsigned long long om = __ballot(open);
-      const int n = psm92_point(T, c0, c1, lane, first);
-      double w = 0.0, uu = 0.0, g = 0.0, r = 0.0;
-      double K[LAB + 1];
-#pragma unroll
-      for (int l = 0; l <= LAB; l++) K[l] = 0.0;
-      if (n >= 0) {
-        r = M.i1 * T.xl[n] + M.i2;
-        const double expo = expo_of(r);
-        if (expo >= minExp) {
-          g = exp(expo);
-          bessel_k<LAB>(T.bessel, G.s * r, K);
-          uu = eval_ecp(J, tr.centre, Cn.L, r);
-          w = T.wl[n] * M.i1;
-        }
+    int lv = tail ? head : T.s93.nlevels;
+    while (lv < T.s93.nlevels) {
+      const int b0 = T.s93.lvl_begin[lv];
+      int l1 = lv + 1;
+      while (l1 < T.s93.nlevels && T.s93.lvl_begin[l1 + 1] - b0 <= 64) l1++;
+      const int tot = T.s93.lvl_begin[l1] - b0;
+      // the lane's pair: which of its points count, contribute, overflow
+      bool in = false, liveL = false, liveR = false, over = false;
+      if (lane < tot) {
+        const int li = T.p93l[b0 + lane], ri = T.p93r[b0 + lane];
+        const double rl = T.xs[li], rr = T.xs[ri];
+        const double el = (G.z * rl + G.s) * rl, er = (G.z * rr + G.s) * rr;
+        in = li >= gs || ri <= ge;
+        liveL = li >= gs && li < ge && el >= minExp;
+        liveR = ri >= gs && ri < ge && er >= minExp;
+        over = (liveL && el > kOverflowExpo) || (liveR && er > kOverflowExpo);
       }
-      // the open entries' pair sums
-      double rn = 1.0;
-      int e = 0;
+      // levels [lv, ls) are evaluated: those before the first overflow
+      const unsigned long long ovm = __ballot(over);
+      int ls = l1;
+      if (ovm) {
+        const int k = __ffsll((long long)ovm) - 1;
+        ls = lv;
+        while (T.s93.lvl_begin[ls + 1] - b0 <= k) ls++;
+      }
+      if (ls > lv) {
+        const int ne = T.s93.lvl_begin[ls] - b0;
+        const unsigned long long cmask = __ballot(in);
+        const unsigned long long mL = __ballot(liveL && lane < ne), mR = __ballot(liveR && lane < ne);
+        const int nL = __popcll(mL), n = nL + __popcll(mR);
+        const unsigned long long below = (1ull << lane) - 1ull;
+        if ((mL >> lane) & 1ull) s_pt[__popcll(mL & below)] = lane;
+        if ((mR >> lane) & 1ull) s_pt[nL + __popcll(mR & below)] = lane | 64;
+        if (lane < ne)
 #pragma unroll
-      for (int l1 = 0; l1 <= LAB; l1++) {
-        const double a = (Cc * rn) * uu;
+          for (int e = 0; e < NQ; e++) s_T[e * kTS + lane] = 0.0;
+        __syncthreads();
+        // live points, the left ones first (at most 64 of them)
+        for (int b = 0; b < n; b += 64) {
+          const int j = b + lane;
+          int k = 0;
+          double t[NQ];
+          if (j < n) {
+            k = s_pt[j] & 63;
+            const int i = j < nL ? T.p93l[b0 + k] : T.p93r[b0 + k];
+            const double r = T.xs[i];
+            const double g = exp((G.z * r + G.s) * r);
+            double K[LAB + 1];
+            bessel_k<LAB>(T.bessel, G.s * r, K);
+            const double Un = UL[i], wn = T.ws[i];
+            double rn = 1.0;
+            int e = 0;
 #pragma unroll
-        for (int l2 = l1; l2 >= 0; l2 -= 2, e++)
-          if ((om >> e) & 1ull) {
-            const double t = pair_sum(w * ((a * K[l2]) * g));
-            if (!(lane & 1)) s_t[e * kFbTS + (lane >> 1)] = t;
+            for (int a1 = 0; a1 <= LAB; a1++) {
+              const double a = (C0 * rn) * Un;
+#pragma unroll
+              for (int a2 = a1; a2 >= 0; a2 -= 2, e++) t[e] = wn * ((a * K[a2]) * g);
+              rn *= r;
+            }
           }
-        rn = r * rn;
-      }
-      __syncthreads();
-      const bool level_end = !first && c1 == T.s92.lvl_begin[lv + 1];
-      if (open) {
-        bool done;
-        if (first) {
-          done = S.first_round(T, s_t + lane * kFbTS, &res);
-        } else {
-          S.I = sum_in_order(S.I, s_t + lane * kFbTS, c1 - c0);
-          done = level_end && S.test(T, lv, &res);
+          if (j < nL)
+#pragma unroll
+            for (int e = 0; e < NQ; e++) s_T[e * kTS + k] = 0.0 + t[e];
+          __syncthreads();
+          if (j >= nL && j < n)
+#pragma unroll
+            for (int e = 0; e < NQ; e++) s_T[e * kTS + k] += t[e];
+          __syncthreads();
         }
-        if (done) {
-          out[lane] = res;
-          open = false;
+        bool stop = false;
+        for (int l = lv; l < ls; l++) {
+          const int o = T.s93.lvl_begin[l] - b0, np = T.s93.lvl_begin[l + 1] - T.s93.lvl_begin[l];
+          const unsigned long long lm = (np >= 64) ? ~0ull : (((1ull << np) - 1ull) << o);
+          const bool any = (cmask & lm) != 0ull;
+          // the level's sums from its first pair with a live point on (the
+          // ones before it are 0)
+          const unsigned long long lp = (mL | mR) & lm;
+          if (lp && lane < NQ) {
+            const int k = __ffsll((long long)lp) - 1;
+            I = sum_in_order(I, s_T + lane * kTS + k, o + np - k);
+          }
+          if (!mydone) {
+            const int j = T.s93.lvl_j[l], nn = T.s93.lvl_n[l];
+            double err;
+            if (j == 0) {
+              p += (I - q);
+              err = 16 * fabs(q - 3 * p / 2) / (3 * nn);
+            } else {
+              err = 16 * fabs(I - 2 * q) / (3 * nn);
+              q = I;
+            }
+            if (any && err < T.tol) {
+              mydone = true;
+              p = 16 * q / (3 * nn);
+            } else {
+              lost = t1_lost(I);
+            }
+          }
+          if (!wave_any(!mydone && !lost)) {
+            stop = true;
+            break;
+          }
         }
+        __syncthreads();
+        if (stop) break;
       }
-      __syncthreads();
-      lv += level_end;
-      if (lv >= T.s92.nlevels || !wave_any(open)) break;
-      if (first || level_end) S.step();
-      c0 = c1;
-      c1 = min(c0 + 32, T.s92.lvl_begin[lv + 1]);
+      if (ls < l1) break;
+      lv = l1;
     }
-    if constexpr (SPEC) {
-      const unsigned long long failed = __ballot(open);
-      if (lane == 0) qfbf[u] = failed;
-    } else if (open) {
-      status[2 * U.trip] = 1;
+    unsigned long long failed = done0;  // of a pair that failed in the head
+    if (tail) {
+      if (lane < NQ) qout[U.qoff + lane] = mydone ? p : 0.0;
+      failed = __ballot(lane < NQ && !mydone);
+      if (lane == 0) qfail[u] = failed;
+      if (!failed || t1_fb_dead(T, G)) continue;
     }
+    fb1_unit<LAB>(T, J, U, tr, Cn.L, G, failed, qout + U.qoff, status, s_T);
   }
 }
 
 template <int LAB>
-__global__ __launch_bounds__(64) void k_fb1(DevTables T, DevJob J, const T1Unit *__restrict__ units,
-                                            double *__restrict__ qout, const unsigned long long *__restrict__ qfail,
-                                            const int *__restrict__ fbq, const int *__restrict__ fbcount,
-                                            unsigned char *__restrict__ status) {
-  __shared__ double s_t[nq_of(LAB) * kFbTS];
-  fb1_body<LAB>(blockIdx.x, gridDim.x, T, J, units, qout, qfail, fbq, fbcount, status, s_t);
+__global__ __launch_bounds__(64) void k_t1tail(DevTables T, DevJob J, const T1Unit *__restrict__ units,
+                                               double *__restrict__ qout, unsigned long long *__restrict__ qfail,
+                                               const int *__restrict__ fbq, const int *__restrict__ fbcount, int head,
+                                               const double *__restrict__ state, size_t plane,
+                                               const int *__restrict__ tq, const int *__restrict__ tcount,
+                                               unsigned char *__restrict__ status) {
+  __shared__ double s_T[nq_of(LAB) * kTS];
+  __shared__ int s_pt[128];
+  t1tail_body<LAB>(blockIdx.x, gridDim.x, T, J, units, qout, qfail, fbq, fbcount, head, state, plane, tq, tcount,
+                   status, s_T, s_pt);
 }
 
 // ---------------------------------------------------------------------------
@@ -1113,53 +1117,92 @@ struct T2Group {
   int trip, l, eoff, ne, tmpl, lmb;
 };
 
-__device__ __forceinline__ int find_group(const int *__restrict__ goff, int ng, int gid) {
-  int lo = 0, hi = ng;  // goff[lo] <= gid < goff[hi]
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (goff[mid] <= gid) lo = mid;
-    else hi = mid;
+struct T2Args {
+  const T2Group *groups;
+  const int *goff;
+  const int *gfirst;  // per wave of 64 entries: the group of its first entry (one more at the end)
+  int ngroups, ntotal;
+  const int *tmpl;
+  double *Tout;
+  unsigned char *tfail;
+  int *gflag, *fbq, *fbcount;  // fbq: per class, the triplets with failed entries (qstride apart)
+  int qstride;
+  int *flist;
+  int *tclaim;                  // per triplet: queued for the fallback
+  const unsigned char *tcls2;   // per triplet: its fallback class max(la, lb) + L - 1
+};
+
+// A failed entry, for the large-grid fallback: gflag[g] counts the group's
+// entries, listed (in any order) at flist[eoff ...]; the triplet's first one
+// queues the triplet, whose listed entries of all groups the fallback takes
+// together
+__device__ __forceinline__ void t2_enlist(const T2Args &A, int gid, int g, const T2Group &G) {
+  const int k = atomicAdd(&A.gflag[g], 1);
+  A.flist[G.eoff + k] = gid - G.eoff;
+  if (k == 0 && atomicExch(&A.tclaim[G.trip], 1) == 0) {
+    const int c = A.tcls2[G.trip];
+    const int slot = atomicAdd(&A.fbcount[c], 1);
+    A.fbq[(size_t)c * A.qstride + slot] = G.trip;
   }
-  return lo;
 }
 
-// One T entry: PS93 up to level lv_end (exclusive).  Returns 0 when it
-// converged (result in *res), 1 when every level ran without convergence,
-// 2 when it stopped unconverged at lv_end.
-__device__ __forceinline__ int t2_entry(const DevTables &T, const DevJob &J, const T2Group &G, int code, int lv_end,
-                                        double *res) {
+// v of lane (quad base + X) in all four lanes of each quad
+template <int X>
+__device__ __forceinline__ double quad_value(double v) {
+  constexpr int perm = X * 0x55;  // quad_perm [X, X, X, X]
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), perm, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), perm, 0xF, 0xF, true);
+  return __hiloint2double(hi, lo);
+}
+
+__device__ __forceinline__ double lane_get(double v, int src) {
+  return __hiloint2double(__shfl(__double2hiint(v), src, 64), __shfl(__double2loint(v), src, 64));
+}
+
+// Type-2 small grid: one wave per 64 T entries.  First a lane per entry runs
+// PS93 levels 0 to 4, eleven points whose reads are all issued before their
+// sums are formed: all but a few per cent of the entries converge there.
+// The few left are then dealt to the lanes four to an entry, sixteen entries
+// at a time: sixteen point pairs a step, four per lane with their reads
+// issued together, whose sums every lane of the quad adds in pair order with
+// the PS93 test at each level's end, so the arithmetic is that of the
+// lane-serial integrator.  (One lane per entry to the end, a straggler held
+// its wave for 372 more points read one level at a time: 107 us alone on the
+// 50-atom cluster, 3.4 ms on 256 uneven molecules.)
+constexpr int kT2Head = 5;  // levels of the first part
+
+struct T2Rows {
+  const double *Fa, *Fb, *Uu;
+  int pF, pU, gs, ge;
+};
+
+__device__ __forceinline__ T2Rows t2_rows(const DevJob &J, const T2Group &G, int code) {
   const int l1 = code & 0xff, l2 = (code >> 8) & 0xff, l3 = (code >> 16) & 0xff;
   const ecp_triplet tr = J.trip[G.trip];
-  const ecp_centre C = J.cent[tr.centre];
+  const ecp_centre *__restrict__ C = J.cent + tr.centre;
   // point and row strides of the F and U rows (layouts as the tables kernel writes them)
-  const int pF = J.ptmajor ? J.FL : 1, pU = J.ptmajor ? J.UK : 1, rs = J.ptmajor ? 1 : SO;
-  const double *__restrict__ Fa =
-      J.F + C.F_off + ((size_t)tr.powa * C.nsh + (tr.sa - C.shell0)) * J.FL * SO + (size_t)l1 * rs;
-  const double *__restrict__ Fb =
-      J.F + C.F_off + ((size_t)tr.powb * C.nsh + (tr.sb - C.shell0)) * J.FL * SO + (size_t)l2 * rs;
-  const double *__restrict__ Uu = J.Ut + C.Ut_off + (size_t)G.l * J.UK * SO + (size_t)l3 * rs;
-  const int gs = tr.gs, ge = tr.ge;
-  auto f = [&](int n) { return T.ws[n] * ((Fa[n * pF] * Fb[n * pF]) * Uu[n * pU]); };
-  double p = f(T.s93.centre);
-  double q = f(T.s93.first_l) + f(T.s93.first_r);
-  double I = p + q;
-  *res = 0.0;
-  for (int lv = 2; lv < lv_end; lv++) {
+  const int rs = J.ptmajor ? 1 : SO;
+  const int F_off = C->F_off, nsh = C->nsh, shell0 = C->shell0;
+  T2Rows R;
+  R.pF = J.ptmajor ? J.FL : 1;
+  R.pU = J.ptmajor ? J.UK : 1;
+  R.Fa = J.F + F_off + ((size_t)tr.powa * nsh + (tr.sa - shell0)) * J.FL * SO + (size_t)l1 * rs;
+  R.Fb = J.F + F_off + ((size_t)tr.powb * nsh + (tr.sb - shell0)) * J.FL * SO + (size_t)l2 * rs;
+  R.Uu = J.Ut + C->Ut_off + (size_t)G.l * J.UK * SO + (size_t)l3 * rs;
+  R.gs = tr.gs;
+  R.ge = tr.ge;
+  return R;
+}
+
+// integrator state of an entry after the first part
+struct T2State {
+  double p, q, I, res;
+  bool done;
+  // the PS93 recurrences and test after level lv (gc_integrators.c:156-217);
+  // any: the level had a point in the window
+  __device__ __forceinline__ void level(const DevTables &T, int lv, bool any) {
+    if (done) return;
     const int j = T.s93.lvl_j[lv], nn = T.s93.lvl_n[lv];
-    int cnt = 0;
-    for (int k = T.s93.lvl_begin[lv]; k < T.s93.lvl_begin[lv + 1]; k++) {
-      const int li = T.p93l[k], ri = T.p93r[k];
-      double t = 0.0;
-      if (li >= gs) {
-        cnt++;
-        t += f(li);
-      }
-      if (ri <= ge) {
-        cnt++;
-        t += f(ri);
-      }
-      I += t;
-    }
     double err;
     if (j == 0) {
       p += (I - q);
@@ -1168,162 +1211,184 @@ __device__ __forceinline__ int t2_entry(const DevTables &T, const DevJob &J, con
       err = 16 * fabs(I - 2 * q) / (3 * nn);
       q = I;
     }
-    if (cnt > 0 && err < T.tol) {
-      *res = 16 * q / (3 * nn);
-      return 0;
+    if (any && err < T.tol) {
+      res = 16 * q / (3 * nn);
+      done = true;
     }
   }
-  return lv_end < T.s93.nlevels ? 2 : 1;
-}
-
-struct T2Args {
-  const T2Group *groups;
-  const int *goff;
-  int ngroups, ntotal;
-  const int *tmpl;
-  double *Tout;
-  unsigned char *tfail;
-  int *gflag, *fbq, *fbcount;  // fbq: per class, the triplets with failed entries (qstride apart)
-  int qstride;
-  unsigned char *fbflag;
-  int *flist;
-  int *tq, *tcount;  // entries left open by the head
-  int *tclaim;                  // per triplet: queued for the fallback
-  const unsigned char *tcls2;   // per triplet: its fallback class max(la, lb) + L - 1
-  int spec;                     // the fallback takes every entry the head leaves open
-  unsigned char *fbf2;          // spec: per entry, the fallback failed on the large grid
 };
 
-// An entry for the large-grid fallback: gflag[g] counts the group's
-// entries, listed (in any order) at flist[eoff ...]; the triplet's first one
-// queues the triplet, whose listed entries of all groups the fallback takes
-// together
-__device__ __forceinline__ void t2_enlist(const T2Args &A, int gid, int g, const T2Group &G) {
-  // the speculative fallback's failure flag of the entry, read only for
-  // enlisted entries: cleared here, before the fallback runs
-  if (A.spec) A.fbf2[gid] = 0;
-  const int k = atomicAdd(&A.gflag[g], 1);
-  A.flist[G.eoff + k] = gid - G.eoff;
-  if (k == 0 && atomicExch(&A.tclaim[G.trip], 1) == 0) {
-    const int c = A.tcls2[G.trip];
-    const int slot = atomicAdd(&A.fbcount[c], 1);
-    A.fbq[(size_t)c * A.qstride + slot] = G.trip;
-    A.fbflag[G.trip] = 1;
-  }
-}
-
-// A decided entry: its small-grid result and failure flag; a failed entry
-// goes to the fallback, unless the fallback already took it speculatively
-__device__ __forceinline__ void t2_store(const T2Args &A, int gid, int g, const T2Group &G, int st, double res) {
-  A.Tout[gid] = res;
-  A.tfail[gid] = st == 0 ? 0 : 1;
-  if (st != 0 && !A.spec) t2_enlist(A, gid, g, G);
-}
-
-// One lane per T entry.  With head < the level count, entries still open
-// after `head` levels are queued instead for k_type2_tail, so that the few
-// stragglers neither hold a wave of converged lanes nor run their remaining
-// levels one point at a time.
-__global__ __launch_bounds__(128) void k_type2(DevTables T, DevJob J, T2Args A, int head) {
-  const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= A.ntotal) return;
-  const int g = find_group(A.goff, A.ngroups, gid);
-  const T2Group G = A.groups[g];
-  const int code = A.tmpl[G.tmpl + (gid - G.eoff)];
-  double res;
-  const int st = t2_entry(T, J, G, code, min(head, T.s93.nlevels), &res);
-  if (st == 2) {
-    A.tq[atomicAdd(A.tcount, 1)] = gid;
-    if (A.spec) t2_enlist(A, gid, g, G);
-    return;
-  }
-  t2_store(A, gid, g, G, st, res);
-}
-
-// Tail: the entries left open by the head, rerun whole by kT2Group lanes
-// each (64 / kT2Group entries per wave).  Per level the group's lanes form
-// the point-pair sums T_k = (0 + f(left)) + f(right) into LDS and the
-// group's first lane adds them to I in pair order and applies the PS93 test,
-// so the arithmetic is that of the lane-serial integrator.
-constexpr int kT2Group = 4;
-
-__global__ __launch_bounds__(64) void k_type2_tail(DevTables T, DevJob J, T2Args A) {
-  constexpr int NE = 64 / kT2Group;
-  __shared__ double s_t[NE][64];
-  __shared__ int s_done[NE];
-  const int lane = threadIdx.x, e = lane / kT2Group, r = lane % kT2Group;
-  const int count = *A.tcount;
-  for (int it0 = blockIdx.x * NE; it0 < count; it0 += gridDim.x * NE) {
-    const int it = it0 + e;
-    const bool live = it < count;
-    int gid = 0, g = 0, code = 0;
-    T2Group G{};
-    if (live) {
-      gid = A.tq[it];
-      g = find_group(A.goff, A.ngroups, gid);
-      G = A.groups[g];
-      code = A.tmpl[G.tmpl + (gid - G.eoff)];
+__device__ __forceinline__ void type2_body(int bid, const DevTables &T, const DevJob &J, const T2Args &A, int *s_off,
+                                           int *s_open) {
+  const int lane = threadIdx.x;
+  const int gid = bid * 64 + lane;
+  // the wave's groups: at most 64 from gfirst on
+  const int g0 = A.gfirst[bid];
+  s_off[lane] = g0 + 1 + lane <= A.ngroups ? A.goff[g0 + 1 + lane] : INT_MAX;
+  __syncthreads();
+  const bool live = gid < A.ntotal;
+  int g = 0;
+  {
+    // the number of following groups that start at or before this entry
+    int lo = 0, hi = 64;
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (s_off[mid] <= gid) lo = mid + 1;
+      else hi = mid;
     }
-    const int l1 = code & 0xff, l2 = (code >> 8) & 0xff, l3 = (code >> 16) & 0xff;
-    const ecp_triplet tr = J.trip[G.trip];
-    const ecp_centre C = J.cent[tr.centre];
-    // point and row strides of the F and U rows (layouts as the tables kernel writes them)
-    const int pF = J.ptmajor ? J.FL : 1, pU = J.ptmajor ? J.UK : 1, rs = J.ptmajor ? 1 : SO;
-    const double *__restrict__ Fa =
-        J.F + C.F_off + ((size_t)tr.powa * C.nsh + (tr.sa - C.shell0)) * J.FL * SO + (size_t)l1 * rs;
-    const double *__restrict__ Fb =
-        J.F + C.F_off + ((size_t)tr.powb * C.nsh + (tr.sb - C.shell0)) * J.FL * SO + (size_t)l2 * rs;
-    const double *__restrict__ Uu = J.Ut + C.Ut_off + (size_t)G.l * J.UK * SO + (size_t)l3 * rs;
-    const int gs = tr.gs, ge = tr.ge;
-    auto f = [&](int n) { return T.ws[n] * ((Fa[n * pF] * Fb[n * pF]) * Uu[n * pU]); };
-    double p = 0.0, q = 0.0, I = 0.0, res = 0.0;
-    bool done = !live;
-    if (live && r == 0) {
-      p = f(T.s93.centre);
-      q = f(T.s93.first_l) + f(T.s93.first_r);
-      I = p + q;
+    g = g0 + lo;
+  }
+  T2Group G{};
+  int code = 0;
+  T2State S{0.0, 0.0, 0.0, 0.0, true};
+  if (live) {
+    G = A.groups[g];
+    code = A.tmpl[G.tmpl + (gid - G.eoff)];
+    const T2Rows R = t2_rows(J, G, code);
+    constexpr int NP = 4;  // point pairs of levels 2 to 4
+    double fa[2 * NP + 3], fb[2 * NP + 3], fu[2 * NP + 3];
+    const int n0[3] = {T.s93.centre, T.s93.first_l, T.s93.first_r};
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+      fa[i] = R.Fa[n0[i] * R.pF];
+      fb[i] = R.Fb[n0[i] * R.pF];
+      fu[i] = R.Uu[n0[i] * R.pU];
     }
-    int st = 1;
-    for (int lv = 2; lv < T.s93.nlevels; lv++) {
-      if (!wave_any(!done)) break;
-      const int b0 = T.s93.lvl_begin[lv], np = T.s93.lvl_begin[lv + 1] - b0;
-      if (!done)
-        for (int k = r; k < np; k += kT2Group) {
-          const int li = T.p93l[b0 + k], ri = T.p93r[b0 + k];
-          double t = 0.0;
-          if (li >= gs) t += f(li);
-          if (ri <= ge) t += f(ri);
-          s_t[e][k] = t;
-        }
-      __syncthreads();
-      if (!done && r == 0) {
-        int cnt = 0;
-        for (int k = 0; k < np; k++) {
-          cnt += (T.p93l[b0 + k] >= gs) + (T.p93r[b0 + k] <= ge);
-          I += s_t[e][k];
-        }
-        const int j = T.s93.lvl_j[lv], nn = T.s93.lvl_n[lv];
-        double err;
-        if (j == 0) {
-          p += (I - q);
-          err = 16 * fabs(q - 3 * p / 2) / (3 * nn);
-        } else {
-          err = 16 * fabs(I - 2 * q) / (3 * nn);
-          q = I;
-        }
-        if (cnt > 0 && err < T.tol) {
-          res = 16 * q / (3 * nn);
-          st = 0;
-          done = true;
-        }
-        s_done[e] = done;
+#pragma unroll
+    for (int k = 0; k < NP; k++) {
+      const int li = T.p93l[k], ri = T.p93r[k], i = 3 + 2 * k;
+      fa[i] = fb[i] = fu[i] = fa[i + 1] = fb[i + 1] = fu[i + 1] = 0.0;
+      if (li >= R.gs) {
+        fa[i] = R.Fa[li * R.pF];
+        fb[i] = R.Fb[li * R.pF];
+        fu[i] = R.Uu[li * R.pU];
       }
-      __syncthreads();
-      done = s_done[e] || !live;
-      __syncthreads();
+      if (ri <= R.ge) {
+        fa[i + 1] = R.Fa[ri * R.pF];
+        fb[i + 1] = R.Fb[ri * R.pF];
+        fu[i + 1] = R.Uu[ri * R.pU];
+      }
     }
-    if (live && r == 0) t2_store(A, gid, g, G, st, res);
+    auto f = [&](int i, int n) { return T.ws[n] * ((fa[i] * fb[i]) * fu[i]); };
+    S.p = f(0, n0[0]);
+    S.q = f(1, n0[1]) + f(2, n0[2]);
+    S.I = S.p + S.q;
+    S.done = false;
+    int k = 0;
+    bool any = false;
+#pragma unroll
+    for (int lv = 2; lv < kT2Head; lv++) {
+      any = false;
+#pragma unroll
+      for (int x = 0; x < (lv == 4 ? 2 : 1); x++, k++) {
+        const int li = T.p93l[k], ri = T.p93r[k], i = 3 + 2 * k;
+        any = any || li >= R.gs || ri <= R.ge;
+        S.I += (0.0 + f(i, li)) + f(i + 1, ri);
+      }
+      S.level(T, lv, any);
+    }
   }
+  // the entries still open, four lanes each
+  unsigned long long failed = 0ull;
+  const unsigned long long om = __ballot(!S.done);
+  const int nopen = __popcll(om);
+  if (nopen) {
+    if (!S.done) s_open[__popcll(om & ((1ull << lane) - 1ull))] = lane;
+    __syncthreads();
+    const int r = lane & 3;
+    for (int o0 = 0; o0 < nopen; o0 += 16) {
+      const int oi = o0 + (lane >> 2);
+      const bool on = oi < nopen;
+      const int src = on ? s_open[oi] : s_open[o0];
+      T2State Q{lane_get(S.p, src), lane_get(S.q, src), lane_get(S.I, src), 0.0, !on};
+      T2Group Gq;
+      Gq.trip = __shfl(G.trip, src, 64);
+      Gq.l = __shfl(G.l, src, 64);
+      const T2Rows R = t2_rows(J, Gq, __shfl(code, src, 64));
+      // steps of 16 pairs, c0 + 4 i + x in lane x of the quad; the points of
+      // the next step are read ahead
+      const int np = T.s93.npairs;
+      int lv = kT2Head, c0 = T.s93.lvl_begin[kT2Head];
+      int li[4], ri[4];
+      auto points = [&](int b) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int k = min(b + 4 * i + r, np - 1);
+          li[i] = T.p93l[k];
+          ri[i] = T.p93r[k];
+        }
+      };
+      points(c0);
+      for (; c0 < np; c0 += 16) {
+        if (!wave_any(!Q.done)) break;
+        double t[4];
+        {
+          double fa[8], fb[8], fu[8], w[8];
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            fa[2 * i] = fb[2 * i] = fu[2 * i] = w[2 * i] = 0.0;
+            fa[2 * i + 1] = fb[2 * i + 1] = fu[2 * i + 1] = w[2 * i + 1] = 0.0;
+            if (!Q.done && li[i] >= R.gs) {
+              w[2 * i] = T.ws[li[i]];
+              fa[2 * i] = R.Fa[li[i] * R.pF];
+              fb[2 * i] = R.Fb[li[i] * R.pF];
+              fu[2 * i] = R.Uu[li[i] * R.pU];
+            }
+            if (!Q.done && ri[i] <= R.ge) {
+              w[2 * i + 1] = T.ws[ri[i]];
+              fa[2 * i + 1] = R.Fa[ri[i] * R.pF];
+              fb[2 * i + 1] = R.Fb[ri[i] * R.pF];
+              fu[2 * i + 1] = R.Uu[ri[i] * R.pU];
+            }
+          }
+          points(c0 + 16);
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+            t[i] = (0.0 + w[2 * i] * ((fa[2 * i] * fb[2 * i]) * fu[2 * i])) +
+                   w[2 * i + 1] * ((fa[2 * i + 1] * fb[2 * i + 1]) * fu[2 * i + 1]);
+        }
+        // the pairs of this step that end a level
+        unsigned int ends = 0;
+        for (int x = lv; x < T.s93.nlevels && T.s93.lvl_begin[x + 1] <= c0 + 16; x++)
+          ends |= 1u << (T.s93.lvl_begin[x + 1] - 1 - c0);
+        // (past the last pair, nothing ends and nothing reads the sums.)
+        // The last pair of a level is its closest to the centre: the level
+        // has a point in the window where this pair does.
+        auto add = [&](int j, double v) {
+          Q.I += v;
+          if ((ends >> j) & 1u) {
+            Q.level(T, lv, T.p93l[c0 + j] >= R.gs || T.p93r[c0 + j] <= R.ge);
+            lv++;
+          }
+        };
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          add(4 * i, quad_value<0>(t[i]));
+          add(4 * i + 1, quad_value<1>(t[i]));
+          add(4 * i + 2, quad_value<2>(t[i]));
+          add(4 * i + 3, quad_value<3>(t[i]));
+        }
+      }
+      // back to the entries' own lanes
+      const int mine = __popcll(om & ((1ull << lane) - 1ull)) - o0;
+      const bool back = !S.done && mine >= 0 && mine < 16;
+      const int from = back ? 4 * mine : 0;
+      const double res = lane_get(Q.res, from);
+      const int ok = __shfl((int)Q.done, from, 64);
+      if (back) S.res = res;
+      failed |= __ballot(back && !ok);
+    }
+  }
+  if (!live) return;
+  const bool fail = (failed >> lane) & 1ull;
+  A.Tout[gid] = S.res;
+  A.tfail[gid] = fail;
+  if (fail) t2_enlist(A, gid, g, G);
+}
+
+__global__ __launch_bounds__(64) void k_type2(DevTables T, DevJob J, T2Args A) {
+  __shared__ int s_off[64], s_open[64];
+  type2_body(blockIdx.x, T, J, A, s_off, s_open);
 }
 
 // type-2 fallback (calcT_FM06, type2.c:417-528): one wave per (triplet with
@@ -1358,8 +1423,7 @@ __device__ __forceinline__ void fb2_body(int bid, int nb, const DevTables &T, co
                                          double *__restrict__ fbT, unsigned char *__restrict__ status,
                                          const int *__restrict__ gcount, const int *__restrict__ flist,
                                          const int *__restrict__ tgfirst, int nslot, int nsplit, int share, double *s_cu,
-                                         double *s_rn, double *s_ka, double *s_kb, double *s_t,
-                                         unsigned char *__restrict__ fbf2) {
+                                         double *s_rn, double *s_ka, double *s_kb, double *s_t) {
   const int lane = threadIdx.x;
   const int count = *fbcount;
   // items (split, slot, triplet): split k takes the k-th share of the entries
@@ -1565,9 +1629,7 @@ __device__ __forceinline__ void fb2_body(int bid, int nb, const DevTables &T, co
           }
 #pragma unroll
           for (int i = 0; i < OWN; i++) {
-            if (!open[i]) continue;
-            if (fbf2) fbf2[eo[i]] = 1;
-            else status[2 * t + 1] = 1;
+            if (open[i]) status[2 * t + 1] = 1;
           }
         }
       }
@@ -1602,29 +1664,25 @@ struct T1Set {
   int *fbq, *fbc, *tq;
   double *st;
   size_t plane;
-  unsigned char *stat, *fbflag;
+  unsigned char *stat;
   int ubeg[ECP_MAX_LAB + 1], ucnt[ECP_MAX_LAB + 1];
-  int head[ECP_MAX_LAB + 1];  // PS93 levels of the head per class (>= the level count: no tail)
-  // speculative fallback (nullptr: off): open entries after the head, the
-  // fallback's results and its failed-entry masks
-  unsigned long long *qopen, *qfbf;
-  double *qfb;
+  int head;  // PS93 levels of the head (>= the level count: no tail)
 };
 
 #define ECP_CASES_LAB(X) X(0) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12)
 #define ECP_CASES_LMB(X) X(0) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12)
 
-template <int MAXLAB, int MODE>
-__global__ __launch_bounds__(64) void k_type1_fused(DevTables T, DevJob J, T1Set S, ClassMap cm) {
+template <int MAXLAB>
+__global__ __launch_bounds__(64, MAXLAB <= 6 ? 2 : 1) void k_type1_fused(DevTables T, DevJob J, T1Set S, ClassMap cm) {
   const int i = class_entry(cm, blockIdx.x);
-  const int c = cm.cls[i], bid = blockIdx.x - cm.bbeg[i], nb = cm.bbeg[i + 1] - cm.bbeg[i];
+  const int c = cm.cls[i], bid = blockIdx.x - cm.bbeg[i];
   const int ub = S.ubeg[c];
   switch (c) {
-#define X(L)                                                                                                   \
-  case L:                                                                                                      \
-    if constexpr (L <= MAXLAB)                                                                                 \
-      type1_body<L, MODE>(bid, nb, T, J, S.units + ub, S.ucnt[c], S.q, S.qf + ub, S.fbq + ub, S.fbc + c, S.head[c], \
-                          S.st, S.plane, S.tq + ub, S.fbc + 32 + c, S.fbflag, S.qopen ? S.qopen + ub : nullptr); \
+#define X(L)                                                                                                     \
+  case L:                                                                                                        \
+    if constexpr (L <= MAXLAB)                                                                                   \
+      type1_body<L>(bid, T, J, S.units + ub, S.ucnt[c], S.q, S.qf + ub, S.fbq + ub, S.fbc + c, S.head, S.st,     \
+                    S.plane, S.tq + ub, S.fbc + 32 + c);                                                         \
     break;
     ECP_CASES_LAB(X)
 #undef X
@@ -1634,24 +1692,7 @@ __global__ __launch_bounds__(64) void k_type1_fused(DevTables T, DevJob J, T1Set
 template <int MAXLAB>
 __global__ __launch_bounds__(64) void k_t1tail_fused(DevTables T, DevJob J, T1Set S, ClassMap cm) {
   __shared__ double s_T[nq_of(MAXLAB) * kTS];
-  const int i = class_entry(cm, blockIdx.x);
-  const int c = cm.cls[i], bid = blockIdx.x - cm.bbeg[i], nb = cm.bbeg[i + 1] - cm.bbeg[i];
-  const int ub = S.ubeg[c];
-  switch (c) {
-#define X(L)                                                                                                   \
-  case L:                                                                                                      \
-    if constexpr (L <= MAXLAB)                                                                                 \
-      t1tail_body<L>(bid, nb, T, J, S.units + ub, S.q, S.qf + ub, S.fbq + ub, S.fbc + c, S.head[c], S.st, S.plane, \
-                     S.tq + ub, S.fbc + 32 + c, S.fbflag, s_T, S.qfb != nullptr);                                \
-    break;
-    ECP_CASES_LAB(X)
-#undef X
-  }
-}
-
-template <int MAXLAB, bool SPEC>
-__global__ __launch_bounds__(64) void k_fb1_fused(DevTables T, DevJob J, T1Set S, ClassMap cm) {
-  __shared__ double s_t[nq_of(MAXLAB) * kFbTS];
+  __shared__ int s_pt[128];
   const int i = class_entry(cm, blockIdx.x);
   const int c = cm.cls[i], bid = blockIdx.x - cm.bbeg[i], nb = cm.bbeg[i + 1] - cm.bbeg[i];
   const int ub = S.ubeg[c];
@@ -1659,8 +1700,8 @@ __global__ __launch_bounds__(64) void k_fb1_fused(DevTables T, DevJob J, T1Set S
 #define X(L)                                                                                                     \
   case L:                                                                                                        \
     if constexpr (L <= MAXLAB)                                                                                   \
-      fb1_body<L, SPEC>(bid, nb, T, J, S.units + ub, S.q, S.qf + ub, S.fbq + ub, S.fbc + c, S.stat, s_t, S.tq + ub, \
-                        S.fbc + 32 + c, SPEC ? S.qopen + ub : nullptr, S.qfb, SPEC ? S.qfbf + ub : nullptr);     \
+      t1tail_body<L>(bid, nb, T, J, S.units + ub, S.q, S.qf + ub, S.fbq + ub, S.fbc + c, S.head, S.st, S.plane,  \
+                     S.tq + ub, S.fbc + 32 + c, S.stat, s_T, s_pt);                                              \
     break;
     ECP_CASES_LAB(X)
 #undef X
@@ -1678,7 +1719,6 @@ struct T2Set {
   const int *gcount, *flist, *tgfirst;
   int nslot, nsplit, share;
   int cu_rows, rn_rows, k_rows;  // LDS rows: U_l of the job's channels, powers of r, K of its largest class
-  unsigned char *fbf2;  // speculative fallback: per entry, the large grid failed (nullptr: off)
 };
 
 // two entries per lane where registers set the waves per SIMD (three), four
@@ -1697,7 +1737,7 @@ __global__ __launch_bounds__(64, MAXLMB <= 7 ? 3 : 2) void k_fb2_fused(DevTables
   case L:                                                                                                        \
     if constexpr (L <= MAXLMB)                                                                                   \
       fb2_body<L, OWN>(bid, nb, T, J, S.groups, S.tmpl, S.fbq2 + (size_t)L * S.nt, S.fbc + kFb2Cnt + L, S.fbT, S.stat, \
-                  S.gcount, S.flist, S.tgfirst, S.nslot, S.nsplit, S.share, s_cu, s_rn, s_ka, s_kb, s_t, S.fbf2); \
+                  S.gcount, S.flist, S.tgfirst, S.nslot, S.nsplit, S.share, s_cu, s_rn, s_ka, s_kb, s_t);         \
     break;
     ECP_CASES_LMB(X)
 #undef X
@@ -1720,7 +1760,6 @@ struct AsmArgs {
   const int *tmpl;
   const double *Tout;
   const unsigned char *tfail;
-  const unsigned char *fbf2;  // speculative type-2 fallback: per entry, the large grid failed (nullptr: off)
   const double *fbT;
   const double *fac, *dfac;
   double *blocks;
@@ -1730,11 +1769,6 @@ struct AsmArgs {
   int lds_S1, lds_S2, shift_lm;  // shift factor tables (aliasing rsph/Q resp. T) for shells up to shift_lm
   const double *udir;             // type 1: per unit, cos theta, phi, sin phi, cos phi of its pair direction
   int lds_group;                  // packed type-1 assembly: LDS doubles per triplet
-  // speculative type-1 fallback (qfb != nullptr): an entry whose small grid
-  // failed (qfail bit) takes the fallback's result qfb; the triplet failed
-  // where the fallback failed too (qfbf bit)
-  const unsigned long long *qfail, *qfbf;
-  const double *qfb;
 };
 
 // binomial shift of a block over C-centred monomials to the IJK(la) x IJK(lb)
@@ -1912,9 +1946,8 @@ __device__ __forceinline__ double asm1_monomial(double acc, const double *__rest
 // here.
 template <int G = 1, int MAXD = 6>
 __global__ __launch_bounds__(kAsmThreads, 3) void k_asm1(DevTables T, DevJob J, AsmArgs A,
-                                                      unsigned char *__restrict__ status,
-                                                      const int *__restrict__ tlist, int ntl,
-                                                      const unsigned char *__restrict__ fbflag, int filter) {
+                                                      const unsigned char *__restrict__ status,
+                                                      const int *__restrict__ tlist, int ntl) {
   extern __shared__ double lds_all[];
   constexpr int W = kAsmThreads / G;
   const int grp = G == 1 ? 0 : (int)threadIdx.x / W;
@@ -1928,44 +1961,18 @@ __global__ __launch_bounds__(kAsmThreads, 3) void k_asm1(DevTables T, DevJob J, 
   bool active = true;
   if constexpr (G == 1) {
     t = tlist[blockIdx.x];
-    // filter 1: only triplets without large-grid work, 2: only those with it
-    if ((filter == 1 && fbflag[t]) || (filter == 2 && !fbflag[t])) return;
     if (status[2 * t]) return;
   } else {
     const int ti = blockIdx.x * G + grp;
     active = ti < ntl;
     t = active ? tlist[ti] : tlist[0];
-    if (active && ((filter == 1 && fbflag[t]) || (filter == 2 && !fbflag[t]) || status[2 * t])) active = false;
+    if (active && status[2 * t]) active = false;
     if (!wave_any(active)) return;
   }
   const ecp_triplet tr = J.trip[t];
   const ecp_centre Cn = J.cent[tr.centre];
   const ecp_shell Sa = J.shells[tr.sa], Sb = J.shells[tr.sb];
   const int la = tr.la, lb = tr.lb, lab = la + lb;  // shifted for derivatives
-  if (A.qfb) {
-    // speculative fallback: an integral failed where the small grid and
-    // the large grid both failed (type1.c:182-190, code 1)
-    bool bad = false;
-    if (active)
-      for (int k = lid; k < Sa.K * Sb.K; k += W) {
-        const int ug = A.t1first[t] + k;
-        bad = bad || (A.qfail[ug] & A.qfbf[ug]) != 0ull;
-      }
-    if constexpr (G == 1) {
-      if (wave_any(bad)) {
-        if (lid == 0) status[2 * t] = 1;
-        return;
-      }
-    } else {
-      // the decision of the lane group's W lanes
-      const unsigned long long m = __ballot(bad);
-      if ((m >> (grp * W)) & ((1ull << W) - 1ull)) {
-        if (lid == 0) status[2 * t] = 1;
-        active = false;
-      }
-      if (!wave_any(active)) return;
-    }
-  }
   const ecp_xyz rc = J.atoms[Cn.atom], ra = J.atoms[Sa.atom], rb = J.atoms[Sb.atom];
   const V3 vA{ra.x - rc.x, ra.y - rc.y, ra.z - rc.z}, vB{rb.x - rc.x, rb.y - rc.y, rb.z - rc.z};
   const int D = T.ijkDim;
@@ -1992,9 +1999,7 @@ __global__ __launch_bounds__(kAsmThreads, 3) void k_asm1(DevTables T, DevJob J, 
     }
     for (int it = lid; it < nc * nql; it += W) {
       const int k = it / nql, e = it - k * nql;
-      const int ug = u0 + c0 + k;
-      const int qo = A.units1[ug].qoff + e;
-      Qs[k * nql + e] = (A.qfb && ((A.qfail[ug] >> e) & 1ull)) ? A.qfb[qo] : A.qout[qo];
+      Qs[k * nql + e] = A.qout[A.units1[u0 + c0 + k].qoff + e];
     }
     __syncthreads();
     for (int p = lid; p < np; p += W) {
@@ -2041,28 +2046,113 @@ __global__ __launch_bounds__(kAsmThreads, 3) void k_asm1(DevTables T, DevJob J, 
                 active);
 }
 
+// degree of the C-centred monomial at ordering position p (l <= 6)
+__device__ __forceinline__ int deg_of(int p) {
+  return (p >= 1) + (p >= 4) + (p >= 10) + (p >= 20) + (p >= 35) + (p >= 56);
+}
+
+// One channel's part of a type-2 block (type2.c:583-623): for the elements
+// (pp, qq) of the lanes lid, lid + nlanes, ... the sum over lambda1 and
+// lambda2 of (sum_m A[lambda1][m][pp] B[lambda2][m][qq]) T[lambda1][lambda2],
+// added to blk.  The channel is a template argument, so that its 2 l + 1
+// factors and its at most (NB - 1 + l) / 2 + 1 values of lambda2 are the
+// only ones in the code: with both padded to the largest channel's, the
+// kernel's time was that of instructions for absent values.
+// NB > 0 (basis l < NB): the angular factors of atom B for every lambda2 in
+// registers, those of atom A per lambda1; NB = 0: both read for each pair.
+template <int NB, int L>
+__device__ __forceinline__ void asm2_channel(const double *__restrict__ angA, const double *__restrict__ angB,
+                                             int ang_c, int nlm2, const double *Tl, int la, int lb, int nca, int ncb,
+                                             float inv_ncb, double *blk, int lid, int nlanes) {
+  constexpr int NM = 2 * L + 1;
+  constexpr int NBL = NB == 0 ? 1 : (NB - 1 + L) / 2 + 1 < NB ? (NB - 1 + L) / 2 + 1 : NB;
+  const int d2 = lb + L + 1, d3 = la + lb + 1;
+  const size_t lam_stride = (size_t)nlm2 * ang_c;
+  for (int idx = lid; idx < nca * ncb; idx += nlanes) {
+    const int pp = (int)(((float)idx + 0.5f) * inv_ncb), qq = idx - pp * ncb;
+    const int alpha = deg_of(pp), beta = deg_of(qq);
+    const int par1 = (alpha + L) & 1, par2 = (beta + L) & 1;
+    const int ll1 = max(par1, L - alpha), ll2 = max(par2, L - beta);
+    const double *pA = angA + L * L * ang_c + pp, *pB = angB + L * L * ang_c + qq;
+    const double *Te = Tl + alpha + beta;
+    double tmp = 0.0;
+    if constexpr (NB > 0) {
+      double Bv[NBL][NM];
+#pragma unroll
+      for (int i = 0; i < NBL; i++) {
+        const bool on = ll2 + 2 * i <= lb + L;
+        const double *pb = pB + (on ? ll2 + 2 * i : ll2) * lam_stride;
+#pragma unroll
+        for (int m = 0; m < NM; m++) Bv[i][m] = pb[m * ang_c];
+      }
+      for (int lam1 = ll1; lam1 <= la + L; lam1 += 2) {
+        const double *pa = pA + lam1 * lam_stride;
+        double Av[NM];
+#pragma unroll
+        for (int m = 0; m < NM; m++) Av[m] = pa[m * ang_c];
+#pragma unroll
+        for (int i = 0; i < NBL; i++) {
+          const int lam2 = ll2 + 2 * i;
+          if (lam2 <= lb + L) {
+            double factor = 0.0;
+#pragma unroll
+            for (int m = 0; m < NM; m++) factor += Av[m] * Bv[i][m];
+            tmp += factor * Te[(lam1 * d2 + lam2) * d3];
+          }
+        }
+      }
+    } else {
+      for (int lam1 = ll1; lam1 <= la + L; lam1 += 2)
+        for (int lam2 = ll2; lam2 <= lb + L; lam2 += 2) {
+          const double *pa = pA + lam1 * lam_stride, *pb = pB + lam2 * lam_stride;
+          double x[NM], y[NM];
+#pragma unroll
+          for (int m = 0; m < NM; m++) {
+            x[m] = pa[m * ang_c];
+            y[m] = pb[m * ang_c];
+          }
+          double factor = 0.0;
+#pragma unroll
+          for (int m = 0; m < NM; m++) factor += x[m] * y[m];
+          tmp += factor * Te[(lam1 * d2 + lam2) * d3];
+        }
+    }
+    blk[idx] += tmp;
+  }
+}
+
+// channels l < MAXL
+template <int NB, int MAXL>
+__device__ __forceinline__ void asm2_channel_of(int l, const double *__restrict__ angA,
+                                                const double *__restrict__ angB, int ang_c, int nlm2,
+                                                const double *Tl, int la, int lb, int nca, int ncb, float inv_ncb,
+                                                double *blk, int lid, int nlanes) {
+  switch (l) {
+#define CH(x)                                                                                                \
+  case x:                                                                                                    \
+    if constexpr (x < MAXL)                                                                                  \
+      asm2_channel<NB, x>(angA, angB, ang_c, nlm2, Tl, la, lb, nca, ncb, inv_ncb, blk, lid, nlanes);         \
+    break;
+    CH(0) CH(1) CH(2) CH(3) CH(4) CH(5) CH(6)
+#undef CH
+  }
+}
+
 // Type-2 block of one triplet per wave: for each projector l, the T_l
 // entries (small-grid results, or the sum of the per-pair fallback results)
 // are placed in LDS and contracted with the angular tables of both atoms
 // (type2.c:583-623), then the block is shifted (util.c:246-334).
-// NB > 0: the angular factors of atom B for every lambda2 (at most NB
-// values) and m (at most NM) are held in registers for each l, those of atom
-// A per lambda1; NB = 0: both read for each (lambda1, lambda2), with NM > 1
-// the 2 l + 1 values of each loaded together (NM >= 2 l + 1 of every
-// projector l).
-// tlist: the triplets of the launch, one per workgroup (nullptr: workgroup
-// t takes triplet t).
-template <int NB, int NM, int TPB = kAsmThreads>
-__global__ __launch_bounds__(TPB) void k_asm2(DevTables T, DevJob J, AsmArgs A,
-                                                      unsigned char *__restrict__ status,
-                                                      const unsigned char *__restrict__ fbflag, int filter,
+// NB, MAXL: as in asm2_channel, channels l < MAXL.
+// tlist: the triplets of the launch, one per workgroup.
+template <int NB, int MAXL>
+__global__ __launch_bounds__(kAsmThreads) void k_asm2(DevTables T, DevJob J, AsmArgs A,
+                                                      const unsigned char *__restrict__ status,
                                                       const int *__restrict__ tlist) {
   extern __shared__ double lds[];
   double *blk = lds + A.lds_blk;
   double *Jbuf = lds + A.lds_J;
   double *Tl = lds + A.lds_T;
-  const int t = tlist ? tlist[blockIdx.x] : (int)blockIdx.x;
-  if ((filter == 1 && fbflag[t]) || (filter == 2 && !fbflag[t])) return;
+  const int t = tlist[blockIdx.x];
   if (status[2 * t + 1]) return;
   const ecp_triplet tr = J.trip[t];
   const ecp_centre Cn = J.cent[tr.centre];
@@ -2075,20 +2165,6 @@ __global__ __launch_bounds__(TPB) void k_asm2(DevTables T, DevJob J, AsmArgs A,
   const V3 vA{rAC[0], rAC[1], rAC[2]}, vB{rBC[0], rBC[1], rBC[2]};
   const int D = T.ijkDim;
   const int g0 = A.tgfirst[t];
-  if (A.fbf2 && filter == 2) {
-    // speculative fallback: the triplet failed where an entry failed on the
-    // small grid and on the large grid (type2.c:417-528, code 1)
-    bool bad = false;
-    for (int l = 0; l < Cn.L; l++) {
-      const T2Group G = A.groups[g0 + l];
-      for (int e = threadIdx.x; e < G.ne; e += blockDim.x) bad = bad || (A.tfail[G.eoff + e] && A.fbf2[G.eoff + e]);
-    }
-    if (__syncthreads_or(bad)) {
-      if (threadIdx.x == 0) status[2 * t + 1] = 1;
-      return;
-    }
-  }
-
   for (int i = threadIdx.x; i < nca * ncb; i += blockDim.x) blk[i] = 0.0;
   __syncthreads();
   const int nlm2 = J.angL * J.angL;
@@ -2099,7 +2175,6 @@ __global__ __launch_bounds__(TPB) void k_asm2(DevTables T, DevJob J, AsmArgs A,
     const int d1 = la + l + 1, d2 = lb + l + 1, d3 = lab + 1;
     for (int i = threadIdx.x; i < d1 * d2 * d3; i += blockDim.x) Tl[i] = 0.0;
     __syncthreads();
-    const int nm = 2 * l + 1;
     for (int e = threadIdx.x; e < G.ne; e += blockDim.x) {
       const int code = A.tmpl[G.tmpl + e];
       const int l1 = code & 0xff, l2 = (code >> 8) & 0xff, l3 = (code >> 16) & 0xff;
@@ -2112,71 +2187,8 @@ __global__ __launch_bounds__(TPB) void k_asm2(DevTables T, DevJob J, AsmArgs A,
       Tl[(l1 * d2 + l2) * d3 + l3] = v;
     }
     __syncthreads();
-    for (int idx = threadIdx.x; idx < nca * ncb; idx += blockDim.x) {
-      const int pp = idx / ncb, qq = idx % ncb;
-      int alpha = 0, beta = 0;
-      while (ECP_DIM_C(alpha) <= pp) alpha++;
-      while (ECP_DIM_C(beta) <= qq) beta++;
-      const int par1 = (alpha + l) % 2, par2 = (beta + l) % 2;
-      const int ll1 = (par1 > l - alpha) ? par1 : l - alpha;
-      const int ll2 = (par2 > l - beta) ? par2 : l - beta;
-      double tmp = 0.0;
-      if constexpr (NB > 0) {
-        double Bv[NB][NM];
-#pragma unroll
-        for (int i = 0; i < NB; i++) {
-          const int lam2 = ll2 + 2 * i;
-          const double *pb = angB + ((size_t)lam2 * nlm2 + l * l) * J.ang_c + qq;
-#pragma unroll
-          for (int m = 0; m < NM; m++) Bv[i][m] = (lam2 <= lb + l && m < nm) ? pb[m * J.ang_c] : 0.0;
-        }
-        for (int lam1 = ll1; lam1 <= la + l; lam1 += 2) {
-          const double *pa = angA + ((size_t)lam1 * nlm2 + l * l) * J.ang_c + pp;
-          double Av[NM];
-#pragma unroll
-          for (int m = 0; m < NM; m++) Av[m] = m < nm ? pa[m * J.ang_c] : 0.0;
-#pragma unroll
-          for (int i = 0; i < NB; i++) {
-            const int lam2 = ll2 + 2 * i;
-            if (lam2 <= lb + l) {
-              double factor = 0.0;
-#pragma unroll
-              for (int m = 0; m < NM; m++)
-                if (m < nm) factor += Av[m] * Bv[i][m];
-              tmp += factor * Tl[(lam1 * d2 + lam2) * d3 + alpha + beta];
-            }
-          }
-        }
-      } else if constexpr (NM > 1) {
-        // all 2 l + 1 factor pairs of an angular factor loaded together (NM
-        // >= 2 l + 1), then summed in m order
-        for (int lam1 = ll1; lam1 <= la + l; lam1 += 2)
-          for (int lam2 = ll2; lam2 <= lb + l; lam2 += 2) {
-            const double *pa = angA + ((size_t)lam1 * nlm2 + l * l) * J.ang_c + pp;
-            const double *pb = angB + ((size_t)lam2 * nlm2 + l * l) * J.ang_c + qq;
-            double x[NM], y[NM];
-#pragma unroll
-            for (int m = 0; m < NM; m++) {
-              x[m] = m < nm ? pa[m * J.ang_c] : 0.0;
-              y[m] = m < nm ? pb[m * J.ang_c] : 0.0;
-            }
-            double factor = 0.0;
-#pragma unroll
-            for (int m = 0; m < NM; m++)
-              if (m < nm) factor += x[m] * y[m];
-            tmp += factor * Tl[(lam1 * d2 + lam2) * d3 + alpha + beta];
-          }
-      } else {
-        for (int lam1 = ll1; lam1 <= la + l; lam1 += 2)
-          for (int lam2 = ll2; lam2 <= lb + l; lam2 += 2) {
-            const double *pa = angA + ((size_t)lam1 * nlm2 + l * l) * J.ang_c + pp;
-            const double *pb = angB + ((size_t)lam2 * nlm2 + l * l) * J.ang_c + qq;
-            const double factor = dot_in_order<2>(0.0, pa, J.ang_c, pb, J.ang_c, nm);
-            tmp += factor * Tl[(lam1 * d2 + lam2) * d3 + alpha + beta];
-          }
-      }
-      blk[idx] += tmp;
-    }
+    asm2_channel_of<NB, MAXL>(l, angA, angB, J.ang_c, nlm2, Tl, la, lb, nca, ncb, 1.0f / ncb, blk, threadIdx.x,
+                              kAsmThreads);
     __syncthreads();
   }
   const double norm2 = (4.0 * M_PI) * (4.0 * M_PI);
@@ -2187,15 +2199,12 @@ __global__ __launch_bounds__(TPB) void k_asm2(DevTables T, DevJob J, AsmArgs A,
 // Type-2 blocks of classes la + lb <= kAsmPackLab (at most 9 elements),
 // kAsmPack triplets per wave (tlist[0 .. ntl)): lane groups of
 // kAsmThreads / kAsmPack lanes, each with an LDS slice of A.lds_group
-// doubles, run k_asm2's phases side by side with the same arithmetic (NM as
-// there: the 2 l + 1 angular factors loaded together, or dot_in_order for
-// NM = 1).  The channel loop runs to the wave's largest L, a group past its
+// doubles, run k_asm2's phases side by side with the same arithmetic.  The channel loop runs to the wave's largest L, a group past its
 // own with empty loops; every group synchronises with the wave.
-template <int NM>
+template <int MAXL>
 __global__ __launch_bounds__(kAsmThreads) void k_asm2p(DevTables T, DevJob J, AsmArgs A,
-                                                    unsigned char *__restrict__ status,
-                                                    const int *__restrict__ tlist, int ntl,
-                                                    const unsigned char *__restrict__ fbflag, int filter) {
+                                                    const unsigned char *__restrict__ status,
+                                                    const int *__restrict__ tlist, int ntl) {
   extern __shared__ double lds_all[];
   constexpr int G = kAsmPack, W = kAsmThreads / G;
   const int grp = (int)threadIdx.x / W, lid = (int)threadIdx.x % W;
@@ -2206,7 +2215,7 @@ __global__ __launch_bounds__(kAsmThreads) void k_asm2p(DevTables T, DevJob J, As
   const int ti = blockIdx.x * G + grp;
   bool active = ti < ntl;
   const int t = active ? tlist[ti] : tlist[0];
-  if (active && ((filter == 1 && fbflag[t]) || (filter == 2 && !fbflag[t]) || status[2 * t + 1])) active = false;
+  if (active && status[2 * t + 1]) active = false;
   if (!wave_any(active)) return;
   const ecp_triplet tr = J.trip[t];
   const ecp_centre Cn = J.cent[tr.centre];
@@ -2216,23 +2225,6 @@ __global__ __launch_bounds__(kAsmThreads) void k_asm2p(DevTables T, DevJob J, As
   const ecp_xyz rc = J.atoms[Cn.atom], ra = J.atoms[Sa.atom], rb = J.atoms[Sb.atom];
   const V3 vA{ra.x - rc.x, ra.y - rc.y, ra.z - rc.z}, vB{rb.x - rc.x, rb.y - rc.y, rb.z - rc.z};
   const int g0 = A.tgfirst[t];
-  if (A.fbf2 && filter == 2) {
-    // speculative fallback: the triplet failed where an entry failed on the
-    // small grid and on the large grid (type2.c:417-528, code 1); the
-    // decision of the group's lanes
-    bool bad = false;
-    if (active)
-      for (int l = 0; l < Cn.L; l++) {
-        const T2Group Gr = A.groups[g0 + l];
-        for (int e = lid; e < Gr.ne; e += W) bad = bad || (A.tfail[Gr.eoff + e] && A.fbf2[Gr.eoff + e]);
-      }
-    const unsigned long long m = __ballot(bad);
-    if ((m >> (grp * W)) & ((1ull << W) - 1ull)) {
-      if (lid == 0) status[2 * t + 1] = 1;
-      active = false;
-    }
-    if (!wave_any(active)) return;
-  }
   if (active)
     for (int i = lid; i < nca * ncb; i += W) blk[i] = 0.0;
   int Lw = active ? Cn.L : 0;
@@ -2250,7 +2242,6 @@ __global__ __launch_bounds__(kAsmThreads) void k_asm2p(DevTables T, DevJob J, As
       for (int i = lid; i < d1 * d2 * d3; i += W) Tl[i] = 0.0;
     }
     __syncthreads();
-    const int nm = 2 * l + 1;
     if (on)
       for (int e = lid; e < Gr.ne; e += W) {
         const int code = A.tmpl[Gr.tmpl + e];
@@ -2265,38 +2256,8 @@ __global__ __launch_bounds__(kAsmThreads) void k_asm2p(DevTables T, DevJob J, As
       }
     __syncthreads();
     if (on)
-      for (int idx = lid; idx < nca * ncb; idx += W) {
-        const int pp = idx / ncb, qq = idx % ncb;
-        int alpha = 0, beta = 0;
-        while (ECP_DIM_C(alpha) <= pp) alpha++;
-        while (ECP_DIM_C(beta) <= qq) beta++;
-        const int par1 = (alpha + l) % 2, par2 = (beta + l) % 2;
-        const int ll1 = (par1 > l - alpha) ? par1 : l - alpha;
-        const int ll2 = (par2 > l - beta) ? par2 : l - beta;
-        double tmp = 0.0;
-        for (int lam1 = ll1; lam1 <= la + l; lam1 += 2)
-          for (int lam2 = ll2; lam2 <= lb + l; lam2 += 2) {
-            const double *pa = angA + ((size_t)lam1 * nlm2 + l * l) * J.ang_c + pp;
-            const double *pb = angB + ((size_t)lam2 * nlm2 + l * l) * J.ang_c + qq;
-            double factor;
-            if constexpr (NM > 1) {
-              double x[NM], y[NM];
-#pragma unroll
-              for (int m = 0; m < NM; m++) {
-                x[m] = m < nm ? pa[m * J.ang_c] : 0.0;
-                y[m] = m < nm ? pb[m * J.ang_c] : 0.0;
-              }
-              factor = 0.0;
-#pragma unroll
-              for (int m = 0; m < NM; m++)
-                if (m < nm) factor += x[m] * y[m];
-            } else {
-              factor = dot_in_order<2>(0.0, pa, J.ang_c, pb, J.ang_c, nm);
-            }
-            tmp += factor * Tl[(lam1 * d2 + lam2) * d3 + alpha + beta];
-          }
-        blk[idx] += tmp;
-      }
+      asm2_channel_of<kAsmPackLab + 1, MAXL>(l, angA, angB, J.ang_c, nlm2, Tl, la, lb, nca, ncb, 1.0f / ncb, blk, lid,
+                                             W);
     __syncthreads();
   }
   const double norm2 = (4.0 * M_PI) * (4.0 * M_PI);
@@ -2389,10 +2350,10 @@ __global__ __launch_bounds__(128) void k_ang(DevTables T, DevJob J, const int2 *
 // first, then device-only buffers
 struct JobLayout {
   size_t i_atoms = 0, i_amaxl = 0, i_sh = 0, i_pa = 0, i_pd = 0, i_cent = 0, i_gauss = 0, i_win = 0, i_trip = 0,
-         i_u1 = 0, i_t1f = 0, i_grp = 0, i_goff = 0, i_tgf = 0, i_fit = 0, i_ait = 0, i_tcls = 0, i_tcls2 = 0,
+         i_u1 = 0, i_t1f = 0, i_grp = 0, i_goff = 0, i_tgf = 0, i_fit = 0, i_ait = 0, i_tcls = 0, i_tcls2 = 0, i_gfirst = 0,
          in_bytes = 0;
-  size_t d_zero = 0, d_fbc = 0, d_gflag = 0, d_stat = 0, d_t1fb = 0, d_t2fb = 0, d_tclaim = 0, d_fbf2 = 0, d_zero_end = 0, d_UL = 0, d_Ut = 0, d_F = 0, d_ang = 0,
-         d_q = 0, d_t1s = 0, d_tq1 = 0, d_qf = 0, d_qfb = 0, d_qopen = 0, d_qfbf = 0, d_udir = 0, d_fbq1 = 0, d_T = 0, d_tf = 0, d_flist = 0, d_tq2 = 0, d_fbq2 = 0, d_fbT = 0, d_blk = 0, total = 0;
+  size_t d_zero = 0, d_fbc = 0, d_gflag = 0, d_stat = 0, d_tclaim = 0, d_zero_end = 0, d_UL = 0, d_Ut = 0, d_F = 0, d_ang = 0,
+         d_q = 0, d_t1s = 0, d_tq1 = 0, d_qf = 0, d_udir = 0, d_fbq1 = 0, d_T = 0, d_tf = 0, d_flist = 0, d_fbq2 = 0, d_fbT = 0, d_blk = 0, total = 0;
   int FL = 0, UK = 0, angL = 0, ang_lam = 0, ang_c = 0, deriv = 0;
 };
 
@@ -2413,29 +2374,23 @@ struct Prepared {
   double *t1s = nullptr;  // type-1 head -> tail state: p, q, I planes of nq doubles
   int *tq1 = nullptr;     // type-1 tail queues (per class, indexed like the units)
   unsigned long long *qf = nullptr;
-  unsigned long long *qopen = nullptr, *qfbf = nullptr;  // speculative type-1 fallback
-  double *qfb = nullptr;
   double *udir = nullptr;  // per type-1 unit: its pair direction (4 values)
   int *fbq1 = nullptr, *fbc = nullptr;
   unsigned char *stat = nullptr;
-  unsigned char *t1fb = nullptr, *t2fb = nullptr;  // per triplet: has large-grid work (type 1 / type 2)
-  ClassMap cm_head, cm_tail, cm_fb1, cm_fb2;      // fused launches
   int max_lab = 0, max_lmb = 0;
   int tcount2[kMaxLMB + 1] = {0};  // triplets per type-2 fallback class
   int max_cls2 = 0;
   int max_ent2 = 0;  // T entries of a triplet, at most
   int *tclaim = nullptr;
-  unsigned char *fbf2 = nullptr;  // per T entry: the speculative fallback failed on the large grid
   const unsigned char *tcls2 = nullptr;
   const int *tgf = nullptr;
   int max_lbs = 0, max_L = 0;  // largest basis l and ECP local label of the job
   const T2Group *grp = nullptr;
-  const int *goff = nullptr;
+  const int *goff = nullptr, *gfirst = nullptr;
   double *Tout = nullptr;
   unsigned char *tf = nullptr;
   int *gflag = nullptr, *fbq2 = nullptr;
   int *flist = nullptr;  // per group: its failed T entries (gflag[g] of them) at eoff
-  int *tq2 = nullptr;    // type-2 entries left open by the head kernel
   double *fbT = nullptr;
   const int2 *fit = nullptr, *ait = nullptr;
   AsmArgs aa{};
@@ -2456,15 +2411,13 @@ struct Prepared {
 
 }  // namespace
 
-constexpr int kWorkers = 4;
+constexpr int kWorkers = 3;
 constexpr int kSpanGraphs = 8;  // graph copies with their own quadrature event pair
 
 struct ecp_dev {
   hipStream_t stream = nullptr;
   hipStream_t workers[kWorkers] = {};
-  hipEvent_t fork = nullptr, t2done = nullptr, t1done = nullptr, angdone = nullptr, join[kWorkers] = {};
-  hipEvent_t h1done = nullptr;  // type-1 head finished (speculative fallback)
-  hipEvent_t h2done = nullptr;  // type-2 head finished (speculative fallback)
+  hipEvent_t fork = nullptr, join[kWorkers] = {};
   // the type-1 small-grid quadrature (head and tail launches), recorded on
   // its stream: event pair k belongs to captured graph k (replays cycle over
   // the graphs, so the last kSpanGraphs replays can be read); the eager
@@ -2493,7 +2446,7 @@ struct ecp_dev {
   int *tmpl_dev = nullptr;
   Prepared P;
   JobLayout L;
-  ecp_tuning tune{8, 8, 100000, 8192, 2, 1, 15, 2048, 0, 1, 0};
+  ecp_tuning tune{5, 8, 100000, 8192, 2, 1, 15, 2048, 0, 1, 0};
   bool planned = false, prepared = false, eager_done = false;
   hipGraph_t graph[kSpanGraphs] = {};
   hipGraphExec_t gexec[kSpanGraphs] = {};
@@ -2617,11 +2570,6 @@ extern "C" ecp_dev *ecp_dev_create(const ecp_static *st, char *err, size_t errle
       return fail("hipEventCreate", e);
   }
   if ((e = hipEventCreateWithFlags(&d->fork, hipEventDisableTiming)) != hipSuccess) return fail("hipEventCreate", e);
-  if ((e = hipEventCreateWithFlags(&d->t2done, hipEventDisableTiming)) != hipSuccess) return fail("hipEventCreate", e);
-  if ((e = hipEventCreateWithFlags(&d->t1done, hipEventDisableTiming)) != hipSuccess) return fail("hipEventCreate", e);
-  if ((e = hipEventCreateWithFlags(&d->angdone, hipEventDisableTiming)) != hipSuccess) return fail("hipEventCreate", e);
-  if ((e = hipEventCreateWithFlags(&d->h1done, hipEventDisableTiming)) != hipSuccess) return fail("hipEventCreate", e);
-  if ((e = hipEventCreateWithFlags(&d->h2done, hipEventDisableTiming)) != hipSuccess) return fail("hipEventCreate", e);
   for (int k = 0; k < kSpanGraphs; k++)
     for (int i = 0; i < 2; i++)
       if ((e = hipEventCreate(&d->span[k][i])) != hipSuccess) return fail("hipEventCreate", e);
@@ -2734,11 +2682,6 @@ extern "C" void ecp_dev_destroy(ecp_dev *d) {
     if (d->join[i]) (void)hipEventDestroy(d->join[i]);
   }
   if (d->fork) (void)hipEventDestroy(d->fork);
-  if (d->t2done) (void)hipEventDestroy(d->t2done);
-  if (d->t1done) (void)hipEventDestroy(d->t1done);
-  if (d->angdone) (void)hipEventDestroy(d->angdone);
-  if (d->h1done) (void)hipEventDestroy(d->h1done);
-  if (d->h2done) (void)hipEventDestroy(d->h2done);
   for (int k = 0; k < kSpanGraphs; k++)
     for (int i = 0; i < 2; i++)
       if (d->span[k][i]) (void)hipEventDestroy(d->span[k][i]);
@@ -2758,176 +2701,105 @@ extern "C" int ecp_dev_last_timing(ecp_dev *d, double *ms, int n) {
 
 namespace {
 
-// Type-1 small grid of one class: the head kernel, then -- for the pairs
-// still open after `head` levels -- the wave-cooperative tail when the class
-// is small (latency-bound: few waves on the device) or the compacted
-// lane-serial tail when it is large (throughput-bound).
-// Type-1 small grid of one class: without a tail (head >= the level count)
-// one lane-serial kernel; otherwise the head kernel, then for the pairs still
-// open the wave-cooperative tail when the class is small (latency-bound: few
-// waves on the device) or the compacted lane-serial tail when it is large.
-// type-2 small grid: the lane-per-entry kernel, split into head and
-// compacted tail when t2_head is below the level count
-// PS93 levels of the type-2 head (t2_head; 0: automatic -- 6 when the small
-// grid is on the critical chain (fused launches), none in large per-class
-// jobs)
-int t2_head_levels(const ecp_dev *d, bool fused) {
-  return d->tune.t2_head > 0 ? d->tune.t2_head : (fused ? 6 : 15);
-}
-
-// spec: the head enlists every entry it leaves open for the fallback, which
-// can start at `mid` (recorded after the head) beside the tail
-void launch_type2(ecp_dev *d, hipStream_t s, bool fused, bool spec = false, hipEvent_t mid = nullptr) {
+void launch_type2(ecp_dev *d, hipStream_t s) {
   const Prepared &P = d->P;
   if (P.ntot2 <= 0) return;
-  T2Args A{P.grp, P.goff, P.ngroups, P.ntot2, d->tmpl_dev, P.Tout, P.tf, P.gflag, P.fbq2, P.fbc + kFb2Cnt, P.nt,
-           P.t2fb, P.flist, P.tq2, P.fbc + 48, P.tclaim, P.tcls2, spec ? 1 : 0, P.fbf2};
-  const int head = t2_head_levels(d, fused);
-  {
-    Span sp(d, s, FAM_TYPE2);
-    k_type2<<<(P.ntot2 + 127) / 128, 128, 0, s>>>(d->T, P.J, A, head);
-  }
-  if (mid) (void)hipEventRecord(mid, s);
-  if (head < d->T.s93.nlevels) {
-    Span sp(d, s, FAM_TYPE2);
-    k_type2_tail<<<std::min((P.ntot2 + 15) / 16, d->tune.t2_tail_grid), 64, 0, s>>>(d->T, P.J, A);
-  }
+  T2Args A{P.grp, P.goff, P.gfirst, P.ngroups, P.ntot2, d->tmpl_dev, P.Tout, P.tf, P.gflag, P.fbq2, P.fbc + kFb2Cnt,
+           P.nt, P.flist, P.tclaim, P.tcls2};
+  Span sp(d, s, FAM_TYPE2);
+  k_type2<<<(P.ntot2 + 63) / 64, 64, 0, s>>>(d->T, P.J, A);
 }
 
 // type-2 assembly: the register-cached variant fits basis l <= 3 with
-// projectors l <= 3 (NB = 4 lambda2 values, NM = 7 m values) or basis
-// l <= 4 with projectors l <= 4; larger jobs read the tables directly.  The
-// cache costs occupancy: it pays where the assembly is on the critical path
-// of a small job (fused launches), not in large throughput-bound ones.
-// pack: the triplets of classes la + lb <= kAsmPackLab (the first of the
-// class-ordered list) kAsmPack to a wave, the others one per workgroup
-template <int TPB>
-void launch_asm2_tpb(ecp_dev *d, hipStream_t s, int filter, bool cache, bool spec, bool pack) {
+// projectors l <= 3, or basis l <= 4 with projectors l <= 4; larger jobs (and
+// asm2_cache 0) read the tables directly.  The triplets of classes la + lb
+// <= kAsmPackLab (the first of the class-ordered list) go kAsmPack to a
+// wave, the others one per workgroup.
+void launch_asm2(ecp_dev *d, hipStream_t s) {
   const Prepared &P = d->P;
-  AsmArgs aa = P.aa;
-  aa.fbf2 = spec ? P.fbf2 : nullptr;
-  const int m = pack ? P.tcls_begin[kAsmPackLab + 1] : 0;
+  Span sp(d, s, FAM_ASM);
+  const int m = P.tcls_begin[kAsmPackLab + 1];
   if (m > 0) {
-    AsmArgs a2 = P.aa2p;
-    a2.fbf2 = aa.fbf2;
     const int g = (m + kAsmPack - 1) / kAsmPack;
-    // the 2 l + 1 angular factors loaded together where l < 4 (148
-    // registers, three waves per SIMD, against 84 and five read pair by
-    // pair: the uneven batch 0.7 ms faster)
-    if (P.max_L <= 4) k_asm2p<7><<<g, kAsmThreads, P.asm2_lds4, s>>>(d->T, P.J, a2, P.stat, P.tcls, m, P.t2fb, filter);
-    else k_asm2p<1><<<g, kAsmThreads, P.asm2_lds4, s>>>(d->T, P.J, a2, P.stat, P.tcls, m, P.t2fb, filter);
+    if (P.max_L <= 4) k_asm2p<4><<<g, kAsmThreads, P.asm2_lds4, s>>>(d->T, P.J, P.aa2p, P.stat, P.tcls, m);
+    else if (P.max_L == 5) k_asm2p<5><<<g, kAsmThreads, P.asm2_lds4, s>>>(d->T, P.J, P.aa2p, P.stat, P.tcls, m);
+    else k_asm2p<7><<<g, kAsmThreads, P.asm2_lds4, s>>>(d->T, P.J, P.aa2p, P.stat, P.tcls, m);
   }
   const int n = P.nt - m;
   if (n <= 0) return;
-  const int *tl = m > 0 ? P.tcls + m : nullptr;
-  if (!cache && P.max_L <= 4)
-    k_asm2<0, 7, TPB><<<n, TPB, P.asm2_lds, s>>>(d->T, P.J, aa, P.stat, P.t2fb, filter, tl);
-  else if (!cache)
-    k_asm2<0, 1, TPB><<<n, TPB, P.asm2_lds, s>>>(d->T, P.J, aa, P.stat, P.t2fb, filter, tl);
-  else if (P.max_lbs <= 3 && P.max_L <= 4)
-    k_asm2<4, 7, TPB><<<n, TPB, P.asm2_lds, s>>>(d->T, P.J, aa, P.stat, P.t2fb, filter, tl);
-  else if (P.max_lbs <= 4 && P.max_L <= 5)
-    k_asm2<5, 9, TPB><<<n, TPB, P.asm2_lds, s>>>(d->T, P.J, aa, P.stat, P.t2fb, filter, tl);
+  const int *tl = P.tcls + m;
+  const bool cache = d->tune.asm2_cache != 0;
+  if (cache && P.max_lbs <= 3 && P.max_L <= 4)
+    k_asm2<4, 4><<<n, kAsmThreads, P.asm2_lds, s>>>(d->T, P.J, P.aa, P.stat, tl);
+  else if (cache && P.max_lbs <= 4 && P.max_L <= 5)
+    k_asm2<5, 5><<<n, kAsmThreads, P.asm2_lds, s>>>(d->T, P.J, P.aa, P.stat, tl);
   else
-    k_asm2<0, 1, TPB><<<n, TPB, P.asm2_lds, s>>>(d->T, P.J, aa, P.stat, P.t2fb, filter, tl);
+    k_asm2<0, 7><<<n, kAsmThreads, P.asm2_lds, s>>>(d->T, P.J, P.aa, P.stat, tl);
 }
 
 // type-1 assembly of the triplets tcls[b .. e) (class-ordered), one per
-// wave, or with pack those of classes la + lb <= kAsmPackLab kAsmPack to a
-// wave (one more launch: it pays in large per-class launches, not on the
-// critical chain of fused ones)
+// wave, those of classes la + lb <= kAsmPackLab kAsmPack to a wave
 // cls >= 0: every triplet of the range is of class la + lb = cls (per-class
 // launches), which bounds the monomial degrees the kernel holds in registers
-// spec: the type-1 fallback ran speculatively (T1Set::qfb), the assembly
-// picks its results where the small grid failed
-void launch_asm1(ecp_dev *d, hipStream_t s, int b, int e, int filter, bool pack, int cls = -1, bool spec = false) {
+void launch_asm1(ecp_dev *d, hipStream_t s, int b, int e, int cls = -1) {
   const Prepared &P = d->P;
-  AsmArgs aa = P.aa;
-  if (spec) {
-    aa.qfail = P.qf;
-    aa.qfbf = P.qfbf;
-    aa.qfb = P.qfb;
-  }
-  const int m = pack ? std::min(std::max(b, P.tcls_begin[kAsmPackLab + 1]), e) : b;
-  if (m > b) {
-    AsmArgs a4 = P.aa4;
-    if (spec) {
-      a4.qfail = P.qf;
-      a4.qfbf = P.qfbf;
-      a4.qfb = P.qfb;
-    }
+  Span sp(d, s, FAM_ASM);
+  const int m = std::min(std::max(b, P.tcls_begin[kAsmPackLab + 1]), e);
+  if (m > b)
     k_asm1<kAsmPack, kAsmPackLab><<<(m - b + kAsmPack - 1) / kAsmPack, kAsmThreads, P.asm1_lds4, s>>>(
-        d->T, P.J, a4, P.stat, P.tcls + b, m - b, P.t1fb, filter);
-  }
+        d->T, P.J, P.aa4, P.stat, P.tcls + b, m - b);
   if (e <= m) return;
   const dim3 g(e - m);
   switch (cls) {
-#define ASM1(D)                                                                                               \
-  case D:                                                                                                   \
-    k_asm1<1, D><<<g, kAsmThreads, P.asm1_lds, s>>>(d->T, P.J, aa, P.stat, P.tcls + m, e - m, P.t1fb, filter); \
+#define ASM1(D)                                                                              \
+  case D:                                                                                  \
+    k_asm1<1, D><<<g, kAsmThreads, P.asm1_lds, s>>>(d->T, P.J, P.aa, P.stat, P.tcls + m, e - m); \
     break;
-    ASM1(0) ASM1(1) ASM1(2) ASM1(3) ASM1(4) ASM1(5)
+    ASM1(3) ASM1(4) ASM1(5)
 #undef ASM1
     default:
       // classes above 5 and mixed-class launches: rows up to degree 6 in
       // registers (the uneven batch's class-6 chain 0.7 ms slower with
       // degree 6 in the general loop)
-      k_asm1<1, 6><<<g, kAsmThreads, P.asm1_lds, s>>>(d->T, P.J, aa, P.stat, P.tcls + m, e - m, P.t1fb, filter);
+      k_asm1<1, 6><<<g, kAsmThreads, P.asm1_lds, s>>>(d->T, P.J, P.aa, P.stat, P.tcls + m, e - m);
   }
 }
 
-// The assembly of the triplets with large-grid work (filter 2) comes last
-// and covers few triplets: with fused launches it runs 4 waves per triplet,
-// so that each triplet's elements finish sooner.
-// spec: the fallback ran speculatively; a triplet failed where an entry
-// failed on both grids
-// The small classes go four triplets to a wave (they are about half of the
-// triplets: the medium cluster 2.5 % and the uneven batch 0.5 % faster),
-// except in the fused sequence's last assembly, which covers the few
-// triplets with fallback work at four waves each.
-void launch_asm2(ecp_dev *d, hipStream_t s, int filter, bool fused, bool spec = false) {
-  const int mode = d->tune.asm2_cache;
-  const bool cache = mode == 1 || (mode == 2 && fused);
-  if (fused && filter == 2)
-    launch_asm2_tpb<4 * kAsmThreads>(d, s, filter, cache, spec, false);
-  else
-    launch_asm2_tpb<kAsmThreads>(d, s, filter, cache, spec, true);
+T1Set t1_set(const ecp_dev *d) {
+  const Prepared &P = d->P;
+  T1Set S{};
+  S.units = P.u1;
+  S.q = P.q;
+  S.qf = P.qf;
+  S.fbq = P.fbq1;
+  S.fbc = P.fbc;
+  S.tq = P.tq1;
+  S.st = P.t1s;
+  S.plane = P.nq;
+  S.stat = P.stat;
+  for (int c = 0; c <= ECP_MAX_LAB; c++) {
+    S.ubeg[c] = P.cls_begin[c];
+    S.ucnt[c] = P.cls_count[c];
+  }
+  S.head = d->tune.t1_head_coop;
+  return S;
 }
 
+// Type-1 quadrature of one class: the head, then the tail and the large-grid
+// fallbacks in one persistent launch
 template <int LAB>
-void launch_type1(ecp_dev *d, hipStream_t s, const DevTables &T, const DevJob &J, const T1Unit *u, int n, double *q,
-                  unsigned long long *qf, int *fbq, int *fbc, double *st, size_t plane, int *tq, int *tc,
-                  unsigned char *ff) {
+void launch_type1(ecp_dev *d, hipStream_t s, const T1Set &S) {
+  const int n = S.ucnt[LAB], ub = S.ubeg[LAB];
   if (n <= 0) return;
-  const bool coop = n <= d->tune.t1_coop_max;
-  const int head = coop ? d->tune.t1_head_coop : d->tune.t1_head_serial;
-  const int grid = (n + 63) / 64;
-  if (head >= T.s93.nlevels) {
-    Span sp(d, s, FAM_TYPE1);
-    k_type1<LAB, 0><<<grid, 64, 0, s>>>(T, J, u, n, q, qf, fbq, fbc, head, st, plane, tq, tc, ff);
-    return;
-  }
   {
     Span sp(d, s, FAM_TYPE1);
-    k_type1<LAB, 1><<<grid, 64, 0, s>>>(T, J, u, n, q, qf, fbq, fbc, head, st, plane, tq, tc, ff);
+    k_type1<LAB><<<(n + 63) / 64, 64, 0, s>>>(d->T, d->P.J, S.units + ub, n, S.q, S.qf + ub, S.fbq + ub, S.fbc + LAB,
+                                              S.head, S.st, S.plane, S.tq + ub, S.fbc + 32 + LAB);
   }
   Span sp(d, s, FAM_T1TAIL);
-  if (coop)
-    k_t1tail<LAB><<<std::min(n, d->tune.t1_tail_grid), 64, 0, s>>>(T, J, u, q, qf, fbq, fbc, head, st, plane, tq,
-                                                                    tc, ff);
-  else
-    k_type1<LAB, 2><<<std::min(grid, d->tune.t1_tail_grid), 64, 0, s>>>(T, J, u, n, q, qf, fbq, fbc, head, st,
-                                                                         plane, tq, tc, ff);
-}
-
-template <int LAB>
-void launch_fb1(ecp_dev *d, hipStream_t s, const DevTables &T, const DevJob &J, const T1Unit *u, int n, double *q,
-                const unsigned long long *qf, const int *fbq, const int *fbc, unsigned char *st) {
-  if (n > 0) {
-    Span sp(d, s, FAM_FB1);
-    const int blocks = std::min(n, 4096);
-    k_fb1<LAB><<<blocks, 64, 0, s>>>(T, J, u, q, qf, fbq, fbc, st);
-  }
+  k_t1tail<LAB><<<std::min(n, d->tune.t1_tail_grid), 64, 0, s>>>(d->T, d->P.J, S.units + ub, S.q, S.qf + ub,
+                                                                 S.fbq + ub, S.fbc + LAB, S.head, S.st, S.plane,
+                                                                 S.tq + ub, S.fbc + 32 + LAB, S.stat);
 }
 
 // workgroup ranges of the classes with work; blocks(c) = workgroups of class c
@@ -3014,30 +2886,22 @@ void launch_tables(ecp_dev *d, hipStream_t s) {
   k_tables<<<A.nzb + A.nub + A.nfit + (A.nunits + 127) / 128, 128, 0, s>>>(d->T, P.J, A);
 }
 
-// the angular tables on stream s, concurrent with the quadratures; the
-// type-2 assembly waits for d->angdone
+// the angular tables on stream s, ahead of the type-2 chain
 void launch_ang(ecp_dev *d, hipStream_t s) {
   const Prepared &P = d->P;
   if (P.nait) k_ang<<<P.nait, 128, 0, s>>>(d->T, P.J, P.ait, d->fac_dev, d->dfac_dev);
-  (void)hipEventRecord(d->angdone, s);
 }
 
 // fuse = 2 (automatic): fused launches for jobs of up to this many type-1
 // primitive pairs (latency-bound: per-class launches hold few waves each)
 constexpr int kFuseAutoMaxUnits = 150000;
 
-// one type-1 class of the per-class sequence: small grid, fallback, assembly
+// one type-1 class of the per-class sequence: quadrature, assembly
 template <int c>
 void enqueue_t1_class_t(ecp_dev *d, hipStream_t ws) {
   const Prepared &P = d->P;
-  launch_type1<c>(d, ws, d->T, P.J, P.u1 + P.cls_begin[c], P.cls_count[c], P.q, P.qf + P.cls_begin[c],
-                  P.fbq1 + P.cls_begin[c], P.fbc + c, P.t1s, P.nq, P.tq1 + P.cls_begin[c], P.fbc + 32 + c, P.t1fb);
-  launch_fb1<c>(d, ws, d->T, P.J, P.u1 + P.cls_begin[c], P.cls_count[c], P.q, P.qf + P.cls_begin[c],
-                P.fbq1 + P.cls_begin[c], P.fbc + c, P.stat);
-  if (P.tcls_begin[c + 1] > P.tcls_begin[c]) {
-    Span sp(d, ws, FAM_ASM);
-    launch_asm1(d, ws, P.tcls_begin[c], P.tcls_begin[c + 1], 0, true, c);
-  }
+  launch_type1<c>(d, ws, t1_set(d));
+  if (P.tcls_begin[c + 1] > P.tcls_begin[c]) launch_asm1(d, ws, P.tcls_begin[c], P.tcls_begin[c + 1], c);
 }
 
 void enqueue_t1_class(ecp_dev *d, hipStream_t ws, int c) {
@@ -3075,59 +2939,36 @@ void enqueue(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
   if (evs) (void)hipEventRecord(evs[1], s);
   (void)hipEventRecord(d->fork, s);
   for (int i = 0; i < kWorkers; i++) (void)hipStreamWaitEvent(w[i], d->fork, 0);
-  // Two layouts.  Jobs whose type-1 classes stay at la + lb <= 6: four
-  // streams, one per hardware queue the device gives a process -- the
-  // type-2 chain (small grid, fallbacks, assembly of the triplets with
-  // fallback work) on the main stream, the assembly of the other triplets
-  // on the third worker, the type-1 classes on the first two.  Jobs with
-  // larger classes, where type 1 carries more of the work: the type-2 small
-  // grid and the assembly without fallback work on the fourth worker, the
-  // fallbacks and the rest of the assembly on the main stream, the type-1
-  // classes on the first three workers.
-  const bool four = P.max_lab <= 6;
-  const int nw1 = four ? 2 : kWorkers - 1;
-  hipStream_t w2 = four ? s : w[kWorkers - 1];
-  hipStream_t wa = four ? w[2] : w2;  // the assembly without fallback work
+  // the type-2 chain (small grid, fallbacks, assembly) on the main stream,
+  // beside it the type-1 classes on three workers: one stream per hardware
+  // queue the device gives a process
+  const int nw1 = kWorkers;
   {
     Span sp(d, s, FAM_TABLES);
     launch_ang(d, s);
   }
   if (P.ntot2 > 0) {
-    launch_type2(d, w2, false);
-    (void)hipEventRecord(d->t2done, w2);
-    // the angular tables are on the main stream: behind the small grid in
-    // the four-stream layout, a wait otherwise
-    (void)hipStreamWaitEvent(wa, four ? d->t2done : d->angdone, 0);
-    {
-      Span sp(d, wa, FAM_ASM);
-      launch_asm2(d, wa, 1, false);
-    }
-    if (!four) (void)hipStreamWaitEvent(s, d->t2done, 0);
+    launch_type2(d, s);
     // every fallback class in one persistent grid: the classes' items run
     // side by side instead of one class after another on this stream
-    {
-      T2Set S2{P.grp, d->tmpl_dev, P.fbq2, P.fbc, P.fbT, P.stat, P.nt, P.gflag, P.flist, P.tgf, 1, 1, 1, 0, 0, 0, nullptr};
-      fb2_slots(d, S2);
-      const ClassMap cm2 = fb2_classes(d, S2);
-      if (cm2.n > 0) {
-        Span sp(d, s, FAM_FB2);
-        launch_fb2_fused(d, s, S2, cm2);
-      }
+    T2Set S2{P.grp, d->tmpl_dev, P.fbq2, P.fbc, P.fbT, P.stat, P.nt, P.gflag, P.flist, P.tgf, 1, 1, 1, 0, 0, 0};
+    fb2_slots(d, S2);
+    const ClassMap cm2 = fb2_classes(d, S2);
+    if (cm2.n > 0) {
+      Span sp(d, s, FAM_FB2);
+      launch_fb2_fused(d, s, S2, cm2);
     }
-    {
-      Span sp(d, s, FAM_ASM);
-      launch_asm2(d, s, 2, false);
-    }
+    launch_asm2(d, s);
   }
-  // type-1 classes, each followed by its fallback and assembly on one of the
-  // type-1 workers: the costliest class first, each on the worker with the
+  // type-1 classes, each followed by its assembly, on one of the
+  // workers: the costliest class first, each on the worker with the
   // least work so far (the cost of a class: its algorithmic small-grid
   // FLOPs), so that no large class starts last and runs alone at the end
   int order[ECP_MAX_LAB + 1], nord = 0;
   for (int c = 0; c <= ECP_MAX_LAB; c++)
     if (P.cls_count[c] > 0) order[nord++] = c;
   std::stable_sort(order, order + nord, [&](int a, int b) { return P.flops_t1[a] > P.flops_t1[b]; });
-  double load[kWorkers - 1] = {};
+  double load[kWorkers] = {};
   for (int i = 0; i < nord; i++) {
     int k = 0;
     for (int j = 1; j < nw1; j++)
@@ -3146,16 +2987,15 @@ void enqueue(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
 }
 
 
-// The fused sequence: tables on the main stream, then two chains.  Type 1:
-// head (all classes) -> tail -> [assembly of triplets without large-grid
-// work] while, on a second stream, large-grid fallback -> assembly of the
-// rest.  Type 2 likewise: small grid -> [assembly without fallback] while
-// fallback -> assembly of the rest.  evs: stage boundaries as in enqueue.
+// The fused sequence: tables on the main stream, then the two chains side by
+// side, each stage one launch over every class.  Type 1: head, then tail and
+// large-grid fallbacks, then assembly.  Type 2: small grid, fallbacks,
+// assembly.  evs: stage boundaries as in enqueue.
 void enqueue_fused(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
   const Prepared &P = d->P;
   const DevTables &T = d->T;
   const DevJob &J = P.J;
-  hipStream_t *w = d->workers;
+  hipStream_t w = d->workers[0];
   d->span_valid = false;
   if (evs) (void)hipEventRecord(evs[0], s);
   {
@@ -3164,92 +3004,33 @@ void enqueue_fused(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
   }
   if (evs) (void)hipEventRecord(evs[1], s);
   (void)hipEventRecord(d->fork, s);
-  for (int i = 0; i < kWorkers; i++) (void)hipStreamWaitEvent(w[i], d->fork, 0);
-  const ecp_tuning &tu = d->tune;
+  (void)hipStreamWaitEvent(w, d->fork, 0);
   // ---- type 1 ----
-  T1Set S{};
-  S.units = P.u1;
-  S.q = P.q;
-  S.qf = P.qf;
-  S.fbq = P.fbq1;
-  S.fbc = P.fbc;
-  S.tq = P.tq1;
-  S.st = P.t1s;
-  S.plane = P.nq;
-  S.stat = P.stat;
-  S.fbflag = P.t1fb;
-  // cooperative tail for classes up to t1_coop_max pairs, none for larger
-  // ones (throughput-bound: the lane-serial head runs every level)
-  int tailcnt[ECP_MAX_LAB + 1];
-  bool tail = false;
-  for (int c = 0; c <= ECP_MAX_LAB; c++) {
-    S.ubeg[c] = P.cls_begin[c];
-    S.ucnt[c] = P.cls_count[c];
-    const bool coop = P.cls_count[c] <= tu.t1_coop_max && tu.t1_head_coop < T.s93.nlevels;
-    S.head[c] = coop ? tu.t1_head_coop : T.s93.nlevels;
-    tailcnt[c] = coop ? P.cls_count[c] : 0;
-    tail = tail || (coop && P.cls_count[c] > 0);
-  }
+  const T1Set S = t1_set(d);
   // the fused kernels hold the registers of their largest class: three
   // instantiations, classes up to 6, 10 and 12
   const int tier1 = P.max_lab > 10 ? 2 : P.max_lab > 6 ? 1 : 0;
-  // speculative fallback: with a tail, the large-grid fallback starts after
-  // the head on every entry the head left open, beside the tail, instead of
-  // after the tail on the failed ones (most of the entries open after the
-  // head fail; the tail only decides which results the assembly takes)
-  const bool spec = tail && tu.t1_spec != 0;
-  if (spec) {
-    S.qopen = P.qopen;
-    S.qfb = P.qfb;
-    S.qfbf = P.qfbf;
-  }
   const ClassMap cmh = class_map(ECP_MAX_LAB + 1, P.cls_count, [&](int c) { return (P.cls_count[c] + 63) / 64; });
   if (cmh.n > 0) {
     // external event nodes when captured, so that replays record them too
-    (void)hipEventRecordWithFlags(d->span[d->span_k][0], w[0], d->capturing ? hipEventRecordExternal : 0);
+    (void)hipEventRecordWithFlags(d->span[d->span_k][0], w, d->capturing ? hipEventRecordExternal : 0);
     {
-      Span sp(d, w[0], FAM_TYPE1);
-      if (tier1 == 2) k_type1_fused<12, 1><<<cmh.bbeg[cmh.n], 64, 0, w[0]>>>(T, J, S, cmh);
-      else if (tier1 == 1) k_type1_fused<10, 1><<<cmh.bbeg[cmh.n], 64, 0, w[0]>>>(T, J, S, cmh);
-      else k_type1_fused<6, 1><<<cmh.bbeg[cmh.n], 64, 0, w[0]>>>(T, J, S, cmh);
+      Span sp(d, w, FAM_TYPE1);
+      if (tier1 == 2) k_type1_fused<12><<<cmh.bbeg[cmh.n], 64, 0, w>>>(T, J, S, cmh);
+      else if (tier1 == 1) k_type1_fused<10><<<cmh.bbeg[cmh.n], 64, 0, w>>>(T, J, S, cmh);
+      else k_type1_fused<6><<<cmh.bbeg[cmh.n], 64, 0, w>>>(T, J, S, cmh);
     }
-    if (spec) (void)hipEventRecord(d->h1done, w[0]);
-    if (tail) {
-      const ClassMap cmt = class_map(ECP_MAX_LAB + 1, tailcnt,
-                                     [&](int c) { return std::min(tailcnt[c], tu.t1_tail_grid); });
-      Span sp(d, w[0], FAM_T1TAIL);
-      if (tier1 == 2) k_t1tail_fused<12><<<cmt.bbeg[cmt.n], 64, 0, w[0]>>>(T, J, S, cmt);
-      else if (tier1 == 1) k_t1tail_fused<10><<<cmt.bbeg[cmt.n], 64, 0, w[0]>>>(T, J, S, cmt);
-      else k_t1tail_fused<6><<<cmt.bbeg[cmt.n], 64, 0, w[0]>>>(T, J, S, cmt);
+    {
+      const ClassMap cmt = class_map(ECP_MAX_LAB + 1, P.cls_count,
+                                     [&](int c) { return std::min(P.cls_count[c], d->tune.t1_tail_grid); });
+      Span sp(d, w, FAM_T1TAIL);
+      if (tier1 == 2) k_t1tail_fused<12><<<cmt.bbeg[cmt.n], 64, 0, w>>>(T, J, S, cmt);
+      else if (tier1 == 1) k_t1tail_fused<10><<<cmt.bbeg[cmt.n], 64, 0, w>>>(T, J, S, cmt);
+      else k_t1tail_fused<6><<<cmt.bbeg[cmt.n], 64, 0, w>>>(T, J, S, cmt);
     }
-    (void)hipEventRecordWithFlags(d->span[d->span_k][1], w[0], d->capturing ? hipEventRecordExternal : 0);
+    (void)hipEventRecordWithFlags(d->span[d->span_k][1], w, d->capturing ? hipEventRecordExternal : 0);
     d->span_valid = true;
-    // the fallback is captured before the assembly beside it: a graph
-    // continues a node's queue with its first dependent, and the fallback
-    // is the critical one
-    (void)hipEventRecord(d->t1done, w[0]);
-    (void)hipStreamWaitEvent(w[1], spec ? d->h1done : d->t1done, 0);
-    const ClassMap cmf = class_map(ECP_MAX_LAB + 1, P.cls_count, [&](int c) { return std::min(P.cls_count[c], 4096); });
-    {
-      Span sp(d, w[1], FAM_FB1);
-      if (tier1 == 2 && spec) k_fb1_fused<12, true><<<cmf.bbeg[cmf.n], 64, 0, w[1]>>>(T, J, S, cmf);
-      else if (tier1 == 2) k_fb1_fused<12, false><<<cmf.bbeg[cmf.n], 64, 0, w[1]>>>(T, J, S, cmf);
-      else if (tier1 == 1 && spec) k_fb1_fused<10, true><<<cmf.bbeg[cmf.n], 64, 0, w[1]>>>(T, J, S, cmf);
-      else if (tier1 == 1) k_fb1_fused<10, false><<<cmf.bbeg[cmf.n], 64, 0, w[1]>>>(T, J, S, cmf);
-      else if (spec) k_fb1_fused<6, true><<<cmf.bbeg[cmf.n], 64, 0, w[1]>>>(T, J, S, cmf);
-      else k_fb1_fused<6, false><<<cmf.bbeg[cmf.n], 64, 0, w[1]>>>(T, J, S, cmf);
-    }
-    {
-      Span sp(d, w[0], FAM_ASM);
-      launch_asm1(d, w[0], 0, P.nt, 1, false);
-    }
-    // the assembly of the triplets with large-grid work reads the tail's
-    // decisions and the fallback's results
-    if (spec) (void)hipStreamWaitEvent(w[1], d->t1done, 0);
-    {
-      Span sp(d, w[1], FAM_ASM);
-      launch_asm1(d, w[1], 0, P.nt, 2, false, -1, spec);
-    }
+    launch_asm1(d, w, 0, P.nt);
   }
   // ---- type 2 ----
   {
@@ -3257,39 +3038,18 @@ void enqueue_fused(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
     launch_ang(d, s);
   }
   if (P.ntot2 > 0) {
-    // likewise the fallback first (it needs no angular tables), then the
-    // assembly beside it, then the assembly that waits for the fallback
-    // t2_spec: the fallback starts after the head, beside the tail, on every
-    // entry the head left open (most of them fail); the assembly then takes
-    // the fallback's result where the tail failed too
-    const bool spec2 = tu.t2_spec != 0 && t2_head_levels(d, true) < T.s93.nlevels;
-    launch_type2(d, w[2], true, spec2, spec2 ? d->h2done : nullptr);
-    (void)hipEventRecord(d->t2done, w[2]);
-    (void)hipStreamWaitEvent(w[3], spec2 ? d->h2done : d->t2done, 0);
-    T2Set S2{P.grp, d->tmpl_dev, P.fbq2, P.fbc, P.fbT, P.stat, P.nt, P.gflag, P.flist, P.tgf, 1, 1, 1, 0, 0, 0,
-             spec2 ? P.fbf2 : nullptr};
+    launch_type2(d, s);
+    T2Set S2{P.grp, d->tmpl_dev, P.fbq2, P.fbc, P.fbT, P.stat, P.nt, P.gflag, P.flist, P.tgf, 1, 1, 1, 0, 0, 0};
     fb2_slots(d, S2);
     const ClassMap cm2 = fb2_classes(d, S2);
     if (cm2.n > 0) {
-      Span sp(d, w[3], FAM_FB2);
-      launch_fb2_fused(d, w[3], S2, cm2);
+      Span sp(d, s, FAM_FB2);
+      launch_fb2_fused(d, s, S2, cm2);
     }
-    (void)hipStreamWaitEvent(w[2], d->angdone, 0);
-    {
-      Span sp(d, w[2], FAM_ASM);
-      launch_asm2(d, w[2], 1, true);
-    }
-    if (spec2) (void)hipStreamWaitEvent(w[3], d->t2done, 0);
-    (void)hipStreamWaitEvent(w[3], d->angdone, 0);
-    {
-      Span sp(d, w[3], FAM_ASM);
-      launch_asm2(d, w[3], 2, true, spec2);
-    }
+    launch_asm2(d, s);
   }
-  for (int i = 0; i < kWorkers; i++) {
-    (void)hipEventRecord(d->join[i], w[i]);
-    (void)hipStreamWaitEvent(s, d->join[i], 0);
-  }
+  (void)hipEventRecord(d->join[0], w);
+  (void)hipStreamWaitEvent(s, d->join[0], 0);
   if (evs) {
     (void)hipEventRecord(evs[2], s);
     (void)hipEventRecord(evs[3], s);
@@ -3389,6 +3149,13 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
   for (int c = 0; c <= kMaxLMB; c++)
     if (P.lmb_count[c]) P.max_lmb = c;
   goff.push_back(ntot2);
+  // the group of every 64th T entry: a wave of the type-2 small grid finds
+  // its entries' groups among those from there on
+  std::vector<int> gfirst((size_t)(ntot2 + 63) / 64);
+  for (size_t w = 0, g = 0; w < gfirst.size(); w++) {
+    while (goff[g + 1] <= (int)(64 * w)) g++;
+    gfirst[w] = (int)g;
+  }
   std::vector<int2> fitems, aitems;
   for (int c = 0; c < job->ncent; c++) {
     const ecp_centre &C = job->cent[c];
@@ -3422,6 +3189,7 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
   Ly.i_grp = in_take(sizeof(T2Group) * groups.size());
   Ly.i_goff = in_take(4 * goff.size());
   Ly.i_tgf = in_take(4 * (size_t)nt);
+  Ly.i_gfirst = in_take(4 * gfirst.size());
   Ly.i_tcls2 = in_take((size_t)nt);
   Ly.i_fit = in_take(sizeof(int2) * fitems.size());
   Ly.i_ait = in_take(sizeof(int2) * aitems.size());
@@ -3437,11 +3205,8 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
   Ly.d_fbc = dv_take(4 * kFbcSlots);
   Ly.d_gflag = dv_take(4 * (size_t)P.ngroups);
   Ly.d_stat = dv_take(2 * (size_t)nt);
-  Ly.d_t1fb = dv_take((size_t)nt);
-  Ly.d_t2fb = dv_take((size_t)nt);
   Ly.d_tclaim = dv_take(4 * (size_t)nt);
   Ly.d_zero_end = dv_off;
-  Ly.d_fbf2 = dv_take((size_t)ntot2);
   Ly.d_UL = dv_take(8 * job->nUL);
   Ly.d_Ut = dv_take(8 * job->nUt);
   Ly.d_F = dv_take(8 * job->nF);
@@ -3453,15 +3218,11 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
   Ly.d_T = dv_take(8 * (size_t)ntot2);
   Ly.d_tf = dv_take((size_t)ntot2);
   Ly.d_flist = dv_take(4 * (size_t)ntot2);
-  Ly.d_tq2 = dv_take(4 * (size_t)ntot2);
   Ly.d_fbq2 = dv_take(4 * (size_t)(kMaxLMB + 1) * nt);
   Ly.d_fbT = dv_take(8 * (size_t)ntot2 * P.maxPairs);
   Ly.d_blk = dv_take(8 * job->nblk);
   Ly.d_t1s = dv_take(3 * 8 * nq);
   Ly.d_tq1 = dv_take(4 * units1.size());
-  Ly.d_qfb = dv_take(8 * nq);
-  Ly.d_qopen = dv_take(8 * units1.size());
-  Ly.d_qfbf = dv_take(8 * units1.size());
   Ly.d_udir = dv_take(32 * units1.size());
   Ly.total = dv_off;
   Ly.FL = job->FL;
@@ -3566,6 +3327,7 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
   cp(Ly.i_grp, groups.data(), sizeof(T2Group) * groups.size());
   cp(Ly.i_goff, goff.data(), 4 * goff.size());
   cp(Ly.i_tgf, tgfirst.data(), 4 * (size_t)nt);
+  cp(Ly.i_gfirst, gfirst.data(), 4 * gfirst.size());
   cp(Ly.i_tcls2, tcls2.data(), (size_t)nt);
   cp(Ly.i_fit, fitems.data(), sizeof(int2) * fitems.size());
   cp(Ly.i_ait, aitems.data(), sizeof(int2) * aitems.size());
@@ -3635,26 +3397,20 @@ extern "C" int ecp_dev_bind(ecp_dev *d, void *mem, size_t cap, char *err, size_t
   P.t1s = (double *)(A + Ly.d_t1s);
   P.tq1 = (int *)(A + Ly.d_tq1);
   P.qf = (unsigned long long *)(A + Ly.d_qf);
-  P.qfb = (double *)(A + Ly.d_qfb);
-  P.qopen = (unsigned long long *)(A + Ly.d_qopen);
-  P.qfbf = (unsigned long long *)(A + Ly.d_qfbf);
   P.udir = (double *)(A + Ly.d_udir);
   P.fbq1 = (int *)(A + Ly.d_fbq1);
   P.fbc = (int *)(A + Ly.d_fbc);  // [0..12] type-1 fallback queues, [32..44] type-1 tails, [48] type-2
                                   // tail, [kFb2Cnt + 0..12] type-2 fallback queues
   P.stat = (unsigned char *)(A + Ly.d_stat);
-  P.t1fb = (unsigned char *)(A + Ly.d_t1fb);
-  P.t2fb = (unsigned char *)(A + Ly.d_t2fb);
   P.grp = (const T2Group *)(A + Ly.i_grp);
   P.goff = (const int *)(A + Ly.i_goff);
+  P.gfirst = (const int *)(A + Ly.i_gfirst);
   P.Tout = (double *)(A + Ly.d_T);
   P.tf = (unsigned char *)(A + Ly.d_tf);
   P.gflag = (int *)(A + Ly.d_gflag);
   P.flist = (int *)(A + Ly.d_flist);
-  P.tq2 = (int *)(A + Ly.d_tq2);
   P.fbq2 = (int *)(A + Ly.d_fbq2);
   P.tclaim = (int *)(A + Ly.d_tclaim);
-  P.fbf2 = (unsigned char *)(A + Ly.d_fbf2);
   P.tcls2 = (const unsigned char *)(A + Ly.i_tcls2);
   P.tgf = (const int *)(A + Ly.i_tgf);
   P.fbT = (double *)(A + Ly.d_fbT);
