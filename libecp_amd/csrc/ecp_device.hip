@@ -7,8 +7,8 @@
 //            (evalECP / tabECP_FM06: ecp.c:41-60, type2.c:184-219); and
 //            F_lambda(r_n) per (centre, shell) on its screened window
 //            (calcF_FM06: type2.c:222-310)
-//   k_ang    per-(centre, atom) angular tables (evalAngularIntegrals:
-//            angular_integrals.c:104-142), concurrent with the quadratures
+//            and per-(centre, atom) angular tables (evalAngularIntegrals:
+//            angular_integrals.c:104-142)
 //   k_type1 / k_t1tail  type-1 radial integrals Q[l1][l2] per (triplet,
 //            primitive pair) with the PS93 sequence (calcQ: type1.c:94-203):
 //            lane-serial head, wave-cooperative tail for the open pairs
@@ -97,14 +97,66 @@ namespace {
 constexpr int SO = ECP_SMALL_ORDER;
 constexpr int kMaxLMB = ECP_MAX_L - 1 + ECP_MAX_LBS;  // largest Bessel order of F / K_a / K_b
 
+// A table that no kernel writes: its elements are read through the constant
+// address space, so that a uniform index is a scalar load wherever it stands.
+// Through a plain pointer the compiler falls back to vector loads behind
+// every barrier and store, which wait in order with the data loads in
+// flight.
+template <typename V>
+struct CPtr {
+  const V *p;
+  CPtr() = default;
+  __host__ __device__ CPtr(const V *q) : p(q) {}
+  __host__ __device__ operator const V *() const { return p; }
+  template <typename I>
+  __device__ __forceinline__ V operator[](I i) const {
+    return at(p + i);
+  }
+  static __device__ __forceinline__ V at(const V *q) {
+    if constexpr (sizeof(V) <= 8) {
+      return *(const __attribute__((address_space(4))) V *)q;
+    } else {
+      static_assert(sizeof(V) % 4 == 0, "whole words");
+      const __attribute__((address_space(4))) int *w = (const __attribute__((address_space(4))) int *)q;
+      V out;
+#pragma unroll
+      for (size_t k = 0; k < sizeof(V) / 4; k++) {
+        const int x = w[k];
+        __builtin_memcpy((char *)&out + 4 * k, &x, 4);
+      }
+      return out;
+    }
+  }
+};
+// one element, or member, likewise
+template <typename V>
+__device__ __forceinline__ V cload(const V *q) {
+  return CPtr<V>::at(q);
+}
+
+// A point pair of the PS93 sequence, in visit order: its points, their
+// weights, and the level it is the last pair of (0: none).  A level's last
+// pair is its closest to the centre, so the level has a point in a window
+// where this pair does.
+struct Ps93Pair {
+  double wl, wr;
+  int li, ri, ends, pad;
+};
+constexpr int kPs93Pad = 16;  // copies of the last pair (ending nothing) past the end of the list
+
 struct DevTables {
-  const double *xs, *ws, *xl, *wl;
-  const int *p93l, *p93r, *p92l, *p92r;
+  CPtr<double> xs, ws, xl, wl;
+  CPtr<int> p93l, p93r, p92l, p92r;
+  CPtr<Ps93Pair> v93;
+  CPtr<int> vis;  // a small-grid point's place in the PS93 visit order
+  // T entries of a triplet (build_templates): packed (lambda1, lambda2, alpha + beta, l), channel after channel; those
+  // of channel l < L at [toff(la, lb, l), toff(la, lb, l + 1)) (t2_off)
+  CPtr<int> tmpl, toff;
   const double *bessel;
   const double *poly2sph;
   const double *omega;
-  const int *ijk, *ijkIndex;
-  const double *binom;  // binom[n*16+k], n,k <= 15
+  CPtr<int> ijk, ijkIndex;
+  CPtr<double> binom;  // binom[n*16+k], n,k <= 15
   int ijkDim, tmDim, lorder;
   int omL, omLambda, omAlpha;
   double tol, lnAcc1, lnAcc2, accuracy;
@@ -112,24 +164,52 @@ struct DevTables {
 };
 
 struct DevJob {
-  const ecp_xyz *atoms;
-  const int *atom_maxl;
-  const ecp_shell *shells;
-  const double *pa, *pd;
-  const ecp_centre *cent;
-  const ecp_gauss *gauss;
-  const ecp_window *win;
-  const ecp_triplet *trip;
+  CPtr<ecp_xyz> atoms;
+  CPtr<int> atom_maxl;
+  CPtr<ecp_shell> shells;
+  CPtr<double> pa, pd;
+  CPtr<ecp_centre> cent;
+  CPtr<ecp_gauss> gauss;
+  CPtr<ecp_window> win;
+  CPtr<ecp_triplet> trip;
   int ntrip;
   double *UL, *Ut, *F, *ang;
   int FL, UK, angL, ang_lam, ang_c;
   int maxPairs;
   int deriv;  // derivative order: F slabs per run 0..deriv, angular tables to lmax + deriv
-  int ptmajor;  // the type-2 F and U rows point-major (per-class sequence), else row-major
+  CPtr<int> teoff;  // per triplet: its first T entry in the job's T arrays
+  int US;            // U row stride: channels times powers
 };
 
 // ---------------------------------------------------------------------------
 // numerical primitives
+
+// The PS93 recurrences and test after level lv (gc_integrators.c:156-217);
+// any: the level had a point in the window.  True when the integral has
+// converged, to *res.  After level lv the rule has n = 3 2^(lv / 2) points in
+// its estimate, and the levels take turns (j = 0 after odd ones): the
+// divisions are by 9 2^h, three operations each (div_const's, with a
+// reciprocal that is exact but for the factor 1 / 9).
+__device__ __forceinline__ bool ps93_level(int lv, bool any, double tol, double I, double &p, double &q,
+                                           double *res) {
+  const int h = lv >> 1;
+  const double b = (double)(9 << h), y = ldexp(1.0 / 9.0, -h);
+  auto over = [&](double x) {
+    const double d = x * y;
+    return __builtin_fma(__builtin_fma(-b, d, x), y, d);
+  };
+  double err;
+  if (lv & 1) {
+    p += (I - q);
+    err = over(16 * fabs(q - 3 * p / 2));
+  } else {
+    err = over(16 * fabs(I - 2 * q));
+    q = I;
+  }
+  if (!(any && err < tol)) return false;
+  *res = over(16 * q);
+  return true;
+}
 
 // Radial powers other than 0, 1, 2 (rare in ECPs) through a call: inlined,
 // pow's registers set the fallbacks' budget (the type-1 fallback 152
@@ -150,10 +230,13 @@ __device__ __forceinline__ double ecp_pow(double r, double n) {
 __device__ __forceinline__ double eval_ecp(const DevJob &J, int centre, int l, double r) {
   double pot = 0.0;
   const double r2 = r * r;
-  const ecp_centre *__restrict__ C = J.cent + centre;
-  const ecp_gauss *__restrict__ g = J.gauss + C->g0;
-  const int end = C->gl[l + 1];
-  for (int i = C->gl[l]; i < end; i++) pot += ecp_pow(r, g[i].n) * g[i].d * exp(-g[i].a * r2);
+  const ecp_centre *C = J.cent + centre;
+  const ecp_gauss *g = J.gauss + cload(&C->g0);
+  const int end = cload(&C->gl[l + 1]);
+  for (int i = cload(&C->gl[l]); i < end; i++) {
+    const ecp_gauss x = cload(g + i);
+    pot += ecp_pow(r, x.n) * x.d * exp(-x.a * r2);
+  }
   return pot;
 }
 
@@ -244,67 +327,13 @@ __device__ __forceinline__ void bessel_k(const double *__restrict__ tab, double 
   }
 }
 
-// Real spherical harmonics written in place into out[(lmax+1)^2] (LDS or
-// global), with the arithmetic of spherical_harmonics.c:15-114: associated
-// Legendre recurrences without Condon-Shortley phase, normalisation
-// sqrt((2l+1)/(2pi) (l-m)!/(l+m)!), 1/sqrt(2) for m = 0, sin/cos(m phi) by
-// the angle-addition recurrence.
-__device__ void real_sph_inplace(int lmax, double theta, double phi, const double *__restrict__ fac,
-                                 const double *__restrict__ dfac, double *out) {
-#define RSH(l, m) ((l) * (l) + (l) + (m))
-  const double x = cos(theta);
-  for (int i = 0; i < (lmax + 1) * (lmax + 1); i++) out[i] = 0.0;
-  if (1.0 == x) {
-    for (int l = 0; l <= lmax; l++) out[RSH(l, 0)] = 1.0;
-  } else if (-1.0 == x) {
-    out[0] = 1.0;
-    for (int l = 1; l <= lmax; l++) out[RSH(l, 0)] = -out[RSH(l - 1, 0)];
-  } else {
-    const double s1 = sqrt(1.0 - x * x);
-    double sl = 1.0;
-    out[0] = 1.0;
-    for (int l = 1; l <= lmax; l++) {
-      sl = (l == 1) ? s1 : sl * s1;
-      out[RSH(l, l)] = sl * dfac[2 * l - 1];
-      int m = l - 1;
-      out[RSH(l, m)] = x * (2 * m + 1) * out[RSH(l - 1, m)];
-      if (l > 1)
-        for (m = 0; m <= l - 2; m++)
-          out[RSH(l, m)] = (x * (2 * l - 1) * out[RSH(l - 1, m)] - (l + m - 1) * out[RSH(l - 2, m)]) / (l - m);
-    }
-  }
-  const double sp = sin(phi), cp = cos(phi);
-  for (int l = 0; l <= lmax; l++) {
-    const double norm0 = sqrt((2.0 * l + 1.0) / (2.0 * M_PI));
-    out[RSH(l, 0)] = norm0 * out[RSH(l, 0)];
-    for (int m = 1; m <= l; m++) out[RSH(l, m)] = (sqrt(fac[l - m] / fac[l + m]) * norm0) * out[RSH(l, m)];
-    out[RSH(l, 0)] = out[RSH(l, 0)] / sqrt(2.0);
-    double sm = 0.0, cm = 1.0;
-    for (int m = 1; m <= l; m++) {
-      if (0.0 == phi) {
-        sm = 0.0;
-        cm = 1.0;
-      } else if (m == 1) {
-        sm = sp;
-        cm = cp;
-      } else {
-        const double ns = sp * cm + cp * sm;
-        cm = cp * cm - sp * sm;
-        sm = ns;
-      }
-      const double P = out[RSH(l, m)];
-      out[RSH(l, -m)] = P * sm;
-      out[RSH(l, m)] = P * cm;
-    }
-  }
-#undef RSH
-}
-
-// Column m >= 0 of real_sph_inplace (entries (l, +-m), l = m..lmax) with
-// the same arithmetic, so that the columns of one direction can be formed by
-// different lanes: s1^m by repeated multiplication, the diagonal, the first
-// subdiagonal and the three-term recurrence in l, the normalisation per
-// (l, m), and sin/cos(m phi) by the angle-addition recurrence from m = 1.
+// Column m >= 0 of the real spherical harmonics (entries (l, +-m), l =
+// m..lmax) with the arithmetic of spherical_harmonics.c:15-114, a column per
+// lane: associated Legendre recurrences without Condon-Shortley phase (s1^m
+// by repeated multiplication, the diagonal, the first subdiagonal and the
+// three-term recurrence in l), the normalisation sqrt((2l+1)/(2pi)
+// (l-m)!/(l+m)!), 1/sqrt(2) for m = 0, and sin/cos(m phi) by the
+// angle-addition recurrence from m = 1.
 // x = cos(theta), sp = sin(phi), cp = cos(phi): the direction's trigonometric
 // values, formed once per direction by the caller.
 __device__ void real_sph_column(int lmax, int m, double x, double phi, double sp, double cp,
@@ -391,8 +420,10 @@ __device__ __forceinline__ double dist(const ecp_xyz &a, const ecp_xyz &b) {
 // U tables of one (centre, row, chunk of 128 points): row C.L is the local
 // channel U_L (type 1), rows l < L the semi-local channels times r^k,
 // k < UK (type 2), zero past the channel's cut-off end[l].  The type-2 rows
-// are Ut[l][k][n], or with J.ptmajor point-major, Ut[l][n][k]: the lanes of
-// a type-2 group then read the same point of neighbouring k together.
+// are Ut[vis(n)][l][k]: the type-2 small grid reads all of a point's values
+// together, and the points in visit order, so that consecutive reads are
+// consecutive in memory (three of four of its integrals read the first
+// fifteen points only).
 __device__ void utab_rows(const DevTables &T, const DevJob &J, int c, int row, int chunk) {
   const ecp_centre C = J.cent[c];
   if (row > C.L) return;
@@ -405,19 +436,16 @@ __device__ void utab_rows(const DevTables &T, const DevJob &J, int c, int row, i
   }
   const int l = row;
   double P = (n <= C.end[l]) ? eval_ecp(J, c, l, r) : 0.0;
-  const size_t rs = J.ptmajor ? 1 : SO;  // stride between the powers k
-  double *dst = J.Ut + C.Ut_off + (size_t)l * J.UK * SO + (J.ptmajor ? (size_t)n * J.UK : (size_t)n);
+  double *dst = J.Ut + C.Ut_off + (size_t)T.vis[n] * J.US + l * J.UK;
   dst[0] = P;
   for (int k = 1; k < J.UK; k++) {
     P = P * r;
-    dst[k * rs] = P;
+    dst[k] = P;
   }
 }
 
-// F[centre][run][shell][lambda][n] (type2.c:263-303), or with J.ptmajor
-// F[centre][run][shell][n][lambda] (the lanes of a type-2 group then read
-// the same point of neighbouring lambda together), one block per
-// non-skipped (centre, shell, run); the whole slab is written (zeros outside
+// F[centre][run][shell][vis(n)][lambda] (type2.c:263-303; points in visit
+// order like the U rows), one block per non-skipped (centre, shell, run); the whole slab is written (zeros outside
 // the window).
 template <int LM>
 __device__ void ftab_slab(const DevTables &T, const DevJob &J, const ecp_centre &C, int sl, int run,
@@ -444,11 +472,10 @@ __device__ void ftab_slab(const DevTables &T, const DevJob &J, const ecp_centre 
         for (int i = 0; i <= LM; i++) acc[i] += da * K[i] * e;
       }
     }
-    const size_t rs = J.ptmajor ? 1 : SO;  // stride between the orders lambda
-    double *row = slab + (J.ptmajor ? (size_t)n * J.FL : (size_t)n);
+    double *row = slab + (size_t)T.vis[n] * J.FL;
 #pragma unroll
-    for (int i = 0; i <= LM; i++) row[i * rs] = acc[i];
-    for (int i = LM + 1; i < J.FL; i++) row[i * rs] = 0.0;
+    for (int i = 0; i <= LM; i++) row[i] = acc[i];
+    for (int i = LM + 1; i < J.FL; i++) row[i] = 0.0;
   }
 }
 
@@ -473,7 +500,7 @@ __device__ void ftab_item(const DevTables &T, const DevJob &J, int2 it) {
 constexpr int kAngRsph = (ECP_MAX_L + ECP_MAX_LBS) * (ECP_MAX_L + ECP_MAX_LBS);
 
 __device__ void ang_item(const DevTables &T, const DevJob &J, int2 it, const double *__restrict__ fac,
-                         const double *__restrict__ dfac, double *rsph) {
+                         const double *__restrict__ dfac, double *rsph, double *s_dir, int part, int nparts) {
   const ecp_centre C = J.cent[it.x];
   const int A = C.atom0 + it.y;
   const int lmax_a = J.atom_maxl[A] + J.deriv;
@@ -482,14 +509,21 @@ __device__ void ang_item(const DevTables &T, const DevJob &J, int2 it, const dou
     const ecp_xyz a = J.atoms[A], c = J.atoms[C.atom];
     double r, th, ph;
     sph_coords(a.x - c.x, a.y - c.y, a.z - c.z, r, th, ph);
-    real_sph_inplace(lmax, th, ph, fac, dfac, rsph);
+    s_dir[0] = cos(th);
+    s_dir[1] = ph;
+    s_dir[2] = sin(ph);
+    s_dir[3] = cos(ph);
   }
+  __syncthreads();
+  // one column m of the harmonics per lane
+  if ((int)threadIdx.x <= lmax)
+    real_sph_column(lmax, threadIdx.x, s_dir[0], s_dir[1], s_dir[2], s_dir[3], fac, dfac, rsph);
   __syncthreads();
   const int d1 = ECP_DIM_L(T.omLambda), d2 = ECP_DIM_C(T.omAlpha);
   const int nlm = C.L * C.L, nc = ECP_DIM_C(lmax_a);
   double *out = J.ang + C.ang_off + (size_t)it.y * J.ang_lam * J.angL * J.angL * J.ang_c;
   const int total = (lmax + 1) * nlm * nc;
-  for (int idx = threadIdx.x; idx < total; idx += blockDim.x) {
+  for (int idx = part * 128 + (int)threadIdx.x; idx < total; idx += 128 * nparts) {
     const int cc = idx % nc;
     const int lm = (idx / nc) % nlm;
     const int lambda = idx / (nc * nlm);
@@ -681,7 +715,6 @@ __device__ __forceinline__ void type1_body(int bid, const DevTables &T, const De
       I[e] = p[e] + t;
     });
     for (int lv = 2; lv < lv1; lv++) {
-      const int j = T.s93.lvl_j[lv], nn = T.s93.lvl_n[lv];
       int cnt = 0;
       for (int k = T.s93.lvl_begin[lv]; k < T.s93.lvl_begin[lv + 1]; k++) {
         const int li = T.p93l[k], ri = T.p93r[k];
@@ -692,17 +725,10 @@ __device__ __forceinline__ void type1_body(int bid, const DevTables &T, const De
 #pragma unroll
       for (int e = 0; e < NQ; e++) {
         if (done & (1ull << e)) continue;
-        double err;
-        if (j == 0) {
-          p[e] += (I[e] - q[e]);
-          err = 16 * fabs(q[e] - 3 * p[e] / 2) / (3 * nn);
-        } else {
-          err = 16 * fabs(I[e] - 2 * q[e]) / (3 * nn);
-          q[e] = I[e];
-        }
-        if (cnt > 0 && err < T.tol) {
+        double res;
+        if (ps93_level(lv, cnt > 0, T.tol, I[e], p[e], q[e], &res)) {
           done |= (1ull << e);
-          p[e] = 16 * q[e] / (3 * nn);
+          p[e] = res;
         } else if (t1_lost(I[e])) {
           lost |= (1ull << e);
         }
@@ -954,12 +980,12 @@ __device__ __forceinline__ void t1tail_body(int bid, int nb, const DevTables &T,
                                             unsigned char *__restrict__ status, double *s_T, int *s_pt) {
   constexpr int NQ = nq_of(LAB);
   static_assert(NQ <= 64, "one lane per Q entry");
-  const int ntail = *tcount, count = ntail + *fbcount;
+  const int ntail = cload(tcount), count = ntail + cload(fbcount);
   const int lane = threadIdx.x;
   for (int it = bid; it < count; it += nb) {
     const bool tail = it < ntail;
-    const int u = tail ? tq[it] : fbq[it - ntail];
-    const T1Unit U = units[u];
+    const int u = cload(tail ? tq + it : fbq + (it - ntail));
+    const T1Unit U = cload(units + u);
     const ecp_triplet tr = J.trip[U.trip];
     const ecp_centre Cn = J.cent[tr.centre];
     T1Geom G;
@@ -1059,18 +1085,10 @@ __device__ __forceinline__ void t1tail_body(int bid, int nb, const DevTables &T,
             I = sum_in_order(I, s_T + lane * kTS + k, o + np - k);
           }
           if (!mydone) {
-            const int j = T.s93.lvl_j[l], nn = T.s93.lvl_n[l];
-            double err;
-            if (j == 0) {
-              p += (I - q);
-              err = 16 * fabs(q - 3 * p / 2) / (3 * nn);
-            } else {
-              err = 16 * fabs(I - 2 * q) / (3 * nn);
-              q = I;
-            }
-            if (any && err < T.tol) {
+            double res;
+            if (ps93_level(l, any, T.tol, I, p, q, &res)) {
               mydone = true;
-              p = 16 * q / (3 * nn);
+              p = res;
             } else {
               lost = t1_lost(I);
             }
@@ -1113,282 +1131,289 @@ __global__ __launch_bounds__(64) void k_t1tail(DevTables T, DevJob J, const T1Un
 // ---------------------------------------------------------------------------
 // type 2: one lane per T entry
 
-struct T2Group {
-  int trip, l, eoff, ne, tmpl, lmb;
-};
+// first entry of channel l in the T entries of shells la, lb
+__device__ __forceinline__ int t2_off(const DevTables &T, int la, int lb, int l) {
+  return T.toff[(la * (ECP_MAX_LBS + 1) + lb) * (ECP_MAX_L + 1) + l];
+}
 
 struct T2Args {
-  const T2Group *groups;
-  const int *goff;
-  const int *gfirst;  // per wave of 64 entries: the group of its first entry (one more at the end)
-  int ngroups, ntotal;
-  const int *tmpl;
   double *Tout;
   unsigned char *tfail;
-  int *gflag, *fbq, *fbcount;  // fbq: per class, the triplets with failed entries (qstride apart)
+  int *tnfail, *flist;  // per triplet: number of failed entries, listed at flist[teoff ...] in entry order
+  int *fbq, *fbcount;   // per fallback class, the triplets with failed entries (qstride apart)
   int qstride;
-  int *flist;
-  int *tclaim;                  // per triplet: queued for the fallback
-  const unsigned char *tcls2;   // per triplet: its fallback class max(la, lb) + L - 1
+  const unsigned char *tcls2;  // per triplet: its fallback class max(la, lb) + L - 1
 };
 
-// A failed entry, for the large-grid fallback: gflag[g] counts the group's
-// entries, listed (in any order) at flist[eoff ...]; the triplet's first one
-// queues the triplet, whose listed entries of all groups the fallback takes
-// together
-__device__ __forceinline__ void t2_enlist(const T2Args &A, int gid, int g, const T2Group &G) {
-  const int k = atomicAdd(&A.gflag[g], 1);
-  A.flist[G.eoff + k] = gid - G.eoff;
-  if (k == 0 && atomicExch(&A.tclaim[G.trip], 1) == 0) {
-    const int c = A.tcls2[G.trip];
-    const int slot = atomicAdd(&A.fbcount[c], 1);
-    A.fbq[(size_t)c * A.qstride + slot] = G.trip;
-  }
-}
-
-// v of lane (quad base + X) in all four lanes of each quad
-template <int X>
-__device__ __forceinline__ double quad_value(double v) {
-  constexpr int perm = X * 0x55;  // quad_perm [X, X, X, X]
-  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), perm, 0xF, 0xF, true);
-  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), perm, 0xF, 0xF, true);
-  return __hiloint2double(hi, lo);
-}
-
-__device__ __forceinline__ double lane_get(double v, int src) {
-  return __hiloint2double(__shfl(__double2hiint(v), src, 64), __shfl(__double2loint(v), src, 64));
-}
-
-// Type-2 small grid: one wave per 64 T entries.  First a lane per entry runs
-// PS93 levels 0 to 4, eleven points whose reads are all issued before their
-// sums are formed: all but a few per cent of the entries converge there.
-// The few left are then dealt to the lanes four to an entry, sixteen entries
-// at a time: sixteen point pairs a step, four per lane with their reads
-// issued together, whose sums every lane of the quad adds in pair order with
-// the PS93 test at each level's end, so the arithmetic is that of the
-// lane-serial integrator.  (One lane per entry to the end, a straggler held
-// its wave for 372 more points read one level at a time: 107 us alone on the
-// 50-atom cluster, 3.4 ms on 256 uneven molecules.)
-constexpr int kT2Head = 5;  // levels of the first part
-
-struct T2Rows {
-  const double *Fa, *Fb, *Uu;
-  int pF, pU, gs, ge;
-};
-
-__device__ __forceinline__ T2Rows t2_rows(const DevJob &J, const T2Group &G, int code) {
-  const int l1 = code & 0xff, l2 = (code >> 8) & 0xff, l3 = (code >> 16) & 0xff;
-  const ecp_triplet tr = J.trip[G.trip];
-  const ecp_centre *__restrict__ C = J.cent + tr.centre;
-  // point and row strides of the F and U rows (layouts as the tables kernel writes them)
-  const int rs = J.ptmajor ? 1 : SO;
-  const int F_off = C->F_off, nsh = C->nsh, shell0 = C->shell0;
-  T2Rows R;
-  R.pF = J.ptmajor ? J.FL : 1;
-  R.pU = J.ptmajor ? J.UK : 1;
-  R.Fa = J.F + F_off + ((size_t)tr.powa * nsh + (tr.sa - shell0)) * J.FL * SO + (size_t)l1 * rs;
-  R.Fb = J.F + F_off + ((size_t)tr.powb * nsh + (tr.sb - shell0)) * J.FL * SO + (size_t)l2 * rs;
-  R.Uu = J.Ut + C->Ut_off + (size_t)G.l * J.UK * SO + (size_t)l3 * rs;
-  R.gs = tr.gs;
-  R.ge = tr.ge;
-  return R;
-}
-
-// integrator state of an entry after the first part
+// integrator state of a T entry
 struct T2State {
   double p, q, I, res;
   bool done;
-  // the PS93 recurrences and test after level lv (gc_integrators.c:156-217);
-  // any: the level had a point in the window
   __device__ __forceinline__ void level(const DevTables &T, int lv, bool any) {
-    if (done) return;
-    const int j = T.s93.lvl_j[lv], nn = T.s93.lvl_n[lv];
-    double err;
-    if (j == 0) {
-      p += (I - q);
-      err = 16 * fabs(q - 3 * p / 2) / (3 * nn);
-    } else {
-      err = 16 * fabs(I - 2 * q) / (3 * nn);
-      q = I;
-    }
-    if (any && err < T.tol) {
-      res = 16 * q / (3 * nn);
-      done = true;
-    }
+    if (!done) done = ps93_level(lv, any, T.tol, I, p, q, &res);
   }
 };
 
-__device__ __forceinline__ void type2_body(int bid, const DevTables &T, const DevJob &J, const T2Args &A, int *s_off,
-                                           int *s_open) {
-  const int lane = threadIdx.x;
-  const int gid = bid * 64 + lane;
-  // the wave's groups: at most 64 from gfirst on
-  const int g0 = A.gfirst[bid];
-  s_off[lane] = g0 + 1 + lane <= A.ngroups ? A.goff[g0 + 1 + lane] : INT_MAX;
-  __syncthreads();
-  const bool live = gid < A.ntotal;
-  int g = 0;
-  {
-    // the number of following groups that start at or before this entry
-    int lo = 0, hi = 64;
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if (s_off[mid] <= gid) lo = mid + 1;
-      else hi = mid;
-    }
-    g = g0 + lo;
-  }
-  T2Group G{};
-  int code = 0;
-  T2State S{0.0, 0.0, 0.0, 0.0, true};
-  if (live) {
-    G = A.groups[g];
-    code = A.tmpl[G.tmpl + (gid - G.eoff)];
-    const T2Rows R = t2_rows(J, G, code);
-    constexpr int NP = 4;  // point pairs of levels 2 to 4
-    double fa[2 * NP + 3], fb[2 * NP + 3], fu[2 * NP + 3];
-    const int n0[3] = {T.s93.centre, T.s93.first_l, T.s93.first_r};
-#pragma unroll
-    for (int i = 0; i < 3; i++) {
-      fa[i] = R.Fa[n0[i] * R.pF];
-      fb[i] = R.Fb[n0[i] * R.pF];
-      fu[i] = R.Uu[n0[i] * R.pU];
-    }
-#pragma unroll
-    for (int k = 0; k < NP; k++) {
-      const int li = T.p93l[k], ri = T.p93r[k], i = 3 + 2 * k;
-      fa[i] = fb[i] = fu[i] = fa[i + 1] = fb[i + 1] = fu[i + 1] = 0.0;
-      if (li >= R.gs) {
-        fa[i] = R.Fa[li * R.pF];
-        fb[i] = R.Fb[li * R.pF];
-        fu[i] = R.Uu[li * R.pU];
-      }
-      if (ri <= R.ge) {
-        fa[i + 1] = R.Fa[ri * R.pF];
-        fb[i + 1] = R.Fb[ri * R.pF];
-        fu[i + 1] = R.Uu[ri * R.pU];
-      }
-    }
-    auto f = [&](int i, int n) { return T.ws[n] * ((fa[i] * fb[i]) * fu[i]); };
-    S.p = f(0, n0[0]);
-    S.q = f(1, n0[1]) + f(2, n0[2]);
-    S.I = S.p + S.q;
-    S.done = false;
-    int k = 0;
-    bool any = false;
-#pragma unroll
-    for (int lv = 2; lv < kT2Head; lv++) {
-      any = false;
-#pragma unroll
-      for (int x = 0; x < (lv == 4 ? 2 : 1); x++, k++) {
-        const int li = T.p93l[k], ri = T.p93r[k], i = 3 + 2 * k;
-        any = any || li >= R.gs || ri <= R.ge;
-        S.I += (0.0 + f(i, li)) + f(i + 1, ri);
-      }
-      S.level(T, lv, any);
-    }
-  }
-  // the entries still open, four lanes each
-  unsigned long long failed = 0ull;
-  const unsigned long long om = __ballot(!S.done);
-  const int nopen = __popcll(om);
-  if (nopen) {
-    if (!S.done) s_open[__popcll(om & ((1ull << lane) - 1ull))] = lane;
-    __syncthreads();
-    const int r = lane & 3;
-    for (int o0 = 0; o0 < nopen; o0 += 16) {
-      const int oi = o0 + (lane >> 2);
-      const bool on = oi < nopen;
-      const int src = on ? s_open[oi] : s_open[o0];
-      T2State Q{lane_get(S.p, src), lane_get(S.q, src), lane_get(S.I, src), 0.0, !on};
-      T2Group Gq;
-      Gq.trip = __shfl(G.trip, src, 64);
-      Gq.l = __shfl(G.l, src, 64);
-      const T2Rows R = t2_rows(J, Gq, __shfl(code, src, 64));
-      // steps of 16 pairs, c0 + 4 i + x in lane x of the quad; the points of
-      // the next step are read ahead
-      const int np = T.s93.npairs;
-      int lv = kT2Head, c0 = T.s93.lvl_begin[kT2Head];
-      int li[4], ri[4];
-      auto points = [&](int b) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const int k = min(b + 4 * i + r, np - 1);
-          li[i] = T.p93l[k];
-          ri[i] = T.p93r[k];
-        }
-      };
-      points(c0);
-      for (; c0 < np; c0 += 16) {
-        if (!wave_any(!Q.done)) break;
-        double t[4];
-        {
-          double fa[8], fb[8], fu[8], w[8];
-#pragma unroll
-          for (int i = 0; i < 4; i++) {
-            fa[2 * i] = fb[2 * i] = fu[2 * i] = w[2 * i] = 0.0;
-            fa[2 * i + 1] = fb[2 * i + 1] = fu[2 * i + 1] = w[2 * i + 1] = 0.0;
-            if (!Q.done && li[i] >= R.gs) {
-              w[2 * i] = T.ws[li[i]];
-              fa[2 * i] = R.Fa[li[i] * R.pF];
-              fb[2 * i] = R.Fb[li[i] * R.pF];
-              fu[2 * i] = R.Uu[li[i] * R.pU];
-            }
-            if (!Q.done && ri[i] <= R.ge) {
-              w[2 * i + 1] = T.ws[ri[i]];
-              fa[2 * i + 1] = R.Fa[ri[i] * R.pF];
-              fb[2 * i + 1] = R.Fb[ri[i] * R.pF];
-              fu[2 * i + 1] = R.Uu[ri[i] * R.pU];
-            }
-          }
-          points(c0 + 16);
-#pragma unroll
-          for (int i = 0; i < 4; i++)
-            t[i] = (0.0 + w[2 * i] * ((fa[2 * i] * fb[2 * i]) * fu[2 * i])) +
-                   w[2 * i + 1] * ((fa[2 * i + 1] * fb[2 * i + 1]) * fu[2 * i + 1]);
-        }
-        // the pairs of this step that end a level
-        unsigned int ends = 0;
-        for (int x = lv; x < T.s93.nlevels && T.s93.lvl_begin[x + 1] <= c0 + 16; x++)
-          ends |= 1u << (T.s93.lvl_begin[x + 1] - 1 - c0);
-        // (past the last pair, nothing ends and nothing reads the sums.)
-        // The last pair of a level is its closest to the centre: the level
-        // has a point in the window where this pair does.
-        auto add = [&](int j, double v) {
-          Q.I += v;
-          if ((ends >> j) & 1u) {
-            Q.level(T, lv, T.p93l[c0 + j] >= R.gs || T.p93r[c0 + j] <= R.ge);
-            lv++;
-          }
-        };
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          add(4 * i, quad_value<0>(t[i]));
-          add(4 * i + 1, quad_value<1>(t[i]));
-          add(4 * i + 2, quad_value<2>(t[i]));
-          add(4 * i + 3, quad_value<3>(t[i]));
-        }
-      }
-      // back to the entries' own lanes
-      const int mine = __popcll(om & ((1ull << lane) - 1ull)) - o0;
-      const bool back = !S.done && mine >= 0 && mine < 16;
-      const int from = back ? 4 * mine : 0;
-      const double res = lane_get(Q.res, from);
-      const int ok = __shfl((int)Q.done, from, 64);
-      if (back) S.res = res;
-      failed |= __ballot(back && !ok);
-    }
-  }
-  if (!live) return;
-  const bool fail = (failed >> lane) & 1ull;
-  A.Tout[gid] = S.res;
-  A.tfail[gid] = fail;
-  if (fail) t2_enlist(A, gid, g, G);
+// Type-2 small grid: a lane group of 64 / G lanes per triplet, all channels.
+// Every entry's integrand is a product of one value each of the triplet's
+// rows at a point -- F_a (la + L of them), F_b, and r^k U_l (L (la + lb +
+// 1)), 12 to 42 doubles up to f shells and projectors -- which the group reads
+// once into LDS, one value per lane; the lanes then own the entries (R each
+// per pass) and form the integrands from LDS.  Read per entry instead, the
+// kernel was bound by the L1 cache's rate of accesses (1.9 G on 256 uneven
+// molecules, 3.1 ms at one per clock and CU, of 3.3 ms).
+// Levels 0 to 5, fifteen points read together, decide nearly all entries of
+// most triplets; where entries stay open, the levels up to 14 follow in
+// steps of NP = 4 point pairs (each ends its level or lies inside it),
+// the next step's values read ahead.  Point pairs
+// are added in order, with the PS93 test at each level's end.  Points outside
+// the pair's window need no test: F_a or F_b is 0 there; a step with all of
+// its points outside is passed over.
+constexpr int kT2Head = 6;      // levels of the first part
+constexpr int kT2HeadPairs = 6; // their point pairs from level 2 on
+constexpr int kT2HeadPts = 3 + 2 * kT2HeadPairs;
+
+// Workgroups go to the eight XCDs, each with its own L2, in turn: workgroup b
+// of n takes the item that leaves runs of 64 consecutive items -- the
+// triplets of one centre, which share its tables -- to one XCD.  (Items in
+// turn, every XCD read every centre's F rows: 25 GB from HBM on 256 uneven
+// molecules where the tables hold 1.8 GB, the type-2 small grid at 7.7 TB/s.)
+__device__ __forceinline__ int xcd_item(int b, int n) {
+  constexpr int S = 64, N = 8 * S;
+  if (b >= n / N * N) return b;
+  const int r = b % N;
+  return b - r + (r % 8) * S + r / 8;
 }
 
-__global__ __launch_bounds__(64) void k_type2(DevTables T, DevJob J, T2Args A) {
-  __shared__ int s_off[64], s_open[64];
-  type2_body(blockIdx.x, T, J, A, s_off, s_open);
+// doubles of LDS of a wave; CH: 16-byte chunks of a point's values
+__host__ __device__ constexpr int t2_lds(int G, int NP, int CH) {
+  return G * 2 * CH * (2 * NP > kT2HeadPts ? 2 * NP : kT2HeadPts);
+}
+
+typedef double dpair __attribute__((ext_vector_type(2)));
+
+// LP: lanes that read a point together, two values (16 bytes) each; the F and
+// U rows have even lengths, so that every chunk is aligned
+template <int G, int NP, int R, int CH>
+__device__ __forceinline__ void type2_body(int bid, const DevTables &T, const DevJob &J, const T2Args &A,
+                                           const int *__restrict__ tlist, int ntl, double *s_all) {
+  constexpr int W = 64 / G, LP = G == 1 ? 32 : 16, PT = W / LP, X = (CH + LP - 1) / LP, ROW = 2 * CH;
+  const int grp = (int)threadIdx.x / W, lid = (int)threadIdx.x % W;
+  const int pt = lid / LP, pl = lid % LP;  // point of a read, lane of the point
+  double *s_v = s_all + grp * t2_lds(1, NP, CH);
+  const int ti = bid * G + grp;
+  const bool active = ti < ntl;
+  const int t = cload(tlist + (active ? ti : 0));
+  const ecp_triplet tr = J.trip[t];
+  const ecp_centre C = J.cent[tr.centre];
+  const int L = C.L, la = tr.la, lb = tr.lb, na = la + L, nb = lb + L, nu = la + lb + 1;
+  const int ca = (na + 1) >> 1, cb = (nb + 1) >> 1, cu = (nu + 1) >> 1;  // chunks of F_a, F_b, a channel's U
+  const int nch = ca + cb + L * cu, gs = tr.gs, ge = tr.ge;
+  const int t0 = t2_off(T, la, lb, 0), ne = active ? t2_off(T, la, lb, L) - t0 : 0, eoff = J.teoff[t];
+  // this lane's chunks of a point: where they are, and their point stride
+  const double *src[X];
+  int st[X];
+#pragma unroll
+  for (int x = 0; x < X; x++) {
+    const int v = pl + x * LP;
+    if (v < ca + cb) {
+      const bool b = v >= ca;
+      const int run = b ? tr.powb : tr.powa, sh = (b ? tr.sb : tr.sa) - C.shell0;
+      src[x] = J.F + C.F_off + ((size_t)run * C.nsh + sh) * J.FL * SO + 2 * (b ? v - ca : v);
+      st[x] = J.FL;
+    } else {
+      const int y = v - ca - cb, l = (int)(((float)y + 0.5f) / (float)cu);
+      src[x] = J.Ut + C.Ut_off + l * J.UK + 2 * (y - l * cu);
+      st[x] = J.US;
+    }
+    if (v >= nch) {  // none: any readable place
+      src[x] = J.Ut + C.Ut_off;
+      st[x] = 0;
+    }
+  }
+  int nfail = 0;
+  for (int e0 = 0; __ballot(e0 < ne) != 0ull; e0 += W * R) {
+    // LDS offsets of the entries' values, and their states
+    int oa[R], ob[R], ou[R];
+    T2State S[R];
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+      const int e = e0 + i * W + lid;
+      S[i] = T2State{0.0, 0.0, 0.0, 0.0, e >= ne};
+      const int code = e < ne ? T.tmpl[t0 + e] : 0;
+      oa[i] = code & 0xff;
+      ob[i] = 2 * ca + ((code >> 8) & 0xff);
+      ou[i] = 2 * (ca + cb) + (code >> 24) * 2 * cu + ((code >> 16) & 0xff);
+    }
+    // value of point slot P of entry i, weighted
+    auto f = [&](int i, int P, double w) {
+      const double *v = s_v + P * ROW;
+      return w * ((v[oa[i]] * v[ob[i]]) * v[ou[i]]);
+    };
+    Ps93Pair hp[kT2HeadPairs];
+#pragma unroll
+    for (int k = 0; k < kT2HeadPairs; k++) hp[k] = T.v93[k];
+    {
+      // rows in visit order: the centre, the first pair, the pairs hp
+      constexpr int NI = (kT2HeadPts + PT - 1) / PT;
+      dpair v[X][NI];
+#pragma unroll
+      for (int P = 0; P < NI; P++) {
+        const int n = min(P * PT + pt, kT2HeadPts - 1);
+#pragma unroll
+        for (int x = 0; x < X; x++) v[x][P] = *(const dpair *)(src[x] + n * st[x]);
+      }
+#pragma unroll
+      for (int P = 0; P < NI; P++)
+#pragma unroll
+        for (int x = 0; x < X; x++)
+          if (pl + x * LP < CH && P * PT + pt < kT2HeadPts)
+            *(dpair *)(s_v + (P * PT + pt) * ROW + 2 * (pl + x * LP)) = v[x][P];
+    }
+    __syncthreads();
+    {
+      const double w0 = T.ws[T.s93.centre], w1 = T.ws[T.s93.first_l], w2 = T.ws[T.s93.first_r];
+#pragma unroll
+      for (int i = 0; i < R; i++) {
+        S[i].p = f(i, 0, w0);
+        S[i].q = f(i, 1, w1) + f(i, 2, w2);
+        S[i].I = S[i].p + S[i].q;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int k = 0; k < kT2HeadPairs; k++) {
+        // (a few pairs' reads in flight at a time: registers)
+        if (k & 1) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < R; i++) {
+          S[i].I += (0.0 + f(i, 3 + 2 * k, hp[k].wl)) + f(i, 4 + 2 * k, hp[k].wr);
+          if (hp[k].ends) S[i].level(T, hp[k].ends, hp[k].li >= gs || hp[k].ri <= ge);
+        }
+      }
+    }
+    __syncthreads();
+    // the levels left, for the groups with an entry still open
+    const int np = T.s93.npairs;
+    int c0 = T.s93.lvl_begin[kT2Head];
+    auto group_open = [&]() {
+      bool o = false;
+#pragma unroll
+      for (int i = 0; i < R; i++) o = o || !S[i].done;
+      const unsigned long long m = __ballot(o);
+      return G == 1 ? m != 0ull : ((m >> (grp * W)) & ((1ull << (W & 63)) - 1ull)) != 0ull;
+    };
+    if (wave_any(group_open())) {
+      // a step's pairs (read ahead with their values) and the values
+      Ps93Pair pr[NP];
+      constexpr int NI = 2 * NP / PT;
+      dpair v[X][NI];
+      auto read = [&](int b) {
+#pragma unroll
+        for (int j = 0; j < NP; j++) pr[j] = T.v93[b + j];
+        // (opaque to the loop optimiser, which would keep an address per
+        // read in registers, and spill)
+        int n0 = 3 + 2 * b;
+        asm volatile("" : "+s"(n0));
+#pragma unroll
+        for (int x = 0; x < X; x++) {
+          const double *q = src[x] + (n0 + pt) * st[x];
+          const int step = PT * st[x];
+#pragma unroll
+          for (int P = 0; P < NI; P++, q += step) v[x][P] = *(const dpair *)q;
+        }
+      };
+      // the step from b on has a point in a group's window
+      auto inside = [&](int b) {
+        const Ps93Pair z = T.v93[b + NP - 1];
+        return wave_any(z.li >= gs || z.ri <= ge);
+      };
+      bool on = inside(c0);
+      if (on) read(c0);
+      for (;;) {
+        Ps93Pair cur[NP];
+        const bool now = on;
+        if (now) {
+#pragma unroll
+          for (int P = 0; P < NI; P++)
+#pragma unroll
+            for (int x = 0; x < X; x++)
+              if (pl + x * LP < CH) *(dpair *)(s_v + (P * PT + pt) * ROW + 2 * (pl + x * LP)) = v[x][P];
+#pragma unroll
+          for (int j = 0; j < NP; j++) cur[j] = pr[j];
+        }
+        __syncthreads();
+        const int b = c0;
+        c0 += NP;
+        const bool last = c0 >= np;
+        on = !last && inside(c0);
+        if (on) read(c0);
+        if (now) {
+#pragma unroll
+          for (int i = 0; i < R; i++) {
+            if (!wave_any(!S[i].done)) continue;
+#pragma unroll
+            for (int j0 = 0; j0 < NP; j0 += 4) {
+              double t[4];
+#pragma unroll
+              for (int j = 0; j < 4; j++)
+                t[j] = (0.0 + f(i, 2 * (j0 + j), cur[j0 + j].wl)) + f(i, 2 * (j0 + j) + 1, cur[j0 + j].wr);
+#pragma unroll
+              for (int j = 0; j < 4; j++) S[i].I += t[j];
+              // level 6 ends with the first four pairs of its step
+              const Ps93Pair &z = cur[j0 + 3];
+              if (z.ends) S[i].level(T, z.ends, z.li >= gs || z.ri <= ge);
+              __builtin_amdgcn_sched_barrier(0);
+            }
+          }
+        } else {
+          const Ps93Pair z = T.v93[b + NP - 1];
+          if (z.ends)
+#pragma unroll
+            for (int i = 0; i < R; i++) S[i].level(T, z.ends, false);
+        }
+        __syncthreads();
+        if (last || !wave_any(group_open())) break;
+      }
+    }
+    // results; the failed entries in entry order
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+      const int e = e0 + i * W + lid;
+      const bool fail = e < ne && !S[i].done;
+      if (e < ne) {
+        A.Tout[eoff + e] = S[i].res;
+        A.tfail[eoff + e] = fail;
+      }
+      unsigned long long m = __ballot(fail);
+      if (G > 1) m = (m >> (grp * W)) & ((1ull << (W & 63)) - 1ull);
+      if (fail) A.flist[eoff + nfail + __popcll(m & ((1ull << lid) - 1ull))] = e;
+      nfail += __popcll(m);
+    }
+  }
+  if (active && lid == 0) {
+    A.tnfail[t] = nfail;
+    if (nfail) {
+      const int c = A.tcls2[t];
+      A.fbq[(size_t)c * A.qstride + atomicAdd(&A.fbcount[c], 1)] = t;
+    }
+  }
+}
+
+// The triplets of classes above kT2PackLab (tlist[m .. nt)), one per wave,
+// then those up to it (tlist[0 .. m)), kT2Pack to a wave.  CH, CHP: 16-byte
+// chunks of a point's values, of a triplet of either kind.
+constexpr int kT2Pack = 2, kT2PackLab = 2, kT2Pairs = 4;
+
+
+template <int CH, int CHP>
+__global__ __launch_bounds__(64, CH <= 24 ? 4 : 3) void k_type2(DevTables T, DevJob J, T2Args A, const int *__restrict__ tlist,
+                                                int m) {
+  __shared__ __align__(16) double s_v[t2_lds(1, kT2Pairs, CH) > t2_lds(kT2Pack, kT2Pairs, CHP)
+                                          ? t2_lds(1, kT2Pairs, CH)
+                                          : t2_lds(kT2Pack, kT2Pairs, CHP)];
+  const int n = J.ntrip - m, np = (m + kT2Pack - 1) / kT2Pack, b = blockIdx.x;
+  if (b < n) type2_body<1, kT2Pairs, 2, CH>(xcd_item(b, n), T, J, A, tlist + m, n, s_v);
+  else type2_body<kT2Pack, kT2Pairs, 2, CHP>(xcd_item(b - n, np), T, J, A, tlist, m, s_v);
 }
 
 // type-2 fallback (calcT_FM06, type2.c:417-528): one wave per (triplet with
@@ -1418,14 +1443,13 @@ static_assert(ECP_MAX_LAB < 16 && kFb2Cnt + kMaxLMB < kFbcSlots, "queue counter 
 // OWN: entries owned per lane and pass
 template <int LMB, int OWN>
 __device__ __forceinline__ void fb2_body(int bid, int nb, const DevTables &T, const DevJob &J,
-                                         const T2Group *__restrict__ groups, const int *__restrict__ tmpl,
                                          const int *__restrict__ fbq, const int *__restrict__ fbcount,
                                          double *__restrict__ fbT, unsigned char *__restrict__ status,
-                                         const int *__restrict__ gcount, const int *__restrict__ flist,
-                                         const int *__restrict__ tgfirst, int nslot, int nsplit, int share, double *s_cu,
+                                         const int *__restrict__ tnfail, const int *__restrict__ flist,
+                                         int nslot, int nsplit, int share, double *s_cu,
                                          double *s_rn, double *s_ka, double *s_kb, double *s_t) {
   const int lane = threadIdx.x;
-  const int count = *fbcount;
+  const int count = cload(fbcount);
   // items (split, slot, triplet): split k takes the k-th share of the entries
   const long per_split = (long)count * nslot;
   const long total = per_split * nsplit;
@@ -1433,24 +1457,20 @@ __device__ __forceinline__ void fb2_body(int bid, int nb, const DevTables &T, co
     const int split = (int)(it / per_split);
     const int rest = (int)(it - split * per_split);
     const int slot = rest / count;
-    const int t = fbq[rest - slot * count];
+    const int t = cload(fbq + (rest - slot * count));
     const ecp_triplet tr = J.trip[t];
     const ecp_shell Sa = J.shells[tr.sa], Sb = J.shells[tr.sb];
     const int npairs = Sa.K * Sb.K;
     const ecp_centre Cn = J.cent[tr.centre];
-    // the triplet's groups (one per semi-local channel l): their failed
-    // entries, listed one group after another
-    const int g0 = tgfirst[t], L = Cn.L;
-    int nfail = 0, lmax = 0;
+    // the triplet's failed entries, and the channels they are of
+    const int L = Cn.L, nfail = cload(tnfail + t), eoff = J.teoff[t], t0 = t2_off(T, tr.la, tr.lb, 0);
     unsigned int chan = 0;
-    for (int l = 0; l < L; l++) {
-      const int c = gcount[g0 + l];
-      nfail += c;
-      if (c) {
-        lmax = l;
-        chan |= 1u << l;
-      }
+    {
+      unsigned int m = 0;
+      for (int k = lane; k < nfail; k += 64) m |= 1u << (T.tmpl[t0 + flist[eoff + k]] >> 24);
+      for (int l = 0; l < L; l++) chan |= wave_any((m >> l) & 1u) ? 1u << l : 0u;
     }
+    const int lmax = 31 - __clz((int)chan);
     // shares of at least `share` entries, in whole chunks
     const int ns = max(1, min(nsplit, (nfail + share - 1) / share));
     const int per = ((nfail + ns - 1) / ns + kFb2Chunk - 1) / kFb2Chunk * kFb2Chunk;
@@ -1469,17 +1489,10 @@ __device__ __forceinline__ void fb2_body(int bid, int nb, const DevTables &T, co
       for (int i = 0; i < OWN; i++) {
         code[i] = 0;
         eo[i] = -1;
-        int kk = w0 + i * 64 + lane;
         if (i * 64 + lane >= nhere) continue;
-        int l = 0, c = gcount[g0];
-        while (kk >= c) {
-          kk -= c;
-          c = gcount[g0 + ++l];
-        }
-        const T2Group G = groups[g0 + l];
-        const int e = flist[G.eoff + kk];
-        code[i] = tmpl[G.tmpl + e] | (l << 24);
-        eo[i] = G.eoff + e;
+        const int e = flist[eoff + w0 + i * 64 + lane];
+        code[i] = T.tmpl[t0 + e];
+        eo[i] = eoff + e;
       }
       for (int pb0 = 0; pb0 < npairs; pb0 += 64) {
         bool mine_live = false;
@@ -1709,14 +1722,12 @@ __global__ __launch_bounds__(64) void k_t1tail_fused(DevTables T, DevJob J, T1Se
 }
 
 struct T2Set {
-  const T2Group *groups;
-  const int *tmpl;
   const int *fbq2;  // per class, the triplets with failed entries (nt apart)
   const int *fbc;
   double *fbT;
   unsigned char *stat;
   int nt;
-  const int *gcount, *flist, *tgfirst;
+  const int *tnfail, *flist;
   int nslot, nsplit, share;
   int cu_rows, rn_rows, k_rows;  // LDS rows: U_l of the job's channels, powers of r, K of its largest class
 };
@@ -1736,8 +1747,8 @@ __global__ __launch_bounds__(64, MAXLMB <= 7 ? 3 : 2) void k_fb2_fused(DevTables
 #define X(L)                                                                                                     \
   case L:                                                                                                        \
     if constexpr (L <= MAXLMB)                                                                                   \
-      fb2_body<L, OWN>(bid, nb, T, J, S.groups, S.tmpl, S.fbq2 + (size_t)L * S.nt, S.fbc + kFb2Cnt + L, S.fbT, S.stat, \
-                  S.gcount, S.flist, S.tgfirst, S.nslot, S.nsplit, S.share, s_cu, s_rn, s_ka, s_kb, s_t);         \
+      fb2_body<L, OWN>(bid, nb, T, J, S.fbq2 + (size_t)L * S.nt, S.fbc + kFb2Cnt + L, S.fbT, S.stat, S.tnfail,   \
+                       S.flist, S.nslot, S.nsplit, S.share, s_cu, s_rn, s_ka, s_kb, s_t);                       \
     break;
     ECP_CASES_LMB(X)
 #undef X
@@ -1755,9 +1766,6 @@ struct AsmArgs {
   const T1Unit *units1;
   const int *t1first;        // per triplet: first type-1 unit
   const double *qout;
-  const T2Group *groups;
-  const int *tgfirst;        // per triplet: first group
-  const int *tmpl;
   const double *Tout;
   const unsigned char *tfail;
   const double *fbT;
@@ -2164,26 +2172,23 @@ __global__ __launch_bounds__(kAsmThreads) void k_asm2(DevTables T, DevJob J, Asm
   const double rBC[3] = {rb.x - rc.x, rb.y - rc.y, rb.z - rc.z};
   const V3 vA{rAC[0], rAC[1], rAC[2]}, vB{rBC[0], rBC[1], rBC[2]};
   const int D = T.ijkDim;
-  const int g0 = A.tgfirst[t];
+  const int t0 = t2_off(T, la, lb, 0), eoff = J.teoff[t];
   for (int i = threadIdx.x; i < nca * ncb; i += blockDim.x) blk[i] = 0.0;
   __syncthreads();
   const int nlm2 = J.angL * J.angL;
   const double *angA = J.ang + Cn.ang_off + (size_t)(Sa.atom - Cn.atom0) * J.ang_lam * nlm2 * J.ang_c;
   const double *angB = J.ang + Cn.ang_off + (size_t)(Sb.atom - Cn.atom0) * J.ang_lam * nlm2 * J.ang_c;
   for (int l = 0; l < Cn.L; l++) {
-    const T2Group G = A.groups[g0 + l];
+    const int eb = t2_off(T, la, lb, l) - t0, ee = t2_off(T, la, lb, l + 1) - t0;
     const int d1 = la + l + 1, d2 = lb + l + 1, d3 = lab + 1;
     for (int i = threadIdx.x; i < d1 * d2 * d3; i += blockDim.x) Tl[i] = 0.0;
     __syncthreads();
-    for (int e = threadIdx.x; e < G.ne; e += blockDim.x) {
-      const int code = A.tmpl[G.tmpl + e];
+    for (int e = eb + (int)threadIdx.x; e < ee; e += kAsmThreads) {
+      const int code = T.tmpl[t0 + e];
       const int l1 = code & 0xff, l2 = (code >> 8) & 0xff, l3 = (code >> 16) & 0xff;
-      double v;
-      if (!A.tfail[G.eoff + e]) {
-        v = A.Tout[G.eoff + e];
-      } else {
-        v = sum_in_order(0.0, A.fbT + (size_t)(G.eoff + e) * J.maxPairs, Sa.K * Sb.K);
-      }
+      const double v = !A.tfail[eoff + e]
+                           ? A.Tout[eoff + e]
+                           : sum_in_order(0.0, A.fbT + (size_t)(eoff + e) * J.maxPairs, Sa.K * Sb.K);
       Tl[(l1 * d2 + l2) * d3 + l3] = v;
     }
     __syncthreads();
@@ -2224,7 +2229,7 @@ __global__ __launch_bounds__(kAsmThreads) void k_asm2p(DevTables T, DevJob J, As
   const int nca = ECP_DIM_C(la), ncb = ECP_DIM_C(lb);
   const ecp_xyz rc = J.atoms[Cn.atom], ra = J.atoms[Sa.atom], rb = J.atoms[Sb.atom];
   const V3 vA{ra.x - rc.x, ra.y - rc.y, ra.z - rc.z}, vB{rb.x - rc.x, rb.y - rc.y, rb.z - rc.z};
-  const int g0 = A.tgfirst[t];
+  const int t0 = t2_off(T, la, lb, 0), eoff = J.teoff[t];
   if (active)
     for (int i = lid; i < nca * ncb; i += W) blk[i] = 0.0;
   int Lw = active ? Cn.L : 0;
@@ -2236,22 +2241,20 @@ __global__ __launch_bounds__(kAsmThreads) void k_asm2p(DevTables T, DevJob J, As
   for (int l = 0; l < Lw; l++) {
     const bool on = active && l < Cn.L;
     const int d1 = la + l + 1, d2 = lb + l + 1, d3 = lab + 1;
-    T2Group Gr{};
+    int eb = 0, ee = 0;
     if (on) {
-      Gr = A.groups[g0 + l];
+      eb = t2_off(T, la, lb, l) - t0;
+      ee = t2_off(T, la, lb, l + 1) - t0;
       for (int i = lid; i < d1 * d2 * d3; i += W) Tl[i] = 0.0;
     }
     __syncthreads();
     if (on)
-      for (int e = lid; e < Gr.ne; e += W) {
-        const int code = A.tmpl[Gr.tmpl + e];
+      for (int e = eb + lid; e < ee; e += W) {
+        const int code = T.tmpl[t0 + e];
         const int l1 = code & 0xff, l2 = (code >> 8) & 0xff, l3 = (code >> 16) & 0xff;
-        double v;
-        if (!A.tfail[Gr.eoff + e]) {
-          v = A.Tout[Gr.eoff + e];
-        } else {
-          v = sum_in_order(0.0, A.fbT + (size_t)(Gr.eoff + e) * J.maxPairs, Sa.K * Sb.K);
-        }
+        const double v = !A.tfail[eoff + e]
+                             ? A.Tout[eoff + e]
+                             : sum_in_order(0.0, A.fbT + (size_t)(eoff + e) * J.maxPairs, Sa.K * Sb.K);
         Tl[(l1 * d2 + l2) * d3 + l3] = v;
       }
     __syncthreads();
@@ -2280,8 +2283,8 @@ size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 // The per-job tables in one launch of 128-thread blocks: the zero-fill of
 // per-run counters and flags (a kernel, so that the sequence can be captured
 // in a HIP graph without memset nodes), the U tables per (centre, row, point
-// chunk), the F slabs per (centre, shell, run) and the pair directions of
-// the type-1 units.  They are independent of each other; every consumer is
+// chunk), the F slabs per (centre, shell, run), the pair directions of
+// the type-1 units and the angular tables per (centre, atom).  They are independent of each other; every consumer is
 // a later launch.
 struct TabArgs {
   unsigned int *zero_base;
@@ -2291,6 +2294,9 @@ struct TabArgs {
   const T1Unit *units;       // type-1 units and their pair directions, 128 per workgroup
   int nunits;
   double *udir;
+  const int2 *ait;           // (centre, atom) pairs of the angular tables, aparts workgroups each
+  int nait, aparts;
+  const double *fac, *dfac;
 };
 
 // The pair direction k = 2 (za rAC + zb rBC) of a type-1 unit (type1.c:
@@ -2316,7 +2322,14 @@ __device__ void unit_dir(const DevJob &J, const T1Unit &U, double *out) {
 constexpr int kUtabChunks = (SO + 127) / 128;
 
 __global__ __launch_bounds__(128, 4) void k_tables(DevTables T, DevJob J, TabArgs A) {
+  __shared__ double rsph[kAngRsph], s_dir[4];
   int b = blockIdx.x;
+  // the longest items first
+  if (b < A.nait * A.aparts) {
+    ang_item(T, J, A.ait[b / A.aparts], A.fac, A.dfac, rsph, s_dir, b % A.aparts, A.aparts);
+    return;
+  }
+  b -= A.nait * A.aparts;
   if (b < A.nzb) {
     for (size_t i = (size_t)b * 128 + threadIdx.x; i < A.zero_words; i += (size_t)A.nzb * 128) A.zero_base[i] = 0u;
     return;
@@ -2338,23 +2351,15 @@ __global__ __launch_bounds__(128, 4) void k_tables(DevTables T, DevJob J, TabArg
   if (u < A.nunits) unit_dir(J, A.units[u], A.udir + 4 * (size_t)u);
 }
 
-// angular tables: a launch of their own (few registers, high occupancy),
-// needed only by the type-2 assembly
-__global__ __launch_bounds__(128) void k_ang(DevTables T, DevJob J, const int2 *__restrict__ items,
-                                             const double *__restrict__ fac, const double *__restrict__ dfac) {
-  __shared__ double rsph[kAngRsph];
-  ang_item(T, J, items[blockIdx.x], fac, dfac, rsph);
-}
-
 // byte offsets of a job's arrays inside its device block: inputs (uploaded)
 // first, then device-only buffers
 struct JobLayout {
   size_t i_atoms = 0, i_amaxl = 0, i_sh = 0, i_pa = 0, i_pd = 0, i_cent = 0, i_gauss = 0, i_win = 0, i_trip = 0,
-         i_u1 = 0, i_t1f = 0, i_grp = 0, i_goff = 0, i_tgf = 0, i_fit = 0, i_ait = 0, i_tcls = 0, i_tcls2 = 0, i_gfirst = 0,
+         i_u1 = 0, i_t1f = 0, i_teoff = 0, i_fit = 0, i_ait = 0, i_tcls = 0, i_tcls2 = 0,
          in_bytes = 0;
-  size_t d_zero = 0, d_fbc = 0, d_gflag = 0, d_stat = 0, d_tclaim = 0, d_zero_end = 0, d_UL = 0, d_Ut = 0, d_F = 0, d_ang = 0,
-         d_q = 0, d_t1s = 0, d_tq1 = 0, d_qf = 0, d_udir = 0, d_fbq1 = 0, d_T = 0, d_tf = 0, d_flist = 0, d_fbq2 = 0, d_fbT = 0, d_blk = 0, total = 0;
-  int FL = 0, UK = 0, angL = 0, ang_lam = 0, ang_c = 0, deriv = 0;
+  size_t d_zero = 0, d_fbc = 0, d_stat = 0, d_zero_end = 0, d_UL = 0, d_Ut = 0, d_F = 0, d_ang = 0,
+         d_q = 0, d_t1s = 0, d_tq1 = 0, d_qf = 0, d_udir = 0, d_fbq1 = 0, d_T = 0, d_tf = 0, d_flist = 0, d_tnf = 0, d_fbq2 = 0, d_fbT = 0, d_blk = 0, total = 0;
+  int FL = 0, UK = 0, US = 0, angL = 0, ang_lam = 0, ang_c = 0, deriv = 0;
 };
 
 struct Prepared {
@@ -2363,8 +2368,7 @@ struct Prepared {
   int nfit = 0, nait = 0;
   int cls_begin[ECP_MAX_LAB + 2] = {0};
   int cls_count[ECP_MAX_LAB + 1] = {0};
-  int lmb_count[kMaxLMB + 1] = {0};
-  int ngroups = 0, ntot2 = 0, maxPairs = 0;
+  int ntot2 = 0, maxPairs = 0;
   size_t nblk = 0;
   // device pointers
   DevJob J{};
@@ -2377,20 +2381,16 @@ struct Prepared {
   double *udir = nullptr;  // per type-1 unit: its pair direction (4 values)
   int *fbq1 = nullptr, *fbc = nullptr;
   unsigned char *stat = nullptr;
-  int max_lab = 0, max_lmb = 0;
+  int max_lab = 0;
   int tcount2[kMaxLMB + 1] = {0};  // triplets per type-2 fallback class
   int max_cls2 = 0;
   int max_ent2 = 0;  // T entries of a triplet, at most
-  int *tclaim = nullptr;
   const unsigned char *tcls2 = nullptr;
-  const int *tgf = nullptr;
   int max_lbs = 0, max_L = 0;  // largest basis l and ECP local label of the job
-  const T2Group *grp = nullptr;
-  const int *goff = nullptr, *gfirst = nullptr;
   double *Tout = nullptr;
   unsigned char *tf = nullptr;
-  int *gflag = nullptr, *fbq2 = nullptr;
-  int *flist = nullptr;  // per group: its failed T entries (gflag[g] of them) at eoff
+  int *tnfail = nullptr, *fbq2 = nullptr;
+  int *flist = nullptr;  // per triplet: its failed T entries (tnfail[t] of them) at teoff[t]
   double *fbT = nullptr;
   const int2 *fit = nullptr, *ait = nullptr;
   AsmArgs aa{};
@@ -2405,7 +2405,6 @@ struct Prepared {
   // algorithmic FLOPs per evaluation (the per-unit models of the reference's
   // eager algorithm): type-1 radial work per class, type-2 radial work
   double flops_t1[ECP_MAX_LAB + 1] = {0};
-  double flops_t2 = 0;
   double model[ECP_FL_N] = {0};  // the model's terms known before evaluation (ecp_model_flops)
 };
 
@@ -2442,8 +2441,7 @@ struct ecp_dev {
   hipEvent_t ev[8] = {};
   float last_ms[8] = {};
   int nev = 0;
-  std::vector<int> tmpl, tmpl_off, tmpl_cnt;
-  int *tmpl_dev = nullptr;
+  std::vector<int> tmpl, toff;
   Prepared P;
   JobLayout L;
   ecp_tuning tune{5, 8, 100000, 8192, 2, 1, 15, 2048, 0, 1, 0};
@@ -2498,7 +2496,7 @@ struct Span {
 
 namespace {
 
-int tmpl_key(int la, int lb, int l) { return (la * 16 + lb) * 16 + l; }
+int toff_key(int la, int lb, int l) { return (la * (ECP_MAX_LBS + 1) + lb) * (ECP_MAX_L + 1) + l; }
 
 // T_l entries (lambda1, lambda2, alpha+beta) with a possibly non-zero angular
 // factor: lambda1 from max((alpha+l) mod 2, l-alpha) to l+alpha in steps of 2
@@ -2506,13 +2504,11 @@ int tmpl_key(int la, int lb, int l) { return (la * 16 + lb) * 16 + l; }
 // l+alpha, angular_integrals.c:77), likewise lambda2 with beta.
 void build_templates(ecp_dev *d) {
   d->tmpl.clear();
-  d->tmpl_off.assign(16 * 16 * 16, 0);
-  d->tmpl_cnt.assign(16 * 16 * 16, 0);
+  d->toff.clear();
   for (int la = 0; la <= ECP_MAX_LBS; la++)
-    for (int lb = 0; lb <= ECP_MAX_LBS; lb++)
+    for (int lb = 0; lb <= ECP_MAX_LBS; lb++) {
       for (int l = 0; l < ECP_MAX_L; l++) {
-        const int key = tmpl_key(la, lb, l);
-        d->tmpl_off[key] = (int)d->tmpl.size();
+        d->toff.push_back((int)d->tmpl.size());
         const int d1 = la + l + 1, d2 = lb + l + 1, d3 = la + lb + 1;
         std::vector<char> used((size_t)d1 * d2 * d3, 0);
         for (int alpha = 0; alpha <= la; alpha++)
@@ -2523,9 +2519,10 @@ void build_templates(ecp_dev *d) {
         for (int l1 = 0; l1 < d1; l1++)
           for (int l2 = 0; l2 < d2; l2++)
             for (int l3 = 0; l3 < d3; l3++)
-              if (used[((size_t)l1 * d2 + l2) * d3 + l3]) d->tmpl.push_back(l1 | (l2 << 8) | (l3 << 16));
-        d->tmpl_cnt[key] = (int)d->tmpl.size() - d->tmpl_off[key];
+              if (used[((size_t)l1 * d2 + l2) * d3 + l3]) d->tmpl.push_back(l1 | (l2 << 8) | (l3 << 16) | (l << 24));
       }
+      d->toff.push_back((int)d->tmpl.size());
+    }
 }
 
 void reset_graph(ecp_dev *d) {
@@ -2605,10 +2602,11 @@ extern "C" ecp_dev *ecp_dev_create(const ecp_static *st, char *err, size_t errle
   };
   const size_t o_xs = take(so * 8), o_ws = take(so * 8), o_xl = take(lo * 8), o_wl = take(lo * 8);
   const size_t o_p93l = take(so * 4), o_p93r = take(so * 4), o_p92l = take(lo * 4), o_p92r = take(lo * 4);
+  const size_t o_vis = take(so * 4), o_v93 = take((st->s93.npairs + kPs93Pad) * sizeof(Ps93Pair));
   const size_t o_bess = take(nbess * 8), o_poly = take(npoly * 8), o_om = take(nom * 8);
   const size_t o_ijk = take(nijk * 4), o_idx = take(nidx * 4), o_bin = take(256 * 8);
   const size_t o_fac = take(nfac * 8), o_dfac = take(nfac * 8);
-  const size_t o_tmpl = take(d->tmpl.size() * 4 + 4);
+  const size_t o_tmpl = take(d->tmpl.size() * 4 + 4), o_toff = take(d->toff.size() * 4);
   std::vector<char> h(off, 0);
   auto put = [&](size_t o, const void *src, size_t bytes) { memcpy(h.data() + o, src, bytes); };
   put(o_xs, st->xs, so * 8);
@@ -2619,6 +2617,32 @@ extern "C" ecp_dev *ecp_dev_create(const ecp_static *st, char *err, size_t errle
   put(o_p93r, st->p93r, so * 4);
   put(o_p92l, st->p92l, lo * 4);
   put(o_p92r, st->p92r, lo * 4);
+  {
+    std::vector<Ps93Pair> v(st->s93.npairs + kPs93Pad);
+    for (int k = 0; k < (int)v.size(); k++) {
+      const int i = std::min(k, st->s93.npairs - 1), li = st->p93l[i], ri = st->p93r[i];
+      v[k] = Ps93Pair{st->ws[li], st->ws[ri], li, ri, 0, 0};
+    }
+    for (int lv = 2; lv < st->s93.nlevels; lv++) {
+      v[st->s93.lvl_begin[lv + 1] - 1].ends = lv;
+      // what ps93_level relies on
+      if (3 * st->s93.lvl_n[lv] != 9 << (lv >> 1) || st->s93.lvl_j[lv] != 1 - (lv & 1)) {
+        snprintf(err, errlen, "unexpected PS93 schedule");
+        ecp_dev_destroy(d);
+        return nullptr;
+      }
+    }
+    put(o_v93, v.data(), v.size() * sizeof(Ps93Pair));
+    std::vector<int> vis(so, -1);
+    vis[st->s93.centre] = 0;
+    vis[st->s93.first_l] = 1;
+    vis[st->s93.first_r] = 2;
+    for (int k = 0; k < st->s93.npairs; k++) {
+      vis[st->p93l[k]] = 3 + 2 * k;
+      vis[st->p93r[k]] = 4 + 2 * k;
+    }
+    put(o_vis, vis.data(), so * 4);
+  }
   put(o_bess, st->bessel, nbess * 8);
   put(o_poly, st->poly2sph, npoly * 8);
   put(o_om, st->omega, nom * 8);
@@ -2628,6 +2652,7 @@ extern "C" ecp_dev *ecp_dev_create(const ecp_static *st, char *err, size_t errle
   put(o_fac, st->fac, nfac * 8);
   put(o_dfac, st->dfac, nfac * 8);
   put(o_tmpl, d->tmpl.data(), d->tmpl.size() * 4);
+  put(o_toff, d->toff.data(), d->toff.size() * 4);
   if ((e = hipMalloc(&d->static_mem, off)) != hipSuccess) return fail("hipMalloc(static tables)", e);
   if ((e = hipMemcpy(d->static_mem, h.data(), off, hipMemcpyHostToDevice)) != hipSuccess)
     return fail("hipMemcpy(static tables)", e);
@@ -2641,6 +2666,8 @@ extern "C" ecp_dev *ecp_dev_create(const ecp_static *st, char *err, size_t errle
   T.p93r = (const int *)(b + o_p93r);
   T.p92l = (const int *)(b + o_p92l);
   T.p92r = (const int *)(b + o_p92r);
+  T.v93 = (const Ps93Pair *)(b + o_v93);
+  T.vis = (const int *)(b + o_vis);
   T.bessel = (const double *)(b + o_bess);
   T.poly2sph = (const double *)(b + o_poly);
   T.omega = (const double *)(b + o_om);
@@ -2649,7 +2676,8 @@ extern "C" ecp_dev *ecp_dev_create(const ecp_static *st, char *err, size_t errle
   T.binom = (const double *)(b + o_bin);
   d->fac_dev = (double *)(b + o_fac);
   d->dfac_dev = (double *)(b + o_dfac);
-  d->tmpl_dev = (int *)(b + o_tmpl);
+  T.tmpl = (const int *)(b + o_tmpl);
+  T.toff = (const int *)(b + o_toff);
   T.ijkDim = st->ijkDim;
   T.tmDim = st->tmDim;
   T.lorder = st->lorder;
@@ -2701,13 +2729,19 @@ extern "C" int ecp_dev_last_timing(ecp_dev *d, double *ms, int n) {
 
 namespace {
 
+// chunks of a point's values in the type-2 small grid: basis l <= 3 with
+// projectors l <= 3 (24; packed triplets 14), basis l <= 4 with projectors
+// l <= 4 (35; 17), and the largest (63; 23)
 void launch_type2(ecp_dev *d, hipStream_t s) {
   const Prepared &P = d->P;
   if (P.ntot2 <= 0) return;
-  T2Args A{P.grp, P.goff, P.gfirst, P.ngroups, P.ntot2, d->tmpl_dev, P.Tout, P.tf, P.gflag, P.fbq2, P.fbc + kFb2Cnt,
-           P.nt, P.flist, P.tclaim, P.tcls2};
+  T2Args A{P.Tout, P.tf, P.tnfail, P.flist, P.fbq2, P.fbc + kFb2Cnt, P.nt, P.tcls2};
   Span sp(d, s, FAM_TYPE2);
-  k_type2<<<(P.ntot2 + 63) / 64, 64, 0, s>>>(d->T, P.J, A);
+  const int m = P.tcls_begin[kT2PackLab + 1];
+  const int grid = P.nt - m + (m + kT2Pack - 1) / kT2Pack;
+  if (P.max_lbs <= 3 && P.max_L <= 4) k_type2<24, 14><<<grid, 64, 0, s>>>(d->T, P.J, A, P.tcls, m);
+  else if (P.max_lbs <= 4 && P.max_L <= 5) k_type2<35, 17><<<grid, 64, 0, s>>>(d->T, P.J, A, P.tcls, m);
+  else k_type2<63, 23><<<grid, 64, 0, s>>>(d->T, P.J, A, P.tcls, m);
 }
 
 // type-2 assembly: the register-cached variant fits basis l <= 3 with
@@ -2883,13 +2917,15 @@ void launch_tables(ecp_dev *d, hipStream_t s) {
   A.units = P.u1;
   A.nunits = P.cls_begin[ECP_MAX_LAB + 1];
   A.udir = P.udir;
-  k_tables<<<A.nzb + A.nub + A.nfit + (A.nunits + 127) / 128, 128, 0, s>>>(d->T, P.J, A);
-}
-
-// the angular tables on stream s, ahead of the type-2 chain
-void launch_ang(ecp_dev *d, hipStream_t s) {
-  const Prepared &P = d->P;
-  if (P.nait) k_ang<<<P.nait, 128, 0, s>>>(d->T, P.J, P.ait, d->fac_dev, d->dfac_dev);
+  A.ait = P.ait;
+  A.nait = P.nait;
+  // few pairs: several workgroups each (20 atoms with g shells, 160 pairs:
+  // the launch 116 us at one, 4556 workgroups in all)
+  A.aparts = P.nait < 1024 ? 4 : 1;
+  A.fac = d->fac_dev;
+  A.dfac = d->dfac_dev;
+  Span sp(d, s, FAM_TABLES);
+  k_tables<<<A.nait * A.aparts + A.nzb + A.nub + A.nfit + (A.nunits + 127) / 128, 128, 0, s>>>(d->T, P.J, A);
 }
 
 // fuse = 2 (automatic): fused launches for jobs of up to this many type-1
@@ -2918,10 +2954,6 @@ void enqueue_t1_class(ecp_dev *d, hipStream_t ws, int c) {
 void enqueue(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
   const int units = d->P.cls_begin[ECP_MAX_LAB + 1];
   const bool fused = d->tune.fuse == 1 || (d->tune.fuse == 2 && units <= kFuseAutoMaxUnits);
-  // point-major type-2 rows in the throughput-bound per-class sequence (the
-  // uneven batch 1.8 % faster); row-major in the fused one, where the
-  // point-major tables cost the medium cluster 2.7 %
-  d->P.J.ptmajor = fused ? 0 : 1;
   if (fused) {
     enqueue_fused(d, s, evs);
     return;
@@ -2932,10 +2964,7 @@ void enqueue(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
   hipStream_t *w = d->workers;
   d->span_valid = false;  // type-1 classes run on several streams
   if (evs) (void)hipEventRecord(evs[0], s);
-  {
-    Span sp(d, s, FAM_TABLES);
-    launch_tables(d, s);
-  }
+  launch_tables(d, s);
   if (evs) (void)hipEventRecord(evs[1], s);
   (void)hipEventRecord(d->fork, s);
   for (int i = 0; i < kWorkers; i++) (void)hipStreamWaitEvent(w[i], d->fork, 0);
@@ -2943,15 +2972,11 @@ void enqueue(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
   // beside it the type-1 classes on three workers: one stream per hardware
   // queue the device gives a process
   const int nw1 = kWorkers;
-  {
-    Span sp(d, s, FAM_TABLES);
-    launch_ang(d, s);
-  }
   if (P.ntot2 > 0) {
     launch_type2(d, s);
     // every fallback class in one persistent grid: the classes' items run
     // side by side instead of one class after another on this stream
-    T2Set S2{P.grp, d->tmpl_dev, P.fbq2, P.fbc, P.fbT, P.stat, P.nt, P.gflag, P.flist, P.tgf, 1, 1, 1, 0, 0, 0};
+    T2Set S2{P.fbq2, P.fbc, P.fbT, P.stat, P.nt, P.tnfail, P.flist, 1, 1, 1, 0, 0, 0};
     fb2_slots(d, S2);
     const ClassMap cm2 = fb2_classes(d, S2);
     if (cm2.n > 0) {
@@ -2998,10 +3023,7 @@ void enqueue_fused(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
   hipStream_t w = d->workers[0];
   d->span_valid = false;
   if (evs) (void)hipEventRecord(evs[0], s);
-  {
-    Span sp(d, s, FAM_TABLES);
-    launch_tables(d, s);
-  }
+  launch_tables(d, s);
   if (evs) (void)hipEventRecord(evs[1], s);
   (void)hipEventRecord(d->fork, s);
   (void)hipStreamWaitEvent(w, d->fork, 0);
@@ -3033,13 +3055,9 @@ void enqueue_fused(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
     launch_asm1(d, w, 0, P.nt);
   }
   // ---- type 2 ----
-  {
-    Span sp(d, s, FAM_TABLES);
-    launch_ang(d, s);
-  }
   if (P.ntot2 > 0) {
     launch_type2(d, s);
-    T2Set S2{P.grp, d->tmpl_dev, P.fbq2, P.fbc, P.fbT, P.stat, P.nt, P.gflag, P.flist, P.tgf, 1, 1, 1, 0, 0, 0};
+    T2Set S2{P.fbq2, P.fbc, P.fbT, P.stat, P.nt, P.tnfail, P.flist, 1, 1, 1, 0, 0, 0};
     fb2_slots(d, S2);
     const ClassMap cm2 = fb2_classes(d, S2);
     if (cm2.n > 0) {
@@ -3112,8 +3130,7 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
     std::vector<int> fill(P.tcls_begin, P.tcls_begin + ECP_MAX_LAB + 1);
     for (int t = 0; t < nt; t++) tcls[fill[job->trip[t].la + job->trip[t].lb]++] = t;
   }
-  std::vector<T2Group> groups;
-  std::vector<int> goff, tgfirst(nt);
+  std::vector<int> teoff(nt);
   std::vector<unsigned char> tcls2(nt);
   for (int c = 0; c <= kMaxLMB; c++) P.tcount2[c] = 0;
   P.max_cls2 = 0;
@@ -3121,41 +3138,21 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
   for (int t = 0; t < nt; t++) {
     const ecp_triplet &tr = job->trip[t];
     const int la = tr.la, lb = tr.lb;
-    tgfirst[t] = (int)groups.size();
+    teoff[t] = ntot2;
     {
       const int c2 = std::max(la, lb) + job->cent[tr.centre].L - 1;
       tcls2[t] = (unsigned char)c2;
       P.tcount2[c2]++;
       P.max_cls2 = std::max(P.max_cls2, c2);
     }
-    const int ent0 = ntot2;
-    for (int l = 0; l < job->cent[tr.centre].L; l++) {
-      const int key = tmpl_key(la, lb, l);
-      T2Group g{t, l, ntot2, d->tmpl_cnt[key], d->tmpl_off[key], std::max(la, lb) + l};
-      groups.push_back(g);
-      // per entry: 4 FLOPs per window point + 150 for the integrator
-      P.flops_t2 += (double)g.ne * (4.0 * (tr.ge - tr.gs) + 150.0);
-      goff.push_back(ntot2);
-      ntot2 += g.ne;
-      P.lmb_count[g.lmb]++;
-    }
-    P.max_ent2 = std::max(P.max_ent2, ntot2 - ent0);
+    const int ne = d->toff[toff_key(la, lb, job->cent[tr.centre].L)] - d->toff[toff_key(la, lb, 0)];
+    ntot2 += ne;
+    P.max_ent2 = std::max(P.max_ent2, ne);
   }
-  P.ngroups = (int)groups.size();
   P.ntot2 = ntot2;
   ecp_model_flops(job, P.model);
   for (int c = 0; c <= ECP_MAX_LAB; c++)
     if (P.cls_count[c]) P.max_lab = c;
-  for (int c = 0; c <= kMaxLMB; c++)
-    if (P.lmb_count[c]) P.max_lmb = c;
-  goff.push_back(ntot2);
-  // the group of every 64th T entry: a wave of the type-2 small grid finds
-  // its entries' groups among those from there on
-  std::vector<int> gfirst((size_t)(ntot2 + 63) / 64);
-  for (size_t w = 0, g = 0; w < gfirst.size(); w++) {
-    while (goff[g + 1] <= (int)(64 * w)) g++;
-    gfirst[w] = (int)g;
-  }
   std::vector<int2> fitems, aitems;
   for (int c = 0; c < job->ncent; c++) {
     const ecp_centre &C = job->cent[c];
@@ -3186,10 +3183,7 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
   Ly.i_trip = in_take(sizeof(ecp_triplet) * nt);
   Ly.i_u1 = in_take(sizeof(T1Unit) * units1.size());
   Ly.i_t1f = in_take(4 * (size_t)nt);
-  Ly.i_grp = in_take(sizeof(T2Group) * groups.size());
-  Ly.i_goff = in_take(4 * goff.size());
-  Ly.i_tgf = in_take(4 * (size_t)nt);
-  Ly.i_gfirst = in_take(4 * gfirst.size());
+  Ly.i_teoff = in_take(4 * (size_t)nt);
   Ly.i_tcls2 = in_take((size_t)nt);
   Ly.i_fit = in_take(sizeof(int2) * fitems.size());
   Ly.i_ait = in_take(sizeof(int2) * aitems.size());
@@ -3203,9 +3197,7 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
   };
   Ly.d_zero = dv_off;
   Ly.d_fbc = dv_take(4 * kFbcSlots);
-  Ly.d_gflag = dv_take(4 * (size_t)P.ngroups);
   Ly.d_stat = dv_take(2 * (size_t)nt);
-  Ly.d_tclaim = dv_take(4 * (size_t)nt);
   Ly.d_zero_end = dv_off;
   Ly.d_UL = dv_take(8 * job->nUL);
   Ly.d_Ut = dv_take(8 * job->nUt);
@@ -3218,6 +3210,7 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
   Ly.d_T = dv_take(8 * (size_t)ntot2);
   Ly.d_tf = dv_take((size_t)ntot2);
   Ly.d_flist = dv_take(4 * (size_t)ntot2);
+  Ly.d_tnf = dv_take(4 * (size_t)nt);
   Ly.d_fbq2 = dv_take(4 * (size_t)(kMaxLMB + 1) * nt);
   Ly.d_fbT = dv_take(8 * (size_t)ntot2 * P.maxPairs);
   Ly.d_blk = dv_take(8 * job->nblk);
@@ -3227,6 +3220,7 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
   Ly.total = dv_off;
   Ly.FL = job->FL;
   Ly.UK = job->UK;
+  Ly.US = job->maxL * job->UK;
   Ly.angL = job->angL;
   Ly.ang_lam = job->ang_lam;
   Ly.ang_c = job->ang_c;
@@ -3324,10 +3318,7 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
   cp(Ly.i_trip, job->trip, sizeof(ecp_triplet) * nt);
   cp(Ly.i_u1, units1.data(), sizeof(T1Unit) * units1.size());
   cp(Ly.i_t1f, t1first.data(), 4 * (size_t)nt);
-  cp(Ly.i_grp, groups.data(), sizeof(T2Group) * groups.size());
-  cp(Ly.i_goff, goff.data(), 4 * goff.size());
-  cp(Ly.i_tgf, tgfirst.data(), 4 * (size_t)nt);
-  cp(Ly.i_gfirst, gfirst.data(), 4 * gfirst.size());
+  cp(Ly.i_teoff, teoff.data(), 4 * (size_t)nt);
   cp(Ly.i_tcls2, tcls2.data(), (size_t)nt);
   cp(Ly.i_fit, fitems.data(), sizeof(int2) * fitems.size());
   cp(Ly.i_ait, aitems.data(), sizeof(int2) * aitems.size());
@@ -3392,6 +3383,8 @@ extern "C" int ecp_dev_bind(ecp_dev *d, void *mem, size_t cap, char *err, size_t
   J.ang_c = Ly.ang_c;
   J.deriv = Ly.deriv;
   J.maxPairs = P.maxPairs;
+  J.teoff = (const int *)(A + Ly.i_teoff);
+  J.US = Ly.US;
   P.u1 = (const T1Unit *)(A + Ly.i_u1);
   P.q = (double *)(A + Ly.d_q);
   P.t1s = (double *)(A + Ly.d_t1s);
@@ -3402,17 +3395,12 @@ extern "C" int ecp_dev_bind(ecp_dev *d, void *mem, size_t cap, char *err, size_t
   P.fbc = (int *)(A + Ly.d_fbc);  // [0..12] type-1 fallback queues, [32..44] type-1 tails, [48] type-2
                                   // tail, [kFb2Cnt + 0..12] type-2 fallback queues
   P.stat = (unsigned char *)(A + Ly.d_stat);
-  P.grp = (const T2Group *)(A + Ly.i_grp);
-  P.goff = (const int *)(A + Ly.i_goff);
-  P.gfirst = (const int *)(A + Ly.i_gfirst);
   P.Tout = (double *)(A + Ly.d_T);
   P.tf = (unsigned char *)(A + Ly.d_tf);
-  P.gflag = (int *)(A + Ly.d_gflag);
+  P.tnfail = (int *)(A + Ly.d_tnf);
   P.flist = (int *)(A + Ly.d_flist);
   P.fbq2 = (int *)(A + Ly.d_fbq2);
-  P.tclaim = (int *)(A + Ly.d_tclaim);
   P.tcls2 = (const unsigned char *)(A + Ly.i_tcls2);
-  P.tgf = (const int *)(A + Ly.i_tgf);
   P.fbT = (double *)(A + Ly.d_fbT);
   P.fit = (const int2 *)(A + Ly.i_fit);
   P.ait = (const int2 *)(A + Ly.i_ait);
@@ -3426,9 +3414,6 @@ extern "C" int ecp_dev_bind(ecp_dev *d, void *mem, size_t cap, char *err, size_t
     aa.udir = P.udir;
     aa.t1first = (const int *)(A + Ly.i_t1f);
     aa.qout = P.q;
-    aa.groups = P.grp;
-    aa.tgfirst = (const int *)(A + Ly.i_tgf);
-    aa.tmpl = d->tmpl_dev;
     aa.Tout = P.Tout;
     aa.tfail = P.tf;
     aa.fbT = P.fbT;
@@ -3530,9 +3515,8 @@ namespace {
 // term is an integer below 2^53, so the atomic sum is exact in any order.
 __global__ __launch_bounds__(256) void k_fb_flops(DevJob J, const T1Unit *__restrict__ units,
                                                   const unsigned long long *__restrict__ qf, int nunits,
-                                                  const T2Group *__restrict__ groups, const int *__restrict__ gflag,
-                                                  const int *__restrict__ flist, const unsigned char *__restrict__ tfail,
-                                                  int ngroups, int N, double *out) {
+                                                  DevTables T, const int *__restrict__ tnfail,
+                                                  const int *__restrict__ flist, int N, double *out) {
   double s1 = 0.0, s2 = 0.0;
   const int stride = gridDim.x * blockDim.x;
   for (int u = blockIdx.x * blockDim.x + threadIdx.x; u < nunits; u += stride) {
@@ -3541,19 +3525,19 @@ __global__ __launch_bounds__(256) void k_fb_flops(DevJob J, const T1Unit *__rest
     const ecp_triplet tr = J.trip[units[u].trip];
     s1 += ecp_fb1_flops(tr.la + tr.lb, f, N);
   }
-  for (int g = blockIdx.x * blockDim.x + threadIdx.x; g < ngroups; g += stride) {
-    // the group's failed entries among those listed for the fallback (a
-    // speculative fallback also lists entries the small grid then decided)
-    const T2Group G = groups[g];
-    int f = 0;
-    for (int k = 0; k < gflag[g]; k++) f += tfail[G.eoff + flist[G.eoff + k]];
-    if (!f) continue;
-    const ecp_triplet tr = J.trip[G.trip];
-    const ecp_centre C = J.cent[tr.centre];
-    int ng = 0;
-    for (int i = 0; i < C.ng; i++) ng += J.gauss[C.g0 + i].l == G.l;
-    const int KK = J.shells[tr.sa].K * J.shells[tr.sb].K;
-    s2 += KK * ecp_fb2_flops(tr.la, tr.lb, G.l, ng, f, N);
+  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < J.ntrip; t += stride) {
+    const int nf = tnfail[t];
+    if (!nf) continue;
+    const ecp_triplet tr = J.trip[t];
+    const ecp_centre *C = J.cent + tr.centre;
+    const int KK = J.shells[tr.sa].K * J.shells[tr.sb].K, t0 = t2_off(T, tr.la, tr.lb, 0);
+    // listed in entry order, channel after channel
+    for (int k = 0; k < nf;) {
+      const int l = T.tmpl[t0 + flist[J.teoff[t] + k]] >> 24;
+      int f = 0;
+      for (; k < nf && T.tmpl[t0 + flist[J.teoff[t] + k]] >> 24 == l; k++) f++;
+      s2 += KK * ecp_fb2_flops(tr.la, tr.lb, l, C->gl[l + 1] - C->gl[l], f, N);
+    }
   }
   if (s1 != 0.0) atomicAdd(&out[0], s1);
   if (s2 != 0.0) atomicAdd(&out[1], s2);
@@ -3597,9 +3581,8 @@ extern "C" int ecp_dev_profile(ecp_dev *d, int *launches, double *ms, double *fl
   if (!d->fbf) ECP_CHECK(hipMalloc(&d->fbf, 2 * sizeof(double)));
   ECP_CHECK(hipMemsetAsync(d->fbf, 0, 2 * sizeof(double), d->stream));
   const int nunits = P.cls_begin[ECP_MAX_LAB + 1];
-  const int nb = std::max(1, std::min(1024, (std::max(nunits, P.ngroups) + 255) / 256));
-  k_fb_flops<<<nb, 256, 0, d->stream>>>(P.J, P.u1, P.qf, nunits, P.grp, P.gflag, P.flist, P.tf, P.ngroups,
-                                        d->T.lorder, d->fbf);
+  const int nb = std::max(1, std::min(1024, (std::max(nunits, P.nt) + 255) / 256));
+  k_fb_flops<<<nb, 256, 0, d->stream>>>(P.J, P.u1, P.qf, nunits, d->T, P.tnfail, P.flist, d->T.lorder, d->fbf);
   ECP_CHECK(hipGetLastError());
   double fb[2] = {0.0, 0.0};
   ECP_CHECK(hipMemcpyAsync(fb, d->fbf, sizeof(fb), hipMemcpyDeviceToHost, d->stream));

@@ -317,8 +317,9 @@ int ecp_job_build(const ecp_mol *mols, int nmol, int deriv, const ecp_static *st
   job->ngauss = ngauss;
   job->nwin = nwin;
   job->maxL = maxL;
-  job->FL = maxL + maxLBS + deriv;          /* rows lambda = 0 .. L-1+l_s+run */
-  job->UK = 2 * (maxLBS + deriv) + 1;       /* r^k, k = 0 .. la+lb (shifted) */
+  /* even: the device reads both in 16-byte chunks */
+  job->FL = (maxL + maxLBS + deriv + 1) & ~1;  /* rows lambda = 0 .. L-1+l_s+run */
+  job->UK = 2 * (maxLBS + deriv) + 2;          /* r^k, k = 0 .. la+lb (shifted) */
   job->angL = maxL;
   job->ang_lam = maxL + maxLBS + deriv;     /* lambda = 0 .. L-1+lmax_a+n */
   job->ang_c = ECP_DIM_C(maxLBS + deriv);
