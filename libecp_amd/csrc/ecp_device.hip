@@ -138,6 +138,8 @@ __device__ __forceinline__ V cload(const V *q) {
 // weights, and the level it is the last pair of (0: none).  A level's last
 // pair is its closest to the centre, so the level has a point in a window
 // where this pair does.
+constexpr int kSphDim = 16;  // more than any l of the harmonics
+
 struct Ps93Pair {
   double wl, wr;
   int li, ri, ends, pad;
@@ -149,6 +151,13 @@ struct DevTables {
   CPtr<int> p93l, p93r, p92l, p92r;
   CPtr<Ps93Pair> v93;
   CPtr<int> vis;  // a small-grid point's place in the PS93 visit order
+  // harmonics: norms sqrt((l-m)!/(l+m)!) sqrt((2l+1)/(2 pi)) (m = 0: the
+  // second factor) at [l * kSphDim + m], double factorials, 1 / n
+  CPtr<double> snorm, dfac, inv;
+  // position of the product of the monomials at positions r and q, of degree
+  // up to the basis's each, at [r * prodN + q]
+  CPtr<int> prod;
+  int prodN;
   // T entries of a triplet (build_templates): packed (lambda1, lambda2, alpha + beta, l), channel after channel; those
   // of channel l < L at [toff(la, lb, l), toff(la, lb, l + 1)) (t2_off)
   CPtr<int> tmpl, toff;
@@ -335,38 +344,13 @@ __device__ __forceinline__ void bessel_k(const double *__restrict__ tab, double 
 // (l-m)!/(l+m)!), 1/sqrt(2) for m = 0, and sin/cos(m phi) by the
 // angle-addition recurrence from m = 1.
 // x = cos(theta), sp = sin(phi), cp = cos(phi): the direction's trigonometric
-// values, formed once per direction by the caller.
-__device__ void real_sph_column(int lmax, int m, double x, double phi, double sp, double cp,
-                                const double *__restrict__ fac, const double *__restrict__ dfac, double *out) {
+// values, formed once per direction by the caller.  The norms come from a
+// table and the divisions by l - m and sqrt(2) take three operations
+// (div_const's): a square root and the divisions per entry were most of the
+// type-1 assembly's instructions.
+__device__ __forceinline__ void real_sph_column(const DevTables &T, int lmax, int m, double x, double phi, double sp,
+                                                double cp, double *out) {
 #define RSH(l, mm) ((l) * (l) + (l) + (mm))
-  if (1.0 == x || -1.0 == x) {
-    for (int l = m; l <= lmax; l++) {
-      out[RSH(l, m)] = 0.0;
-      out[RSH(l, -m)] = 0.0;
-    }
-    if (m == 0) {
-      double v = 1.0;
-      for (int l = 0; l <= lmax; l++) {
-        if (l > 0 && -1.0 == x) v = -v;
-        out[RSH(l, 0)] = v;
-      }
-    }
-  } else {
-    const double s1 = sqrt(1.0 - x * x);
-    // P_mm, P_(m+1)m, then the recurrence
-    double pmm;
-    if (m == 0) {
-      pmm = 1.0;
-    } else {
-      double sl = s1;
-      for (int l = 2; l <= m; l++) sl = sl * s1;
-      pmm = sl * dfac[2 * m - 1];
-    }
-    out[RSH(m, m)] = pmm;
-    if (m + 1 <= lmax) out[RSH(m + 1, m)] = x * (2 * m + 1) * out[RSH(m, m)];
-    for (int l = m + 2; l <= lmax; l++)
-      out[RSH(l, m)] = (x * (2 * l - 1) * out[RSH(l - 1, m)] - (l + m - 1) * out[RSH(l - 2, m)]) / (l - m);
-  }
   double sm = 0.0, cm = 1.0;
   for (int k = 1; k <= m; k++) {
     if (0.0 == phi) {
@@ -381,15 +365,44 @@ __device__ void real_sph_column(int lmax, int m, double x, double phi, double sp
       sm = ns;
     }
   }
+  const bool pole = 1.0 == x || -1.0 == x;
+  double p1 = 0.0, p2 = 0.0;  // P_(l-1)m, P_(l-2)m
+  if (pole) {
+    p1 = m == 0 ? 1.0 : 0.0;
+  } else if (m == 0) {
+    p1 = 1.0;
+  } else {
+    const double s1 = sqrt(1.0 - x * x);
+    double sl = s1;
+    for (int l = 2; l <= m; l++) sl = sl * s1;
+    p1 = sl * T.dfac[2 * m - 1];
+  }
+  const double *__restrict__ nrm = T.snorm + m;
+  const double rt2 = sqrt(2.0), irt2 = 1.0 / rt2;
   for (int l = m; l <= lmax; l++) {
-    const double norm0 = sqrt((2.0 * l + 1.0) / (2.0 * M_PI));
-    if (m == 0) {
-      out[RSH(l, 0)] = norm0 * out[RSH(l, 0)];
-      out[RSH(l, 0)] = out[RSH(l, 0)] / sqrt(2.0);
+    double P;
+    if (l == m) {
+      P = p1;
     } else {
-      const double P = (sqrt(fac[l - m] / fac[l + m]) * norm0) * out[RSH(l, m)];
-      out[RSH(l, -m)] = P * sm;
-      out[RSH(l, m)] = P * cm;
+      if (pole) {
+        P = -1.0 == x ? -p1 : p1;
+      } else if (l == m + 1) {
+        P = x * (2 * m + 1) * p1;
+      } else {
+        const double a = x * (2 * l - 1) * p1 - (l + m - 1) * p2, b = l - m, y = T.inv[l - m];
+        const double q = a * y;
+        P = __builtin_fma(__builtin_fma(-b, q, a), y, q);
+      }
+      p2 = p1;
+      p1 = P;
+    }
+    const double v = nrm[l * kSphDim] * P;
+    if (m == 0) {
+      const double q = v * irt2;
+      out[RSH(l, 0)] = __builtin_fma(__builtin_fma(-rt2, q, v), irt2, q);
+    } else {
+      out[RSH(l, -m)] = v * sm;
+      out[RSH(l, m)] = v * cm;
     }
   }
 #undef RSH
@@ -499,8 +512,8 @@ __device__ void ftab_item(const DevTables &T, const DevJob &J, int2 it) {
 // per-(centre, atom) angular table ang[lambda][LM(l,m)][C(la,c)]
 constexpr int kAngRsph = (ECP_MAX_L + ECP_MAX_LBS) * (ECP_MAX_L + ECP_MAX_LBS);
 
-__device__ void ang_item(const DevTables &T, const DevJob &J, int2 it, const double *__restrict__ fac,
-                         const double *__restrict__ dfac, double *rsph, double *s_dir, int part, int nparts) {
+__device__ void ang_item(const DevTables &T, const DevJob &J, int2 it, double *rsph, double *s_dir, int part,
+                         int nparts) {
   const ecp_centre C = J.cent[it.x];
   const int A = C.atom0 + it.y;
   const int lmax_a = J.atom_maxl[A] + J.deriv;
@@ -517,7 +530,7 @@ __device__ void ang_item(const DevTables &T, const DevJob &J, int2 it, const dou
   __syncthreads();
   // one column m of the harmonics per lane
   if ((int)threadIdx.x <= lmax)
-    real_sph_column(lmax, threadIdx.x, s_dir[0], s_dir[1], s_dir[2], s_dir[3], fac, dfac, rsph);
+    real_sph_column(T, lmax, threadIdx.x, s_dir[0], s_dir[1], s_dir[2], s_dir[3], rsph);
   __syncthreads();
   const int d1 = ECP_DIM_L(T.omLambda), d2 = ECP_DIM_C(T.omAlpha);
   const int nlm = C.L * C.L, nc = ECP_DIM_C(lmax_a);
@@ -703,6 +716,8 @@ __device__ __forceinline__ void type1_body(int bid, const DevTables &T, const De
           each(e, (0.0 + a.w * ((ca * a.K[l2]) * a.g)) + b.w * ((cb * b.K[l2]) * b.g));
         ra *= a.r;
         rb *= b.r;
+        // (many entries: no more of them in flight than registers hold)
+        if constexpr (LAB > 8) __builtin_amdgcn_sched_barrier(0);
       }
     };
     double p[NQ], q[NQ], I[NQ];
@@ -1769,7 +1784,6 @@ struct AsmArgs {
   const double *Tout;
   const unsigned char *tfail;
   const double *fbT;
-  const double *fac, *dfac;
   double *blocks;
   // dynamic LDS layout (doubles): J is shared; the type-1 region (rsph, H)
   // and the type-2 region (blk, T) overlap
@@ -1858,6 +1872,26 @@ __device__ void shift_factors(const DevTables &T, int l, const V3 v, bool with_n
   }
 }
 
+// sum of f[t] get(r[t]) over t < n, in order; the reads of up to four terms
+// are issued together
+template <typename Get>
+__device__ __forceinline__ double shift_sum(const double *f, const int *r, int n, Get get) {
+  double acc = 0.0;
+  int t = 0;
+  for (; t + 4 <= n; t += 4) {
+    double x[4], y[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      x[i] = f[t + i];
+      y[i] = get(r[t + i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) acc += x[i] * y[i];
+  }
+  for (; t < n; t++) acc += f[t] * get(r[t]);
+  return acc;
+}
+
 // binomial shift of a block over C-centred monomials to the IJK(la) x IJK(lb)
 // output (util.c:246-334).  The block is read through get(r, q): row r is an
 // ordering position of degree <= la, column q a position of degree <= lb.
@@ -1887,9 +1921,7 @@ __device__ void shift_block(const DevTables &T, Get get, int la, int lb, const V
     const double *f = SA.f + c1 * SA.mt;
     const int *r = SA.r + c1 * SA.mt;
     const int n = SA.n[c1];
-    double acc = 0.0;
-    for (int t = 0; t < n; t++) acc += f[t] * get(r[t], q);
-    Jbuf[idx] = acc;
+    Jbuf[idx] = shift_sum(f, r, n, [&](int x) { return get(x, q); });
   }
   __syncthreads();
   for (int idx = lid; idx < nia * nib; idx += nlanes) {
@@ -1897,9 +1929,7 @@ __device__ void shift_block(const DevTables &T, Get get, int la, int lb, const V
     const double *f = SB.f + c2 * SB.mt;
     const int *r = SB.r + c2 * SB.mt;
     const int n = SB.n[c2];
-    double acc = 0.0;
-    for (int t = 0; t < n; t++) acc += f[t] * Jbuf[c1 * ncb + r[t]];
-    out[idx] = acc;
+    out[idx] = shift_sum(f, r, n, [&](int x) { return Jbuf[c1 * ncb + x]; });
   }
   __syncthreads();
 }
@@ -1983,7 +2013,6 @@ __global__ __launch_bounds__(kAsmThreads, 3) void k_asm1(DevTables T, DevJob J, 
   const int la = tr.la, lb = tr.lb, lab = la + lb;  // shifted for derivatives
   const ecp_xyz rc = J.atoms[Cn.atom], ra = J.atoms[Sa.atom], rb = J.atoms[Sb.atom];
   const V3 vA{ra.x - rc.x, ra.y - rc.y, ra.z - rc.z}, vB{rb.x - rc.x, rb.y - rc.y, rb.z - rc.z};
-  const int D = T.ijkDim;
   const int tmd = ECP_DIM_L(T.tmDim);
 
   const int np = active ? ECP_DIM_C(lab) : 0;
@@ -2003,7 +2032,7 @@ __global__ __launch_bounds__(kAsmThreads, 3) void k_asm1(DevTables T, DevJob J, 
     for (int it = lid; it < nc * (lab + 1); it += W) {
       const int k = it / (lab + 1), m = it - k * (lab + 1);
       const double *d = A.udir + 4 * (size_t)(u0 + c0 + k);
-      real_sph_column(lab, m, d[0], d[1], d[2], d[3], A.fac, A.dfac, rsph + k * A.lds_rs_stride);
+      real_sph_column(T, lab, m, d[0], d[1], d[2], d[3], rsph + k * A.lds_rs_stride);
     }
     for (int it = lid; it < nc * nql; it += W) {
       const int k = it / nql, e = it - k * nql;
@@ -2043,10 +2072,7 @@ __global__ __launch_bounds__(kAsmThreads, 3) void k_asm1(DevTables T, DevJob J, 
     __syncthreads();
   }
   const double norm1 = 4.0 * M_PI;
-  auto get1 = [&](int r, int q) {
-    const int *ea = T.ijk + 3 * r, *eb = T.ijk + 3 * q;
-    return H[T.ijkIndex[((ea[0] + eb[0]) * D + ea[1] + eb[1]) * D + ea[2] + eb[2]]];
-  };
+  auto get1 = [&](int r, int q) { return H[T.prod[r * T.prodN + q]]; };
   if constexpr (G == 1)
     shift_block(T, get1, tr.oa, tr.ob, vA, vB, norm1, Jbuf, lds + A.lds_S1, A.shift_lm, A.blocks + tr.blk1);
   else
@@ -2059,210 +2085,158 @@ __device__ __forceinline__ int deg_of(int p) {
   return (p >= 1) + (p >= 4) + (p >= 10) + (p >= 20) + (p >= 35) + (p >= 56);
 }
 
-// One channel's part of a type-2 block (type2.c:583-623): for the elements
-// (pp, qq) of the lanes lid, lid + nlanes, ... the sum over lambda1 and
-// lambda2 of (sum_m A[lambda1][m][pp] B[lambda2][m][qq]) T[lambda1][lambda2],
-// added to blk.  The channel is a template argument, so that its 2 l + 1
-// factors and its at most (NB - 1 + l) / 2 + 1 values of lambda2 are the
-// only ones in the code: with both padded to the largest channel's, the
-// kernel's time was that of instructions for absent values.
+// T values of a triplet in LDS, every channel: entry (l, lambda1, lambda2,
+// k = alpha + beta).  lambda1 + alpha, lambda2 + beta and l have the same
+// parity, so k and lambda1 + lambda2 do too, and half of the k suffice.
+__device__ __forceinline__ int t2_slot(int la, int lb, int l, int l1, int l2, int k) {
+  const int a = la + 1, b = lb + 1, d3 = (la + lb + 2) >> 1;
+  // the channels before l: sum of (a + i)(b + i), i < l
+  const int before = l * a * b + (a + b) * (l * (l - 1) >> 1) + (l - 1) * l * (2 * l - 1) / 6;
+  return (before + l1 * (b + l) + l2) * d3 + (k >> 1);
+}
+__host__ __device__ constexpr int t2_slots(int la, int lb, int L) {
+  int n = 0;
+  for (int l = 0; l < L; l++) n += (la + l + 1) * (lb + l + 1);
+  return n * ((la + lb + 2) / 2);
+}
+
+// One channel's part of element (pp, qq) of a type-2 block (type2.c:583-623):
+// the sum over lambda1 and lambda2 of (sum_m A[lambda1][m][pp]
+// B[lambda2][m][qq]) T[lambda1][lambda2].  The channel is a template
+// argument, so that its 2 l + 1 factors and its at most (NB - 1 + l) / 2 + 1
+// values of lambda2 are the only ones in the code: with both padded to the
+// largest channel's, the kernel's time was that of instructions for absent
+// values.
 // NB > 0 (basis l < NB): the angular factors of atom B for every lambda2 in
-// registers, those of atom A per lambda1; NB = 0: both read for each pair.
+// registers, those of atom A for the next lambda1 read ahead; NB = 0: both
+// read for each pair.
 template <int NB, int L>
-__device__ __forceinline__ void asm2_channel(const double *__restrict__ angA, const double *__restrict__ angB,
-                                             int ang_c, int nlm2, const double *Tl, int la, int lb, int nca, int ncb,
-                                             float inv_ncb, double *blk, int lid, int nlanes) {
+__device__ __forceinline__ double asm2_channel(const double *__restrict__ pA, const double *__restrict__ pB,
+                                               int ang_c, int lam_stride, const double *Tl, int la, int lb, int alpha,
+                                               int beta) {
   constexpr int NM = 2 * L + 1;
   constexpr int NBL = NB == 0 ? 1 : (NB - 1 + L) / 2 + 1 < NB ? (NB - 1 + L) / 2 + 1 : NB;
-  const int d2 = lb + L + 1, d3 = la + lb + 1;
-  const size_t lam_stride = (size_t)nlm2 * ang_c;
-  for (int idx = lid; idx < nca * ncb; idx += nlanes) {
-    const int pp = (int)(((float)idx + 0.5f) * inv_ncb), qq = idx - pp * ncb;
-    const int alpha = deg_of(pp), beta = deg_of(qq);
-    const int par1 = (alpha + L) & 1, par2 = (beta + L) & 1;
-    const int ll1 = max(par1, L - alpha), ll2 = max(par2, L - beta);
-    const double *pA = angA + L * L * ang_c + pp, *pB = angB + L * L * ang_c + qq;
-    const double *Te = Tl + alpha + beta;
-    double tmp = 0.0;
-    if constexpr (NB > 0) {
-      double Bv[NBL][NM];
+  const int ll1 = max((alpha + L) & 1, L - alpha), ll2 = max((beta + L) & 1, L - beta);
+  const int ds = (la + lb + 2) >> 1, d2 = (lb + L + 1) * ds;
+  const double *Te = Tl + t2_slot(la, lb, L, ll1, ll2, alpha + beta);
+  pA += L * L * ang_c + ll1 * lam_stride;
+  pB += L * L * ang_c + ll2 * lam_stride;
+  const int n1 = (la + L - ll1) >> 1, n2 = (lb + L - ll2) >> 1;  // values of lambda1, lambda2, less one
+  double tmp = 0.0;
+  if constexpr (NB > 0) {
+    double Bv[NBL][NM], Av[NM];
 #pragma unroll
-      for (int i = 0; i < NBL; i++) {
-        const bool on = ll2 + 2 * i <= lb + L;
-        const double *pb = pB + (on ? ll2 + 2 * i : ll2) * lam_stride;
+    for (int m = 0; m < NM; m++) Av[m] = pA[m * ang_c];
 #pragma unroll
-        for (int m = 0; m < NM; m++) Bv[i][m] = pb[m * ang_c];
-      }
-      for (int lam1 = ll1; lam1 <= la + L; lam1 += 2) {
-        const double *pa = pA + lam1 * lam_stride;
-        double Av[NM];
+    for (int i = 0; i < NBL; i++) {
+      const double *pb = pB + 2 * min(i, n2) * lam_stride;
 #pragma unroll
-        for (int m = 0; m < NM; m++) Av[m] = pa[m * ang_c];
+      for (int m = 0; m < NM; m++) Bv[i][m] = pb[m * ang_c];
+    }
+    for (int i1 = 0; i1 <= n1; i1++, Te += 2 * d2) {
+      double An[NM];
+      pA += i1 < n1 ? 2 * lam_stride : 0;
 #pragma unroll
-        for (int i = 0; i < NBL; i++) {
-          const int lam2 = ll2 + 2 * i;
-          if (lam2 <= lb + L) {
-            double factor = 0.0;
+      for (int m = 0; m < NM; m++) An[m] = pA[m * ang_c];
 #pragma unroll
-            for (int m = 0; m < NM; m++) factor += Av[m] * Bv[i][m];
-            tmp += factor * Te[(lam1 * d2 + lam2) * d3];
-          }
-        }
-      }
-    } else {
-      for (int lam1 = ll1; lam1 <= la + L; lam1 += 2)
-        for (int lam2 = ll2; lam2 <= lb + L; lam2 += 2) {
-          const double *pa = pA + lam1 * lam_stride, *pb = pB + lam2 * lam_stride;
-          double x[NM], y[NM];
-#pragma unroll
-          for (int m = 0; m < NM; m++) {
-            x[m] = pa[m * ang_c];
-            y[m] = pb[m * ang_c];
-          }
+      for (int i = 0; i < NBL; i++)
+        if (i <= n2) {
           double factor = 0.0;
 #pragma unroll
-          for (int m = 0; m < NM; m++) factor += x[m] * y[m];
-          tmp += factor * Te[(lam1 * d2 + lam2) * d3];
+          for (int m = 0; m < NM; m++) factor += Av[m] * Bv[i][m];
+          tmp += factor * Te[2 * i * ds];
         }
+#pragma unroll
+      for (int m = 0; m < NM; m++) Av[m] = An[m];
     }
-    blk[idx] += tmp;
+  } else {
+    for (int i1 = 0; i1 <= n1; i1++, pA += 2 * lam_stride, Te += 2 * d2)
+      for (int i = 0; i <= n2; i++) {
+        const double *pb = pB + 2 * i * lam_stride;
+        double x[NM], y[NM];
+#pragma unroll
+        for (int m = 0; m < NM; m++) {
+          x[m] = pA[m * ang_c];
+          y[m] = pb[m * ang_c];
+        }
+        double factor = 0.0;
+#pragma unroll
+        for (int m = 0; m < NM; m++) factor += x[m] * y[m];
+        tmp += factor * Te[2 * i * ds];
+      }
   }
+  return tmp;
 }
 
-// channels l < MAXL
-template <int NB, int MAXL>
-__device__ __forceinline__ void asm2_channel_of(int l, const double *__restrict__ angA,
-                                                const double *__restrict__ angB, int ang_c, int nlm2,
-                                                const double *Tl, int la, int lb, int nca, int ncb, float inv_ncb,
-                                                double *blk, int lid, int nlanes) {
-  switch (l) {
-#define CH(x)                                                                                                \
-  case x:                                                                                                    \
-    if constexpr (x < MAXL)                                                                                  \
-      asm2_channel<NB, x>(angA, angB, ang_c, nlm2, Tl, la, lb, nca, ncb, inv_ncb, blk, lid, nlanes);         \
-    break;
-    CH(0) CH(1) CH(2) CH(3) CH(4) CH(5) CH(6)
-#undef CH
-  }
-}
-
-// Type-2 block of one triplet per wave: for each projector l, the T_l
-// entries (small-grid results, or the sum of the per-pair fallback results)
-// are placed in LDS and contracted with the angular tables of both atoms
-// (type2.c:583-623), then the block is shifted (util.c:246-334).
-// NB, MAXL: as in asm2_channel, channels l < MAXL.
-// tlist: the triplets of the launch, one per workgroup.
-template <int NB, int MAXL>
+// Type-2 blocks, a lane group of 64 / G lanes and an LDS slice per triplet
+// (tlist[0 .. ntl); G = kAsmPack: classes la + lb <= kAsmPackLab, at most 9
+// elements): the T values of every channel (small-grid results, or the sum
+// of the per-pair fallback results) are read together and placed in LDS, the
+// lanes form the elements, contracting them with the angular tables of both
+// atoms (type2.c:583-623), and the block is shifted (util.c:246-334).
+// NB: as in asm2_channel; channels l < MAXL.
+template <int G, int NB, int MAXL>
 __global__ __launch_bounds__(kAsmThreads) void k_asm2(DevTables T, DevJob J, AsmArgs A,
                                                       const unsigned char *__restrict__ status,
-                                                      const int *__restrict__ tlist) {
-  extern __shared__ double lds[];
-  double *blk = lds + A.lds_blk;
-  double *Jbuf = lds + A.lds_J;
-  double *Tl = lds + A.lds_T;
-  const int t = tlist[blockIdx.x];
-  if (status[2 * t + 1]) return;
-  const ecp_triplet tr = J.trip[t];
-  const ecp_centre Cn = J.cent[tr.centre];
-  const ecp_shell Sa = J.shells[tr.sa], Sb = J.shells[tr.sb];
-  const int la = tr.la, lb = tr.lb, lab = la + lb;  // shifted for derivatives
-  const int nca = ECP_DIM_C(la), ncb = ECP_DIM_C(lb);
-  const ecp_xyz rc = J.atoms[Cn.atom], ra = J.atoms[Sa.atom], rb = J.atoms[Sb.atom];
-  const double rAC[3] = {ra.x - rc.x, ra.y - rc.y, ra.z - rc.z};
-  const double rBC[3] = {rb.x - rc.x, rb.y - rc.y, rb.z - rc.z};
-  const V3 vA{rAC[0], rAC[1], rAC[2]}, vB{rBC[0], rBC[1], rBC[2]};
-  const int D = T.ijkDim;
-  const int t0 = t2_off(T, la, lb, 0), eoff = J.teoff[t];
-  for (int i = threadIdx.x; i < nca * ncb; i += blockDim.x) blk[i] = 0.0;
-  __syncthreads();
-  const int nlm2 = J.angL * J.angL;
-  const double *angA = J.ang + Cn.ang_off + (size_t)(Sa.atom - Cn.atom0) * J.ang_lam * nlm2 * J.ang_c;
-  const double *angB = J.ang + Cn.ang_off + (size_t)(Sb.atom - Cn.atom0) * J.ang_lam * nlm2 * J.ang_c;
-  for (int l = 0; l < Cn.L; l++) {
-    const int eb = t2_off(T, la, lb, l) - t0, ee = t2_off(T, la, lb, l + 1) - t0;
-    const int d1 = la + l + 1, d2 = lb + l + 1, d3 = lab + 1;
-    for (int i = threadIdx.x; i < d1 * d2 * d3; i += blockDim.x) Tl[i] = 0.0;
-    __syncthreads();
-    for (int e = eb + (int)threadIdx.x; e < ee; e += kAsmThreads) {
-      const int code = T.tmpl[t0 + e];
-      const int l1 = code & 0xff, l2 = (code >> 8) & 0xff, l3 = (code >> 16) & 0xff;
-      const double v = !A.tfail[eoff + e]
-                           ? A.Tout[eoff + e]
-                           : sum_in_order(0.0, A.fbT + (size_t)(eoff + e) * J.maxPairs, Sa.K * Sb.K);
-      Tl[(l1 * d2 + l2) * d3 + l3] = v;
-    }
-    __syncthreads();
-    asm2_channel_of<NB, MAXL>(l, angA, angB, J.ang_c, nlm2, Tl, la, lb, nca, ncb, 1.0f / ncb, blk, threadIdx.x,
-                              kAsmThreads);
-    __syncthreads();
-  }
-  const double norm2 = (4.0 * M_PI) * (4.0 * M_PI);
-  auto get2 = [&](int r, int q) { return blk[r * ncb + q]; };
-  shift_block(T, get2, tr.oa, tr.ob, vA, vB, norm2, Jbuf, lds + A.lds_S2, A.shift_lm, A.blocks + tr.blk2);
-}
-
-// Type-2 blocks of classes la + lb <= kAsmPackLab (at most 9 elements),
-// kAsmPack triplets per wave (tlist[0 .. ntl)): lane groups of
-// kAsmThreads / kAsmPack lanes, each with an LDS slice of A.lds_group
-// doubles, run k_asm2's phases side by side with the same arithmetic.  The channel loop runs to the wave's largest L, a group past its
-// own with empty loops; every group synchronises with the wave.
-template <int MAXL>
-__global__ __launch_bounds__(kAsmThreads) void k_asm2p(DevTables T, DevJob J, AsmArgs A,
-                                                    const unsigned char *__restrict__ status,
-                                                    const int *__restrict__ tlist, int ntl) {
+                                                      const int *__restrict__ tlist, int ntl) {
   extern __shared__ double lds_all[];
-  constexpr int G = kAsmPack, W = kAsmThreads / G;
-  const int grp = (int)threadIdx.x / W, lid = (int)threadIdx.x % W;
-  double *lds = lds_all + (size_t)grp * A.lds_group;
-  double *blk = lds + A.lds_blk;
-  double *Jbuf = lds + A.lds_J;
-  double *Tl = lds + A.lds_T;
-  const int ti = blockIdx.x * G + grp;
+  constexpr int W = kAsmThreads / G;
+  const int grp = G == 1 ? 0 : (int)threadIdx.x / W, lid = (int)threadIdx.x % W;
+  double *lds = lds_all + (G == 1 ? 0 : (size_t)grp * A.lds_group);
+  double *blk = lds + A.lds_blk, *Jbuf = lds + A.lds_J, *Tl = lds + A.lds_T;
+  const int ti = xcd_item(blockIdx.x, gridDim.x) * G + grp;
   bool active = ti < ntl;
-  const int t = active ? tlist[ti] : tlist[0];
-  if (active && status[2 * t + 1]) active = false;
+  const int t = cload(tlist + (active ? ti : 0));
+  if (status[2 * t + 1]) active = false;
   if (!wave_any(active)) return;
   const ecp_triplet tr = J.trip[t];
   const ecp_centre Cn = J.cent[tr.centre];
   const ecp_shell Sa = J.shells[tr.sa], Sb = J.shells[tr.sb];
-  const int la = tr.la, lb = tr.lb, lab = la + lb;  // shifted for derivatives
+  const int la = tr.la, lb = tr.lb;  // shifted for derivatives
   const int nca = ECP_DIM_C(la), ncb = ECP_DIM_C(lb);
   const ecp_xyz rc = J.atoms[Cn.atom], ra = J.atoms[Sa.atom], rb = J.atoms[Sb.atom];
   const V3 vA{ra.x - rc.x, ra.y - rc.y, ra.z - rc.z}, vB{rb.x - rc.x, rb.y - rc.y, rb.z - rc.z};
   const int t0 = t2_off(T, la, lb, 0), eoff = J.teoff[t];
-  if (active)
-    for (int i = lid; i < nca * ncb; i += W) blk[i] = 0.0;
-  int Lw = active ? Cn.L : 0;
-  for (int o = 32; o > 0; o >>= 1) Lw = max(Lw, __shfl_xor(Lw, o, 64));
+  const int ne = active ? t2_off(T, la, lb, Cn.L) - t0 : 0, npairs = Sa.K * Sb.K;
+  const int nslots = active ? t2_slots(la, lb, Cn.L) : 0;
+  for (int i = lid; i < nslots; i += W) Tl[i] = 0.0;
   __syncthreads();
-  const int nlm2 = J.angL * J.angL;
-  const double *angA = J.ang + Cn.ang_off + (size_t)(Sa.atom - Cn.atom0) * J.ang_lam * nlm2 * J.ang_c;
-  const double *angB = J.ang + Cn.ang_off + (size_t)(Sb.atom - Cn.atom0) * J.ang_lam * nlm2 * J.ang_c;
-  for (int l = 0; l < Lw; l++) {
-    const bool on = active && l < Cn.L;
-    const int d1 = la + l + 1, d2 = lb + l + 1, d3 = lab + 1;
-    int eb = 0, ee = 0;
-    if (on) {
-      eb = t2_off(T, la, lb, l) - t0;
-      ee = t2_off(T, la, lb, l + 1) - t0;
-      for (int i = lid; i < d1 * d2 * d3; i += W) Tl[i] = 0.0;
+  for (int e0 = lid; e0 < ne; e0 += 4 * W) {
+    double v[4];
+    int code[4];
+    unsigned char f[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int e = min(e0 + i * W, ne - 1);
+      v[i] = A.Tout[eoff + e];
+      f[i] = A.tfail[eoff + e];
+      code[i] = T.tmpl[t0 + e];
     }
-    __syncthreads();
-    if (on)
-      for (int e = eb + lid; e < ee; e += W) {
-        const int code = T.tmpl[t0 + e];
-        const int l1 = code & 0xff, l2 = (code >> 8) & 0xff, l3 = (code >> 16) & 0xff;
-        const double v = !A.tfail[eoff + e]
-                             ? A.Tout[eoff + e]
-                             : sum_in_order(0.0, A.fbT + (size_t)(eoff + e) * J.maxPairs, Sa.K * Sb.K);
-        Tl[(l1 * d2 + l2) * d3 + l3] = v;
-      }
-    __syncthreads();
-    if (on)
-      asm2_channel_of<kAsmPackLab + 1, MAXL>(l, angA, angB, J.ang_c, nlm2, Tl, la, lb, nca, ncb, 1.0f / ncb, blk, lid,
-                                             W);
-    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int e = e0 + i * W;
+      if (e >= ne) break;
+      if (f[i]) v[i] = sum_in_order(0.0, A.fbT + (size_t)(eoff + e) * J.maxPairs, npairs);
+      Tl[t2_slot(la, lb, code[i] >> 24, code[i] & 0xff, (code[i] >> 8) & 0xff, (code[i] >> 16) & 0xff)] = v[i];
+    }
   }
+  __syncthreads();
+  const int lam_stride = J.angL * J.angL * J.ang_c;
+  const double *angA = J.ang + Cn.ang_off + (size_t)(Sa.atom - Cn.atom0) * J.ang_lam * lam_stride;
+  const double *angB = J.ang + Cn.ang_off + (size_t)(Sb.atom - Cn.atom0) * J.ang_lam * lam_stride;
+  const float inv_ncb = 1.0f / ncb;
+  for (int idx = active ? lid : nca * ncb; idx < nca * ncb; idx += W) {
+    const int pp = (int)(((float)idx + 0.5f) * inv_ncb), qq = idx - pp * ncb;
+    const int alpha = deg_of(pp), beta = deg_of(qq);
+    double v = 0.0;
+#define CH(x)                                                                                          \
+  if constexpr (x < MAXL)                                                                              \
+    if (x < Cn.L) v += asm2_channel<NB, x>(angA + pp, angB + qq, J.ang_c, lam_stride, Tl, la, lb, alpha, beta);
+    CH(0) CH(1) CH(2) CH(3) CH(4) CH(5) CH(6)
+#undef CH
+    blk[idx] = v;
+  }
+  __syncthreads();
   const double norm2 = (4.0 * M_PI) * (4.0 * M_PI);
   auto get2 = [&](int r, int q) { return blk[r * ncb + q]; };
   shift_block(T, get2, tr.oa, tr.ob, vA, vB, norm2, Jbuf, lds + A.lds_S2, A.shift_lm, A.blocks + tr.blk2, lid, W,
@@ -2296,7 +2270,6 @@ struct TabArgs {
   double *udir;
   const int2 *ait;           // (centre, atom) pairs of the angular tables, aparts workgroups each
   int nait, aparts;
-  const double *fac, *dfac;
 };
 
 // The pair direction k = 2 (za rAC + zb rBC) of a type-1 unit (type1.c:
@@ -2326,7 +2299,7 @@ __global__ __launch_bounds__(128, 4) void k_tables(DevTables T, DevJob J, TabArg
   int b = blockIdx.x;
   // the longest items first
   if (b < A.nait * A.aparts) {
-    ang_item(T, J, A.ait[b / A.aparts], A.fac, A.dfac, rsph, s_dir, b % A.aparts, A.aparts);
+    ang_item(T, J, A.ait[b / A.aparts], rsph, s_dir, b % A.aparts, A.aparts);
     return;
   }
   b -= A.nait * A.aparts;
@@ -2436,7 +2409,6 @@ struct ecp_dev {
   size_t pin_in_cap = 0;
   char *pin_out = nullptr;
   size_t pin_out_cap = 0;
-  double *dfac_dev = nullptr, *fac_dev = nullptr;
   int lds_max = 64 * 1024;  // LDS per workgroup of the device (160 KiB on gfx950)
   hipEvent_t ev[8] = {};
   float last_ms[8] = {};
@@ -2605,7 +2577,9 @@ extern "C" ecp_dev *ecp_dev_create(const ecp_static *st, char *err, size_t errle
   const size_t o_vis = take(so * 4), o_v93 = take((st->s93.npairs + kPs93Pad) * sizeof(Ps93Pair));
   const size_t o_bess = take(nbess * 8), o_poly = take(npoly * 8), o_om = take(nom * 8);
   const size_t o_ijk = take(nijk * 4), o_idx = take(nidx * 4), o_bin = take(256 * 8);
-  const size_t o_fac = take(nfac * 8), o_dfac = take(nfac * 8);
+  const size_t o_snorm = take(kSphDim * kSphDim * 8), o_dfac = take(nfac * 8), o_inv = take(kSphDim * 8);
+  const int prodN = ECP_DIM_C(st->omAlpha);
+  const size_t o_prod = take((size_t)prodN * prodN * 4);
   const size_t o_tmpl = take(d->tmpl.size() * 4 + 4), o_toff = take(d->toff.size() * 4);
   std::vector<char> h(off, 0);
   auto put = [&](size_t o, const void *src, size_t bytes) { memcpy(h.data() + o, src, bytes); };
@@ -2649,7 +2623,24 @@ extern "C" ecp_dev *ecp_dev_create(const ecp_static *st, char *err, size_t errle
   put(o_ijk, st->ijk, nijk * 4);
   put(o_idx, st->ijkIndex, nidx * 4);
   put(o_bin, binom.data(), 256 * 8);
-  put(o_fac, st->fac, nfac * 8);
+  {
+    std::vector<double> nrm(kSphDim * kSphDim, 0.0), inv(kSphDim, 0.0);
+    for (int l = 0; l < kSphDim; l++) {
+      const double norm0 = sqrt((2.0 * l + 1.0) / (2.0 * M_PI));
+      for (int m = 0; m <= l && l + m < (int)nfac; m++)
+        nrm[l * kSphDim + m] = m == 0 ? norm0 : sqrt(st->fac[l - m] / st->fac[l + m]) * norm0;
+      if (l > 0) inv[l] = 1.0 / l;
+    }
+    put(o_snorm, nrm.data(), nrm.size() * 8);
+    put(o_inv, inv.data(), inv.size() * 8);
+    std::vector<int> prod((size_t)prodN * prodN);
+    for (int r = 0; r < prodN; r++)
+      for (int q = 0; q < prodN; q++) {
+        const int *a = st->ijk + 3 * r, *c = st->ijk + 3 * q, D = st->ijkDim;
+        prod[(size_t)r * prodN + q] = st->ijkIndex[((a[0] + c[0]) * D + a[1] + c[1]) * D + a[2] + c[2]];
+      }
+    put(o_prod, prod.data(), prod.size() * 4);
+  }
   put(o_dfac, st->dfac, nfac * 8);
   put(o_tmpl, d->tmpl.data(), d->tmpl.size() * 4);
   put(o_toff, d->toff.data(), d->toff.size() * 4);
@@ -2674,8 +2665,11 @@ extern "C" ecp_dev *ecp_dev_create(const ecp_static *st, char *err, size_t errle
   T.ijk = (const int *)(b + o_ijk);
   T.ijkIndex = (const int *)(b + o_idx);
   T.binom = (const double *)(b + o_bin);
-  d->fac_dev = (double *)(b + o_fac);
-  d->dfac_dev = (double *)(b + o_dfac);
+  T.snorm = (const double *)(b + o_snorm);
+  T.dfac = (const double *)(b + o_dfac);
+  T.inv = (const double *)(b + o_inv);
+  T.prod = (const int *)(b + o_prod);
+  T.prodN = prodN;
   T.tmpl = (const int *)(b + o_tmpl);
   T.toff = (const int *)(b + o_toff);
   T.ijkDim = st->ijkDim;
@@ -2752,23 +2746,19 @@ void launch_type2(ecp_dev *d, hipStream_t s) {
 void launch_asm2(ecp_dev *d, hipStream_t s) {
   const Prepared &P = d->P;
   Span sp(d, s, FAM_ASM);
-  const int m = P.tcls_begin[kAsmPackLab + 1];
-  if (m > 0) {
-    const int g = (m + kAsmPack - 1) / kAsmPack;
-    if (P.max_L <= 4) k_asm2p<4><<<g, kAsmThreads, P.asm2_lds4, s>>>(d->T, P.J, P.aa2p, P.stat, P.tcls, m);
-    else if (P.max_L == 5) k_asm2p<5><<<g, kAsmThreads, P.asm2_lds4, s>>>(d->T, P.J, P.aa2p, P.stat, P.tcls, m);
-    else k_asm2p<7><<<g, kAsmThreads, P.asm2_lds4, s>>>(d->T, P.J, P.aa2p, P.stat, P.tcls, m);
-  }
-  const int n = P.nt - m;
-  if (n <= 0) return;
-  const int *tl = P.tcls + m;
   const bool cache = d->tune.asm2_cache != 0;
-  if (cache && P.max_lbs <= 3 && P.max_L <= 4)
-    k_asm2<4, 4><<<n, kAsmThreads, P.asm2_lds, s>>>(d->T, P.J, P.aa, P.stat, tl);
-  else if (cache && P.max_lbs <= 4 && P.max_L <= 5)
-    k_asm2<5, 5><<<n, kAsmThreads, P.asm2_lds, s>>>(d->T, P.J, P.aa, P.stat, tl);
-  else
-    k_asm2<0, 7><<<n, kAsmThreads, P.asm2_lds, s>>>(d->T, P.J, P.aa, P.stat, tl);
+  const int m = P.tcls_begin[kAsmPackLab + 1], n = P.nt - m;
+  auto go = [&](auto kernel, int g, size_t lds, const AsmArgs &aa, const int *tl, int ntl) {
+    if (g > 0) kernel<<<g, kAsmThreads, lds, s>>>(d->T, P.J, aa, P.stat, tl, ntl);
+  };
+  const int *tl = P.tcls + m;
+  if (cache && P.max_lbs <= 3 && P.max_L <= 4) go(k_asm2<1, 4, 4>, n, P.asm2_lds, P.aa, tl, n);
+  else if (cache && P.max_lbs <= 4 && P.max_L <= 5) go(k_asm2<1, 5, 5>, n, P.asm2_lds, P.aa, tl, n);
+  else go(k_asm2<1, 0, 7>, n, P.asm2_lds, P.aa, tl, n);
+  const int gp = (m + kAsmPack - 1) / kAsmPack;
+  if (P.max_L <= 4) go(k_asm2<kAsmPack, kAsmPackLab + 1, 4>, gp, P.asm2_lds4, P.aa2p, P.tcls, m);
+  else if (P.max_L == 5) go(k_asm2<kAsmPack, kAsmPackLab + 1, 5>, gp, P.asm2_lds4, P.aa2p, P.tcls, m);
+  else go(k_asm2<kAsmPack, 0, 7>, gp, P.asm2_lds4, P.aa2p, P.tcls, m);
 }
 
 // type-1 assembly of the triplets tcls[b .. e) (class-ordered), one per
@@ -2922,8 +2912,6 @@ void launch_tables(ecp_dev *d, hipStream_t s) {
   // few pairs: several workgroups each (20 atoms with g shells, 160 pairs:
   // the launch 116 us at one, 4556 workgroups in all)
   A.aparts = P.nait < 1024 ? 4 : 1;
-  A.fac = d->fac_dev;
-  A.dfac = d->dfac_dev;
   Span sp(d, s, FAM_TABLES);
   k_tables<<<A.nait * A.aparts + A.nzb + A.nub + A.nfit + (A.nunits + 127) / 128, 128, 0, s>>>(d->T, P.J, A);
 }
@@ -3249,7 +3237,7 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
     o = base;
     aa.lds_blk = o; o += ECP_DIM_C(LM) * ECP_DIM_C(LM);
     aa.lds_S2 = o;
-    aa.lds_T = o; o += (LM + LC) * (LM + LC) * (2 * LM + 1);
+    aa.lds_T = o; o += t2_slots(LM, LM, LC);
     const int end2 = std::max(o, aa.lds_S2 + ns);
     P.asm1_lds = (size_t)end1 * sizeof(double);
     // packed type 1 (la + lb <= kAsmPackLab): one slice of LDS per triplet
@@ -3277,7 +3265,12 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
       a2.lds_J = o2; o2 += ECP_DIM_IJK(LS) * ECP_DIM_C(LS);
       a2.lds_blk = o2; o2 += ECP_DIM_C(LS) * ECP_DIM_C(LS);
       a2.lds_S2 = o2;
-      a2.lds_T = o2; o2 += (LS + LC) * (LS + LC) * (2 * LS + 1);
+      a2.lds_T = o2;
+      int ts = 0;
+      for (int x = 0; x <= LS; x++)
+        for (int y = 0; y <= LS; y++)
+          if (x + y <= kAsmPackLab) ts = std::max(ts, t2_slots(x, y, LC));
+      o2 += ts;
       a2.lds_group = std::max(o2, a2.lds_S2 + shift_tab_doubles(LS));
       P.asm2_lds4 = (size_t)kAsmPack * a2.lds_group * sizeof(double);
     }
@@ -3417,8 +3410,6 @@ extern "C" int ecp_dev_bind(ecp_dev *d, void *mem, size_t cap, char *err, size_t
     aa.Tout = P.Tout;
     aa.tfail = P.tf;
     aa.fbT = P.fbT;
-    aa.fac = d->fac_dev;
-    aa.dfac = d->dfac_dev;
     aa.blocks = P.blk;
   }
   d->prepared = true;
