@@ -1154,7 +1154,7 @@ __device__ __forceinline__ int t2_off(const DevTables &T, int la, int lb, int l)
 struct T2Args {
   double *Tout;
   unsigned char *tfail;
-  int *tnfail, *flist;  // per triplet: number of failed entries, listed at flist[teoff ...] in entry order
+  int *tnfail, *flist;  // per triplet: number of failed entries, listed at flist[teoff ...]
   int *fbq, *fbcount;   // per fallback class, the triplets with failed entries (qstride apart)
   int qstride;
   const unsigned char *tcls2;  // per triplet: its fallback class max(la, lb) + L - 1
@@ -1211,7 +1211,8 @@ typedef double dpair __attribute__((ext_vector_type(2)));
 // U rows have even lengths, so that every chunk is aligned
 template <int G, int NP, int R, int CH>
 __device__ __forceinline__ void type2_body(int bid, const DevTables &T, const DevJob &J, const T2Args &A,
-                                           const int *__restrict__ tlist, int ntl, double *s_all) {
+                                           const int *__restrict__ tlist, int ntl, int slice, int nslices,
+                                           double *s_all) {
   constexpr int W = 64 / G, LP = G == 1 ? 32 : 16, PT = W / LP, X = (CH + LP - 1) / LP, ROW = 2 * CH;
   const int grp = (int)threadIdx.x / W, lid = (int)threadIdx.x % W;
   const int pt = lid / LP, pl = lid % LP;  // point of a read, lane of the point
@@ -1246,8 +1247,7 @@ __device__ __forceinline__ void type2_body(int bid, const DevTables &T, const De
       st[x] = 0;
     }
   }
-  int nfail = 0;
-  for (int e0 = 0; __ballot(e0 < ne) != 0ull; e0 += W * R) {
+  for (int e0 = slice * W * R; __ballot(e0 < ne) != 0ull; e0 += nslices * W * R) {
     // LDS offsets of the entries' values, and their states
     int oa[R], ob[R], ou[R];
     T2State S[R];
@@ -1390,26 +1390,36 @@ __device__ __forceinline__ void type2_body(int bid, const DevTables &T, const De
         if (last || !wave_any(group_open())) break;
       }
     }
-    // results; the failed entries in entry order
+    // results; the pass's failed entries are listed together, and the first
+    // to list any puts the triplet on its fallback queue
+    bool fail[R];
+    int below[R], nfail = 0;
 #pragma unroll
     for (int i = 0; i < R; i++) {
       const int e = e0 + i * W + lid;
-      const bool fail = e < ne && !S[i].done;
+      fail[i] = e < ne && !S[i].done;
       if (e < ne) {
         A.Tout[eoff + e] = S[i].res;
-        A.tfail[eoff + e] = fail;
+        A.tfail[eoff + e] = fail[i];
       }
-      unsigned long long m = __ballot(fail);
+      unsigned long long m = __ballot(fail[i]);
       if (G > 1) m = (m >> (grp * W)) & ((1ull << (W & 63)) - 1ull);
-      if (fail) A.flist[eoff + nfail + __popcll(m & ((1ull << lid) - 1ull))] = e;
+      below[i] = nfail + __popcll(m & ((1ull << lid) - 1ull));
       nfail += __popcll(m);
     }
-  }
-  if (active && lid == 0) {
-    A.tnfail[t] = nfail;
-    if (nfail) {
-      const int c = A.tcls2[t];
-      A.fbq[(size_t)c * A.qstride + atomicAdd(&A.fbcount[c], 1)] = t;
+    if (wave_any(nfail != 0)) {
+      int base = 0;
+      if (lid == 0 && nfail) {
+        base = atomicAdd(&A.tnfail[t], nfail);
+        if (base == 0) {
+          const int c = A.tcls2[t];
+          A.fbq[(size_t)c * A.qstride + atomicAdd(&A.fbcount[c], 1)] = t;
+        }
+      }
+      base = __shfl(base, grp * W);
+#pragma unroll
+      for (int i = 0; i < R; i++)
+        if (fail[i]) A.flist[eoff + base + below[i]] = e0 + i * W + lid;
     }
   }
 }
@@ -1417,18 +1427,26 @@ __device__ __forceinline__ void type2_body(int bid, const DevTables &T, const De
 // The triplets of classes above kT2PackLab (tlist[m .. nt)), one per wave,
 // then those up to it (tlist[0 .. m)), kT2Pack to a wave.  CH, CHP: 16-byte
 // chunks of a point's values, of a triplet of either kind.
-constexpr int kT2Pack = 2, kT2PackLab = 2, kT2Pairs = 4;
-
+// A triplet of many entries takes one wave's passes in turn, kT2Pass entries
+// each; jobs too small to fill the chip (kT2Fill waves, four times what it
+// holds) split the passes over `nslices` waves per triplet.  A pass stages
+// its points' rows in either case, so that the split adds no work: 17 atoms
+// 231 -> 197 us an evaluation, 50 atoms 380 -> 342 us (at a quarter of
+// kT2Fill: no gain on the latter), g shells shifted to h under L = 6 on
+// three atoms 1331 -> 582 us (with the wide assembly below).
+constexpr int kT2Pack = 2, kT2PackLab = 2, kT2Pairs = 4, kT2Fill = 16384, kT2Pass = 128;
 
 template <int CH, int CHP>
 __global__ __launch_bounds__(64, CH <= 24 ? 4 : 3) void k_type2(DevTables T, DevJob J, T2Args A, const int *__restrict__ tlist,
-                                                int m) {
+                                                int m, int nslices) {
   __shared__ __align__(16) double s_v[t2_lds(1, kT2Pairs, CH) > t2_lds(kT2Pack, kT2Pairs, CHP)
                                           ? t2_lds(1, kT2Pairs, CH)
                                           : t2_lds(kT2Pack, kT2Pairs, CHP)];
   const int n = J.ntrip - m, np = (m + kT2Pack - 1) / kT2Pack, b = blockIdx.x;
-  if (b < n) type2_body<1, kT2Pairs, 2, CH>(xcd_item(b, n), T, J, A, tlist + m, n, s_v);
-  else type2_body<kT2Pack, kT2Pairs, 2, CHP>(xcd_item(b - n, np), T, J, A, tlist, m, s_v);
+  if (b < n * nslices)
+    type2_body<1, kT2Pairs, 2, CH>(xcd_item(b % n, n), T, J, A, tlist + m, n, b / n, nslices, s_v);
+  else
+    type2_body<kT2Pack, kT2Pairs, 2, CHP>(xcd_item(b - n * nslices, np), T, J, A, tlist, m, 0, 1, s_v);
 }
 
 // type-2 fallback (calcT_FM06, type2.c:417-528): one wave per (triplet with
@@ -2175,12 +2193,12 @@ __device__ __forceinline__ double asm2_channel(const double *__restrict__ pA, co
 // lanes form the elements, contracting them with the angular tables of both
 // atoms (type2.c:583-623), and the block is shifted (util.c:246-334).
 // NB: as in asm2_channel; channels l < MAXL.
-template <int G, int NB, int MAXL>
-__global__ __launch_bounds__(kAsmThreads) void k_asm2(DevTables T, DevJob J, AsmArgs A,
+template <int G, int NB, int MAXL, int NT = kAsmThreads>
+__global__ __launch_bounds__(NT) void k_asm2(DevTables T, DevJob J, AsmArgs A,
                                                       const unsigned char *__restrict__ status,
                                                       const int *__restrict__ tlist, int ntl) {
   extern __shared__ double lds_all[];
-  constexpr int W = kAsmThreads / G;
+  constexpr int W = NT / G;
   const int grp = G == 1 ? 0 : (int)threadIdx.x / W, lid = (int)threadIdx.x % W;
   double *lds = lds_all + (G == 1 ? 0 : (size_t)grp * A.lds_group);
   double *blk = lds + A.lds_blk, *Jbuf = lds + A.lds_J, *Tl = lds + A.lds_T;
@@ -2732,29 +2750,44 @@ void launch_type2(ecp_dev *d, hipStream_t s) {
   T2Args A{P.Tout, P.tf, P.tnfail, P.flist, P.fbq2, P.fbc + kFb2Cnt, P.nt, P.tcls2};
   Span sp(d, s, FAM_TYPE2);
   const int m = P.tcls_begin[kT2PackLab + 1];
-  const int grid = P.nt - m + (m + kT2Pack - 1) / kT2Pack;
-  if (P.max_lbs <= 3 && P.max_L <= 4) k_type2<24, 14><<<grid, 64, 0, s>>>(d->T, P.J, A, P.tcls, m);
-  else if (P.max_lbs <= 4 && P.max_L <= 5) k_type2<35, 17><<<grid, 64, 0, s>>>(d->T, P.J, A, P.tcls, m);
-  else k_type2<63, 23><<<grid, 64, 0, s>>>(d->T, P.J, A, P.tcls, m);
+  const int n = P.nt - m, npass = (P.max_ent2 + kT2Pass - 1) / kT2Pass;
+  const int ns = std::max(1, std::min(npass, kT2Fill / std::max(n, 1)));
+  const int grid = n * ns + (m + kT2Pack - 1) / kT2Pack;
+  if (P.max_lbs <= 3 && P.max_L <= 4) k_type2<24, 14><<<grid, 64, 0, s>>>(d->T, P.J, A, P.tcls, m, ns);
+  else if (P.max_lbs <= 4 && P.max_L <= 5) k_type2<35, 17><<<grid, 64, 0, s>>>(d->T, P.J, A, P.tcls, m, ns);
+  else k_type2<63, 23><<<grid, 64, 0, s>>>(d->T, P.J, A, P.tcls, m, ns);
 }
+
+// Jobs of up to this many type-2 blocks (of classes above kAsmPackLab) give
+// each 256 threads: 17 atoms 197 -> 180 us an evaluation; 50 atoms (1000 to
+// 4000 such blocks) lose, 379 -> 398 us, and 256 molecules are unchanged to
+// 19 % slower.
+constexpr int kAsm2Wide = 1024;
 
 // type-2 assembly: the register-cached variant fits basis l <= 3 with
 // projectors l <= 3, or basis l <= 4 with projectors l <= 4; larger jobs (and
 // asm2_cache 0) read the tables directly.  The triplets of classes la + lb
 // <= kAsmPackLab (the first of the class-ordered list) go kAsmPack to a
-// wave, the others one per workgroup.
+// wave, the others one per workgroup: a wave where the job fills the chip,
+// 256 threads where it does not and for the largest classes, whose LDS lets
+// few workgroups share a CU (i shells, L = 7: 5477 -> 2092 us with the split
+// small grid).
 void launch_asm2(ecp_dev *d, hipStream_t s) {
   const Prepared &P = d->P;
   Span sp(d, s, FAM_ASM);
   const bool cache = d->tune.asm2_cache != 0;
   const int m = P.tcls_begin[kAsmPackLab + 1], n = P.nt - m;
-  auto go = [&](auto kernel, int g, size_t lds, const AsmArgs &aa, const int *tl, int ntl) {
-    if (g > 0) kernel<<<g, kAsmThreads, lds, s>>>(d->T, P.J, aa, P.stat, tl, ntl);
+  auto go = [&](auto kernel, int g, size_t lds, const AsmArgs &aa, const int *tl, int ntl, int nt = kAsmThreads) {
+    if (g > 0) kernel<<<g, nt, lds, s>>>(d->T, P.J, aa, P.stat, tl, ntl);
   };
   const int *tl = P.tcls + m;
-  if (cache && P.max_lbs <= 3 && P.max_L <= 4) go(k_asm2<1, 4, 4>, n, P.asm2_lds, P.aa, tl, n);
+  const bool wide = n <= kAsm2Wide;
+  if (cache && P.max_lbs <= 3 && P.max_L <= 4 && wide) go(k_asm2<1, 4, 4, 256>, n, P.asm2_lds, P.aa, tl, n, 256);
+  else if (cache && P.max_lbs <= 4 && P.max_L <= 5 && wide)
+    go(k_asm2<1, 5, 5, 256>, n, P.asm2_lds, P.aa, tl, n, 256);
+  else if (cache && P.max_lbs <= 3 && P.max_L <= 4) go(k_asm2<1, 4, 4>, n, P.asm2_lds, P.aa, tl, n);
   else if (cache && P.max_lbs <= 4 && P.max_L <= 5) go(k_asm2<1, 5, 5>, n, P.asm2_lds, P.aa, tl, n);
-  else go(k_asm2<1, 0, 7>, n, P.asm2_lds, P.aa, tl, n);
+  else go(k_asm2<1, 0, 7, 256>, n, P.asm2_lds, P.aa, tl, n, 256);
   const int gp = (m + kAsmPack - 1) / kAsmPack;
   if (P.max_L <= 4) go(k_asm2<kAsmPack, kAsmPackLab + 1, 4>, gp, P.asm2_lds4, P.aa2p, P.tcls, m);
   else if (P.max_L == 5) go(k_asm2<kAsmPack, kAsmPackLab + 1, 5>, gp, P.asm2_lds4, P.aa2p, P.tcls, m);
@@ -2853,7 +2886,10 @@ void launch_fb2_fused(ecp_dev *d, hipStream_t s, const T2Set &S2, const ClassMap
   // the registers (168) allow
   const size_t lds = sizeof(double) * (kFb2Chunk * kFbTS + (S2.cu_rows + S2.rn_rows + 2 * S2.k_rows) * 64);
   if (P.max_cls2 > 11) k_fb2_fused<12><<<nb, 64, lds, s>>>(d->T, P.J, S2, cm);
-  else if (P.max_cls2 > 7) k_fb2_fused<11><<<nb, 64, lds, s>>>(d->T, P.J, S2, cm);
+  // (class 8, g shells under L = 5, without class 11's scratch: 20 atoms
+  // 4450 -> 3864 us an evaluation)
+  else if (P.max_cls2 > 8) k_fb2_fused<11><<<nb, 64, lds, s>>>(d->T, P.J, S2, cm);
+  else if (P.max_cls2 > 7) k_fb2_fused<8><<<nb, 64, lds, s>>>(d->T, P.J, S2, cm);
   else k_fb2_fused<7><<<nb, 64, lds, s>>>(d->T, P.J, S2, cm);
 }
 
@@ -2916,9 +2952,18 @@ void launch_tables(ecp_dev *d, hipStream_t s) {
   k_tables<<<A.nait * A.aparts + A.nzb + A.nub + A.nfit + (A.nunits + 127) / 128, 128, 0, s>>>(d->T, P.J, A);
 }
 
-// fuse = 2 (automatic): fused launches for jobs of up to this many type-1
-// primitive pairs (latency-bound: per-class launches hold few waves each)
-constexpr int kFuseAutoMaxUnits = 150000;
+// fuse = 2 (automatic), by the job's type-1 primitive pairs.  Up to
+// kFuseAutoSmall fused launches: per-class ones hold few waves each (10 503
+// pairs: 180 against 262 us an evaluation).  Up to kFuseAutoLarge per class,
+// each class with its own registers (235 440 pairs: 691 against 720 us;
+// 445 424 pairs of classes up to 8: 3864 against 4057 us).  Above, fused
+// again where the largest class is 6: every stage fills the chip by itself
+// (1 273 608 pairs: 3045 against 3302 us; 6.2 million: 14.44 against 14.82 ms).
+constexpr int kFuseAutoSmall = 150000, kFuseAutoLarge = 800000;
+
+bool fuse_auto(int units, int max_lab) {
+  return units <= kFuseAutoSmall || (units > kFuseAutoLarge && max_lab <= 6);
+}
 
 // one type-1 class of the per-class sequence: quadrature, assembly
 template <int c>
@@ -2941,7 +2986,7 @@ void enqueue_t1_class(ecp_dev *d, hipStream_t ws, int c) {
 
 void enqueue(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
   const int units = d->P.cls_begin[ECP_MAX_LAB + 1];
-  const bool fused = d->tune.fuse == 1 || (d->tune.fuse == 2 && units <= kFuseAutoMaxUnits);
+  const bool fused = d->tune.fuse == 1 || (d->tune.fuse == 2 && fuse_auto(units, d->P.max_lab));
   if (fused) {
     enqueue_fused(d, s, evs);
     return;
@@ -3017,26 +3062,26 @@ void enqueue_fused(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
   (void)hipStreamWaitEvent(w, d->fork, 0);
   // ---- type 1 ----
   const T1Set S = t1_set(d);
-  // the fused kernels hold the registers of their largest class: three
-  // instantiations, classes up to 6, 10 and 12
-  const int tier1 = P.max_lab > 10 ? 2 : P.max_lab > 6 ? 1 : 0;
+  // the fused kernels hold the registers of their largest class: four
+  // instantiations, classes up to 6, 8, 10 and 12 (8 without spills; with
+  // class 10's registers for a class-8 job the evaluation took 2 % longer)
+  auto launch = [&](auto f6, auto f8, auto f10, auto f12, const ClassMap &cm) {
+    auto f = P.max_lab <= 6 ? f6 : P.max_lab <= 8 ? f8 : P.max_lab <= 10 ? f10 : f12;
+    f<<<cm.bbeg[cm.n], 64, 0, w>>>(T, J, S, cm);
+  };
   const ClassMap cmh = class_map(ECP_MAX_LAB + 1, P.cls_count, [&](int c) { return (P.cls_count[c] + 63) / 64; });
   if (cmh.n > 0) {
     // external event nodes when captured, so that replays record them too
     (void)hipEventRecordWithFlags(d->span[d->span_k][0], w, d->capturing ? hipEventRecordExternal : 0);
     {
       Span sp(d, w, FAM_TYPE1);
-      if (tier1 == 2) k_type1_fused<12><<<cmh.bbeg[cmh.n], 64, 0, w>>>(T, J, S, cmh);
-      else if (tier1 == 1) k_type1_fused<10><<<cmh.bbeg[cmh.n], 64, 0, w>>>(T, J, S, cmh);
-      else k_type1_fused<6><<<cmh.bbeg[cmh.n], 64, 0, w>>>(T, J, S, cmh);
+      launch(k_type1_fused<6>, k_type1_fused<8>, k_type1_fused<10>, k_type1_fused<12>, cmh);
     }
     {
       const ClassMap cmt = class_map(ECP_MAX_LAB + 1, P.cls_count,
                                      [&](int c) { return std::min(P.cls_count[c], d->tune.t1_tail_grid); });
       Span sp(d, w, FAM_T1TAIL);
-      if (tier1 == 2) k_t1tail_fused<12><<<cmt.bbeg[cmt.n], 64, 0, w>>>(T, J, S, cmt);
-      else if (tier1 == 1) k_t1tail_fused<10><<<cmt.bbeg[cmt.n], 64, 0, w>>>(T, J, S, cmt);
-      else k_t1tail_fused<6><<<cmt.bbeg[cmt.n], 64, 0, w>>>(T, J, S, cmt);
+      launch(k_t1tail_fused<6>, k_t1tail_fused<8>, k_t1tail_fused<10>, k_t1tail_fused<12>, cmt);
     }
     (void)hipEventRecordWithFlags(d->span[d->span_k][1], w, d->capturing ? hipEventRecordExternal : 0);
     d->span_valid = true;
@@ -3186,6 +3231,7 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
   Ly.d_zero = dv_off;
   Ly.d_fbc = dv_take(4 * kFbcSlots);
   Ly.d_stat = dv_take(2 * (size_t)nt);
+  Ly.d_tnf = dv_take(4 * (size_t)nt);
   Ly.d_zero_end = dv_off;
   Ly.d_UL = dv_take(8 * job->nUL);
   Ly.d_Ut = dv_take(8 * job->nUt);
@@ -3198,7 +3244,6 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
   Ly.d_T = dv_take(8 * (size_t)ntot2);
   Ly.d_tf = dv_take((size_t)ntot2);
   Ly.d_flist = dv_take(4 * (size_t)ntot2);
-  Ly.d_tnf = dv_take(4 * (size_t)nt);
   Ly.d_fbq2 = dv_take(4 * (size_t)(kMaxLMB + 1) * nt);
   Ly.d_fbT = dv_take(8 * (size_t)ntot2 * P.maxPairs);
   Ly.d_blk = dv_take(8 * job->nblk);
