@@ -3867,6 +3867,9 @@ int con_launch(ecp_dev *d, const ecp_job *job, const ConImage &c, char *idx, con
   A.nd = job->deriv == 0 ? 1 : 3;
   A.nunits = c.nunits;
   A.nmol = job->nmol;
+  // a stale error of an earlier call (capturing the fused sequence leaves one)
+  // must not be taken for one of these launches
+  (void)hipGetLastError();
   ECP_CHECK(hipEventRecord(d->con_ev[0], d->stream));
   if (Pp.nt > 0) {
     k_con_part<<<std::min(Pp.nt, 65536), 64, 0, d->stream>>>(d->T, A);

@@ -71,3 +71,29 @@ def test_tile_edges_against_oracle(name):
         a, b, f = np.asarray(a), np.asarray(b), np.asarray(f)
         assert np.all(np.abs(a - b) <= 1e-10 + 1e-8 * np.abs(b) + 2 * np.abs(b - f)), \
             (k, float(np.abs(a - b).max()))
+
+
+def _flat(out):
+    return np.concatenate([np.ravel(np.asarray(x, dtype=float)) for o in out
+                           for x in (o if isinstance(o, (tuple, list)) else [o])])
+
+
+@pytest.mark.parametrize("n", [0, 1])
+def test_contract_after_replays(n):
+    """A contraction after graph replays gives the bits of one after a first
+    evaluation."""
+    m = [plain_small(3)]
+    rng = np.random.default_rng(2)
+    P = [rng.standard_normal((m[0].nao, m[0].nao))]
+    outs = []
+    for repeats in (1, 3):
+        b = native.Batch(m, n=n)
+        try:
+            b.set_param("fuse", 1)
+            b.execute(repeats)
+            codes, out, _ = b.contract(P)
+        finally:
+            b.close()
+        assert not codes.any()
+        outs.append(_flat(out))
+    assert np.array_equal(outs[0], outs[1])
