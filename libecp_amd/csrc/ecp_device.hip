@@ -1991,6 +1991,15 @@ __device__ __forceinline__ double asm1_monomial(double acc, const double *__rest
 // formed once per monomial (same terms, same order as type1.c:266-295 per
 // element), then shifted to the output block (util.c:246-334).
 // G > 1 (classes la + lb <= 2, where a triplet has at most 10 monomials):
+// The block of a triplet whose integration failed: zeros, whatever an earlier
+// job left in the memory (a contraction sums every block and reports the
+// failure beside its result).
+__device__ __forceinline__ void zero_block(const DevJob &J, int t, double *blk, int lid, int nlanes) {
+  const ecp_triplet &tr = J.trip[t];
+  const int n = ECP_DIM_IJK(tr.oa) * ECP_DIM_IJK(tr.ob);
+  for (int i = lid; i < n; i += nlanes) blk[i] = 0.0;
+}
+
 // G triplets per wave, kAsmThreads / G lanes and an LDS slice of
 // A.lds_group doubles each; the wave's lane groups run the same phases and
 // synchronise together, an inactive group with empty loops.
@@ -2017,12 +2026,18 @@ __global__ __launch_bounds__(kAsmThreads, 3) void k_asm1(DevTables T, DevJob J, 
   bool active = true;
   if constexpr (G == 1) {
     t = tlist[blockIdx.x];
-    if (status[2 * t]) return;
+    if (status[2 * t]) {
+      zero_block(J, t, A.blocks + J.trip[t].blk1, lid, W);
+      return;
+    }
   } else {
     const int ti = blockIdx.x * G + grp;
     active = ti < ntl;
     t = active ? tlist[ti] : tlist[0];
-    if (active && status[2 * t]) active = false;
+    if (active && status[2 * t]) {
+      zero_block(J, t, A.blocks + J.trip[t].blk1, lid, W);
+      active = false;
+    }
     if (!wave_any(active)) return;
   }
   const ecp_triplet tr = J.trip[t];
@@ -2205,7 +2220,10 @@ __global__ __launch_bounds__(NT) void k_asm2(DevTables T, DevJob J, AsmArgs A,
   const int ti = xcd_item(blockIdx.x, gridDim.x) * G + grp;
   bool active = ti < ntl;
   const int t = cload(tlist + (active ? ti : 0));
-  if (status[2 * t + 1]) active = false;
+  if (active && status[2 * t + 1]) {
+    zero_block(J, t, A.blocks + J.trip[t].blk2, lid, W);
+    active = false;
+  }
   if (!wave_any(active)) return;
   const ecp_triplet tr = J.trip[t];
   const ecp_centre Cn = J.cent[tr.centre];
@@ -2283,9 +2301,13 @@ struct TabArgs {
   size_t zero_words;
   int nzb, nub, nfit, rows;  // rows: U-table rows per centre (largest L + 1)
   const int2 *fit;
-  const T1Unit *units;       // type-1 units and their pair directions, 128 per workgroup
-  int nunits;
+  // the type-1 units (class after class, in triplet order) and their pair
+  // directions, one (triplet, pair) item per lane
+  T1Unit *units;
   double *udir;
+  const int *t1first;
+  int cls_begin[ECP_MAX_LAB + 1];
+  size_t cls_qbase[ECP_MAX_LAB + 1];
   const int2 *ait;           // (centre, atom) pairs of the angular tables, aparts workgroups each
   int nait, aparts;
 };
@@ -2338,18 +2360,28 @@ __global__ __launch_bounds__(128, 4) void k_tables(DevTables T, DevJob J, TabArg
     return;
   }
   b -= A.nfit;
-  const int u = b * 128 + threadIdx.x;
-  if (u < A.nunits) unit_dir(J, A.units[u], A.udir + 4 * (size_t)u);
+  const size_t item = (size_t)b * 128 + threadIdx.x;
+  const int t = (int)(item / J.maxPairs), k = (int)(item - (size_t)t * J.maxPairs);
+  if (t >= J.ntrip) return;
+  const ecp_triplet tr = J.trip[t];
+  const int Kb = J.shells[tr.sb].K;
+  if (k >= J.shells[tr.sa].K * Kb) return;
+  const int c = tr.la + tr.lb, u = A.t1first[t] + k;
+  // entries of a class: sum of l / 2 + 1 over l <= c
+  const int nq = (c + 2) * (c + 2) / 4;
+  const T1Unit U{t, k / Kb, k % Kb, (int)(A.cls_qbase[c] + (size_t)(u - A.cls_begin[c]) * nq)};
+  A.units[u] = U;
+  unit_dir(J, U, A.udir + 4 * (size_t)u);
 }
 
 // byte offsets of a job's arrays inside its device block: inputs (uploaded)
 // first, then device-only buffers
 struct JobLayout {
   size_t i_atoms = 0, i_amaxl = 0, i_sh = 0, i_pa = 0, i_pd = 0, i_cent = 0, i_gauss = 0, i_win = 0, i_trip = 0,
-         i_u1 = 0, i_t1f = 0, i_teoff = 0, i_fit = 0, i_ait = 0, i_tcls = 0, i_tcls2 = 0,
+         i_t1f = 0, i_teoff = 0, i_fit = 0, i_ait = 0, i_tcls = 0, i_tcls2 = 0,
          in_bytes = 0;
   size_t d_zero = 0, d_fbc = 0, d_stat = 0, d_zero_end = 0, d_UL = 0, d_Ut = 0, d_F = 0, d_ang = 0,
-         d_q = 0, d_t1s = 0, d_tq1 = 0, d_qf = 0, d_udir = 0, d_fbq1 = 0, d_T = 0, d_tf = 0, d_flist = 0, d_tnf = 0, d_fbq2 = 0, d_fbT = 0, d_blk = 0, total = 0;
+         d_q = 0, d_t1s = 0, d_tq1 = 0, d_qf = 0, d_u1 = 0, d_udir = 0, d_fbq1 = 0, d_T = 0, d_tf = 0, d_flist = 0, d_tnf = 0, d_fbq2 = 0, d_fbT = 0, d_blk = 0, total = 0;
   int FL = 0, UK = 0, US = 0, angL = 0, ang_lam = 0, ang_c = 0, deriv = 0;
 };
 
@@ -2363,7 +2395,8 @@ struct Prepared {
   size_t nblk = 0;
   // device pointers
   DevJob J{};
-  const T1Unit *u1 = nullptr;
+  T1Unit *u1 = nullptr;
+  size_t cls_qbase[ECP_MAX_LAB + 2] = {0};  // first Q value of each class
   double *q = nullptr;
   size_t nq = 0;
   double *t1s = nullptr;  // type-1 head -> tail state: p, q, I planes of nq doubles
@@ -2396,13 +2429,14 @@ struct Prepared {
   // algorithmic FLOPs per evaluation (the per-unit models of the reference's
   // eager algorithm): type-1 radial work per class, type-2 radial work
   double flops_t1[ECP_MAX_LAB + 1] = {0};
-  double model[ECP_FL_N] = {0};  // the model's terms known before evaluation (ecp_model_flops)
 };
 
 }  // namespace
 
 constexpr int kWorkers = 3;
 constexpr int kSpanGraphs = 8;  // graph copies with their own quadrature event pair
+
+constexpr ecp_tuning kTuningDefaults{5, 8, 100000, 8192, 2, 1, 15, 2048, 0, 1, 0};
 
 struct ecp_dev {
   hipStream_t stream = nullptr;
@@ -2434,8 +2468,9 @@ struct ecp_dev {
   std::vector<int> tmpl, toff;
   Prepared P;
   JobLayout L;
-  ecp_tuning tune{5, 8, 100000, 8192, 2, 1, 15, 2048, 0, 1, 0};
+  ecp_tuning tune = kTuningDefaults;
   bool planned = false, prepared = false, eager_done = false;
+  bool uploading = false;  // a copy from pin_in may be in flight on stream
   hipGraph_t graph[kSpanGraphs] = {};
   hipGraphExec_t gexec[kSpanGraphs] = {};
   int ngraph = 0;
@@ -2941,15 +2976,19 @@ void launch_tables(ecp_dev *d, hipStream_t s) {
   A.nfit = P.nfit;
   A.fit = P.fit;
   A.units = P.u1;
-  A.nunits = P.cls_begin[ECP_MAX_LAB + 1];
   A.udir = P.udir;
+  A.t1first = P.aa.t1first;
+  for (int c = 0; c <= ECP_MAX_LAB; c++) {
+    A.cls_begin[c] = P.cls_begin[c];
+    A.cls_qbase[c] = P.cls_qbase[c];
+  }
   A.ait = P.ait;
   A.nait = P.nait;
   // few pairs: several workgroups each (20 atoms with g shells, 160 pairs:
   // the launch 116 us at one, 4556 workgroups in all)
   A.aparts = P.nait < 1024 ? 4 : 1;
   Span sp(d, s, FAM_TABLES);
-  k_tables<<<A.nait * A.aparts + A.nzb + A.nub + A.nfit + (A.nunits + 127) / 128, 128, 0, s>>>(d->T, P.J, A);
+  k_tables<<<A.nait * A.aparts + A.nzb + A.nub + A.nfit + (int)(((size_t)P.nt * P.maxPairs + 127) / 128), 128, 0, s>>>(d->T, P.J, A);
 }
 
 // fuse = 2 (automatic), by the job's type-1 primitive pairs.  Up to
@@ -3120,6 +3159,10 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
   d->planned = false;
   d->eager_done = false;
   reset_graph(d);
+  if (d->uploading) {
+    ECP_CHECK(hipStreamSynchronize(d->stream));
+    d->uploading = false;
+  }
   P = Prepared();
   Ly = JobLayout();
   const int nt = job->ntrip;
@@ -3131,71 +3174,29 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
     d->planned = true;
     return 0;
   }
-  // type-1 units grouped by class lab, inside a class in triplet order
+  // type-1 units are grouped by class lab, inside a class in triplet order;
+  // the tables launch writes them
   for (int t = 0; t < nt; t++) {
     const ecp_triplet &tr = job->trip[t];
-    P.cls_count[tr.la + tr.lb] += job->shells[tr.sa].K * job->shells[tr.sb].K;
-  }
-  for (int c = 0; c <= ECP_MAX_LAB; c++) P.cls_begin[c + 1] = P.cls_begin[c] + P.cls_count[c];
-  std::vector<T1Unit> units1(P.cls_begin[ECP_MAX_LAB + 1]);
-  std::vector<int> t1first(nt), cls_fill(P.cls_begin, P.cls_begin + ECP_MAX_LAB + 1);
-  std::vector<size_t> cls_qbase(ECP_MAX_LAB + 2, 0);
-  for (int c = 0; c <= ECP_MAX_LAB; c++) cls_qbase[c + 1] = cls_qbase[c] + (size_t)P.cls_count[c] * nq_of(c);
-  for (int t = 0; t < nt; t++) {
-    const ecp_triplet &tr = job->trip[t];
-    const ecp_shell &Sa = job->shells[tr.sa], &Sb = job->shells[tr.sb];
-    const int c = tr.la + tr.lb;
-    t1first[t] = cls_fill[c];
-    for (int pa = 0; pa < Sa.K; pa++)
-      for (int pb = 0; pb < Sb.K; pb++) {
-        const int u = cls_fill[c]++;
-        units1[u] = T1Unit{t, pa, pb, (int)(cls_qbase[c] + (size_t)(u - P.cls_begin[c]) * nq_of(c))};
-      }
+    const int c = tr.la + tr.lb, KK = job->shells[tr.sa].K * job->shells[tr.sb].K;
+    P.cls_count[c] += KK;
+    P.tcls_begin[c + 1]++;
     // per primitive pair: G (31 lambda + 74 + 4 n_Q) + 150 n_Q
-    const double G = tr.ge - tr.gs;
-    P.flops_t1[c] += (double)Sa.K * Sb.K * (G * (31.0 * c + 74 + 4.0 * nq_of(c)) + 150.0 * nq_of(c));
+    P.flops_t1[c] += KK * ((tr.ge - tr.gs) * (31.0 * c + 74 + 4.0 * nq_of(c)) + 150.0 * nq_of(c));
   }
-  const size_t nq = cls_qbase[ECP_MAX_LAB + 1];
-  std::vector<int> tcls(nt);
-  {
-    for (int t = 0; t < nt; t++) P.tcls_begin[job->trip[t].la + job->trip[t].lb + 1]++;
-    for (int c = 0; c <= ECP_MAX_LAB; c++) P.tcls_begin[c + 1] += P.tcls_begin[c];
-    std::vector<int> fill(P.tcls_begin, P.tcls_begin + ECP_MAX_LAB + 1);
-    for (int t = 0; t < nt; t++) tcls[fill[job->trip[t].la + job->trip[t].lb]++] = t;
-  }
-  std::vector<int> teoff(nt);
-  std::vector<unsigned char> tcls2(nt);
-  for (int c = 0; c <= kMaxLMB; c++) P.tcount2[c] = 0;
-  P.max_cls2 = 0;
-  int ntot2 = 0;
-  for (int t = 0; t < nt; t++) {
-    const ecp_triplet &tr = job->trip[t];
-    const int la = tr.la, lb = tr.lb;
-    teoff[t] = ntot2;
-    {
-      const int c2 = std::max(la, lb) + job->cent[tr.centre].L - 1;
-      tcls2[t] = (unsigned char)c2;
-      P.tcount2[c2]++;
-      P.max_cls2 = std::max(P.max_cls2, c2);
-    }
-    const int ne = d->toff[toff_key(la, lb, job->cent[tr.centre].L)] - d->toff[toff_key(la, lb, 0)];
-    ntot2 += ne;
-    P.max_ent2 = std::max(P.max_ent2, ne);
-  }
-  P.ntot2 = ntot2;
-  ecp_model_flops(job, P.model);
-  for (int c = 0; c <= ECP_MAX_LAB; c++)
+  for (int c = 0; c <= ECP_MAX_LAB; c++) {
+    P.cls_begin[c + 1] = P.cls_begin[c] + P.cls_count[c];
+    P.cls_qbase[c + 1] = P.cls_qbase[c] + (size_t)P.cls_count[c] * nq_of(c);
+    P.tcls_begin[c + 1] += P.tcls_begin[c];
     if (P.cls_count[c]) P.max_lab = c;
-  std::vector<int2> fitems, aitems;
+  }
+  const size_t nunits = P.cls_begin[ECP_MAX_LAB + 1], nq = P.cls_qbase[ECP_MAX_LAB + 1];
   for (int c = 0; c < job->ncent; c++) {
     const ecp_centre &C = job->cent[c];
-    for (int run = 0; run <= job->deriv; run++)
-      for (int s = 0; s < C.nsh; s++)
-        if (!job->win[C.win_off + s].skip) fitems.push_back(make_int2(c, s * 4 + run));
-    for (int a = 0; a < C.nat; a++) aitems.push_back(make_int2(c, a));
+    for (int s = 0; s < C.nsh; s++) P.nfit += !job->win[C.win_off + s].skip;
+    P.nait += C.nat;
   }
-  P.nfit = (int)fitems.size();
-  P.nait = (int)aitems.size();
+  P.nfit *= job->deriv + 1;
   P.maxPairs = job->maxK * job->maxK;
   // layout: inputs (copied), then device-only buffers; the per-run zeroed
   // counters and flags are contiguous
@@ -3214,14 +3215,68 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
   Ly.i_gauss = in_take(sizeof(ecp_gauss) * job->ngauss);
   Ly.i_win = in_take(sizeof(ecp_window) * job->nwin);
   Ly.i_trip = in_take(sizeof(ecp_triplet) * nt);
-  Ly.i_u1 = in_take(sizeof(T1Unit) * units1.size());
   Ly.i_t1f = in_take(4 * (size_t)nt);
   Ly.i_teoff = in_take(4 * (size_t)nt);
   Ly.i_tcls2 = in_take((size_t)nt);
-  Ly.i_fit = in_take(sizeof(int2) * fitems.size());
-  Ly.i_ait = in_take(sizeof(int2) * aitems.size());
+  Ly.i_fit = in_take(sizeof(int2) * P.nfit);
+  Ly.i_ait = in_take(sizeof(int2) * P.nait);
   Ly.i_tcls = in_take(4 * (size_t)nt);
   Ly.in_bytes = in_off;
+  if (Ly.in_bytes > d->pin_in_cap) {
+    if (d->pin_in) ECP_CHECK(hipHostFree(d->pin_in));
+    d->pin_in = nullptr;
+    d->pin_in_cap = 0;
+    ECP_CHECK(hipHostMalloc(&d->pin_in, Ly.in_bytes + Ly.in_bytes / 4));
+    d->pin_in_cap = Ly.in_bytes + Ly.in_bytes / 4;
+  }
+  // the inputs, straight into the staging memory
+  char *H = d->pin_in;
+  auto cp = [&](size_t o, const void *src, size_t b) {
+    if (b) memcpy(H + o, src, b);
+  };
+  cp(Ly.i_atoms, job->atoms, sizeof(ecp_xyz) * job->nat);
+  cp(Ly.i_amaxl, job->atom_maxl, 4 * (size_t)job->nat);
+  cp(Ly.i_sh, job->shells, sizeof(ecp_shell) * job->nsh);
+  cp(Ly.i_pa, job->pa, 8 * (size_t)job->nprim);
+  cp(Ly.i_pd, job->pd, 8 * (size_t)job->nprim);
+  cp(Ly.i_cent, job->cent, sizeof(ecp_centre) * job->ncent);
+  cp(Ly.i_gauss, job->gauss, sizeof(ecp_gauss) * job->ngauss);
+  cp(Ly.i_win, job->win, sizeof(ecp_window) * job->nwin);
+  cp(Ly.i_trip, job->trip, sizeof(ecp_triplet) * nt);
+  int ntot2 = 0;
+  {
+    int *t1first = (int *)(H + Ly.i_t1f), *teoff = (int *)(H + Ly.i_teoff), *tcls = (int *)(H + Ly.i_tcls);
+    unsigned char *tcls2 = (unsigned char *)(H + Ly.i_tcls2);
+    int ufill[ECP_MAX_LAB + 1], tfill[ECP_MAX_LAB + 1];
+    for (int c = 0; c <= ECP_MAX_LAB; c++) {
+      ufill[c] = P.cls_begin[c];
+      tfill[c] = P.tcls_begin[c];
+    }
+    for (int t = 0; t < nt; t++) {
+      const ecp_triplet &tr = job->trip[t];
+      const int la = tr.la, lb = tr.lb, c = la + lb, L = job->cent[tr.centre].L;
+      t1first[t] = ufill[c];
+      ufill[c] += job->shells[tr.sa].K * job->shells[tr.sb].K;
+      tcls[tfill[c]++] = t;
+      const int c2 = std::max(la, lb) + L - 1;
+      tcls2[t] = (unsigned char)c2;
+      P.tcount2[c2]++;
+      P.max_cls2 = std::max(P.max_cls2, c2);
+      const int ne = d->toff[toff_key(la, lb, L)] - d->toff[toff_key(la, lb, 0)];
+      teoff[t] = ntot2;
+      ntot2 += ne;
+      P.max_ent2 = std::max(P.max_ent2, ne);
+    }
+    int2 *fit = (int2 *)(H + Ly.i_fit), *ait = (int2 *)(H + Ly.i_ait);
+    for (int c = 0; c < job->ncent; c++) {
+      const ecp_centre &C = job->cent[c];
+      for (int run = 0; run <= job->deriv; run++)
+        for (int s = 0; s < C.nsh; s++)
+          if (!job->win[C.win_off + s].skip) *fit++ = make_int2(c, s * 4 + run);
+      for (int a = 0; a < C.nat; a++) *ait++ = make_int2(c, a);
+    }
+  }
+  P.ntot2 = ntot2;
   size_t dv_off = align_up(Ly.in_bytes);
   auto dv_take = [&](size_t b) {
     size_t o = dv_off;
@@ -3239,8 +3294,9 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
   Ly.d_ang = dv_take(8 * job->nang);
   Ly.d_q = dv_take(8 * nq);
   P.nq = nq;
-  Ly.d_qf = dv_take(8 * units1.size());
-  Ly.d_fbq1 = dv_take(4 * units1.size());
+  Ly.d_qf = dv_take(8 * nunits);
+  Ly.d_u1 = dv_take(sizeof(T1Unit) * nunits);
+  Ly.d_fbq1 = dv_take(4 * nunits);
   Ly.d_T = dv_take(8 * (size_t)ntot2);
   Ly.d_tf = dv_take((size_t)ntot2);
   Ly.d_flist = dv_take(4 * (size_t)ntot2);
@@ -3248,8 +3304,8 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
   Ly.d_fbT = dv_take(8 * (size_t)ntot2 * P.maxPairs);
   Ly.d_blk = dv_take(8 * job->nblk);
   Ly.d_t1s = dv_take(3 * 8 * nq);
-  Ly.d_tq1 = dv_take(4 * units1.size());
-  Ly.d_udir = dv_take(32 * units1.size());
+  Ly.d_tq1 = dv_take(4 * nunits);
+  Ly.d_udir = dv_take(32 * nunits);
   Ly.total = dv_off;
   Ly.FL = job->FL;
   Ly.UK = job->UK;
@@ -3326,13 +3382,6 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
       return -1;
     }
   }
-  if (Ly.in_bytes > d->pin_in_cap) {
-    if (d->pin_in) ECP_CHECK(hipHostFree(d->pin_in));
-    d->pin_in = nullptr;
-    d->pin_in_cap = 0;
-    ECP_CHECK(hipHostMalloc(&d->pin_in, Ly.in_bytes + Ly.in_bytes / 4));
-    d->pin_in_cap = Ly.in_bytes + Ly.in_bytes / 4;
-  }
   const size_t out_bytes = 8 * job->nblk + 2 * (size_t)nt;
   if (out_bytes > d->pin_out_cap) {
     if (d->pin_out) ECP_CHECK(hipHostFree(d->pin_out));
@@ -3341,26 +3390,6 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
     ECP_CHECK(hipHostMalloc(&d->pin_out, out_bytes + out_bytes / 4));
     d->pin_out_cap = out_bytes + out_bytes / 4;
   }
-  char *H = d->pin_in;
-  auto cp = [&](size_t o, const void *src, size_t b) {
-    if (b) memcpy(H + o, src, b);
-  };
-  cp(Ly.i_atoms, job->atoms, sizeof(ecp_xyz) * job->nat);
-  cp(Ly.i_amaxl, job->atom_maxl, 4 * (size_t)job->nat);
-  cp(Ly.i_sh, job->shells, sizeof(ecp_shell) * job->nsh);
-  cp(Ly.i_pa, job->pa, 8 * (size_t)job->nprim);
-  cp(Ly.i_pd, job->pd, 8 * (size_t)job->nprim);
-  cp(Ly.i_cent, job->cent, sizeof(ecp_centre) * job->ncent);
-  cp(Ly.i_gauss, job->gauss, sizeof(ecp_gauss) * job->ngauss);
-  cp(Ly.i_win, job->win, sizeof(ecp_window) * job->nwin);
-  cp(Ly.i_trip, job->trip, sizeof(ecp_triplet) * nt);
-  cp(Ly.i_u1, units1.data(), sizeof(T1Unit) * units1.size());
-  cp(Ly.i_t1f, t1first.data(), 4 * (size_t)nt);
-  cp(Ly.i_teoff, teoff.data(), 4 * (size_t)nt);
-  cp(Ly.i_tcls2, tcls2.data(), (size_t)nt);
-  cp(Ly.i_fit, fitems.data(), sizeof(int2) * fitems.size());
-  cp(Ly.i_ait, aitems.data(), sizeof(int2) * aitems.size());
-  cp(Ly.i_tcls, tcls.data(), 4 * (size_t)nt);
   if (bytes) *bytes = Ly.total;
   d->planned = true;
   return 0;
@@ -3397,8 +3426,10 @@ extern "C" int ecp_dev_bind(ecp_dev *d, void *mem, size_t cap, char *err, size_t
     snprintf(err, errlen, "job needs %zu bytes of device memory, %zu given", Ly.total, cap);
     return -1;
   }
+  // the evaluation follows on the same stream; the staging memory is not
+  // written again before ecp_dev_plan has waited for the copy
   ECP_CHECK(hipMemcpyAsync(A, d->pin_in, Ly.in_bytes, hipMemcpyHostToDevice, d->stream));
-  ECP_CHECK(hipStreamSynchronize(d->stream));
+  d->uploading = true;
   DevJob &J = P.J;
   J.atoms = (const ecp_xyz *)(A + Ly.i_atoms);
   J.atom_maxl = (const int *)(A + Ly.i_amaxl);
@@ -3423,7 +3454,7 @@ extern "C" int ecp_dev_bind(ecp_dev *d, void *mem, size_t cap, char *err, size_t
   J.maxPairs = P.maxPairs;
   J.teoff = (const int *)(A + Ly.i_teoff);
   J.US = Ly.US;
-  P.u1 = (const T1Unit *)(A + Ly.i_u1);
+  P.u1 = (T1Unit *)(A + Ly.d_u1);
   P.q = (double *)(A + Ly.d_q);
   P.t1s = (double *)(A + Ly.d_t1s);
   P.tq1 = (int *)(A + Ly.d_tq1);
@@ -3581,7 +3612,8 @@ __global__ __launch_bounds__(256) void k_fb_flops(DevJob J, const T1Unit *__rest
 
 }  // namespace
 
-extern "C" int ecp_dev_profile(ecp_dev *d, int *launches, double *ms, double *flops, char *err, size_t errlen) {
+extern "C" int ecp_dev_profile(ecp_dev *d, const ecp_job *job, int *launches, double *ms, double *flops, char *err,
+                               size_t errlen) {
   if (!d->prepared) {
     snprintf(err, errlen, "ecp_dev_profile before ecp_dev_prepare");
     return -1;
@@ -3610,10 +3642,12 @@ extern "C" int ecp_dev_profile(ecp_dev *d, int *launches, double *ms, double *fl
   // algorithmic FLOPs per family: the model's terms known before the
   // evaluation, and the fallbacks from this evaluation's failed integrals
   const Prepared &P = d->P;
-  flops[FAM_TABLES] = P.model[ECP_FL_FTAB];
-  flops[FAM_TYPE1] = P.model[ECP_FL_T1];
-  flops[FAM_TYPE2] = P.model[ECP_FL_T2];
-  flops[FAM_ASM] = P.model[ECP_FL_ASM1] + P.model[ECP_FL_ASM2] + P.model[ECP_FL_SHIFT];
+  double model[ECP_FL_N];
+  ecp_model_flops(job, model);
+  flops[FAM_TABLES] = model[ECP_FL_FTAB];
+  flops[FAM_TYPE1] = model[ECP_FL_T1];
+  flops[FAM_TYPE2] = model[ECP_FL_T2];
+  flops[FAM_ASM] = model[ECP_FL_ASM1] + model[ECP_FL_ASM2] + model[ECP_FL_SHIFT];
   if (!d->fbf) ECP_CHECK(hipMalloc(&d->fbf, 2 * sizeof(double)));
   ECP_CHECK(hipMemsetAsync(d->fbf, 0, 2 * sizeof(double), d->stream));
   const int nunits = P.cls_begin[ECP_MAX_LAB + 1];
@@ -3630,22 +3664,22 @@ extern "C" int ecp_dev_profile(ecp_dev *d, int *launches, double *ms, double *fl
 
 extern "C" const char *ecp_dev_family_name(int f) { return (f >= 0 && f < FAM_N) ? kFamName[f] : ""; }
 
-extern "C" int ecp_dev_fetch(ecp_dev *d, double *blocks_out, unsigned char *status_out, char *err, size_t errlen) {
+extern "C" int ecp_dev_fetch(ecp_dev *d, double **blocks, unsigned char **status, char *err, size_t errlen) {
   const Prepared &P = d->P;
+  *blocks = nullptr;
+  *status = nullptr;
   if (P.nt == 0) return 0;
   ECP_CHECK(hipMemcpyAsync(d->pin_out, P.blk, 8 * P.nblk, hipMemcpyDeviceToHost, d->stream));
   ECP_CHECK(hipMemcpyAsync(d->pin_out + 8 * P.nblk, P.stat, 2 * (size_t)P.nt, hipMemcpyDeviceToHost, d->stream));
   ECP_CHECK(hipStreamSynchronize(d->stream));
-  memcpy(blocks_out, d->pin_out, 8 * P.nblk);
-  memcpy(status_out, d->pin_out + 8 * P.nblk, 2 * (size_t)P.nt);
+  *blocks = (double *)d->pin_out;
+  *status = (unsigned char *)(d->pin_out + 8 * P.nblk);
   return 0;
 }
 
-extern "C" int ecp_dev_run(ecp_dev *d, const ecp_job *job, double *blocks_out, unsigned char *status_out,
-                           char *err, size_t errlen) {
-  if (ecp_dev_prepare(d, job, err, errlen)) return -1;
-  if (ecp_dev_execute(d, 1, nullptr, err, errlen)) return -1;
-  return ecp_dev_fetch(d, blocks_out, status_out, err, errlen);
+// bytes of device and pinned memory a context holds for jobs
+extern "C" size_t ecp_dev_held(const ecp_dev *d) {
+  return d->arena_cap + d->con_cap + d->pin_in_cap + d->pin_out_cap;
 }
 
 // ---------------------------------------------------------------------------
@@ -4045,6 +4079,17 @@ extern "C" int ecp_dev_current(void) {
 }
 
 extern "C" int ecp_dev_use(int device) { return hipSetDevice(device) == hipSuccess ? 0 : -1; }
+
+extern "C" void ecp_dev_renew(ecp_dev *d) {
+  ecp_dev_set_tuning(d, &kTuningDefaults);
+  d->planned = d->prepared = false;
+  d->nev = 0;
+  d->span_valid = false;
+  d->last_eager = false;
+  d->last_replays = 0;
+  d->P = Prepared();
+  d->L = JobLayout();
+}
 
 extern "C" void ecp_dev_get_tuning(const ecp_dev *d, ecp_tuning *t) { *t = d->tune; }
 

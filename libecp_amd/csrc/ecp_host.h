@@ -100,14 +100,14 @@ typedef struct ecp_dev ecp_dev;
 
 ecp_dev *ecp_dev_create(const ecp_static *st, char *err, size_t errlen);
 void ecp_dev_destroy(ecp_dev *d);
-/* Runs the whole pipeline for a job: returns 0 and fills blocks (job->nblk
-   doubles) and status (2 bytes per triplet: type-1 / type-2 failure flags),
-   or a negative value on a device error (message in err). */
-int ecp_dev_run(ecp_dev *d, const ecp_job *job, double *blocks, unsigned char *status, char *err,
-                size_t errlen);
-/* The same in three steps: upload a job (inputs become resident in HBM),
-   execute its kernel sequence `repeats` times (graph replays after the
-   first; *ms_total = device time per repeat), and copy the results back. */
+/* Runs a job in three steps: upload it (its inputs become resident in HBM;
+   nothing waits for the copy before the evaluation behind it), execute its
+   kernel sequence `repeats` times (graph replays after the first; *ms_total =
+   device time per repeat), and copy the results back.  Fetched results
+   (job->nblk doubles; 2 bytes per triplet: type-1 / type-2 failure flags) are
+   in the context's pinned memory, valid until the next fetch or plan on it
+   (NULL for a job without triplets).  0, or a negative value on a device
+   error (message in err). */
 int ecp_dev_prepare(ecp_dev *d, const ecp_job *job, char *err, size_t errlen);
 /* prepare = plan + bind.  plan does the host work (work lists, layout,
    staging in pinned memory) and returns the bytes of device memory the job
@@ -116,7 +116,9 @@ int ecp_dev_prepare(ecp_dev *d, const ecp_job *job, char *err, size_t errlen);
 int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char *err, size_t errlen);
 int ecp_dev_bind(ecp_dev *d, void *mem, size_t cap, char *err, size_t errlen);
 int ecp_dev_execute(ecp_dev *d, int repeats, double *ms_total, char *err, size_t errlen);
-int ecp_dev_fetch(ecp_dev *d, double *blocks, unsigned char *status, char *err, size_t errlen);
+int ecp_dev_fetch(ecp_dev *d, double **blocks, unsigned char **status, char *err, size_t errlen);
+/* bytes of device and pinned memory a context holds for jobs */
+size_t ecp_dev_held(const ecp_dev *d);
 /* Contracts the last evaluation's blocks with densities on the device (job
    of derivative order 0: one energy per molecule; order 1: 3 gradient
    components per atom, molecule after molecule).  P holds nP doubles,
@@ -142,7 +144,8 @@ int ecp_dev_contract_noalloc(ecp_dev *d, const ecp_job *job, const char *img, si
    own stream).  Per kernel family (tables, type1, type2, fallback1,
    fallback2, assemble): launches, summed duration in ms, algorithmic FLOPs
    of one evaluation (type1/type2 only).  Returns the number of families. */
-int ecp_dev_profile(ecp_dev *d, int *launches, double *ms, double *flops, char *err, size_t errlen);
+int ecp_dev_profile(ecp_dev *d, const ecp_job *job, int *launches, double *ms, double *flops, char *err,
+                    size_t errlen);
 const char *ecp_dev_family_name(int f);
 /* Stage timings of the last execute (ms): tables, quadratures (small grid
    and large-grid fallbacks, concurrent), assembly[, mean graph replay]. */
@@ -157,6 +160,9 @@ int ecp_dev_span_ms(ecp_dev *d, double *ms, int *samples, char *err, size_t errl
    graph (the next execute runs eagerly and captures again) */
 void ecp_dev_get_tuning(const ecp_dev *d, ecp_tuning *t);
 void ecp_dev_set_tuning(ecp_dev *d, const ecp_tuning *t);
+/* an idle context as a new one: default parameters, no timings of earlier
+   jobs (its workspaces stay) */
+void ecp_dev_renew(ecp_dev *d);
 /* Waits for every stream of the context (after a failed bind / execute /
    fetch, before its device memory is reused).  0, or -1 when a stream
    reports an error. */

@@ -231,17 +231,36 @@ typedef struct {
   int n, cap;
 } trip_vec;
 
-static int trip_push(trip_vec *tv, const ecp_triplet *t) {
-  if (tv->n == tv->cap) {
+/* room for n more */
+static int trip_room(trip_vec *tv, int n) {
+  if (tv->n + n > tv->cap) {
     int nc = tv->cap ? 2 * tv->cap : 1024;
     ecp_triplet *nv = realloc(tv->v, sizeof(ecp_triplet) * (size_t)nc);
     if (!nv) return -1;
     tv->v = nv;
     tv->cap = nc;
   }
-  tv->v[tv->n++] = *t;
   return 0;
 }
+
+/* the number of leading values of the ascending x[0 .. n) below v (or equal
+   to it, with eq) */
+static int count_below(const double *x, int n, double v, int eq) {
+  int lo = 0, hi = n;
+  while (lo < hi) {
+    const int mid = (lo + hi) / 2;
+    if (eq ? x[mid] <= v : x[mid] < v)
+      lo = mid + 1;
+    else
+      hi = mid;
+  }
+  return lo;
+}
+
+/* a shell with a non-empty window of the centre at hand */
+typedef struct {
+  int shell, atom, l, start, end;
+} active_shell;
 
 /* Orders a centre's Gaussians by channel, keeping the input order inside a
    channel (the order its potential is summed in), and records where each
@@ -336,10 +355,13 @@ int ecp_job_build(const ecp_mol *mols, int nmol, int deriv, const ecp_static *st
   job->trip_mol_begin = calloc((size_t)nmol + 1, sizeof(int));
   job->mol_atom0 = calloc((size_t)nmol + 1, sizeof(int));
   double *radius = calloc((size_t)nsh + 1, sizeof(double));
+  active_shell *act = malloc(sizeof(active_shell) * ((size_t)nsh + 1));
   if (!job->atoms || !job->atom_maxl || !job->atom_shell0 || !job->atom_nsh || !job->shells || !job->pa ||
-      !job->pd || !job->cent || !job->gauss || !job->win || !job->trip_mol_begin || !job->mol_atom0 || !radius) {
+      !job->pd || !job->cent || !job->gauss || !job->win || !job->trip_mol_begin || !job->mol_atom0 || !radius ||
+      !act) {
     snprintf(err, errlen, "out of host memory");
     free(radius);
+    free(act);
     free(dims);
     ecp_job_free(job);
     return -1;
@@ -414,7 +436,7 @@ int ecp_job_build(const ecp_mol *mols, int nmol, int deriv, const ecp_static *st
       for (int l = 0; l < Cn->L; l++) {
         int e = -1;
         for (int i = end; i >= 0; i--)
-          if (fabs(ecp_eval_ecp_host(job->gauss + Cn->g0, Cn->ng, l, st->xs[i])) > 1.0E-14) {
+          if (fabs(ecp_eval_ecp_host(job->gauss + Cn->g0 + Cn->gl[l], Cn->gl[l + 1] - Cn->gl[l], l, st->xs[i])) > 1.0E-14) {
             e = i;
             break;
           }
@@ -435,6 +457,7 @@ int ecp_job_build(const ecp_mol *mols, int nmol, int deriv, const ecp_static *st
       Cn->ang_off = (int)ango;
       ango += (size_t)M->nat * job->ang_lam * job->angL * job->angL * job->ang_c;
       /* basis screening of each shell on [0, end] (type2.c:148-180) */
+      int nact = 0;
       for (int s = 0; s < dims[m].nsh; s++) {
         const ecp_shell *S = &job->shells[s0 + s];
         const ecp_xyz rA = job->atoms[S->atom];
@@ -442,63 +465,60 @@ int ecp_job_build(const ecp_mol *mols, int nmol, int deriv, const ecp_static *st
         const double dAC = sqrt(x * x + y * y + z * z);
         const double rmin = dAC - radius[s0 + s], rmax = dAC + radius[s0 + s];
         ecp_window *W = &job->win[Cn->win_off + s];
-        int j;
-        for (j = end; j >= 0; j--)
-          if (st->xs[j] < rmin) break;
-        W->start = j + 1;
-        for (j = end; j >= 0; j--)
-          if (st->xs[j] <= rmax) break;
-        W->end = (j < 0 || st->xs[j] > rmax) ? -1 : j;
+        /* first point of [0, end] from rmin on, last up to rmax */
+        W->start = count_below(st->xs, end + 1, rmin, 0);
+        W->end = count_below(st->xs, end + 1, rmax, 1) - 1;
         W->skip = !(W->end >= W->start);
+        if (!W->skip) act[nact++] = (active_shell){s0 + s, S->atom, S->l, W->start, W->end};
       }
-      /* triplets in the reference order */
-      for (int A = 0; A < M->nat && !rc; A++) {
-        const int gA = a0 + A;
-        for (int B = A; B < M->nat && !rc; B++) {
-          const int gB = a0 + B;
-          for (int s1 = 0; s1 < job->atom_nsh[gA]; s1++) {
-            const int sa = job->atom_shell0[gA] + s1;
-            const ecp_window *Wa = &job->win[Cn->win_off + (sa - s0)];
-            if (Wa->skip) continue;
-            for (int s2 = (A == B) ? s1 : 0; s2 < job->atom_nsh[gB]; s2++) {
-              const int sb = job->atom_shell0[gB] + s2;
-              const ecp_window *Wb = &job->win[Cn->win_off + (sb - s0)];
-              if (Wb->skip) continue;
-              ecp_triplet t;
-              memset(&t, 0, sizeof(t));
-              t.centre = c;
-              t.sa = sa;
-              t.sb = sb;
-              t.gs = Wa->start > Wb->start ? Wa->start : Wb->start;
-              t.ge = Wa->end > Wb->end ? Wa->end : Wb->end;
-              if (!(t.gs < t.ge)) continue;
-              /* derivatives: A = B = C contributes nothing (libecp.c:305-306) */
-              if (deriv > 0 && gA == Cn->atom && gB == Cn->atom) continue;
-              const int la0 = job->shells[sa].l, lb0 = job->shells[sb].l;
+      /* triplets in the reference order: atoms A <= B, then their shells */
+      for (int ia = 0, ea; ia < nact && !rc; ia = ea) {
+        const int gA = act[ia].atom;
+        for (ea = ia + 1; ea < nact && act[ea].atom == gA;) ea++;
+        for (int ib = ia, eb; ib < nact && !rc; ib = eb) {
+          const int gB = act[ib].atom;
+          for (eb = ib + 1; eb < nact && act[eb].atom == gB;) eb++;
+          /* derivatives: A = B = C contributes nothing (libecp.c:305-306) */
+          if (deriv > 0 && gA == Cn->atom && gB == Cn->atom) continue;
+          for (int i1 = ia; i1 < ea && !rc; i1++) {
+            const active_shell *Sa = &act[i1];
+            for (int i2 = gA == gB ? i1 : ib; i2 < eb && !rc; i2++) {
+              const active_shell *Sb = &act[i2];
+              const int gs = Sa->start > Sb->start ? Sa->start : Sb->start;
+              const int ge = Sa->end > Sb->end ? Sa->end : Sb->end;
+              if (!(gs < ge)) continue;
+              if (trip_room(&tv, kShiftN[deriv])) {
+                set_err(err, errlen, "out of host memory");
+                rc = -1;
+                break;
+              }
               /* one block pair per derivative shift (libecp.c:322-330) */
-              for (int k = 0; k < kShiftN[deriv] && !rc; k++) {
+              for (int k = 0; k < kShiftN[deriv]; k++) {
                 const int sha = kShiftA[deriv][k], shb = kShiftB[deriv][k];
-                if (la0 < -sha || lb0 < -shb || (deriv == 1 && Cn->atom == gA && sha != 0) ||
+                if (Sa->l < -sha || Sb->l < -shb || (deriv == 1 && Cn->atom == gA && sha != 0) ||
                     (deriv == 1 && Cn->atom == gB && shb != 0))
                   continue;
-                t.shifta = sha;
-                t.shiftb = shb;
-                t.la = la0 + sha;
-                t.lb = lb0 + shb;
-                t.powa = sha > 0 ? sha : 0;
-                t.powb = shb > 0 ? shb : 0;
+                ecp_triplet *t = &tv.v[tv.n++];
+                memset(t, 0, sizeof(*t));
+                t->centre = c;
+                t->sa = Sa->shell;
+                t->sb = Sb->shell;
+                t->gs = gs;
+                t->ge = ge;
+                t->shifta = sha;
+                t->shiftb = shb;
+                t->la = Sa->l + sha;
+                t->lb = Sb->l + shb;
+                t->powa = sha > 0 ? sha : 0;
+                t->powb = shb > 0 ? shb : 0;
                 /* second derivatives: the (+1, 0) and (0, +1) blocks are
                    shifted back on the unshifted side (libecp.c:364-369) */
-                t.oa = (deriv == 2 && sha == 1 && shb == 0) ? la0 : t.la;
-                t.ob = (deriv == 2 && sha == 0 && shb == 1) ? lb0 : t.lb;
-                const int nb = ECP_DIM_IJK(t.oa) * ECP_DIM_IJK(t.ob);
-                t.blk1 = (int)blk;
-                t.blk2 = (int)(blk + nb);
+                t->oa = (deriv == 2 && sha == 1 && shb == 0) ? Sa->l : t->la;
+                t->ob = (deriv == 2 && sha == 0 && shb == 1) ? Sb->l : t->lb;
+                const int nb = ECP_DIM_IJK(t->oa) * ECP_DIM_IJK(t->ob);
+                t->blk1 = (int)blk;
+                t->blk2 = (int)(blk + nb);
                 blk += 2 * (size_t)nb;
-                if (trip_push(&tv, &t)) {
-                  set_err(err, errlen, "out of host memory");
-                  rc = -1;
-                }
               }
             }
           }
@@ -523,6 +543,7 @@ int ecp_job_build(const ecp_mol *mols, int nmol, int deriv, const ecp_static *st
   job->nF = fo;
   job->nang = ango;
   free(radius);
+  free(act);
   free(dims);
   if (rc) ecp_job_free(job);
   return rc;

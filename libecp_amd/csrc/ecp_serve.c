@@ -111,10 +111,6 @@ typedef struct {
   struct libecp_server *srv;
   int slot;
   ecp_dev *dev;
-  double *blocks;
-  size_t cap_blocks;
-  unsigned char *status;
-  size_t cap_status;
   req **rs;     /* the requests of the current job */
   ecp_mol *mols;
   int cap_rs;
@@ -268,25 +264,12 @@ static void *worker_main(void *arg) {
 
     /* evaluate */
     int dev_rc = 0;
+    double *blocks = NULL; /* in the context's pinned memory */
+    unsigned char *status = NULL;
     if (job.ntrip > 0) {
-      if (job.nblk + 1 > w->cap_blocks) {
-        free(w->blocks);
-        w->cap_blocks = job.nblk + job.nblk / 4 + 1;
-        w->blocks = malloc(sizeof(double) * w->cap_blocks);
-        if (!w->blocks) w->cap_blocks = 0;
-      }
-      if (2 * (size_t)job.ntrip + 1 > w->cap_status) {
-        free(w->status);
-        w->cap_status = 2 * (size_t)job.ntrip + (size_t)job.ntrip / 2 + 1;
-        w->status = malloc(w->cap_status);
-        if (!w->status) w->cap_status = 0;
-      }
-      if (!w->blocks || !w->status) {
-        snprintf(err, sizeof(err), "out of host memory for the blocks");
-        dev_rc = -1;
-      } else if (ecp_dev_bind(w->dev, s->mem.base + off, bytes, err, sizeof(err)) ||
+      if (ecp_dev_bind(w->dev, s->mem.base + off, bytes, err, sizeof(err)) ||
           ecp_dev_execute(w->dev, 1, NULL, err, sizeof(err)) ||
-          ecp_dev_fetch(w->dev, w->blocks, w->status, err, sizeof(err)))
+          ecp_dev_fetch(w->dev, &blocks, &status, err, sizeof(err)))
         dev_rc = -1;
     }
     /* after a device error, kernels of the job may still be queued on the
@@ -317,7 +300,7 @@ static void *worker_main(void *arg) {
         rcs[i] = -1;
         continue;
       }
-      rcs[i] = job.ntrip > 0 ? ecp_job_scatter(&job, i, aoff, w->blocks, w->status, 0, r->nao, r->upper) : 0;
+      rcs[i] = job.ntrip > 0 ? ecp_job_scatter(&job, i, aoff, blocks, status, 0, r->nao, r->upper) : 0;
     }
     free(aoff);
     ecp_job_free(&job);
@@ -332,8 +315,6 @@ static void *worker_main(void *arg) {
 static void server_release(struct libecp_server *s) {
   for (int i = 0; i < s->nslots; i++) {
     ecp_dev_destroy(s->wk[i].dev);
-    free(s->wk[i].blocks);
-    free(s->wk[i].status);
     free(s->wk[i].rs);
     free(s->wk[i].mols);
   }

@@ -15,7 +15,7 @@ import pytest
 
 import ecp_native as E
 from libecp_amd import native
-from libecp_amd.workloads import build_molecule, plain_small
+from libecp_amd.workloads import build_molecule, high_l, plain_small
 
 pytestmark = pytest.mark.gpu
 
@@ -73,9 +73,76 @@ def test_tile_edges_against_oracle(name):
             (k, float(np.abs(a - b).max()))
 
 
+def _batch_outputs(mols, n, tune=None):
+    """Matrices (n = 0) or contracted gradients, and the parameters seen."""
+    b = native.Batch(mols, n=n)
+    try:
+        params = {k: b.get_param(k) for k in ("fuse", "fb2_split", "t1_tail_grid")}
+        for k, v in (tune or {}).items():
+            b.set_param(k, v)
+        b.execute(3)
+        if n == 0:
+            b.fetch()
+            out = [b.matrix(i) for i in range(len(mols))]
+        else:
+            rng = np.random.default_rng(1)
+            out = b.contract([rng.standard_normal((m.nao, m.nao)) for m in mols])[1]
+        return params, out
+    finally:
+        b.close()
+
+
 def _flat(out):
     return np.concatenate([np.ravel(np.asarray(x, dtype=float)) for o in out
                            for x in (o if isinstance(o, (tuple, list)) else [o])])
+
+
+def test_failed_blocks_are_zero_in_a_used_context():
+    """A molecule with a failed integration contracts to the same energy and
+    code in fresh memory and where another job's blocks were."""
+    bad, other = high_l(1003), high_l(1000)
+    P = {id(m): [np.random.default_rng(3).standard_normal((m.nao, m.nao))] for m in (bad, other)}
+
+    def energy(m):
+        b = native.Batch([m])
+        try:
+            b.execute(1)
+            codes, out, _ = b.contract(P[id(m)])
+            return int(codes[0]), out[0]
+        finally:
+            b.close()
+
+    was = native.cache_enable(False)
+    try:
+        fresh = energy(bad)
+        native.cache_enable(True)
+        energy(other)
+        used = energy(bad)
+    finally:
+        native.cache_clear()
+        native.cache_enable(was)
+    assert fresh[0] != 0
+    assert used == fresh
+
+
+def test_batch_in_a_used_context():
+    """Batches of rising and falling sizes and both orders in contexts that
+    earlier batches of the same tables left (tuned, with their own graphs)
+    give the bits and see the parameters of batches in fresh contexts."""
+    small, many = [plain_small(3)], [plain_small(i) for i in range(4, 10)]
+    seq = [(small, 0), (many, 0), (many[:2], 1), (small, 0), (many, 1), (many[:3], 0)]
+    was = native.cache_enable(False)
+    try:
+        fresh = [_batch_outputs(m, n) for m, n in seq]
+        native.cache_enable(True)
+        for _ in range(2):
+            for (m, n), (params, out) in zip(seq, fresh):
+                p, o = _batch_outputs(m, n, {"fuse": 0, "fb2_split": 2, "t1_tail_grid": 512})
+                assert p == params
+                assert np.array_equal(_flat(o), _flat(out))
+    finally:
+        native.cache_clear()
+        native.cache_enable(was)
 
 
 @pytest.mark.parametrize("n", [0, 1])
