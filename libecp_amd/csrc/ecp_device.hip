@@ -158,6 +158,8 @@ struct DevTables {
   // up to the basis's each, at [r * prodN + q]
   CPtr<int> prod;
   int prodN;
+  // the shift's terms (shift_table)
+  const unsigned *shift;
   // T entries of a triplet (build_templates): packed (lambda1, lambda2, alpha + beta, l), channel after channel; those
   // of channel l < L at [toff(la, lb, l), toff(la, lb, l + 1)) (t2_off)
   CPtr<int> tmpl, toff;
@@ -165,7 +167,6 @@ struct DevTables {
   const double *poly2sph;
   const double *omega;
   CPtr<int> ijk, ijkIndex;
-  CPtr<double> binom;  // binom[n*16+k], n,k <= 15
   int ijkDim, tmDim, lorder;
   int omL, omLambda, omAlpha;
   double tol, lnAcc1, lnAcc2, accuracy;
@@ -1857,36 +1858,48 @@ __device__ __forceinline__ ShiftTab shift_tab_at(double *base, int LM, int side)
   return S;
 }
 
-__device__ void shift_factors(const DevTables &T, int l, const V3 v, bool with_norm, double norm, ShiftTab S,
-                              int lid, int nlanes) {
-  const int D = T.ijkDim;
+// (component, alpha) terms of a shell l, and of the shells before it
+__host__ __device__ constexpr int shift_terms(int l) {
+  return (l + 1) * (l + 2) * (l + 3) * (l + 4) * (l + 5) / 120;
+}
+__host__ __device__ constexpr int shift_terms_before(int l) {
+  return l * (l + 1) * (l + 2) * (l + 3) * (l + 4) * (l + 5) / 720;
+}
+
+// One side's factors, a term per lane of the W (8 to 64) lanes lid of a
+// group, from the term table (shift_table); the terms kept move up inside
+// their component.  (A component per lane took its up to 27 terms one after
+// another, each behind two table reads.)
+__device__ __forceinline__ void shift_factors(const DevTables &T, int l, const V3 v, bool with_norm, double norm,
+                                              ShiftTab S, int lid, int W) {
+  const int n = shift_terms(l);
+  const unsigned *tab = T.shift + shift_terms_before(l);
   const double tol = T.accuracy;
-  for (int c = lid; c < ECP_DIM_IJK(l); c += nlanes) {
-    const int *e = T.ijk + 3 * ECP_IDX_C(l, c);
-    const int ax = e[0], ay = e[1], az = e[2];
-    int n = 0;
-    for (int alx = 0; alx <= ax; alx++) {
-      double x = 1.0;
-      for (int i = 0; i < ax - alx; i++) x = -x * v.x;
-      const double bx = T.binom[ax * 16 + alx];
-      for (int aly = 0; aly <= ay; aly++) {
-        double y = 1.0;
-        for (int i = 0; i < ay - aly; i++) y = -y * v.y;
-        const double by = bx * T.binom[ay * 16 + aly];
-        for (int alz = 0; alz <= az; alz++) {
-          double z = 1.0;
-          for (int i = 0; i < az - alz; i++) z = -z * v.z;
-          const double bz = by * T.binom[az * 16 + alz];
-          double factor = bz * ((x * y) * z);
-          if (fabs(factor) <= tol) continue;
-          if (with_norm) factor *= norm;
-          S.f[c * S.mt + n] = factor;
-          S.r[c * S.mt + n] = T.ijkIndex[(alx * D + aly) * D + alz];
-          n++;
-        }
-      }
+  const int base = (int)(threadIdx.x & 63) & ~(W - 1);
+  const unsigned long long group = W == 64 ? ~0ull : (1ull << W) - 1ull;
+  unsigned long long prev = 0;
+  for (int e0 = 0; e0 < n; e0 += W) {
+    const bool in = e0 + lid < n;
+    const unsigned z = tab[min(e0 + lid, n - 1)];
+    const int c = z & 31, r = (z >> 14) & 127, dist = (z >> 26) & 31;
+    double px = 1.0, py = 1.0, pz = 1.0;
+    for (int i = (z >> 5) & 7; i > 0; i--) px = -px * v.x;
+    for (int i = (z >> 8) & 7; i > 0; i--) py = -py * v.y;
+    for (int i = (z >> 11) & 7; i > 0; i--) pz = -pz * v.z;
+    const double factor = (double)((z >> 21) & 31) * ((px * py) * pz);
+    const bool keep = in && !(fabs(factor) <= tol);
+    const unsigned long long m = (__ballot(keep) >> base) & group;
+    // kept terms of the component before this one; its first term may have
+    // been in the previous round
+    const int first = lid - dist;
+    int pos = __popcll(m & ((1ull << lid) - 1ull) & (~0ull << max(first, 0)));
+    if (first < 0) pos += __popcll(prev >> (W + first));
+    if (keep) {
+      S.f[c * S.mt + pos] = with_norm ? factor * norm : factor;
+      S.r[c * S.mt + pos] = r;
     }
-    S.n[c] = n;
+    if (in && z >> 31) S.n[c] = pos + keep;
+    prev = m;
   }
 }
 
@@ -1930,8 +1943,18 @@ __device__ void shift_block(const DevTables &T, Get get, int la, int lb, const V
   const ShiftTab SA = shift_tab_at(tab, LM, 0), SB = shift_tab_at(tab, LM, 1);
   __syncthreads();
   if (active) {
-    shift_factors(T, la, rA, false, 1.0, SA, lid, nlanes);
-    shift_factors(T, lb, rB, true, norm, SB, lid, nlanes);
+    // the sides beside each other where the lanes suffice
+    const int W = min(nlanes, 64), h = W / 2;
+    if (nlanes > 64) {
+      if (lid < 64) shift_factors(T, la, rA, false, 1.0, SA, lid, 64);
+      else if (lid < 128) shift_factors(T, lb, rB, true, norm, SB, lid - 64, 64);
+    } else if (max(shift_terms(la), shift_terms(lb)) <= h) {
+      const bool b = lid >= h;
+      shift_factors(T, b ? lb : la, b ? rB : rA, b, norm, b ? SB : SA, lid & (h - 1), h);
+    } else {
+      shift_factors(T, la, rA, false, 1.0, SA, lid, W);
+      shift_factors(T, lb, rB, true, norm, SB, lid, W);
+    }
   }
   __syncthreads();
   for (int idx = lid; idx < nia * ncb; idx += nlanes) {
@@ -1952,33 +1975,50 @@ __device__ void shift_block(const DevTables &T, Get get, int la, int lb, const V
   __syncthreads();
 }
 
-// H[p] += sum over the chunk's pairs k, in pair order, of
-// sum_{l = D, D - 2, ..} (sum_m S_lm(k) poly2sph[p][lm]) Q_k[(D - l) / 2]
-// for a monomial p of degree D: the same terms in the same order as the
-// general loop in k_asm1, with the monomial's poly2sph row held in
-// registers across the pairs instead of read again for every pair.
-template <int D>
-__device__ __forceinline__ double asm1_monomial(double acc, const double *__restrict__ pm, const double *rsph,
-                                                int rs_stride, const double *Qs, int nql, int nc) {
-  constexpr int NPM = (D + 1) * (D + 2) / 2;  // sum of 2 l + 1 over l = D, D - 2, ..
-  double pmv[NPM];
-  {
-    int j = 0;
+// One C-centred monomial's sum over the chunk's pairs: acc, then per pair the
+// blocks l = deg, deg - 2, .. of its poly2sph row times the pair's harmonics,
+// each times its Q value, in that order.  The lanes of a wave hold monomials
+// of every degree up to lab <= MAXD: block b is l = 2 b for even degrees and
+// l = 2 b - 1 for odd ones, so that all degrees go through one pass of at most
+// (MAXD + 1)(MAXD + 2) / 2 terms, the last two of a block for even degrees
+// only.  (A pass per degree, with its lanes alone, kept 0.20 of the lanes
+// busy: 84 terms a pair for class 6 instead of 28.)  Terms a lane does not
+// have are computed and not taken.
+template <int MAXD>
+__device__ __forceinline__ double asm1_monomial(double acc, int deg, int lab, const double *__restrict__ pm,
+                                                const double *rsph, int rs_stride, const double *Qs, int nql,
+                                                int nc) {
+  constexpr int NB = (MAXD + 1) / 2 + 1, NT = 4 * (NB - 1) + 1;
+  const int odd = deg & 1;
+  double pmv[NB][NT];
+  int off[NB];  // the block's first harmonic
+  bool on[NB];
 #pragma unroll
-    for (int l = D; l >= 0; l -= 2)
+  for (int b = 0; b < NB; b++) {
+    const int l = 2 * b - odd;
+    on[b] = l >= 0 && l <= deg;
+    off[b] = on[b] ? l * l : 0;
+    if (2 * b - 1 <= lab)
 #pragma unroll
-      for (int m = 0; m < 2 * l + 1; m++) pmv[j++] = pm[ECP_IDX_LM(l, m)];
+      for (int m = 0; m < 4 * b + 1; m++)
+        if (2 * b <= MAXD || m < 4 * b - 1) pmv[b][m] = pm[off[b] + (on[b] ? min(m, 2 * l) : 0)];
   }
   for (int k = 0; k < nc; k++) {
     const double *rs = rsph + k * rs_stride;
     const double *Q = Qs + k * nql;
-    int j = 0;
 #pragma unroll
-    for (int l = D; l >= 0; l -= 2) {
+    for (int b = NB - 1; b >= 0; b--) {
+      if (2 * b - 1 > lab) continue;
+      const double q = Q[on[b] ? (deg - 2 * b + odd) >> 1 : 0];
       double f = 0.0;
 #pragma unroll
-      for (int m = 0; m < 2 * l + 1; m++) f += rs[ECP_IDX_LM(l, m)] * pmv[j++];
-      acc += f * Q[(D - l) / 2];
+      for (int m = 0; m < 4 * b + 1; m++) {
+        if (2 * b > MAXD && m >= 4 * b - 1) continue;
+        const double x = f + rs[off[b] + m] * pmv[b][m];
+        f = m < 4 * b - 1 || !odd ? x : f;
+      }
+      const double a = acc + f * q;
+      acc = on[b] ? a : acc;
     }
   }
   return acc;
@@ -2080,14 +2120,7 @@ __global__ __launch_bounds__(kAsmThreads, 3) void k_asm1(DevTables T, DevJob J, 
       const double *pm = T.poly2sph + (size_t)p * tmd;
       double acc = H[p];
       if (deg <= MAXD) {
-        switch (deg) {
-#define MONO(D)                                                                       \
-  case D:                                                                             \
-    if constexpr (D <= MAXD) acc = asm1_monomial<D>(acc, pm, rsph, A.lds_rs_stride, Qs + qstart, nql, nc); \
-    break;
-          MONO(0) MONO(1) MONO(2) MONO(3) MONO(4) MONO(5) MONO(6)
-#undef MONO
-        }
+        acc = asm1_monomial<MAXD>(acc, deg, lab, pm, rsph, A.lds_rs_stride, Qs + qstart, nql, nc);
         H[p] = acc;
         continue;
       }
@@ -2563,6 +2596,33 @@ void reset_graph(ecp_dev *d) {
 
 }  // namespace
 
+// The terms of the shift of shells l = 0 .. 6, component after component,
+// alpha in the loop order of util.c:277-320, a word each: component (5 bits),
+// a - alpha (3 bits an axis), position of alpha (7), product of the binomials
+// C(a, alpha) (5: at most 20), distance from the component's first term (5)
+// and whether it is the component's last.
+static std::vector<unsigned> shift_table(const ecp_static *st) {
+  std::vector<unsigned> tab;
+  double f[8] = {1.0};
+  for (int i = 1; i < 8; i++) f[i] = f[i - 1] * i;
+  auto binom = [&](int n, int k) { return (unsigned)(f[n] / (f[n - k] * f[k])); };
+  for (int l = 0; l <= 6 && l < st->ijkDim; l++)
+    for (int c = 0; c < ECP_DIM_IJK(l); c++) {
+      const int *e = st->ijk + 3 * ECP_IDX_C(l, c);
+      unsigned d = 0;
+      for (int x = 0; x <= e[0]; x++)
+        for (int y = 0; y <= e[1]; y++)
+          for (int z = 0; z <= e[2]; z++, d++) {
+            const unsigned r = (unsigned)st->ijkIndex[(x * st->ijkDim + y) * st->ijkDim + z];
+            const unsigned b = binom(e[0], x) * binom(e[1], y) * binom(e[2], z);
+            const bool last = x == e[0] && y == e[1] && z == e[2];
+            tab.push_back((unsigned)c | (unsigned)(e[0] - x) << 5 | (unsigned)(e[1] - y) << 8 |
+                          (unsigned)(e[2] - z) << 11 | r << 14 | b << 21 | d << 26 | (unsigned)last << 31);
+          }
+    }
+  return tab;
+}
+
 extern "C" ecp_dev *ecp_dev_create(const ecp_static *st, char *err, size_t errlen) {
   ecp_dev *d = new ecp_dev();
   auto fail = [&](const char *what, hipError_t e) {
@@ -2611,14 +2671,6 @@ extern "C" ecp_dev *ecp_dev_create(const ecp_static *st, char *err, size_t errle
   const size_t nijk = 3 * (size_t)ECP_DIM_C(st->ijkDim - 1);
   const size_t nidx = (size_t)st->ijkDim * st->ijkDim * st->ijkDim;
   const size_t nfac = 2 * (size_t)st->tmDim + 6;
-  std::vector<double> binom(16 * 16, 0.0);
-  {
-    double f[16];
-    f[0] = 1.0;
-    for (int i = 1; i < 16; i++) f[i] = f[i - 1] * i;
-    for (int n = 0; n < 16; n++)
-      for (int k = 0; k <= n; k++) binom[n * 16 + k] = f[n] / (f[n - k] * f[k]);
-  }
   size_t off = 0;
   auto take = [&](size_t bytes) {
     size_t o = off;
@@ -2629,8 +2681,10 @@ extern "C" ecp_dev *ecp_dev_create(const ecp_static *st, char *err, size_t errle
   const size_t o_p93l = take(so * 4), o_p93r = take(so * 4), o_p92l = take(lo * 4), o_p92r = take(lo * 4);
   const size_t o_vis = take(so * 4), o_v93 = take((st->s93.npairs + kPs93Pad) * sizeof(Ps93Pair));
   const size_t o_bess = take(nbess * 8), o_poly = take(npoly * 8), o_om = take(nom * 8);
-  const size_t o_ijk = take(nijk * 4), o_idx = take(nidx * 4), o_bin = take(256 * 8);
+  const size_t o_ijk = take(nijk * 4), o_idx = take(nidx * 4);
   const size_t o_snorm = take(kSphDim * kSphDim * 8), o_dfac = take(nfac * 8), o_inv = take(kSphDim * 8);
+  const std::vector<unsigned> shift = shift_table(st);
+  const size_t o_shift = take(shift.size() * 4 + 4);
   const int prodN = ECP_DIM_C(st->omAlpha);
   const size_t o_prod = take((size_t)prodN * prodN * 4);
   const size_t o_tmpl = take(d->tmpl.size() * 4 + 4), o_toff = take(d->toff.size() * 4);
@@ -2675,7 +2729,6 @@ extern "C" ecp_dev *ecp_dev_create(const ecp_static *st, char *err, size_t errle
   put(o_om, st->omega, nom * 8);
   put(o_ijk, st->ijk, nijk * 4);
   put(o_idx, st->ijkIndex, nidx * 4);
-  put(o_bin, binom.data(), 256 * 8);
   {
     std::vector<double> nrm(kSphDim * kSphDim, 0.0), inv(kSphDim, 0.0);
     for (int l = 0; l < kSphDim; l++) {
@@ -2693,6 +2746,7 @@ extern "C" ecp_dev *ecp_dev_create(const ecp_static *st, char *err, size_t errle
         prod[(size_t)r * prodN + q] = st->ijkIndex[((a[0] + c[0]) * D + a[1] + c[1]) * D + a[2] + c[2]];
       }
     put(o_prod, prod.data(), prod.size() * 4);
+    put(o_shift, shift.data(), shift.size() * 4);
   }
   put(o_dfac, st->dfac, nfac * 8);
   put(o_tmpl, d->tmpl.data(), d->tmpl.size() * 4);
@@ -2717,12 +2771,12 @@ extern "C" ecp_dev *ecp_dev_create(const ecp_static *st, char *err, size_t errle
   T.omega = (const double *)(b + o_om);
   T.ijk = (const int *)(b + o_ijk);
   T.ijkIndex = (const int *)(b + o_idx);
-  T.binom = (const double *)(b + o_bin);
   T.snorm = (const double *)(b + o_snorm);
   T.dfac = (const double *)(b + o_dfac);
   T.inv = (const double *)(b + o_inv);
   T.prod = (const int *)(b + o_prod);
   T.prodN = prodN;
+  T.shift = (const unsigned *)(b + o_shift);
   T.tmpl = (const int *)(b + o_tmpl);
   T.toff = (const int *)(b + o_toff);
   T.ijkDim = st->ijkDim;
