@@ -1869,7 +1869,9 @@ __host__ __device__ constexpr int shift_terms_before(int l) {
 // One side's factors, a term per lane of the W (8 to 64) lanes lid of a
 // group, from the term table (shift_table); the terms kept move up inside
 // their component.  (A component per lane took its up to 27 terms one after
-// another, each behind two table reads.)
+// another, each behind two table reads.  The assembly of 256 molecules,
+// alone: type 1 1978 + 461 -> 1276 + 338 us, type 2 2857 + 682 -> 2177 + 476;
+// waits were 0.6 of its wave cycles.)
 __device__ __forceinline__ void shift_factors(const DevTables &T, int l, const V3 v, bool with_norm, double norm,
                                               ShiftTab S, int lid, int W) {
   const int n = shift_terms(l);
@@ -1982,8 +1984,8 @@ __device__ void shift_block(const DevTables &T, Get get, int la, int lb, const V
 // l = 2 b - 1 for odd ones, so that all degrees go through one pass of at most
 // (MAXD + 1)(MAXD + 2) / 2 terms, the last two of a block for even degrees
 // only.  (A pass per degree, with its lanes alone, kept 0.20 of the lanes
-// busy: 84 terms a pair for class 6 instead of 28.)  Terms a lane does not
-// have are computed and not taken.
+// busy: 84 terms a pair for class 6 instead of 28; 256 molecules 2111 ->
+// 1978 us.)  Terms a lane does not have are computed and not taken.
 template <int MAXD>
 __device__ __forceinline__ double asm1_monomial(double acc, int deg, int lab, const double *__restrict__ pm,
                                                 const double *rsph, int rs_stride, const double *Qs, int nql,
@@ -3019,7 +3021,11 @@ ClassMap fb2_classes(const ecp_dev *d, const T2Set &S) {
 // overlaps the quadratures).
 void enqueue_fused(ecp_dev *d, hipStream_t s, hipEvent_t *evs);
 
-void launch_tables(ecp_dev *d, hipStream_t s) {
+// parts of the tables launch: what type 1 needs (with the zero-fill), and
+// the rest, which only type 2 reads
+constexpr int kTabFront = 1, kTabBack = 2;
+
+void launch_tables(ecp_dev *d, hipStream_t s, int parts) {
   const Prepared &P = d->P;
   TabArgs A{};
   A.zero_base = P.zero_base;
@@ -3041,8 +3047,13 @@ void launch_tables(ecp_dev *d, hipStream_t s) {
   // few pairs: several workgroups each (20 atoms with g shells, 160 pairs:
   // the launch 116 us at one, 4556 workgroups in all)
   A.aparts = P.nait < 1024 ? 4 : 1;
+  int units = (int)(((size_t)P.nt * P.maxPairs + 127) / 128);
+  if (!(parts & kTabFront)) A.nzb = A.nub = units = 0;
+  if (!(parts & kTabBack)) A.nait = A.nfit = 0;
+  const int grid = A.nait * A.aparts + A.nzb + A.nub + A.nfit + units;
+  if (grid == 0) return;
   Span sp(d, s, FAM_TABLES);
-  k_tables<<<A.nait * A.aparts + A.nzb + A.nub + A.nfit + (int)(((size_t)P.nt * P.maxPairs + 127) / 128), 128, 0, s>>>(d->T, P.J, A);
+  k_tables<<<grid, 128, 0, s>>>(d->T, P.J, A);
 }
 
 // fuse = 2 (automatic), by the job's type-1 primitive pairs.  Up to
@@ -3056,6 +3067,22 @@ constexpr int kFuseAutoSmall = 150000, kFuseAutoLarge = 800000;
 
 bool fuse_auto(int units, int max_lab) {
   return units <= kFuseAutoSmall || (units > kFuseAutoLarge && max_lab <= 6);
+}
+
+// The tables, and the fork of the first nw workers, which take the type-1
+// work, off the main stream.  Captured small jobs split the launch, so that
+// the type-1 chain does not wait for the tables of type 2: replays of a tiny
+// molecule 146 -> 137 us, 17 atoms 174 -> 165 us, 50 atoms 330 -> 314 us.
+// Eager, the second launch costs what it gains (tiny molecule 234 -> 242 us a
+// call), and large jobs gain nothing (50-atom gradient 784 -> 799 us, 20
+// atoms with g shells 3509 -> 3523 us, 256 molecules 12458 -> 12392 us).
+void fork_tables(ecp_dev *d, hipStream_t s, int nw, hipEvent_t *evs) {
+  const bool split = d->capturing && d->P.cls_begin[ECP_MAX_LAB + 1] <= kFuseAutoSmall;
+  launch_tables(d, s, split ? kTabFront : kTabFront | kTabBack);
+  (void)hipEventRecord(d->fork, s);
+  for (int i = 0; i < nw; i++) (void)hipStreamWaitEvent(d->workers[i], d->fork, 0);
+  if (split) launch_tables(d, s, kTabBack);
+  if (evs) (void)hipEventRecord(evs[1], s);
 }
 
 // one type-1 class of the per-class sequence: quadrature, assembly
@@ -3090,10 +3117,7 @@ void enqueue(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
   hipStream_t *w = d->workers;
   d->span_valid = false;  // type-1 classes run on several streams
   if (evs) (void)hipEventRecord(evs[0], s);
-  launch_tables(d, s);
-  if (evs) (void)hipEventRecord(evs[1], s);
-  (void)hipEventRecord(d->fork, s);
-  for (int i = 0; i < kWorkers; i++) (void)hipStreamWaitEvent(w[i], d->fork, 0);
+  fork_tables(d, s, kWorkers, evs);
   // the type-2 chain (small grid, fallbacks, assembly) on the main stream,
   // beside it the type-1 classes on three workers: one stream per hardware
   // queue the device gives a process
@@ -3149,10 +3173,7 @@ void enqueue_fused(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
   hipStream_t w = d->workers[0];
   d->span_valid = false;
   if (evs) (void)hipEventRecord(evs[0], s);
-  launch_tables(d, s);
-  if (evs) (void)hipEventRecord(evs[1], s);
-  (void)hipEventRecord(d->fork, s);
-  (void)hipStreamWaitEvent(w, d->fork, 0);
+  fork_tables(d, s, 1, evs);
   // ---- type 1 ----
   const T1Set S = t1_set(d);
   // the fused kernels hold the registers of their largest class: four
