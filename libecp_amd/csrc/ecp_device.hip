@@ -1180,14 +1180,20 @@ struct T2State {
 // molecules, 3.1 ms at one per clock and CU, of 3.3 ms).
 // Levels 0 to 5, fifteen points read together, decide nearly all entries of
 // most triplets; where entries stay open, the levels up to 14 follow in
-// steps of NP = 4 point pairs (each ends its level or lies inside it),
-// the next step's values read ahead.  Point pairs
+// steps of NP = 4 point pairs (each ends its level or lies inside it; in
+// steps of 8, the first takes levels 6 and 7, of 4 pairs each), the next
+// step's values read ahead.  Point pairs
 // are added in order, with the PS93 test at each level's end.  Points outside
 // the pair's window need no test: F_a or F_b is 0 there; a step with all of
 // its points outside is passed over.
 constexpr int kT2Head = 6;      // levels of the first part
 constexpr int kT2HeadPairs = 6; // their point pairs from level 2 on
 constexpr int kT2HeadPts = 3 + 2 * kT2HeadPairs;
+template <bool SMALL>
+struct T2Shape {
+  static constexpr int kStep = SMALL ? 8 : 4;  // point pairs of a later step
+  static constexpr int kOwn = SMALL ? 1 : 2;   // entries a lane owns
+};
 
 // Workgroups go to the eight XCDs, each with its own L2, in turn: workgroup b
 // of n takes the item that leaves runs of 64 consecutive items -- the
@@ -1202,22 +1208,25 @@ __device__ __forceinline__ int xcd_item(int b, int n) {
 }
 
 // doubles of LDS of a wave; CH: 16-byte chunks of a point's values
-__host__ __device__ constexpr int t2_lds(int G, int NP, int CH) {
-  return G * 2 * CH * (2 * NP > kT2HeadPts ? 2 * NP : kT2HeadPts);
+template <bool SMALL>
+__host__ __device__ constexpr int t2_lds(int G, int CH) {
+  constexpr int step = 2 * T2Shape<SMALL>::kStep;
+  return G * 2 * CH * (step > kT2HeadPts ? step : kT2HeadPts);
 }
 
 typedef double dpair __attribute__((ext_vector_type(2)));
 
 // LP: lanes that read a point together, two values (16 bytes) each; the F and
 // U rows have even lengths, so that every chunk is aligned
-template <int G, int NP, int R, int CH>
+template <int G, int CH, bool SMALL>
 __device__ __forceinline__ void type2_body(int bid, const DevTables &T, const DevJob &J, const T2Args &A,
                                            const int *__restrict__ tlist, int ntl, int slice, int nslices,
                                            double *s_all) {
+  constexpr int NP = T2Shape<SMALL>::kStep, R = T2Shape<SMALL>::kOwn;
   constexpr int W = 64 / G, LP = G == 1 ? 32 : 16, PT = W / LP, X = (CH + LP - 1) / LP, ROW = 2 * CH;
   const int grp = (int)threadIdx.x / W, lid = (int)threadIdx.x % W;
   const int pt = lid / LP, pl = lid % LP;  // point of a read, lane of the point
-  double *s_v = s_all + grp * t2_lds(1, NP, CH);
+  double *s_v = s_all + grp * t2_lds<SMALL>(1, CH);
   const int ti = bid * G + grp;
   const bool active = ti < ntl;
   const int t = cload(tlist + (active ? ti : 0));
@@ -1340,8 +1349,13 @@ __device__ __forceinline__ void type2_body(int bid, const DevTables &T, const De
       };
       // the step from b on has a point in a group's window
       auto inside = [&](int b) {
-        const Ps93Pair z = T.v93[b + NP - 1];
-        return wave_any(z.li >= gs || z.ri <= ge);
+        bool in = false;
+#pragma unroll
+        for (int j = 3; j < NP; j += 4) {
+          const Ps93Pair z = T.v93[b + j];
+          in = in || z.li >= gs || z.ri <= ge;
+        }
+        return wave_any(in);
       };
       bool on = inside(c0);
       if (on) read(c0);
@@ -1382,10 +1396,13 @@ __device__ __forceinline__ void type2_body(int bid, const DevTables &T, const De
             }
           }
         } else {
-          const Ps93Pair z = T.v93[b + NP - 1];
-          if (z.ends)
 #pragma unroll
-            for (int i = 0; i < R; i++) S[i].level(T, z.ends, false);
+          for (int j = 3; j < NP; j += 4) {
+            const Ps93Pair z = T.v93[b + j];
+            if (z.ends)
+#pragma unroll
+              for (int i = 0; i < R; i++) S[i].level(T, z.ends, false);
+          }
         }
         __syncthreads();
         if (last || !wave_any(group_open())) break;
@@ -1435,19 +1452,34 @@ __device__ __forceinline__ void type2_body(int bid, const DevTables &T, const De
 // 231 -> 197 us an evaluation, 50 atoms 380 -> 342 us (at a quarter of
 // kT2Fill: no gain on the latter), g shells shifted to h under L = 6 on
 // three atoms 1331 -> 582 us (with the wide assembly below).
-constexpr int kT2Pack = 2, kT2PackLab = 2, kT2Pairs = 4, kT2Fill = 16384, kT2Pass = 128;
+constexpr int kT2Pack = 2, kT2PackLab = 2, kT2Fill = 16384, kT2Pass = 128;
 
 template <int CH, int CHP>
 __global__ __launch_bounds__(64, CH <= 24 ? 4 : 3) void k_type2(DevTables T, DevJob J, T2Args A, const int *__restrict__ tlist,
                                                 int m, int nslices) {
-  __shared__ __align__(16) double s_v[t2_lds(1, kT2Pairs, CH) > t2_lds(kT2Pack, kT2Pairs, CHP)
-                                          ? t2_lds(1, kT2Pairs, CH)
-                                          : t2_lds(kT2Pack, kT2Pairs, CHP)];
+  __shared__ __align__(16) double s_v[t2_lds<false>(1, CH) > t2_lds<false>(kT2Pack, CHP) ? t2_lds<false>(1, CH)
+                                                                                        : t2_lds<false>(kT2Pack, CHP)];
   const int n = J.ntrip - m, np = (m + kT2Pack - 1) / kT2Pack, b = blockIdx.x;
   if (b < n * nslices)
-    type2_body<1, kT2Pairs, 2, CH>(xcd_item(b % n, n), T, J, A, tlist + m, n, b / n, nslices, s_v);
+    type2_body<1, CH, false>(xcd_item(b % n, n), T, J, A, tlist + m, n, b / n, nslices, s_v);
   else
-    type2_body<kT2Pack, kT2Pairs, 2, CHP>(xcd_item(b - n * nslices, np), T, J, A, tlist, m, 0, 1, s_v);
+    type2_body<kT2Pack, CHP, false>(xcd_item(b - n * nslices, np), T, J, A, tlist, m, 0, 1, s_v);
+}
+
+// Jobs of up to kT2Small triplets, whose time is the chain of one wave's
+// steps: an entry per lane, 64 a pass, every triplet in waves of its own, and
+// steps of eight point pairs (half as many).  Alone, on a tiny molecule, 49 ->
+// 29 us; replays of it 129 -> 109 us, 17 atoms (1167 triplets) 156 -> 144 us.
+// From 50 atoms (8001 triplets) on the general shape is the better one, 306
+// against 313 us, 24 674 triplets of a gradient 775 against 884 us.
+constexpr int kT2Small = 4096;
+
+template <int CH>
+__global__ __launch_bounds__(64, 2) void k_type2_small(DevTables T, DevJob J, T2Args A, const int *__restrict__ tlist,
+                                                       int nslices) {
+  __shared__ __align__(16) double s_v[t2_lds<true>(1, CH)];
+  const int n = J.ntrip;
+  type2_body<1, CH, true>(blockIdx.x % n, T, J, A, tlist, n, blockIdx.x / n, nslices, s_v);
 }
 
 // type-2 fallback (calcT_FM06, type2.c:417-528): one wave per (triplet with
@@ -2840,6 +2872,12 @@ void launch_type2(ecp_dev *d, hipStream_t s) {
   if (P.ntot2 <= 0) return;
   T2Args A{P.Tout, P.tf, P.tnfail, P.flist, P.fbq2, P.fbc + kFb2Cnt, P.nt, P.tcls2};
   Span sp(d, s, FAM_TYPE2);
+  if (P.nt <= kT2Small && P.max_lbs <= 4 && P.max_L <= 5) {
+    const int ns = std::max(1, std::min((P.max_ent2 + 63) / 64, kT2Fill / P.nt));
+    if (P.max_lbs <= 3 && P.max_L <= 4) k_type2_small<24><<<P.nt * ns, 64, 0, s>>>(d->T, P.J, A, P.tcls, ns);
+    else k_type2_small<35><<<P.nt * ns, 64, 0, s>>>(d->T, P.J, A, P.tcls, ns);
+    return;
+  }
   const int m = P.tcls_begin[kT2PackLab + 1];
   const int n = P.nt - m, npass = (P.max_ent2 + kT2Pass - 1) / kT2Pass;
   const int ns = std::max(1, std::min(npass, kT2Fill / std::max(n, 1)));

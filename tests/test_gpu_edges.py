@@ -15,7 +15,7 @@ import pytest
 
 import ecp_native as E
 from libecp_amd import native
-from libecp_amd.workloads import build_molecule, high_l, plain_small
+from libecp_amd.workloads import batch_molecule, build_molecule, high_l, plain_small
 
 pytestmark = pytest.mark.gpu
 
@@ -164,3 +164,32 @@ def test_contract_after_replays(n):
         assert not codes.any()
         outs.append(_flat(out))
     assert np.array_equal(outs[0], outs[1])
+
+
+def _pile(mols, n):
+    b = native.Batch(mols, n=n)
+    try:
+        b.execute(3)
+        if n == 0:
+            b.fetch()
+            return [_flat([b.matrix(i)]) for i in range(len(mols))], b.triplets()[1]
+        P = [np.random.default_rng(4).standard_normal((m.nao, m.nao)) for m in mols]
+        return [_flat([g]) for g in b.contract(P)[1]], b.triplets()[1]
+    finally:
+        b.close()
+
+
+@pytest.mark.parametrize("n", [0, 1])
+@pytest.mark.parametrize("name", ["s_to_f", "s_to_g", "few"])
+def test_small_job_equals_large_one(name, n):
+    """A molecule alone (the type-2 shapes of small jobs) and in a batch of
+    copies too large for them: the same bits."""
+    m = {"s_to_f": lambda: batch_molecule(np.random.default_rng(6), 17 if n == 0 else 9),
+         "s_to_g": lambda: high_l(1000, nat=8 if n == 0 else 5, n_ecp=2, box=9.0),
+         "few": entries_few}[name]()
+    alone, nt = _pile([m], n)
+    assert 0 < nt <= 4096
+    copies, many = _pile([m] * (8192 // nt + 1), n)
+    assert many > 4096
+    for c in copies:
+        assert np.array_equal(c, alone[0])
