@@ -155,26 +155,18 @@ const char *libecp_kernel_family(int i);
    launches (the quadrature then spans several streams). */
 int libecp_batch_quadrature_ms(libecp_batch *b, double *ms, int *samples);
 /* Launch parameters of the batch's device pipeline, by name:
-   "t1_head_coop" / "t1_head_serial" (PS93 levels the type-1 head kernel runs
-   before the wave-cooperative / lane-serial tail; 8 and 8 by default),
-   "t1_coop_max" (largest
-   type-1 class, in primitive pairs, that takes the cooperative tail),
-   "t1_tail_grid" (most workgroups of a tail launch), "fuse" (1: one launch
-   per stage covering every class, with assembly overlapping the large-grid
-   fallbacks; 0: per-class launches on forked streams; 2, the default: fused
-   for small jobs), "asm2_cache" (type-2 assembly with the angular factors
-   in registers: 0 no, 1, the default: yes, 2 with fused launches only),
-   "t2_head" (PS93 levels of the type-2 small-grid kernel before the entries
-   still open are rerun compacted; 15, the default: no split; 0: 6 with
-   fused launches, no split otherwise), "t2_tail_grid",
-   "fb2_split" (shares a triplet's type-2 fallback entries are split into,
-   each with its own waves; 0, the default: by the job's size).  "t1_spec" (fused launches: 1, the default, starts
-   the type-1 large-grid fallback beside the small-grid tail on every entry
-   the head left open; 0 after the tail on the failed entries).  "t2_spec"
-   (fused launches with a type-2 head: 1 starts the type-2 large-grid
-   fallback beside the tail on every entry the head left open; 0, the
-   default, after the tail on the failed entries).  Results do not depend on
-   them.  0, or -1 for an unknown name. */
+   "t1_head_coop" (PS93 levels the type-1 head kernel runs before the
+   wave-cooperative tail; 5 by default), "t1_tail_grid" (most workgroups of a
+   class's tail), "fuse" (1: one launch per stage covering every class, the
+   type-1 and type-2 chains side by side; 0: per-class type-1 launches on
+   forked streams; 2, the default: by the job's size), "asm2_cache" (type-2
+   assembly with the angular factors in registers: 0 no, 1, the default, and
+   2 yes), "fb2_split" (shares a triplet's type-2 fallback entries are split
+   into, each with its own waves; 0, the default: by the job's size).
+   "t1_head_serial", "t1_coop_max", "t2_head", "t2_tail_grid", "t1_spec" and
+   "t2_spec" are accepted and read back; the kernels no longer have these
+   choices.  Results do not depend on any of them.  0, or -1 for an unknown
+   name. */
 int libecp_batch_set_param(libecp_batch *b, const char *name, int value);
 int libecp_batch_get_param(libecp_batch *b, const char *name, int *value);
 /* Autotuner: times the batch (graph replays, `repeats` per candidate) over

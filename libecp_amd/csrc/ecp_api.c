@@ -874,14 +874,10 @@ int libecp_batch_autotune(libecp_batch *b, int repeats, char *report, int len) {
     int v[6];
   } space[] = {
       {"fuse", 3, {0, 1, 2}},
-      {"asm2_cache", 3, {0, 1, 2}},
-      {"t2_head", 6, {0, 4, 6, 8, 10, 15}},
-      {"t1_coop_max", 5, {0, 20000, 100000, 400000, 1 << 30}},
-      {"t1_head_coop", 4, {6, 8, 10, 12}},
-      {"t1_head_serial", 4, {6, 8, 10, 15}},
+      {"asm2_cache", 2, {0, 1}},
+      {"t1_head_coop", 4, {4, 5, 6, 8}},
       {"t1_tail_grid", 4, {2048, 8192, 32768, 131072}},
       {"fb2_split", 4, {0, 1, 2, 3}},
-      {"t1_spec", 2, {0, 1}},
   };
   for (size_t k = 0; k < sizeof(space) / sizeof(space[0]); k++) {
     for (int i = 0; i < space[k].n; i++) {
@@ -906,8 +902,8 @@ int libecp_batch_autotune(libecp_batch *b, int repeats, char *report, int len) {
   }
   ecp_dev_set_tuning(b->dev, &best);
   if (report && used < (size_t)len)
-    snprintf(report + used, (size_t)len - used, "; best %.4f ms: fuse=%d asm2_cache=%d t2_head=%d t1_coop_max=%d "
-             "t1_head_coop=%d t1_head_serial=%d t1_tail_grid=%d", tbest, best.fuse, best.asm2_cache, best.t2_head,
-             best.t1_coop_max, best.t1_head_coop, best.t1_head_serial, best.t1_tail_grid);
+    snprintf(report + used, (size_t)len - used, "; best %.4f ms: fuse=%d asm2_cache=%d t1_head_coop=%d "
+             "t1_tail_grid=%d fb2_split=%d", tbest, best.fuse, best.asm2_cache, best.t1_head_coop, best.t1_tail_grid,
+             best.fb2_split);
   return 0;
 }

@@ -8,14 +8,16 @@
 //            F_lambda(r_n) per (centre, shell) on its screened window
 //            (calcF_FM06: type2.c:222-310)
 //            and per-(centre, atom) angular tables (evalAngularIntegrals:
-//            angular_integrals.c:104-142)
+//            angular_integrals.c:104-142); the type-1 units
 //   k_type1 / k_t1tail  type-1 radial integrals Q[l1][l2] per (triplet,
 //            primitive pair) with the PS93 sequence (calcQ: type1.c:94-203):
-//            lane-serial head, wave-cooperative tail for the open pairs
-//   k_type2  type-2 radial integrals T_l[l1][l2][l3] per entry with PS93
-//            (calcT_fast_FM06: type2.c:336-381)
-//   k_fb1 / k_fb2  PSM92 large-grid redo of failed entries on FM06-mapped
-//            grids (type1.c:205-252, calcT_FM06: type2.c:417-528)
+//            lane-serial head, wave-cooperative tail for the open pairs,
+//            which also redoes the failed ones with PSM92 on the FM06-mapped
+//            large grid (type1.c:205-252)
+//   k_type2 / k_type2_small  type-2 radial integrals T_l[l1][l2][l3] per
+//            entry with PS93 (calcT_fast_FM06: type2.c:336-381)
+//   k_fb2    PSM92 large-grid redo of failed type-2 entries (calcT_FM06:
+//            type2.c:417-528)
 //   k_asm1 / k_asm2  type-1 / type-2 blocks, binomial shift and norms
 //            (calcChi: type1.c:211-302, calcGamma: type2.c:532-631,
 //             calcPolynomials: util.c:246-334)

@@ -73,26 +73,18 @@ typedef struct {
 /* ---- launch parameters of the device pipeline (tunable per context) ---- */
 typedef struct {
   int t1_head_coop;   /* PS93 levels of the type-1 head kernel before the wave-cooperative tail */
-  int t1_head_serial; /* ... before the lane-serial tail (>= the level count: no tail) */
-  int t1_coop_max;    /* largest class (primitive pairs) that takes the cooperative tail */
+  int t1_head_serial; /* kept for callers that set it: no effect */
+  int t1_coop_max;    /* likewise */
   int t1_tail_grid;   /* most workgroups of a tail launch (persistent over its queue) */
-  int fuse;           /* 1: one launch per stage over all classes, assembly overlapping the
-                         large-grid fallbacks; 0: per-class launches on forked streams;
-                         2: fused for small jobs, per-class for large ones */
-  int asm2_cache;     /* type-2 assembly with angular factors in registers: 0 no, 1 yes
-                         (the default), 2 with fused launches only */
-  int t2_head;        /* PS93 levels of the type-2 head kernel before the compacted tail
-                         (>= the level count, the default: no tail; 0: 6 with fused
-                         launches, else none) */
-  int t2_tail_grid;   /* most workgroups of the type-2 tail launch */
+  int fuse;           /* 1: one launch per stage over all classes, a chain for either type;
+                         0: per-class type-1 launches on forked streams; 2: by the job's size */
+  int asm2_cache;     /* type-2 assembly with angular factors in registers: 0 no, else yes */
+  int t2_head;        /* kept for callers that set it: no effect */
+  int t2_tail_grid;   /* likewise */
   int fb2_split;      /* shares a triplet's type-2 fallback entries are split into, each with its
                          own waves; 0: by the job's size */
-  int t1_spec;        /* fused launches: the type-1 large-grid fallback starts after the head,
-                         beside the tail, on every entry the head left open (1), or after the
-                         tail on the failed ones only (0) */
-  int t2_spec;        /* fused launches with a type-2 head: the type-2 fallback starts after
-                         the head, beside the tail, on every entry the head left open (1), or
-                         after the tail on the failed ones only (0) */
+  int t1_spec;        /* kept for callers that set it: no effect */
+  int t2_spec;        /* likewise */
 } ecp_tuning;
 
 /* ---- device layer (ecp_device.hip) ---- */
