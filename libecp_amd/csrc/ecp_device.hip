@@ -659,8 +659,9 @@ __device__ __forceinline__ void t1_finish(const DevTables &T, const T1Geom &G, i
 }
 
 // Type-1 small grid, one lane per primitive pair: levels [0, head); a pair
-// still open then saves its integrator state -- p, q, I per entry in planes
-// of `plane` doubles at state -- and its converged-entry mask and is queued
+// still open then saves its integrator state -- p per entry at its results'
+// place, q and I in planes of `plane` doubles at state -- and its
+// converged-entry mask and is queued
 // for the tail (head >= the level count: the whole sequence, no tail).
 // Within a level each point pair's sum T = (0 + f(left)) + f(right) is added
 // to I in pair order, and the PS93 recurrences and test
@@ -767,9 +768,9 @@ __device__ __forceinline__ void type1_body(int bid, const DevTables &T, const De
     if ((done | lost) != all && lv1 < T.s93.nlevels) {
 #pragma unroll
       for (int e = 0; e < NQ; e++) {
-        state[U.qoff + e] = p[e];
-        state[plane + U.qoff + e] = q[e];
-        state[2 * plane + U.qoff + e] = I[e];
+        qout[U.qoff + e] = p[e];
+        state[U.qoff + e] = q[e];
+        state[plane + U.qoff + e] = I[e];
       }
       qfail[u] = done;
       tq[queue_slot(tcount)] = u;
@@ -1016,9 +1017,9 @@ __device__ __forceinline__ void t1tail_body(int bid, int nb, const DevTables &T,
     double p = 0.0, q = 0.0, I = 0.0;
     bool mydone = true, lost = false;
     if (tail && lane < NQ) {
-      p = state[U.qoff + lane];
-      q = state[plane + U.qoff + lane];
-      I = state[2 * plane + U.qoff + lane];
+      p = qout[U.qoff + lane];
+      q = state[U.qoff + lane];
+      I = state[plane + U.qoff + lane];
       mydone = (done0 >> lane) & 1ull;
     }
     int lv = tail ? head : T.s93.nlevels;
@@ -2468,7 +2469,7 @@ struct Prepared {
   size_t cls_qbase[ECP_MAX_LAB + 2] = {0};  // first Q value of each class
   double *q = nullptr;
   size_t nq = 0;
-  double *t1s = nullptr;  // type-1 head -> tail state: p, q, I planes of nq doubles
+  double *t1s = nullptr;  // type-1 head -> tail state: q, I planes of nq doubles (p in q)
   int *tq1 = nullptr;     // type-1 tail queues (per class, indexed like the units)
   unsigned long long *qf = nullptr;
   double *udir = nullptr;  // per type-1 unit: its pair direction (4 values)
@@ -3418,7 +3419,7 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
   Ly.d_fbq2 = dv_take(4 * (size_t)(kMaxLMB + 1) * nt);
   Ly.d_fbT = dv_take(8 * (size_t)ntot2 * P.maxPairs);
   Ly.d_blk = dv_take(8 * job->nblk);
-  Ly.d_t1s = dv_take(3 * 8 * nq);
+  Ly.d_t1s = dv_take(2 * 8 * nq);
   Ly.d_tq1 = dv_take(4 * nunits);
   Ly.d_udir = dv_take(32 * nunits);
   Ly.total = dv_off;
