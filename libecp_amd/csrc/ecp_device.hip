@@ -3793,6 +3793,16 @@ extern "C" int ecp_dev_fetch(ecp_dev *d, double **blocks, unsigned char **status
   return 0;
 }
 
+// Zeros for a job's results, which a context of an earlier job holds other
+// values in (a fetch or contraction before the first evaluation reads them).
+extern "C" int ecp_dev_clear(ecp_dev *d, char *err, size_t errlen) {
+  const Prepared &P = d->P;
+  if (P.nt == 0) return 0;
+  ECP_CHECK(hipMemsetAsync(P.blk, 0, 8 * P.nblk, d->stream));
+  ECP_CHECK(hipMemsetAsync(P.stat, 0, 2 * (size_t)P.nt, d->stream));
+  return 0;
+}
+
 // bytes of device and pinned memory a context holds for jobs
 extern "C" size_t ecp_dev_held(const ecp_dev *d) {
   return d->arena_cap + d->con_cap + d->pin_in_cap + d->pin_out_cap;

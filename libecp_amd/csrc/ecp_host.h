@@ -109,6 +109,8 @@ int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char *err, size_
 int ecp_dev_bind(ecp_dev *d, void *mem, size_t cap, char *err, size_t errlen);
 int ecp_dev_execute(ecp_dev *d, int repeats, double *ms_total, char *err, size_t errlen);
 int ecp_dev_fetch(ecp_dev *d, double **blocks, unsigned char **status, char *err, size_t errlen);
+/* queues zeros for the results of the job at hand */
+int ecp_dev_clear(ecp_dev *d, char *err, size_t errlen);
 /* bytes of device and pinned memory a context holds for jobs */
 size_t ecp_dev_held(const ecp_dev *d);
 /* Contracts the last evaluation's blocks with densities on the device (job

@@ -125,6 +125,24 @@ def test_failed_blocks_are_zero_in_a_used_context():
     assert used == fresh
 
 
+def test_results_before_an_evaluation():
+    """A batch that takes another one's context reads zeros until its first
+    evaluation."""
+    native.cache_clear()
+    for m in (plain_small(4), plain_small(3)):
+        b = native.Batch([m])
+        try:
+            b.fetch()
+            rc, I = b.matrix(0)
+            assert rc == 0 and not I.any()
+            b.execute(1)
+            b.fetch()
+            rc, I = b.matrix(0)
+            assert rc == 0 and I.any()
+        finally:
+            b.close()
+
+
 def test_batch_in_a_used_context():
     """Batches of rising and falling sizes and both orders in contexts that
     earlier batches of the same tables left (tuned, with their own graphs)
