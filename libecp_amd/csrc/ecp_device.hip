@@ -3694,8 +3694,9 @@ extern "C" int ecp_dev_execute(ecp_dev *d, int repeats, double *ms_total, char *
 // own stream; per family: launches, summed duration (ms), algorithmic FLOPs.
 namespace {
 // Algorithmic FLOPs of the large-grid fallbacks of the last evaluation
-// (ecp_fb1_flops / ecp_fb2_flops per failed primitive pair / group): every
-// term is an integer below 2^53, so the atomic sum is exact in any order.
+// (ecp_fb1_flops per failed primitive pair, ecp_fb2_flops per primitive pair of
+// a (triplet, channel) with failed entries): every term is an integer below
+// 2^53, so the atomic sum is exact in any order.
 __global__ __launch_bounds__(256) void k_fb_flops(DevJob J, const T1Unit *__restrict__ units,
                                                   const unsigned long long *__restrict__ qf, int nunits,
                                                   DevTables T, const int *__restrict__ tnfail,
@@ -3714,13 +3715,17 @@ __global__ __launch_bounds__(256) void k_fb_flops(DevJob J, const T1Unit *__rest
     const ecp_triplet tr = J.trip[t];
     const ecp_centre *C = J.cent + tr.centre;
     const int KK = J.shells[tr.sa].K * J.shells[tr.sb].K, t0 = t2_off(T, tr.la, tr.lb, 0);
-    // listed in entry order, channel after channel
-    for (int k = 0; k < nf;) {
+    // one term per channel with failed entries: counted first, since the
+    // waves that share a triplet's passes list their entries in any order
+    int f[ECP_MAX_L] = {0};
+    for (int k = 0; k < nf; k++) {
       const int l = T.tmpl[t0 + flist[J.teoff[t] + k]] >> 24;
-      int f = 0;
-      for (; k < nf && T.tmpl[t0 + flist[J.teoff[t] + k]] >> 24 == l; k++) f++;
-      s2 += KK * ecp_fb2_flops(tr.la, tr.lb, l, C->gl[l + 1] - C->gl[l], f, N);
+#pragma unroll
+      for (int i = 0; i < ECP_MAX_L; i++) f[i] += l == i;
     }
+#pragma unroll
+    for (int l = 0; l < ECP_MAX_L; l++)
+      if (f[l]) s2 += KK * ecp_fb2_flops(tr.la, tr.lb, l, C->gl[l + 1] - C->gl[l], f[l], N);
   }
   if (s1 != 0.0) atomicAdd(&out[0], s1);
   if (s2 != 0.0) atomicAdd(&out[1], s2);
