@@ -156,7 +156,7 @@ const char *libecp_kernel_family(int i);
 int libecp_batch_quadrature_ms(libecp_batch *b, double *ms, int *samples);
 /* Launch parameters of the batch's device pipeline, by name:
    "t1_head_coop" (PS93 levels the type-1 head kernel runs before the
-   wave-cooperative tail; 5 by default), "t1_tail_grid" (most workgroups of a
+   wave-cooperative tail; 5 by default, at least 2), "t1_tail_grid" (most workgroups of a
    class's tail), "fuse" (1: one launch per stage covering every class, the
    type-1 and type-2 chains side by side; 0: per-class type-1 launches on
    forked streams; 2, the default: by the job's size), "asm2_cache" (type-2

@@ -2970,7 +2970,8 @@ T1Set t1_set(const ecp_dev *d) {
     S.ubeg[c] = P.cls_begin[c];
     S.ucnt[c] = P.cls_count[c];
   }
-  S.head = d->tune.t1_head_coop;
+  // the head always takes levels 0 and 1, so the tail starts at 2 or later
+  S.head = std::max(2, d->tune.t1_head_coop);
   return S;
 }
 
