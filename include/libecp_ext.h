@@ -105,7 +105,8 @@ int libecp_batch_execute(libecp_batch *b, int repeats, double *ms);
 int libecp_batch_fetch(libecp_batch *b);
 /* Adds molecule `mol`'s ECP matrix into the upper triangle of I (row stride
    rowdim), as getIntegrals does; returns 0, or 1 / 2 when a type-1 / type-2
-   integration of that molecule failed (blocks up to the failure added). */
+   integration of that molecule failed (blocks up to the failure added), or
+   -1 (libecp_last_error(); also when no results have been fetched). */
 int libecp_batch_matrix(libecp_batch *b, int mol, int rowdim, double *I);
 /* Contracts the last evaluation with one density per molecule on the
    device (see libecp_contract): molecule m's full symmetric nao_m x nao_m

@@ -695,7 +695,11 @@ int libecp_batch_matrix(libecp_batch *b, int mol, int rowdim, double *I) {
     set_last_error("the ECP matrix of a derivative batch is not defined (use libecp_batch_contract)");
     return -1;
   }
-  if (!b->blocks) return 0; /* nothing fetched */
+  if (b->job.ntrip == 0) return 0;
+  if (!b->blocks) {
+    set_last_error("no fetched results (call libecp_batch_fetch first)");
+    return -1;
+  }
   return ecp_job_scatter(&b->job, mol, b->aoff, b->blocks, b->status, rowdim, 0, I);
 }
 

@@ -1,0 +1,63 @@
+"""Host code around the kernels: contexts, graphs, results and error paths,
+with tests/c/host_runtime.c in the place of the HIP runtime (host memory,
+kernels that do nothing, calls that can be made to fail).  Every scenario
+below runs in a process of its own."""
+import ctypes as C
+import os
+import subprocess
+import sys
+
+import pytest
+
+from cases import CASES
+from libecp_amd import native
+from libecp_amd.workloads import plain_small
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+SCENARIOS = {}
+
+
+def scenario(f):
+    SCENARIOS[f.__name__] = f
+    return f
+
+
+def count(name):
+    rt = C.CDLL("libamdhip64.so.7")
+    rt.hrt_get.restype = C.c_long
+    return rt.hrt_get(name.encode())
+
+
+def make(name, value):
+    C.CDLL("libamdhip64.so.7").hrt_set(name.encode(), C.c_long(value))
+
+
+@scenario
+def matrix_before_a_fetch_is_an_error():
+    b = native.Batch([plain_small(0)])
+    assert b.matrix(0)[0] == -1 and "fetch" in native.last_error()
+    b.execute(1)
+    assert b.matrix(0)[0] == -1
+    b.fetch()
+    assert b.matrix(0)[0] == 0
+    b.close()
+    b = native.Batch([CASES["no_ecp"]()])  # nothing to fetch
+    assert b.triplets()[1] == 0 and b.matrix(0)[0] == 0
+    b.close()
+
+
+@pytest.fixture(scope="module")
+def runtime(tmp_path_factory):
+    d = tmp_path_factory.mktemp("runtime")
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-Wl,-soname,libamdhip64.so.7", "-o",
+                    str(d / "libamdhip64.so.7"), os.path.join(HERE, "c", "host_runtime.c")], check=True)
+    return str(d)
+
+
+@pytest.mark.parametrize("name", sorted(SCENARIOS))
+def test_scenario(runtime, name):
+    env = dict(os.environ, LD_LIBRARY_PATH=runtime + os.pathsep + os.environ.get("LD_LIBRARY_PATH", ""),
+               PYTHONPATH=os.pathsep.join([os.path.dirname(HERE), HERE]))
+    p = subprocess.run([sys.executable, "-c", f"import test_host_runtime as t; t.SCENARIOS['{name}']()"],
+                       env=env, capture_output=True, text=True, timeout=120)
+    assert p.returncode == 0, p.stderr[-3000:]
