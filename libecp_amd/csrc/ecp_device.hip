@@ -3204,6 +3204,25 @@ void enqueue(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
 }
 
 
+// Event i of the quadrature's pair, on stream s.  Under capture an event
+// record node of the graph, so that replays record it too: added to the graph
+// itself, since hipEventRecordWithFlags with hipEventRecordExternal is refused
+// by HIP 7.0 runtimes (one may be in the process before this library).
+hipError_t record_span(ecp_dev *d, hipStream_t s, int i) {
+  hipEvent_t ev = d->span[d->span_k][i];
+  if (!d->capturing) return hipEventRecord(ev, s);
+  hipStreamCaptureStatus st;
+  hipGraph_t g = nullptr;
+  const hipGraphNode_t *dep = nullptr;
+  size_t ndep = 0;
+  hipError_t e = hipStreamGetCaptureInfo_v2(s, &st, nullptr, &g, &dep, &ndep);
+  if (e != hipSuccess) return e;
+  if (st != hipStreamCaptureStatusActive) return hipErrorStreamCaptureInvalidated;
+  hipGraphNode_t node;
+  e = hipGraphAddEventRecordNode(&node, g, dep, ndep, ev);
+  return e != hipSuccess ? e : hipStreamUpdateCaptureDependencies(s, &node, 1, hipStreamSetCaptureDependencies);
+}
+
 // The fused sequence: tables on the main stream, then the two chains side by
 // side, each stage one launch over every class.  Type 1: head, then tail and
 // large-grid fallbacks, then assembly.  Type 2: small grid, fallbacks,
@@ -3227,8 +3246,7 @@ void enqueue_fused(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
   };
   const ClassMap cmh = class_map(ECP_MAX_LAB + 1, P.cls_count, [&](int c) { return (P.cls_count[c] + 63) / 64; });
   if (cmh.n > 0) {
-    // external event nodes when captured, so that replays record them too
-    (void)hipEventRecordWithFlags(d->span[d->span_k][0], w, d->capturing ? hipEventRecordExternal : 0);
+    d->span_valid = record_span(d, w, 0) == hipSuccess;
     {
       Span sp(d, w, FAM_TYPE1);
       launch(k_type1_fused<6>, k_type1_fused<8>, k_type1_fused<10>, k_type1_fused<12>, cmh);
@@ -3239,8 +3257,7 @@ void enqueue_fused(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
       Span sp(d, w, FAM_T1TAIL);
       launch(k_t1tail_fused<6>, k_t1tail_fused<8>, k_t1tail_fused<10>, k_t1tail_fused<12>, cmt);
     }
-    (void)hipEventRecordWithFlags(d->span[d->span_k][1], w, d->capturing ? hipEventRecordExternal : 0);
-    d->span_valid = true;
+    d->span_valid = record_span(d, w, 1) == hipSuccess && d->span_valid;
     launch_asm1(d, w, 0, P.nt);
   }
   // ---- type 2 ----
@@ -4033,8 +4050,8 @@ int con_launch(ecp_dev *d, const ecp_job *job, const ConImage &c, char *idx, con
   A.nd = job->deriv == 0 ? 1 : 3;
   A.nunits = c.nunits;
   A.nmol = job->nmol;
-  // a stale error of an earlier call (capturing the fused sequence leaves one)
-  // must not be taken for one of these launches
+  // a stale error of an earlier, unrelated call must not be taken for one of
+  // these launches
   (void)hipGetLastError();
   ECP_CHECK(hipEventRecord(d->con_ev[0], d->stream));
   if (Pp.nt > 0) {

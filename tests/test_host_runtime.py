@@ -46,6 +46,22 @@ def matrix_before_a_fetch_is_an_error():
     b.close()
 
 
+@scenario
+def quadrature_span_is_recorded_by_replays():
+    """Two kernels of 100 ticks each between the pair's events, in the eager
+    evaluation and in replays; no error is left behind where the runtime
+    refuses external event records."""
+    make("external_refused", 1)
+    b = native.Batch([plain_small(0)])
+    b.set_param("fuse", 1)
+    b.execute(1)
+    assert (b.quadrature_ms(), b.quadrature_samples) == (200.0, 1)
+    b.execute(12)
+    assert (b.quadrature_ms(), b.quadrature_samples) == (200.0, 8)
+    assert C.CDLL("libamdhip64.so.7").hipGetLastError() == 0
+    b.close()
+
+
 @pytest.fixture(scope="module")
 def runtime(tmp_path_factory):
     d = tmp_path_factory.mktemp("runtime")
