@@ -2520,6 +2520,7 @@ struct ecp_dev {
   int span_k = 0;
   bool span_valid = false;
   bool capturing = false;  // enqueue runs under stream capture
+  hipError_t seq_err = hipSuccess;  // first error of the sequence being enqueued (seq)
   bool last_eager = false;  // the last execute ran no replay
   long long replays = 0;    // replays since the graphs were captured
   int last_replays = 0;     // replays of the last execute
@@ -2564,6 +2565,11 @@ namespace {
 enum { FAM_TABLES = 0, FAM_TYPE1, FAM_TYPE2, FAM_FB1, FAM_FB2, FAM_ASM, FAM_T1TAIL, FAM_N };
 const char *kFamName[FAM_N] = {"tables", "type1", "type2", "fallback1", "fallback2", "assemble", "type1_tail"};
 
+// keeps the first error of the calls of a kernel sequence (run_sequence)
+void seq(ecp_dev *d, hipError_t e) {
+  if (d->seq_err == hipSuccess) d->seq_err = e;
+}
+
 // records an event pair around one launch on stream s when profiling
 struct Span {
   ecp_dev *d;
@@ -2572,19 +2578,19 @@ struct Span {
   Span(ecp_dev *d_, hipStream_t s_, int fam) : d(d_), s(s_), i(-1) {
     if (!d->profiling) return;
     if ((size_t)(2 * d->npev + 2) > d->pev.size()) {
-      hipEvent_t a, b;
-      (void)hipEventCreate(&a);
-      (void)hipEventCreate(&b);
+      hipEvent_t a = nullptr, b = nullptr;
+      seq(d, hipEventCreate(&a));
+      seq(d, hipEventCreate(&b));
       d->pev.push_back(a);
       d->pev.push_back(b);
       d->pfam.push_back(fam);
     }
     i = d->npev++;
     d->pfam[i] = fam;
-    (void)hipEventRecord(d->pev[2 * i], s);
+    seq(d, hipEventRecord(d->pev[2 * i], s));
   }
   ~Span() {
-    if (i >= 0) (void)hipEventRecord(d->pev[2 * i + 1], s);
+    if (i >= 0) seq(d, hipEventRecord(d->pev[2 * i + 1], s));
   }
 };
 }  // namespace
@@ -3121,10 +3127,10 @@ bool fuse_auto(int units, int max_lab) {
 void fork_tables(ecp_dev *d, hipStream_t s, int nw, hipEvent_t *evs) {
   const bool split = d->capturing && d->P.cls_begin[ECP_MAX_LAB + 1] <= kFuseAutoSmall;
   launch_tables(d, s, split ? kTabFront : kTabFront | kTabBack);
-  (void)hipEventRecord(d->fork, s);
-  for (int i = 0; i < nw; i++) (void)hipStreamWaitEvent(d->workers[i], d->fork, 0);
+  seq(d, hipEventRecord(d->fork, s));
+  for (int i = 0; i < nw; i++) seq(d, hipStreamWaitEvent(d->workers[i], d->fork, 0));
   if (split) launch_tables(d, s, kTabBack);
-  if (evs) (void)hipEventRecord(evs[1], s);
+  if (evs) seq(d, hipEventRecord(evs[1], s));
 }
 
 // one type-1 class of the per-class sequence: quadrature, assembly
@@ -3158,7 +3164,7 @@ void enqueue(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
   const DevJob &J = P.J;
   hipStream_t *w = d->workers;
   d->span_valid = false;  // type-1 classes run on several streams
-  if (evs) (void)hipEventRecord(evs[0], s);
+  if (evs) seq(d, hipEventRecord(evs[0], s));
   fork_tables(d, s, kWorkers, evs);
   // the type-2 chain (small grid, fallbacks, assembly) on the main stream,
   // beside it the type-1 classes on three workers: one stream per hardware
@@ -3194,12 +3200,12 @@ void enqueue(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
     enqueue_t1_class(d, w[k], order[i]);
   }
   for (int i = 0; i < kWorkers; i++) {
-    (void)hipEventRecord(d->join[i], w[i]);
-    (void)hipStreamWaitEvent(s, d->join[i], 0);
+    seq(d, hipEventRecord(d->join[i], w[i]));
+    seq(d, hipStreamWaitEvent(s, d->join[i], 0));
   }
   if (evs) {
-    (void)hipEventRecord(evs[2], s);
-    (void)hipEventRecord(evs[3], s);
+    seq(d, hipEventRecord(evs[2], s));
+    seq(d, hipEventRecord(evs[3], s));
   }
 }
 
@@ -3233,7 +3239,7 @@ void enqueue_fused(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
   const DevJob &J = P.J;
   hipStream_t w = d->workers[0];
   d->span_valid = false;
-  if (evs) (void)hipEventRecord(evs[0], s);
+  if (evs) seq(d, hipEventRecord(evs[0], s));
   fork_tables(d, s, 1, evs);
   // ---- type 1 ----
   const T1Set S = t1_set(d);
@@ -3246,7 +3252,7 @@ void enqueue_fused(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
   };
   const ClassMap cmh = class_map(ECP_MAX_LAB + 1, P.cls_count, [&](int c) { return (P.cls_count[c] + 63) / 64; });
   if (cmh.n > 0) {
-    d->span_valid = record_span(d, w, 0) == hipSuccess;
+    seq(d, record_span(d, w, 0));
     {
       Span sp(d, w, FAM_TYPE1);
       launch(k_type1_fused<6>, k_type1_fused<8>, k_type1_fused<10>, k_type1_fused<12>, cmh);
@@ -3257,7 +3263,8 @@ void enqueue_fused(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
       Span sp(d, w, FAM_T1TAIL);
       launch(k_t1tail_fused<6>, k_t1tail_fused<8>, k_t1tail_fused<10>, k_t1tail_fused<12>, cmt);
     }
-    d->span_valid = record_span(d, w, 1) == hipSuccess && d->span_valid;
+    seq(d, record_span(d, w, 1));
+    d->span_valid = true;
     launch_asm1(d, w, 0, P.nt);
   }
   // ---- type 2 ----
@@ -3272,12 +3279,28 @@ void enqueue_fused(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
     }
     launch_asm2(d, s);
   }
-  (void)hipEventRecord(d->join[0], w);
-  (void)hipStreamWaitEvent(s, d->join[0], 0);
+  seq(d, hipEventRecord(d->join[0], w));
+  seq(d, hipStreamWaitEvent(s, d->join[0], 0));
   if (evs) {
-    (void)hipEventRecord(evs[2], s);
-    (void)hipEventRecord(evs[3], s);
+    seq(d, hipEventRecord(evs[2], s));
+    seq(d, hipEventRecord(evs[3], s));
   }
+}
+
+// enqueue, with every call's and launch's error looked at: under capture a
+// launch that failed would be missing from every replay.  0, or -1 (message
+// in err) with nothing of the sequence left running.
+int run_sequence(ecp_dev *d, hipStream_t s, hipEvent_t *evs, char *err, size_t errlen) {
+  // a stale error of an earlier, unrelated call must not be taken for one of
+  // this sequence's
+  (void)hipGetLastError();
+  d->seq_err = hipSuccess;
+  enqueue(d, s, evs);
+  seq(d, hipGetLastError());
+  if (d->seq_err == hipSuccess) return 0;
+  snprintf(err, errlen, "kernel sequence failed: %s", hipGetErrorString(d->seq_err));
+  if (!d->capturing) (void)ecp_dev_sync(d);
+  return -1;
 }
 
 }  // namespace
@@ -3648,13 +3671,9 @@ extern "C" int ecp_dev_execute(ecp_dev *d, int repeats, double *ms_total, char *
   double total = 0.0;
   d->last_eager = false;
   if (!d->eager_done) {
-    // a stale error of an earlier, unrelated call must not be taken for one
-    // of this enqueue's launches
-    (void)hipGetLastError();
     d->span_k = 0;
     d->last_eager = true;
-    enqueue(d, s, d->ev);
-    ECP_CHECK(hipGetLastError());
+    if (run_sequence(d, s, d->ev, err, errlen)) return -1;
     ECP_CHECK(hipStreamSynchronize(s));
     for (int i = 1; i < 4; i++) {
       float ms = 0.f;
@@ -3678,9 +3697,17 @@ extern "C" int ecp_dev_execute(ecp_dev *d, int repeats, double *ms_total, char *
       ECP_CHECK(hipStreamSynchronize(s));
       ECP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
       d->capturing = true;
-      enqueue(d, s, nullptr);
+      const int rc = run_sequence(d, s, nullptr, err, errlen);
       d->capturing = false;
-      ECP_CHECK(hipStreamEndCapture(s, &d->graph[k]));
+      const hipError_t ec = hipStreamEndCapture(s, &d->graph[k]);
+      if (rc) {
+        // (the capture may have been invalidated: no graph then)
+        (void)hipGetLastError();
+        if (ec == hipSuccess && d->graph[k]) (void)hipGraphDestroy(d->graph[k]);
+        d->graph[k] = nullptr;
+        return -1;
+      }
+      ECP_CHECK(ec);
       ECP_CHECK(hipGraphInstantiate(&d->gexec[k], d->graph[k], nullptr, nullptr, 0));
       d->ngraph = k + 1;
       if (!d->span_valid) break;
@@ -3767,10 +3794,9 @@ extern "C" int ecp_dev_profile(ecp_dev *d, const ecp_job *job, int *launches, do
   d->npev = 0;
   d->span_k = 0;
   d->last_eager = true;
-  (void)hipGetLastError();
-  enqueue(d, d->stream, nullptr);
+  const int rc = run_sequence(d, d->stream, nullptr, err, errlen);
   d->profiling = false;
-  ECP_CHECK(hipGetLastError());
+  if (rc) return -1;
   ECP_CHECK(hipStreamSynchronize(d->stream));
   for (int i = 0; i < d->npev; i++) {
     float t = 0.f;

@@ -62,6 +62,37 @@ def quadrature_span_is_recorded_by_replays():
     b.close()
 
 
+def fails(f, *args):
+    try:
+        f(*args)
+    except RuntimeError:
+        return True
+    return False
+
+
+@scenario
+def failed_calls_of_a_sequence_are_reported():
+    """A launch that fails under capture, and a wait between streams."""
+    for fuse in (0, 1):
+        b = native.Batch([plain_small(0)])
+        b.set_param("fuse", fuse)
+        b.execute(1)
+        make("launch_fail", 1)
+        assert fails(b.execute, 2)
+        make("launch_fail", 0)
+        assert b.execute(2) > 0
+        b.close()
+        assert count("graphs") == count("execs") == 0
+        make("wait_fail", 1)
+        b = native.Batch([plain_small(0)])
+        b.set_param("fuse", fuse)
+        assert fails(b.execute, 1)
+        assert fails(b.profile)
+        make("wait_fail", 0)
+        assert b.execute(1) > 0
+        b.close()
+
+
 @pytest.fixture(scope="module")
 def runtime(tmp_path_factory):
     d = tmp_path_factory.mktemp("runtime")
