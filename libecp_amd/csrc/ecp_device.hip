@@ -3699,16 +3699,17 @@ extern "C" int ecp_dev_execute(ecp_dev *d, int repeats, double *ms_total, char *
       d->capturing = true;
       const int rc = run_sequence(d, s, nullptr, err, errlen);
       d->capturing = false;
-      const hipError_t ec = hipStreamEndCapture(s, &d->graph[k]);
-      if (rc) {
-        // (the capture may have been invalidated: no graph then)
+      hipError_t ec = hipStreamEndCapture(s, &d->graph[k]);
+      if (!rc && ec == hipSuccess) ec = hipGraphInstantiate(&d->gexec[k], d->graph[k], nullptr, nullptr, 0);
+      if (rc || ec != hipSuccess) {
+        // copy k does not exist (an invalidated capture gives no graph)
         (void)hipGetLastError();
-        if (ec == hipSuccess && d->graph[k]) (void)hipGraphDestroy(d->graph[k]);
+        if (d->graph[k]) (void)hipGraphDestroy(d->graph[k]);
         d->graph[k] = nullptr;
+        d->gexec[k] = nullptr;
+        if (!rc) snprintf(err, errlen, "capturing the kernel sequence failed: %s", hipGetErrorString(ec));
         return -1;
       }
-      ECP_CHECK(ec);
-      ECP_CHECK(hipGraphInstantiate(&d->gexec[k], d->graph[k], nullptr, nullptr, 0));
       d->ngraph = k + 1;
       if (!d->span_valid) break;
     }

@@ -93,6 +93,18 @@ def failed_calls_of_a_sequence_are_reported():
         b.close()
 
 
+@scenario
+def graphs_of_a_failed_capture_are_freed():
+    for copy in (1, 3):
+        b = native.Batch([plain_small(0)])
+        b.set_param("fuse", 1)
+        make("instantiate_fail", copy)
+        assert fails(b.execute, 2)
+        assert b.execute(2) > 0
+        b.close()
+        assert count("graphs") == count("execs") == 0
+
+
 @pytest.fixture(scope="module")
 def runtime(tmp_path_factory):
     d = tmp_path_factory.mktemp("runtime")
