@@ -119,10 +119,16 @@ static ecp_dev *cache_take(cache_slot *c, int device) {
   return d;
 }
 
-/* keeps an idle context for the next handle of the same key, or frees it;
-   limit: the bytes all idle contexts may then hold (0: any) */
-static void cache_give(cache_slot *c, ecp_dev *d, int device, size_t limit) {
+/* keeps an idle context for the next handle of the same key, or frees it, as
+   always after a failed device call (work of its job may still be queued, and
+   what failed may fail again); limit: the bytes all idle contexts may then
+   hold (0: any) */
+static void cache_give(cache_slot *c, ecp_dev *d, int device, int failed, size_t limit) {
   if (!d) return;
+  if (failed) {
+    ecp_dev_destroy(d);
+    return;
+  }
   size_t held = ecp_dev_held(d);
   pthread_mutex_lock(&g_cache_mu);
   for (int i = 0; i < kCacheKeys; i++)
@@ -139,17 +145,14 @@ static void cache_give(cache_slot *c, ecp_dev *d, int device, size_t limit) {
 
 /* A batch's context, with the workspaces of its job: kept like a handle's
    where all idle contexts together hold no more than kCacheBytes, and never
-   after a device error.  (48 new molecules, with allocations and the pages
+   after a failed call or an error on its streams.  (48 new molecules, with allocations and the pages
    behind them against without: created in 11.7 and 4.8 ms, matrices read in
    15 and 3.6 ms, freed in 1.9 and 0.1 ms.) */
-static void cache_give_batch(cache_slot *c, ecp_dev *d, int device) {
+static void cache_give_batch(cache_slot *c, ecp_dev *d, int device, int failed) {
   if (!d) return;
-  if (ecp_dev_sync(d)) {
-    ecp_dev_destroy(d);
-    return;
-  }
-  ecp_dev_renew(d);
-  cache_give(c, d, device, kCacheBytes);
+  if (ecp_dev_sync(d)) failed = 1;
+  if (!failed) ecp_dev_renew(d);
+  cache_give(c, d, device, failed, kCacheBytes);
 }
 
 void libecp_cache_clear(void) {
@@ -188,6 +191,7 @@ struct _libECPHandle {
   cache_slot *slot;     /* non-NULL: tables and context come from the cache */
   int dev_id;           /* HIP device of dev */
   ecp_dev *dev;
+  int dev_failed;       /* a call on dev failed */
   ecp_job job;
   int job_ready;
   double *blocks;       /* the fetched results, in the device context's pinned memory */
@@ -204,7 +208,7 @@ void libECP_free(libECPHandle *h) {
   if (!h) return;
   if (h->job_ready) ecp_job_free(&h->job);
   if (h->slot)
-    cache_give(h->slot, h->dev, h->dev_id, 0);
+    cache_give(h->slot, h->dev, h->dev_id, h->dev_failed, 0);
   else
     ecp_dev_destroy(h->dev);
   ecp_static_free(&h->st_own);
@@ -307,6 +311,13 @@ static int ensure_device(libECPHandle *h) {
   return 0;
 }
 
+/* -1 for a failed call on a device context */
+static int dev_error(int *failed, const char *err) {
+  set_last_error(err);
+  *failed = 1;
+  return -1;
+}
+
 /* Evaluates every triplet of the handle's molecule on the device and points
    h->blocks / h->status at the results; returns 0, or -1 on a device/host error. */
 static int run_handle(libECPHandle *h) {
@@ -330,22 +341,13 @@ static int run_handle(libECPHandle *h) {
   g_phase[PH_CONTEXT] = t - t1;
   /* prepare (host work lists, layout; the upload is queued) / execute
      (upload, kernels, waits) / fetch (download, waits) */
-  if (ecp_dev_prepare(h->dev, &h->job, err, sizeof(err))) {
-    set_last_error(err);
-    return -1;
-  }
+  if (ecp_dev_prepare(h->dev, &h->job, err, sizeof(err))) return dev_error(&h->dev_failed, err);
   t1 = now_ms();
   g_phase[PH_UPLOAD] = t1 - t;
-  if (ecp_dev_execute(h->dev, 1, NULL, err, sizeof(err))) {
-    set_last_error(err);
-    return -1;
-  }
+  if (ecp_dev_execute(h->dev, 1, NULL, err, sizeof(err))) return dev_error(&h->dev_failed, err);
   t = now_ms();
   g_phase[PH_KERNELS] = t - t1;
-  if (ecp_dev_fetch(h->dev, &h->blocks, &h->status, err, sizeof(err))) {
-    set_last_error(err);
-    return -1;
-  }
+  if (ecp_dev_fetch(h->dev, &h->blocks, &h->status, err, sizeof(err))) return dev_error(&h->dev_failed, err);
   g_phase[PH_DOWNLOAD] = now_ms() - t;
   return 0;
 }
@@ -456,10 +458,8 @@ int libecp_contract(libECPHandle *h, int rowdim, const double *P, double *out) {
   int code = 0;
   if (ecp_dev_prepare(h->dev, &h->job, err, sizeof(err)) ||
       ecp_dev_execute(h->dev, 1, NULL, err, sizeof(err)) ||
-      ecp_dev_contract(h->dev, &h->job, P, nP, 0, &poff, &prow, out, 0, &code, NULL, err, sizeof(err))) {
-    set_last_error(err);
-    return -1;
-  }
+      ecp_dev_contract(h->dev, &h->job, P, nP, 0, &poff, &prow, out, 0, &code, NULL, err, sizeof(err)))
+    return dev_error(&h->dev_failed, err);
   return code;
 }
 
@@ -538,6 +538,7 @@ struct libecp_batch {
   cache_slot *slot;     /* non-NULL: tables and context come from the cache */
   ecp_dev *dev;
   int dev_id;
+  int dev_failed;       /* a call on dev failed */
   ecp_job job;
   int *aoff;
   double *blocks;       /* the fetched results, in the device context's pinned memory */
@@ -550,7 +551,7 @@ struct libecp_batch {
 void libecp_batch_free(libecp_batch *b) {
   if (!b) return;
   if (b->slot)
-    cache_give_batch(b->slot, b->dev, b->dev_id);
+    cache_give_batch(b->slot, b->dev, b->dev_id, b->dev_failed);
   else
     ecp_dev_destroy(b->dev);
   ecp_job_free(&b->job);
@@ -662,7 +663,7 @@ libecp_batch *libecp_batch_create_n(const libecp_molecule *mols, int nmol, int n
   if (!b->dev) b->dev = ecp_dev_create(b->st, err, sizeof(err));
   if (!b->dev || ecp_dev_prepare(b->dev, &b->job, err, sizeof(err)) || ecp_dev_clear(b->dev, err, sizeof(err)) ||
       ecp_dev_sync(b->dev)) {
-    set_last_error(err[0] ? err : "device error after the upload");
+    dev_error(&b->dev_failed, err[0] ? err : "device error after the upload");
     libecp_batch_free(b);
     return NULL;
   }
@@ -672,20 +673,14 @@ libecp_batch *libecp_batch_create_n(const libecp_molecule *mols, int nmol, int n
 int libecp_batch_execute(libecp_batch *b, int repeats, double *ms) {
   char err[512] = "";
   if (!b) return -1;
-  if (ecp_dev_execute(b->dev, repeats, ms, err, sizeof(err))) {
-    set_last_error(err);
-    return -1;
-  }
+  if (ecp_dev_execute(b->dev, repeats, ms, err, sizeof(err))) return dev_error(&b->dev_failed, err);
   return 0;
 }
 
 int libecp_batch_fetch(libecp_batch *b) {
   char err[512] = "";
   if (!b) return -1;
-  if (ecp_dev_fetch(b->dev, &b->blocks, &b->status, err, sizeof(err))) {
-    set_last_error(err);
-    return -1;
-  }
+  if (ecp_dev_fetch(b->dev, &b->blocks, &b->status, err, sizeof(err))) return dev_error(&b->dev_failed, err);
   return 0;
 }
 
@@ -713,11 +708,8 @@ int libecp_batch_contract_noalloc(libecp_batch *b, const double *P, double *out,
     set_last_error("density contraction supports derivative orders 0 and 1");
     return -1;
   }
-  if (ecp_dev_contract_noalloc(b->dev, &b->job, b->con_img, b->con_img_bytes, P, out, codes, ms, err,
-                               sizeof(err))) {
-    set_last_error(err);
-    return -1;
-  }
+  if (ecp_dev_contract_noalloc(b->dev, &b->job, b->con_img, b->con_img_bytes, P, out, codes, ms, err, sizeof(err)))
+    return dev_error(&b->dev_failed, err);
   return 0;
 }
 
@@ -748,10 +740,8 @@ int libecp_batch_contract(libecp_batch *b, const double *P, double *out, int *co
     nP += (size_t)b->nao[m] * b->nao[m];
   }
   int rc = 0;
-  if (ecp_dev_contract(b->dev, &b->job, P, nP, device, poff, prow, out, device, cd, ms, err, sizeof(err))) {
-    set_last_error(err);
-    rc = -1;
-  }
+  if (ecp_dev_contract(b->dev, &b->job, P, nP, device, poff, prow, out, device, cd, ms, err, sizeof(err)))
+    rc = dev_error(&b->dev_failed, err);
   free(poff);
   free(prow);
   if (!codes) free(cd);
@@ -787,10 +777,7 @@ int libecp_batch_profile(libecp_batch *b, int *launches, double *ms, double *flo
   double m[16], f[16];
   if (!b) return -1;
   int k = ecp_dev_profile(b->dev, &b->job, l, m, f, err, sizeof(err));
-  if (k < 0) {
-    set_last_error(err);
-    return -1;
-  }
+  if (k < 0) return dev_error(&b->dev_failed, err);
   for (int i = 0; i < k && i < n; i++) {
     launches[i] = l[i];
     ms[i] = m[i];
@@ -863,10 +850,7 @@ int libecp_batch_autotune(libecp_batch *b, int repeats, char *report, int len) {
   ecp_tuning best;
   ecp_dev_get_tuning(b->dev, &best);
   double tbest = time_tuning(b, &best, repeats, err, sizeof(err));
-  if (tbest < 0) {
-    set_last_error(err);
-    return -1;
-  }
+  if (tbest < 0) return dev_error(&b->dev_failed, err);
   size_t used = 0;
   if (report && len > 0) {
     report[0] = 0;
@@ -891,9 +875,8 @@ int libecp_batch_autotune(libecp_batch *b, int repeats, char *report, int len) {
       *f = space[k].v[i];
       const double ms = time_tuning(b, &t, repeats, err, sizeof(err));
       if (ms < 0) {
-        set_last_error(err);
         ecp_dev_set_tuning(b->dev, &best);
-        return -1;
+        return dev_error(&b->dev_failed, err);
       }
       if (report && used < (size_t)len)
         used += (size_t)snprintf(report + used, (size_t)len - used, "; %s=%d %.4f ms", space[k].name,

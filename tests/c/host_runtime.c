@@ -1,5 +1,5 @@
 /* The part of the HIP runtime's interface that the library's host code calls,
-   on host memory: allocations are malloc'ed, copies are memcpy, kernels do
+   on host memory: allocations are zeroed, copies are memcpy, kernels do
    nothing but advance a clock.  Tests of the host code (contexts, graphs,
    error paths) load it in place of libamdhip64.so.7; hrt_set makes calls
    fail, hrt_get counts what is alive. */
@@ -167,7 +167,7 @@ int hipLaunchKernel(const void *f, dim3_t g, dim3_t b, void **args, size_t shm, 
 /* ---- memory: the size in front of every block ---- */
 int hipMalloc(void **p, size_t n) {
   if (v_mem_limit && v_device_bytes + (long)n > v_mem_limit) return fail(NO_MEMORY);
-  size_t *q = malloc(n + 4096);
+  size_t *q = calloc(1, n + 4096);
   if (!q) return fail(NO_MEMORY);
   *q = n;
   v_device_bytes += (long)n;

@@ -7,6 +7,7 @@ import os
 import subprocess
 import sys
 
+import numpy as np
 import pytest
 
 from cases import CASES
@@ -103,6 +104,38 @@ def graphs_of_a_failed_capture_are_freed():
         assert b.execute(2) > 0
         b.close()
         assert count("graphs") == count("execs") == 0
+
+
+@scenario
+def contexts_are_not_reused_after_a_failed_call():
+    m = plain_small(0)
+    P = np.eye(m.nao)
+
+    def batch():
+        b = native.Batch([m])
+        try:
+            b.execute(1)
+        finally:
+            b.close()
+
+    def handle():
+        h = native.Handle(m)
+        try:
+            assert h.contract(P)[0] == 0
+        finally:
+            h.close()
+
+    for use in (batch, handle):
+        use()
+        n = count("contexts")
+        use()
+        assert count("contexts") == n      # taken from the cache
+        make("launch_fail", 2)
+        assert fails(use)                  # the same one, which is freed
+        make("launch_fail", 0)
+        assert count("contexts") == n
+        use()
+        assert count("contexts") == n + 1
 
 
 @pytest.fixture(scope="module")
