@@ -45,17 +45,19 @@ double libecp_model_fallback_flops(int type, int la, int lb, int l, int ng_l, in
    matrix accumulation or callbacks.  Returns the number of phases (7). */
 int libecp_last_call_ms(double *ms, int n);
 
-/* Process-wide cache.  Handles with the default Cartesian ordering share
-   the geometry-independent tables of their key (largest ECP label, largest
-   basis l + n, grid order, tolerance, accuracy; at most 8 keys) and reuse
-   device contexts (streams, pinned staging, tables resident in HBM; at most
-   2 idle per key and device): libECP_free returns the context to the cache
-   instead of destroying it, and the next handle of the key takes it, so
-   repeated getIntegrals calls pay for neither.  Idle contexts keep their
-   device and pinned memory until libecp_cache_clear() (which frees them) or
-   the end of the process.  libecp_cache_enable(0) clears the cache and
-   disables it (every handle then builds and frees its own); returns the
-   previous setting. */
+/* Process-wide cache.  Handles with the default Cartesian ordering, and
+   batches, share the geometry-independent tables of their key (largest ECP
+   label, largest basis l + n, grid order, tolerance, accuracy; at most 8 keys)
+   and reuse device contexts (streams, pinned staging, tables resident in HBM,
+   the device memory of their jobs; at most 2 idle per key): libECP_free and
+   libecp_batch_free return the context to the cache instead of destroying it,
+   and the next handle or batch of the key takes it, so repeated calls pay for
+   neither.  A context that a batch has had stays only while all idle contexts
+   hold at most 4 GiB of device and pinned memory together; one with a failed
+   call is destroyed.  Idle contexts keep their memory until
+   libecp_cache_clear() (which frees them) or the end of the process.
+   libecp_cache_enable(0) clears the cache and disables it (every handle and
+   batch then builds and frees its own); returns the previous setting. */
 void libecp_cache_clear(void);
 int libecp_cache_enable(int on);
 

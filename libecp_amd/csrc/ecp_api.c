@@ -60,6 +60,7 @@ typedef struct {
   ecp_static st; /* read-only once built */
   ecp_dev *idle[kCacheIdle];
   int idle_dev[kCacheIdle];
+  int idle_batch[kCacheIdle]; /* a batch has had the context */
   int nidle;
 } cache_slot;
 
@@ -104,26 +105,30 @@ static cache_slot *cache_tables(int maxL, int maxAlpha, int grid, double tol, do
   return hit;
 }
 
-static ecp_dev *cache_take(cache_slot *c, int device) {
+/* an idle context, or NULL; *batch: a batch has had it */
+static ecp_dev *cache_take(cache_slot *c, int device, int *batch) {
   ecp_dev *d = NULL;
   pthread_mutex_lock(&g_cache_mu);
   for (int i = c->nidle - 1; i >= 0; i--)
     if (c->idle_dev[i] == device) {
       d = c->idle[i];
-      c->idle[i] = c->idle[c->nidle - 1];
-      c->idle_dev[i] = c->idle_dev[c->nidle - 1];
+      *batch = c->idle_batch[i];
       c->nidle--;
+      c->idle[i] = c->idle[c->nidle];
+      c->idle_dev[i] = c->idle_dev[c->nidle];
+      c->idle_batch[i] = c->idle_batch[c->nidle];
       break;
     }
   pthread_mutex_unlock(&g_cache_mu);
   return d;
 }
 
-/* keeps an idle context for the next handle of the same key, or frees it, as
-   always after a failed device call (work of its job may still be queued, and
-   what failed may fail again); limit: the bytes all idle contexts may then
-   hold (0: any) */
-static void cache_give(cache_slot *c, ecp_dev *d, int device, int failed, size_t limit) {
+/* Keeps an idle context for the next handle or batch of the same key, or
+   frees it, as always after a failed device call (work of its job may still be
+   queued, and what failed may fail again).  A context that a batch has had,
+   whoever gives it back, is kept only where all idle contexts together hold no
+   more than kCacheBytes; those of handles alone keep what they need. */
+static void cache_give(cache_slot *c, ecp_dev *d, int device, int failed, int batch) {
   if (!d) return;
   if (failed) {
     ecp_dev_destroy(d);
@@ -133,9 +138,10 @@ static void cache_give(cache_slot *c, ecp_dev *d, int device, int failed, size_t
   pthread_mutex_lock(&g_cache_mu);
   for (int i = 0; i < kCacheKeys; i++)
     for (int k = 0; k < g_cache[i].nidle; k++) held += ecp_dev_held(g_cache[i].idle[k]);
-  if (g_cache_on && c->nidle < kCacheIdle && (!limit || held <= limit)) {
+  if (g_cache_on && c->nidle < kCacheIdle && (!batch || held <= kCacheBytes)) {
     c->idle[c->nidle] = d;
     c->idle_dev[c->nidle] = device;
+    c->idle_batch[c->nidle] = batch;
     c->nidle++;
     d = NULL;
   }
@@ -143,16 +149,16 @@ static void cache_give(cache_slot *c, ecp_dev *d, int device, int failed, size_t
   ecp_dev_destroy(d);
 }
 
-/* A batch's context, with the workspaces of its job: kept like a handle's
-   where all idle contexts together hold no more than kCacheBytes, and never
-   after a failed call or an error on its streams.  (48 new molecules, with allocations and the pages
-   behind them against without: created in 11.7 and 4.8 ms, matrices read in
-   15 and 3.6 ms, freed in 1.9 and 0.1 ms.) */
+/* A batch's context, with the workspaces of its job, renewed for the next
+   user; never after a failed call or an error on its streams.  (48 new
+   molecules, with allocations and the pages behind them against without:
+   created in 11.7 and 4.8 ms, matrices read in 15 and 3.6 ms, freed in 1.9
+   and 0.1 ms.) */
 static void cache_give_batch(cache_slot *c, ecp_dev *d, int device, int failed) {
   if (!d) return;
   if (ecp_dev_sync(d)) failed = 1;
   if (!failed) ecp_dev_renew(d);
-  cache_give(c, d, device, failed, kCacheBytes);
+  cache_give(c, d, device, failed, 1);
 }
 
 void libecp_cache_clear(void) {
@@ -192,6 +198,7 @@ struct _libECPHandle {
   int dev_id;           /* HIP device of dev */
   ecp_dev *dev;
   int dev_failed;       /* a call on dev failed */
+  int dev_batch;        /* a batch has had dev */
   ecp_job job;
   int job_ready;
   double *blocks;       /* the fetched results, in the device context's pinned memory */
@@ -208,7 +215,7 @@ void libECP_free(libECPHandle *h) {
   if (!h) return;
   if (h->job_ready) ecp_job_free(&h->job);
   if (h->slot)
-    cache_give(h->slot, h->dev, h->dev_id, h->dev_failed, 0);
+    cache_give(h->slot, h->dev, h->dev_id, h->dev_failed, h->dev_batch);
   else
     ecp_dev_destroy(h->dev);
   ecp_static_free(&h->st_own);
@@ -302,7 +309,7 @@ static int ensure_device(libECPHandle *h) {
   char err[512] = "";
   if (h->dev) return 0;
   h->dev_id = ecp_dev_current();
-  if (h->slot) h->dev = cache_take(h->slot, h->dev_id);
+  if (h->slot) h->dev = cache_take(h->slot, h->dev_id, &h->dev_batch);
   if (!h->dev) h->dev = ecp_dev_create(h->st, err, sizeof(err));
   if (!h->dev) {
     set_last_error(err);
@@ -659,7 +666,8 @@ libecp_batch *libecp_batch_create_n(const libecp_molecule *mols, int nmol, int n
     }
   }
   b->dev_id = ecp_dev_current();
-  if (b->slot) b->dev = cache_take(b->slot, b->dev_id);
+  int batch;
+  if (b->slot) b->dev = cache_take(b->slot, b->dev_id, &batch);
   if (!b->dev) b->dev = ecp_dev_create(b->st, err, sizeof(err));
   if (!b->dev || ecp_dev_prepare(b->dev, &b->job, err, sizeof(err)) || ecp_dev_clear(b->dev, err, sizeof(err)) ||
       ecp_dev_sync(b->dev)) {

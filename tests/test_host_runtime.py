@@ -12,7 +12,7 @@ import pytest
 
 from cases import CASES
 from libecp_amd import native
-from libecp_amd.workloads import plain_small
+from libecp_amd.workloads import plain_small, uneven_batch
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 SCENARIOS = {}
@@ -136,6 +136,27 @@ def contexts_are_not_reused_after_a_failed_call():
         assert count("contexts") == n
         use()
         assert count("contexts") == n + 1
+
+
+@scenario
+def idle_contexts_of_batches_stay_below_4_gib():
+    """Also one that a handle took and gives back after another batch's came."""
+    mols = uneven_batch(0)[:90]
+    big = max(mols, key=lambda m: m.nao)
+
+    def batch():
+        b = native.Batch(mols)
+        b.close()
+
+    batch()
+    one, contexts = count("device_bytes"), count("contexts")
+    assert 2 << 30 < one < 4 << 30
+    h = native.Handle(big)
+    h.contract(np.eye(big.nao))
+    assert count("contexts") == contexts   # the batch's
+    batch()
+    h.close()
+    assert count("device_bytes") < 4 << 30
 
 
 @pytest.fixture(scope="module")
