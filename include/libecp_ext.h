@@ -47,10 +47,10 @@ int libecp_last_call_ms(double *ms, int n);
 
 /* Process-wide cache.  Handles with the default Cartesian ordering, and
    batches, share the geometry-independent tables of their key (largest ECP
-   label, largest basis l + n, grid order, tolerance, accuracy; at most 8 keys)
-   and reuse device contexts (streams, pinned staging, tables resident in HBM,
-   the device memory of their jobs; at most 2 idle per key): libECP_free and
-   libecp_batch_free return the context to the cache instead of destroying it,
+   label, largest basis l + n, grid order, tolerance, accuracy; at most 8 keys
+   that handles bring and 8 that batches bring) and reuse device contexts
+   (streams, pinned staging, tables resident in HBM, the device memory of their
+   jobs; at most 2 idle per key): libECP_free and libecp_batch_free return the context to the cache instead of destroying it,
    and the next handle or batch of the key takes it, so repeated calls pay for
    neither.  A context that a batch has had stays only while all idle contexts
    hold at most 4 GiB of device and pinned memory together; one with a failed

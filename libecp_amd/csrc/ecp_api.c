@@ -48,13 +48,15 @@ int libecp_last_call_ms(double *ms, int n) {
    tolerance, accuracy) and the default Cartesian ordering, so they are kept
    per process: the tables once per key, and up to kCacheIdle idle contexts
    per key and device, which a handle takes at its first calculation and
-   returns when it is freed.  Batches use both in the same way.  Handles with
-   a custom ordering, and every handle and batch while the cache is disabled,
-   own their tables and context. */
-enum { kCacheKeys = 8, kCacheIdle = 2 };
+   returns when it is freed.  Batches use both in the same way, with room for
+   as many keys of their own, so that they take none from the handles.  Handles
+   with a custom ordering, and every handle and batch while the cache is
+   disabled or has no room for the key, own their tables and context. */
+enum { kCacheKeys = 8, kCacheSlots = 2 * kCacheKeys, kCacheIdle = 2 };
 static const size_t kCacheBytes = (size_t)4 << 30;
 typedef struct {
   int used;
+  int batch;     /* the key came with a batch */
   int maxL, maxAlpha, grid;
   double tol, acc;
   ecp_static st; /* read-only once built */
@@ -65,33 +67,36 @@ typedef struct {
 } cache_slot;
 
 static pthread_mutex_t g_cache_mu = PTHREAD_MUTEX_INITIALIZER;
-static cache_slot g_cache[kCacheKeys];
+static cache_slot g_cache[kCacheSlots];
 static int g_cache_on = 1;
 
 /* the slot of a key, built on first use; NULL when the cache is off or full
    (the caller then builds its own tables) */
-static cache_slot *cache_tables(int maxL, int maxAlpha, int grid, double tol, double acc, char *err,
+static cache_slot *cache_tables(int batch, int maxL, int maxAlpha, int grid, double tol, double acc, char *err,
                                 size_t errlen, int *failed) {
   *failed = 0;
   pthread_mutex_lock(&g_cache_mu);
   cache_slot *hit = NULL, *fresh = NULL;
+  int keys = 0; /* that came with a batch, or with a handle */
   if (g_cache_on)
-    for (int i = 0; i < kCacheKeys; i++) {
+    for (int i = 0; i < kCacheSlots; i++) {
       cache_slot *c = &g_cache[i];
       if (!c->used) {
         if (!fresh) fresh = c;
         continue;
       }
+      keys += c->batch == batch;
       if (c->maxL == maxL && c->maxAlpha == maxAlpha && c->grid == grid && c->tol == tol && c->acc == acc) {
         hit = c;
         break;
       }
     }
-  if (!hit && fresh) {
+  if (!hit && fresh && keys < kCacheKeys) {
     if (ecp_static_init(&fresh->st, maxL, maxAlpha, NULL, -1, grid, tol, acc, err, errlen)) {
       *failed = 1;
     } else {
       fresh->used = 1;
+      fresh->batch = batch;
       fresh->maxL = maxL;
       fresh->maxAlpha = maxAlpha;
       fresh->grid = grid;
@@ -136,7 +141,7 @@ static void cache_give(cache_slot *c, ecp_dev *d, int device, int failed, int ba
   }
   size_t held = ecp_dev_held(d);
   pthread_mutex_lock(&g_cache_mu);
-  for (int i = 0; i < kCacheKeys; i++)
+  for (int i = 0; i < kCacheSlots; i++)
     for (int k = 0; k < g_cache[i].nidle; k++) held += ecp_dev_held(g_cache[i].idle[k]);
   if (g_cache_on && c->nidle < kCacheIdle && (!batch || held <= kCacheBytes)) {
     c->idle[c->nidle] = d;
@@ -162,10 +167,10 @@ static void cache_give_batch(cache_slot *c, ecp_dev *d, int device, int failed) 
 }
 
 void libecp_cache_clear(void) {
-  ecp_dev *drop[kCacheKeys * kCacheIdle];
+  ecp_dev *drop[kCacheSlots * kCacheIdle];
   int nd = 0;
   pthread_mutex_lock(&g_cache_mu);
-  for (int i = 0; i < kCacheKeys; i++) {
+  for (int i = 0; i < kCacheSlots; i++) {
     for (int k = 0; k < g_cache[i].nidle; k++) drop[nd++] = g_cache[i].idle[k];
     g_cache[i].nidle = 0;
   }
@@ -287,7 +292,7 @@ libECPHandle *libECP_init(int nrAtoms, double *geometry, int *shellsECP, int *lE
   const double t0 = now_ms();
   int failed = 0;
   if (!shellOrdering)
-    h->slot = cache_tables(maxL, d.maxLBS + n, largeGridOrder, tolerance, accuracy, err, sizeof(err), &failed);
+    h->slot = cache_tables(0, maxL, d.maxLBS + n, largeGridOrder, tolerance, accuracy, err, sizeof(err), &failed);
   if (h->slot) {
     h->st = &h->slot->st;
   } else if (failed || ecp_static_init(&h->st_own, maxL, d.maxLBS + n, shellOrdering, lmax, largeGridOrder,
@@ -624,7 +629,7 @@ libecp_batch *libecp_batch_create_n(const libecp_molecule *mols, int nmol, int n
     if (d.maxLBS > maxLBS) maxLBS = d.maxLBS;
   }
   int failed = 0;
-  b->slot = cache_tables(maxL, maxLBS + n, largeGridOrder, tolerance, accuracy, err, sizeof(err), &failed);
+  b->slot = cache_tables(1, maxL, maxLBS + n, largeGridOrder, tolerance, accuracy, err, sizeof(err), &failed);
   b->st = b->slot ? &b->slot->st : &b->st_own;
   if (failed ||
       (!b->slot && ecp_static_init(&b->st_own, maxL, maxLBS + n, NULL, -1, largeGridOrder, tolerance, accuracy, err,

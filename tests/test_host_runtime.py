@@ -159,6 +159,26 @@ def idle_contexts_of_batches_stay_below_4_gib():
     assert count("device_bytes") < 4 << 30
 
 
+@scenario
+def batches_take_no_cache_keys_from_handles():
+    m = plain_small(0)
+    for k in range(9):
+        native.Batch([m], tol=1e-12 * (1 + k)).close()
+
+    def handle(tol):
+        h = native.Handle(m, tol=tol)
+        h.contract(np.eye(m.nao))
+        h.close()
+
+    keys = [1e-11 * (2 + k) for k in range(8)]
+    for tol in keys:
+        handle(tol)
+    n = count("contexts")
+    for tol in keys:
+        handle(tol)
+    assert count("contexts") == n
+
+
 @pytest.fixture(scope="module")
 def runtime(tmp_path_factory):
     d = tmp_path_factory.mktemp("runtime")
