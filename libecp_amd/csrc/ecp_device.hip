@@ -44,6 +44,7 @@
 #include <mutex>
 #include <vector>
 
+#include "../../include/libecp_ext.h"
 #include "ecp_host.h"
 
 #define ECP_CHECK(call)                                                            \
@@ -68,6 +69,17 @@ namespace {
 constexpr int kScratchDevices = 64;
 std::mutex g_scratch_mu;
 void *g_scratch_ptr[kScratchDevices];
+
+// An allocation; where memory has run out, once more after the idle contexts of
+// the process cache have given theirs back.
+template <typename Alloc>
+hipError_t alloc_or_trim(Alloc alloc) {
+  const hipError_t e = alloc();
+  if (e != hipErrorOutOfMemory) return e;
+  (void)hipGetLastError();
+  libecp_cache_clear();
+  return alloc();
+}
 
 // The scratch address on the current device, looked up once per device.
 // 0, or -1 (message in err).
@@ -2794,7 +2806,8 @@ extern "C" ecp_dev *ecp_dev_create(const ecp_static *st, char *err, size_t errle
   put(o_dfac, st->dfac, nfac * 8);
   put(o_tmpl, d->tmpl.data(), d->tmpl.size() * 4);
   put(o_toff, d->toff.data(), d->toff.size() * 4);
-  if ((e = hipMalloc(&d->static_mem, off)) != hipSuccess) return fail("hipMalloc(static tables)", e);
+  if ((e = alloc_or_trim([&] { return hipMalloc(&d->static_mem, off); })) != hipSuccess)
+    return fail("hipMalloc(static tables)", e);
   if ((e = hipMemcpy(d->static_mem, h.data(), off, hipMemcpyHostToDevice)) != hipSuccess)
     return fail("hipMemcpy(static tables)", e);
   char *b = (char *)d->static_mem;
@@ -3383,7 +3396,7 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
     if (d->pin_in) ECP_CHECK(hipHostFree(d->pin_in));
     d->pin_in = nullptr;
     d->pin_in_cap = 0;
-    ECP_CHECK(hipHostMalloc(&d->pin_in, Ly.in_bytes + Ly.in_bytes / 4));
+    ECP_CHECK(alloc_or_trim([&] { return hipHostMalloc(&d->pin_in, Ly.in_bytes + Ly.in_bytes / 4); }));
     d->pin_in_cap = Ly.in_bytes + Ly.in_bytes / 4;
   }
   // the inputs, straight into the staging memory
@@ -3544,7 +3557,7 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
     if (d->pin_out) ECP_CHECK(hipHostFree(d->pin_out));
     d->pin_out = nullptr;
     d->pin_out_cap = 0;
-    ECP_CHECK(hipHostMalloc(&d->pin_out, out_bytes + out_bytes / 4));
+    ECP_CHECK(alloc_or_trim([&] { return hipHostMalloc(&d->pin_out, out_bytes + out_bytes / 4); }));
     d->pin_out_cap = out_bytes + out_bytes / 4;
   }
   if (bytes) *bytes = Ly.total;
@@ -3575,7 +3588,7 @@ extern "C" int ecp_dev_bind(ecp_dev *d, void *mem, size_t cap, char *err, size_t
       d->arena = nullptr;
       d->arena_cap = 0;
       const size_t c2 = Ly.total + Ly.total / 4;
-      ECP_CHECK(hipMalloc(&d->arena, c2));
+      ECP_CHECK(alloc_or_trim([&] { return hipMalloc(&d->arena, c2); }));
       d->arena_cap = c2;
     }
     A = d->arena;
@@ -4123,7 +4136,7 @@ extern "C" int ecp_dev_contract(ecp_dev *d, const ecp_job *job, const double *P,
     if (d->con_mem) ECP_CHECK(hipFree(d->con_mem));
     d->con_mem = nullptr;
     d->con_cap = 0;
-    ECP_CHECK(hipMalloc(&d->con_mem, o));
+    ECP_CHECK(alloc_or_trim([&] { return hipMalloc(&d->con_mem, o); }));
     d->con_cap = o;
     d->con_idx.clear();
   }
@@ -4233,7 +4246,7 @@ extern "C" int ecp_dev_span_ms(ecp_dev *d, double *ms, int *samples, char *err, 
 
 extern "C" int ecp_dev_mem_alloc(void **p, size_t bytes, char *err, size_t errlen) {
   *p = nullptr;
-  ECP_CHECK(hipMalloc(p, bytes));
+  ECP_CHECK(alloc_or_trim([&] { return hipMalloc(p, bytes); }));
   return 0;
 }
 

@@ -179,6 +179,24 @@ def batches_take_no_cache_keys_from_handles():
     assert count("contexts") == n
 
 
+@scenario
+def idle_contexts_give_way_when_memory_runs_out():
+    """To a batch and to a server whose memory would have been there without
+    them."""
+    mols = uneven_batch(0)[:12]
+    b = native.Batch(mols)
+    size = count("device_bytes")
+    b.close()
+    make("mem_limit", size + (1 << 20))
+    b = native.Batch(mols, tol=1e-11)       # another key: a new context
+    b.close()
+    s = native.Server(slots=1, hbm_budget=size - (32 << 20))
+    s.close()
+    make("mem_limit", size // 4)
+    assert fails(native.Batch, mols)
+    make("mem_limit", 0)
+
+
 @pytest.fixture(scope="module")
 def runtime(tmp_path_factory):
     d = tmp_path_factory.mktemp("runtime")
