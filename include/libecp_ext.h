@@ -41,8 +41,9 @@ double libecp_model_fallback_flops(int type, int la, int lb, int l, int ng_l, in
 /* Phases of the last getIntegrals or calculateECPIntegrals call made by the
    calling thread, in ms, up to n of: host tables (libECP_init; ~0 when they
    come from the process cache), screening (triplet list), device context
-   (created, or taken from the cache), plan + upload, kernels, download,
-   matrix accumulation or callbacks.  Returns the number of phases (7). */
+   (created, or taken from the cache), plan (work lists and staging; the upload
+   is queued), upload and kernels, download, matrix accumulation or callbacks.
+   Returns the number of phases (7). */
 int libecp_last_call_ms(double *ms, int n);
 
 /* Process-wide cache.  Handles with the default Cartesian ordering, and
@@ -146,7 +147,9 @@ int libecp_batch_stage_ms(libecp_batch *b, double *ms, int n);
    stream).  For up to n kernel families (names: libecp_kernel_family(i)):
    number of launches, summed duration (ms), algorithmic FLOPs of one
    evaluation under the reference algorithm's per-unit models (0 where no
-   model is defined).  Returns the number of families, or -1. */
+   model is defined).  The type-1 large grid ("fallback1") is evaluated by the
+   launches of "type1_tail": its FLOPs stand under its own name, its time under
+   theirs.  Returns the number of families, or -1. */
 int libecp_batch_profile(libecp_batch *b, int *launches, double *ms, double *flops, int n);
 const char *libecp_kernel_family(int i);
 /* Device time (ms) of the type-1 small-grid quadrature -- the head and tail

@@ -24,8 +24,8 @@ const char *libecp_last_error(void) { return g_err; }
 void ecp_api_set_error(const char *msg) { set_last_error(msg); }
 
 /* Phases of the last getIntegrals / calculateECPIntegrals call on this
-   thread (ms): host tables, screening, device context, plan + upload,
-   kernels, download, matrix / callbacks. */
+   thread (ms): host tables, screening, device context, plan (the upload is
+   queued), upload + kernels, download, matrix / callbacks. */
 enum { PH_TABLES = 0, PH_SCREEN, PH_CONTEXT, PH_UPLOAD, PH_KERNELS, PH_DOWNLOAD, PH_DELIVER, PH_N };
 static __thread double g_phase[PH_N];
 

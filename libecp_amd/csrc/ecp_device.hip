@@ -148,12 +148,12 @@ __device__ __forceinline__ V cload(const V *q) {
   return CPtr<V>::at(q);
 }
 
+constexpr int kSphDim = 16;  // more than any l of the harmonics
+
 // A point pair of the PS93 sequence, in visit order: its points, their
 // weights, and the level it is the last pair of (0: none).  A level's last
 // pair is its closest to the centre, so the level has a point in a window
 // where this pair does.
-constexpr int kSphDim = 16;  // more than any l of the harmonics
-
 struct Ps93Pair {
   double wl, wr;
   int li, ri, ends, pad;
@@ -236,8 +236,8 @@ __device__ __forceinline__ bool ps93_level(int lv, bool any, double tol, double 
 }
 
 // Radial powers other than 0, 1, 2 (rare in ECPs) through a call: inlined,
-// pow's registers set the fallbacks' budget (the type-1 fallback 152
-// registers and three waves per SIMD, against 128 and four)
+// pow's registers set the budget of the kernel around it (a type-1 fallback
+// kernel of its own held 152 registers with it, 128 without)
 __device__ __attribute__((noinline)) double ecp_pow_general(double r, double n) { return pow(r, n); }
 
 __device__ __forceinline__ double ecp_pow(double r, double n) {
@@ -927,63 +927,63 @@ __device__ __forceinline__ void fb1_unit(const DevTables &T, const DevJob &J, co
   bool open = lane < NQ && ((mask >> lane) & 1ull);
   Psm92 S{0.0, 0.0, 0.0};
   double res = 0.0;
-      // rounds of point pairs [c0, c1): levels 0 to 5 first, then 32 pairs of
-      // level lv at a time
-      int lv = psm92_first(T), c0 = 0, c1 = T.s92.lvl_begin[lv];
-      for (;;) {
-        const bool first = c0 == 0;
-        const unsigned long long om = __ballot(open);
-        const int n = psm92_point(T, c0, c1, lane, first);
-        double w = 0.0, uu = 0.0, g = 0.0, r = 0.0;
-        double K[LAB + 1];
-  #pragma unroll
-        for (int l = 0; l <= LAB; l++) K[l] = 0.0;
-        if (n >= 0) {
-          r = M.i1 * T.xl[n] + M.i2;
-          const double expo = expo_of(r);
-          if (expo >= minExp) {
-            g = exp(expo);
-            bessel_k<LAB>(T.bessel, G.s * r, K);
-            uu = eval_ecp(J, tr.centre, L, r);
-            w = T.wl[n] * M.i1;
-          }
-        }
-        // the open entries' pair sums
-        double rn = 1.0;
-        int e = 0;
-  #pragma unroll
-        for (int l1 = 0; l1 <= LAB; l1++) {
-          const double a = (Cc * rn) * uu;
-  #pragma unroll
-          for (int l2 = l1; l2 >= 0; l2 -= 2, e++)
-            if ((om >> e) & 1ull) {
-              const double t = pair_sum(w * ((a * K[l2]) * g));
-              if (!(lane & 1)) s_t[e * kFbTS + (lane >> 1)] = t;
-            }
-          rn = r * rn;
-        }
-        __syncthreads();
-        const bool level_end = !first && c1 == T.s92.lvl_begin[lv + 1];
-        if (open) {
-          bool done;
-          if (first) {
-            done = S.first_round(T, s_t + lane * kFbTS, &res);
-          } else {
-            S.I = sum_in_order(S.I, s_t + lane * kFbTS, c1 - c0);
-            done = level_end && S.test(T, lv, &res);
-          }
-          if (done) {
-            out[lane] = res;
-            open = false;
-          }
-        }
-        __syncthreads();
-        lv += level_end;
-        if (lv >= T.s92.nlevels || !wave_any(open)) break;
-        if (first || level_end) S.step();
-        c0 = c1;
-        c1 = min(c0 + 32, T.s92.lvl_begin[lv + 1]);
+  // rounds of point pairs [c0, c1): levels 0 to 5 first, then 32 pairs of
+  // level lv at a time
+  int lv = psm92_first(T), c0 = 0, c1 = T.s92.lvl_begin[lv];
+  for (;;) {
+    const bool first = c0 == 0;
+    const unsigned long long om = __ballot(open);
+    const int n = psm92_point(T, c0, c1, lane, first);
+    double w = 0.0, uu = 0.0, g = 0.0, r = 0.0;
+    double K[LAB + 1];
+#pragma unroll
+    for (int l = 0; l <= LAB; l++) K[l] = 0.0;
+    if (n >= 0) {
+      r = M.i1 * T.xl[n] + M.i2;
+      const double expo = expo_of(r);
+      if (expo >= minExp) {
+        g = exp(expo);
+        bessel_k<LAB>(T.bessel, G.s * r, K);
+        uu = eval_ecp(J, tr.centre, L, r);
+        w = T.wl[n] * M.i1;
       }
+    }
+    // the open entries' pair sums
+    double rn = 1.0;
+    int e = 0;
+#pragma unroll
+    for (int l1 = 0; l1 <= LAB; l1++) {
+      const double a = (Cc * rn) * uu;
+#pragma unroll
+      for (int l2 = l1; l2 >= 0; l2 -= 2, e++)
+        if ((om >> e) & 1ull) {
+          const double t = pair_sum(w * ((a * K[l2]) * g));
+          if (!(lane & 1)) s_t[e * kFbTS + (lane >> 1)] = t;
+        }
+      rn = r * rn;
+    }
+    __syncthreads();
+    const bool level_end = !first && c1 == T.s92.lvl_begin[lv + 1];
+    if (open) {
+      bool done;
+      if (first) {
+        done = S.first_round(T, s_t + lane * kFbTS, &res);
+      } else {
+        S.I = sum_in_order(S.I, s_t + lane * kFbTS, c1 - c0);
+        done = level_end && S.test(T, lv, &res);
+      }
+      if (done) {
+        out[lane] = res;
+        open = false;
+      }
+    }
+    __syncthreads();
+    lv += level_end;
+    if (lv >= T.s92.nlevels || !wave_any(open)) break;
+    if (first || level_end) S.step();
+    c0 = c1;
+    c1 = min(c0 + 32, T.s92.lvl_begin[lv + 1]);
+  }
   if (open) status[2 * U.trip] = 1;
 }
 
@@ -1160,7 +1160,7 @@ __global__ __launch_bounds__(64) void k_t1tail(DevTables T, DevJob J, const T1Un
 }
 
 // ---------------------------------------------------------------------------
-// type 2: one lane per T entry
+// type 2: the small grid, a lane group per triplet; then the large grid
 
 // first entry of channel l in the T entries of shells la, lb
 __device__ __forceinline__ int t2_off(const DevTables &T, int la, int lb, int l) {
@@ -2073,13 +2073,6 @@ __device__ __forceinline__ double asm1_monomial(double acc, int deg, int lab, co
   return acc;
 }
 
-// Type-1 block of one triplet per wave (the triplets tlist[0 .. ntl), in
-// class order lambda = la + lb).  chi[i][j] depends on (i, j) only
-// through the monomial p = i + j, so H[p] = sum_pairs sum_l F_pair[p][l]
-// Q[deg p][l] with F_pair[p][l] = sum_m S_lm(k^_pair) poly2sph[p][lm] is
-// formed once per monomial (same terms, same order as type1.c:266-295 per
-// element), then shifted to the output block (util.c:246-334).
-// G > 1 (classes la + lb <= 2, where a triplet has at most 10 monomials):
 // The block of a triplet whose integration failed: zeros, whatever an earlier
 // job left in the memory (a contraction sums every block and reports the
 // failure beside its result).
@@ -2089,13 +2082,20 @@ __device__ __forceinline__ void zero_block(const DevJob &J, int t, double *blk, 
   for (int i = lid; i < n; i += nlanes) blk[i] = 0.0;
 }
 
+// Type-1 block of one triplet per wave (the triplets tlist[0 .. ntl), in
+// class order lambda = la + lb).  chi[i][j] depends on (i, j) only
+// through the monomial p = i + j, so H[p] = sum_pairs sum_l F_pair[p][l]
+// Q[deg p][l] with F_pair[p][l] = sum_m S_lm(k^_pair) poly2sph[p][lm] is
+// formed once per monomial (same terms, same order as type1.c:266-295 per
+// element), then shifted to the output block (util.c:246-334).
+// G > 1 (classes la + lb <= 2, where a triplet has at most 10 monomials):
 // G triplets per wave, kAsmThreads / G lanes and an LDS slice of
 // A.lds_group doubles each; the wave's lane groups run the same phases and
 // synchronise together, an inactive group with empty loops.
 // MAXD: the largest monomial degree whose poly2sph row goes to registers
 // (the triplets' la + lb when a launch covers one class); higher degrees
-// take the general loop.  Registers, without spills: 51 (rows up to degree
-// 2 in registers) to 111 (degree 6), 94 for the packed variant; the pair
+// take the general loop.  Registers, without spills: 64 (rows up to degree
+// 3 in registers) to 98 (degree 6), 92 for the packed variant; the pair
 // directions come from the tables kernel, so no trigonometric code sits
 // here.
 template <int G = 1, int MAXD = 6>
@@ -2398,7 +2398,7 @@ struct TabArgs {
 // 211-302 via util.c:74-106), stored as cos theta, phi, sin phi, cos phi,
 // the values spherical_harmonics.c:15-114 forms from it.  Formed with the
 // tables, so that the type-1 assembly carries no trigonometric code (with
-// it, 168 registers and spills instead of 111).
+// it, it held 168 registers and spilled; 111 when it was taken out).
 __device__ void unit_dir(const DevJob &J, const T1Unit &U, double *out) {
   const ecp_triplet tr = J.trip[U.trip];
   const ecp_centre Cn = J.cent[tr.centre];
@@ -3030,12 +3030,12 @@ ClassMap class_map(int ncls, const int *count, F blocks) {
 }
 
 // the type-2 fallback classes of cm in one grid; like the type-1 kernels,
-// three tiers bound the Bessel orders the grid holds: up to 7, 11 and 12
+// four tiers bound the Bessel orders the grid holds: up to 7, 8, 11 and 12
 void launch_fb2_fused(ecp_dev *d, hipStream_t s, const T2Set &S2, const ClassMap &cm) {
   const Prepared &P = d->P;
   const int nb = cm.bbeg[cm.n];
   // 13.1 KB for projectors up to f and class 6: twelve waves per CU, what
-  // the registers (168) allow
+  // the registers (148) allow
   const size_t lds = sizeof(double) * (kFb2Chunk * kFbTS + (S2.cu_rows + S2.rn_rows + 2 * S2.k_rows) * 64);
   if (P.max_cls2 > 11) k_fb2_fused<12><<<nb, 64, lds, s>>>(d->T, P.J, S2, cm);
   // (class 8, g shells under L = 5, without class 11's scratch: 20 atoms
@@ -3074,12 +3074,6 @@ ClassMap fb2_classes(const ecp_dev *d, const T2Set &S) {
   });
 }
 
-// The kernel sequence of one evaluation, on resident inputs, one launch per
-// class: tables on the main stream, then the type-2 chain and the type-1
-// classes, each class as small grid -> large-grid fallback -> assembly, on
-// forked streams (two layouts, see enqueue).  With evs, stage boundaries are
-// recorded on the main stream: start, tables done, end, end (assembly
-// overlaps the quadratures).
 void enqueue_fused(ecp_dev *d, hipStream_t s, hipEvent_t *evs);
 
 // parts of the tables launch: what type 1 needs (with the zero-fill), and
@@ -3165,6 +3159,12 @@ void enqueue_t1_class(ecp_dev *d, hipStream_t ws, int c) {
   }
 }
 
+// The kernel sequence of one evaluation, on resident inputs: fused launches
+// (enqueue_fused), or tables on the main stream, then there the type-2 chain
+// and beside it, on the workers, the type-1 classes, each as head -> tail and
+// large-grid fallback -> assembly.  With evs, stage boundaries are recorded on
+// the main stream: start, tables done, end, end (assembly overlaps the
+// quadratures).
 void enqueue(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
   const int units = d->P.cls_begin[ECP_MAX_LAB + 1];
   const bool fused = d->tune.fuse == 1 || (d->tune.fuse == 2 && fuse_auto(units, d->P.max_lab));
@@ -3221,7 +3221,6 @@ void enqueue(ecp_dev *d, hipStream_t s, hipEvent_t *evs) {
     seq(d, hipEventRecord(evs[3], s));
   }
 }
-
 
 // Event i of the quadrature's pair, on stream s.  Under capture an event
 // record node of the graph, so that replays record it too: added to the graph
@@ -3566,7 +3565,8 @@ extern "C" int ecp_dev_plan(ecp_dev *d, const ecp_job *job, size_t *bytes, char 
 }
 
 // Device half: places the planned job at `mem` (capacity cap; NULL = the
-// context's own grow-only arena), uploads the staged inputs and waits.
+// context's own grow-only arena) and queues the upload of the staged inputs;
+// nothing waits for it here.
 extern "C" int ecp_dev_bind(ecp_dev *d, void *mem, size_t cap, char *err, size_t errlen) {
   if (!d->planned) {
     snprintf(err, errlen, "ecp_dev_bind before ecp_dev_plan");
@@ -3631,8 +3631,8 @@ extern "C" int ecp_dev_bind(ecp_dev *d, void *mem, size_t cap, char *err, size_t
   P.qf = (unsigned long long *)(A + Ly.d_qf);
   P.udir = (double *)(A + Ly.d_udir);
   P.fbq1 = (int *)(A + Ly.d_fbq1);
-  P.fbc = (int *)(A + Ly.d_fbc);  // [0..12] type-1 fallback queues, [32..44] type-1 tails, [48] type-2
-                                  // tail, [kFb2Cnt + 0..12] type-2 fallback queues
+  P.fbc = (int *)(A + Ly.d_fbc);  // [0..12] type-1 fallback queues, [32..44] type-1 tails,
+                                  // [kFb2Cnt + 0..12] type-2 fallback queues
   P.stat = (unsigned char *)(A + Ly.d_stat);
   P.Tout = (double *)(A + Ly.d_T);
   P.tf = (unsigned char *)(A + Ly.d_tf);
@@ -3749,8 +3749,6 @@ extern "C" int ecp_dev_execute(ecp_dev *d, int repeats, double *ms_total, char *
   return 0;
 }
 
-// One eager evaluation with an event pair around every kernel launch on its
-// own stream; per family: launches, summed duration (ms), algorithmic FLOPs.
 namespace {
 // Algorithmic FLOPs of the large-grid fallbacks of the last evaluation
 // (ecp_fb1_flops per failed primitive pair, ecp_fb2_flops per primitive pair of
@@ -3792,6 +3790,10 @@ __global__ __launch_bounds__(256) void k_fb_flops(DevJob J, const T1Unit *__rest
 
 }  // namespace
 
+// One eager evaluation with an event pair around every kernel launch on its
+// own stream; per family: launches, summed duration (ms), algorithmic FLOPs.
+// The type-1 large grid runs in the tail's launches: its FLOPs are under
+// FAM_FB1, its time is in FAM_T1TAIL's.
 extern "C" int ecp_dev_profile(ecp_dev *d, const ecp_job *job, int *launches, double *ms, double *flops, char *err,
                                size_t errlen) {
   if (!d->prepared) {
