@@ -413,7 +413,8 @@ def leg_main(args):
         fam[k] = e
     out["kernels"] = fam
     out["kernels_note"] = ("eager evaluation, HIP events per launch on its stream; families overlap on the "
-                           "device, so their times do not add up to the step")
+                           "device, so their times do not add up to the step; the type-1 large grid runs in the "
+                           "type1_tail launches: its FLOPs are under fallback1, its time under type1_tail")
     out["stage_ms_first_step"] = dict(zip(["tables", "quadratures", "assembly"], stages[:3]))
     # Roofline of the type-1 small-grid quadrature, the largest algorithmic
     # cost: G (31 lambda + 74 + 4 n_Q) + 150 n_Q per primitive pair, over the

@@ -3112,12 +3112,14 @@ void launch_tables(ecp_dev *d, hipStream_t s, int parts) {
 }
 
 // fuse = 2 (automatic), by the job's type-1 primitive pairs.  Up to
-// kFuseAutoSmall fused launches: per-class ones hold few waves each (10 503
-// pairs: 180 against 262 us an evaluation).  Up to kFuseAutoLarge per class,
-// each class with its own registers (235 440 pairs: 691 against 720 us;
-// 445 424 pairs of classes up to 8: 3864 against 4057 us).  Above, fused
-// again where the largest class is 6: every stage fills the chip by itself
-// (1 273 608 pairs: 3045 against 3302 us; 6.2 million: 14.44 against 14.82 ms).
+// kFuseAutoSmall fused launches: per-class ones hold few waves each.  Up to
+// kFuseAutoLarge per class, each class with its own registers.  Above, fused
+// again where the largest class is 6: every stage fills the chip by itself.
+// Replays, us, fused / per class: 8001 pairs 135 / 214, 119 934 348 / 361,
+// 149 436 443 / 433, 196 659 567 / 556, 290 133 687 / 662, 328 707 865 / 888,
+// 548 541 1146 / 1244, 852 570 1834 / 2003; classes up to 8: 459 360 4823 /
+// 4571, 880 656 7228 / 7503.  So the lower edge is at the crossing; the upper
+// one is above it, and the class limit holds back jobs of classes up to 8.
 constexpr int kFuseAutoSmall = 150000, kFuseAutoLarge = 800000;
 
 bool fuse_auto(int units, int max_lab) {
